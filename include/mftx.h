@@ -15,8 +15,10 @@
  *     asynchronously; the library allocates only context- or plan-owned
  *     workspace, never a caller buffer;
  *   - dtype codes: 0 complex64, 1 float32, 2 complex128, 3 float64;
- *   - precision codes: 0 FP32 (complex64 operands, FP32 MFMA),
- *     1 BF16X3 (split hi/lo BF16 operands, three MFMA passes, FP32 accumulate).
+ *   - precision codes: 0 FP32 (operands as f16 pairs, 22 bits, scaled by a
+ *     power of two to f16's range; three MFMA passes, FP32 accumulate: errors
+ *     below those of FP32 MFMAs), 1 BF16X3 (operands as bf16 pairs, 16 bits,
+ *     three MFMA passes, FP32 accumulate).
  */
 #ifndef MFTX_H
 #define MFTX_H
@@ -83,10 +85,10 @@ int mftx_dft2(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, i
  * reference: this is for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Same arguments, results and errors as mftx_dft2, but the
- * packed operands live in a fixed array of MFTX_NOALLOC_SCRATCH_BYTES of
- * device memory that the library holds on every GPU it runs on until the
- * process ends (its address is looked up once per device, at mftx_create).
- * A transform whose operands need more than that (about a 1024^2 -> 2048^2
+ * packed operands live in a fixed array of device memory that the library
+ * holds on every GPU it runs on until the process ends (its address is looked
+ * up once per device, at mftx_create).  A transform whose operands, counted as
+ * complex64 with padded rows, need more than MFTX_NOALLOC_SCRATCH_BYTES (about a 1024^2 -> 2048^2
  * transform) fails with MFTX_EINVAL and a message giving both sizes.  Every
  * call on one GPU shares that GPU's array: calls that overlap on one GPU
  * (other host threads, or streams with no order between them) race on it;
@@ -329,10 +331,10 @@ typedef struct {
  * and allocates plan-owned workspace.  Tile pointers are kept and re-read on
  * every execute, so amp/opd contents may change between executes.
  * Schedule knobs (no reference counterpart; lentil_amd.PSFPlan can pick
- * them by timing candidates): lambda_group = wavelengths whose |E|^2 one
- * GEMM workgroup sums in registers (0 = 8); tile_n = C columns per GEMM
- * workgroup, 64 (16-wide K steps) or 128 (32-wide K steps; every tile's K is
- * padded to a multiple of 32) (0 = 128). */
+ * them by timing candidates): lambda_group = the most wavelengths whose |E|^2
+ * one GEMM workgroup sums in registers (0 = 8; fewer where that fills the chip
+ * better); tile_n = output slots (column pairs) per GEMM workgroup, 64 or 128,
+ * or 0 to choose per launch. */
 int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles,
                   const double* wavelengths, int32_t nwave,
                   const mftx_problem* problems, int32_t nprob,

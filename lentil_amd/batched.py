@@ -68,8 +68,8 @@ def _round_up(v, q):
 def contraction_cost(shapes, M, N):
     """Complex MACs the two GEMM stages execute for tiles of ``shapes``
     (m, n) summed coherently onto one M x N grid, their stage-2 K
-    concatenated, with the kernels' padding (tiled rows to 128, K to 32),
-    for the cheaper of the two contraction orders."""
+    concatenated, with rows padded to 128 and K to 32, for the cheaper of the
+    two contraction orders (pairing halves every term alike)."""
     row_first = (sum(_round_up(m, 128) * _round_up(n, 32) * N for m, n in shapes)
                  + _round_up(N, 128) * sum(_round_up(m, 32) for m, _ in shapes) * M)
     col_first = (sum(_round_up(n, 128) * _round_up(m, 32) * M for m, n in shapes)
@@ -285,9 +285,9 @@ class PSFPlan:
     Parameters mirror the reference loop: ``pupil`` is a lentil_amd
     ``Pupil`` (2-D mask: one tile; 3-D mask: one tile per segment), ``tilts``
     are Tilt/DispersiveTilt planes applied after the pupil.  ``precision`` is
-    'fp32' or 'bf16x3'; ``lambda_group`` wavelengths share one output tile
-    accumulation in registers; ``tile_n`` is the GEMM workgroup width (64 or
-    128 columns, 0 = library default); ``autotune`` times every
+    'fp32' or 'bf16x3'; at most ``lambda_group`` wavelengths share one output
+    tile accumulation in registers; ``tile_n`` is the GEMM workgroup width (64
+    or 128 slots, 0 = chosen per launch); ``autotune`` times every
     (lambda_group, tile_n) candidate on this device and keeps the fastest
     (remembered per problem shape for the process); ``use_graph`` replays the
     launches from a hipGraph after the first call.  ``copies`` > 1 makes that

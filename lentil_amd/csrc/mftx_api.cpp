@@ -33,7 +33,8 @@ using namespace mftx;
 namespace {
 
 constexpr int kRingSlots = 16;
-constexpr size_t kSlotBytes = 512 * 1024;  // up to ~13k work items per launch
+constexpr size_t kTableCap = 64u << 20;  // twiddle table bytes per stage of one mftx_dft2
+constexpr size_t kSlotBytes = 512 * 1024;
 
 int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 double centre(int64_t k) { return (double)(k / 2); }  // floor(k/2), k >= 0 (fourier.py:117-120)
@@ -42,38 +43,103 @@ double centre(int64_t k) { return (double)(k / 2); }  // floor(k/2), k >= 0 (fou
 double cost_row_first(double m, double n, double M, double N) { return m * n * N + M * m * N; }
 double cost_col_first(double m, double n, double M, double N) { return M * m * n + M * n * N; }
 
-Work empty_work() { return Work{0, 0, 0, 0, nullptr, 0, 0, 0}; }
+Work empty_work() { return Work{}; }
 
-// XCD-aware order: clusters of works that share A rows are assigned round-
-// robin to the 8 XCDs; workgroup i of a launch runs on XCD i % 8, so a
-// cluster's works land on one XCD and share its L2.
-std::vector<Work> xcd_order(const std::vector<std::vector<Work>>& clusters) {
-  std::vector<std::vector<Work>> bins(8);
-  for (size_t c = 0; c < clusters.size(); ++c) {
-    auto& b = bins[c % 8];
-    b.insert(b.end(), clusters[c].begin(), clusters[c].end());
-  }
-  size_t mx = 0;
-  for (auto& b : bins) mx = std::max(mx, b.size());
+// XCD-aware order: the works, listed so that neighbours share operand rows and
+// twiddle tables, are cut into 8 equal runs, one per XCD; workgroup i of a
+// launch runs on XCD i % 8, so each XCD walks its own run and its L2 serves
+// what neighbours share.
+std::vector<Work> xcd_order(const std::vector<Work>& works) {
+  const size_t n = works.size();
   std::vector<Work> out;
-  out.reserve(mx * 8);
-  for (size_t i = 0; i < mx; ++i)
-    for (int x = 0; x < 8; ++x) out.push_back(i < bins[x].size() ? bins[x][i] : empty_work());
+  size_t most = 0;
+  for (size_t x = 0; x < 8; ++x) most = std::max(most, (x + 1) * n / 8 - x * n / 8);
+  out.reserve(most * 8);
+  for (size_t i = 0; i < most; ++i)
+    for (size_t x = 0; x < 8; ++x) {
+      const size_t b = x * n / 8, e = (x + 1) * n / 8;
+      out.push_back(b + i < e ? works[b + i] : empty_work());
+    }
   while (!out.empty() && out.back().pend == 0) out.pop_back();
   return out;
 }
 
-// Works covering rows_tiled C rows x `slots` slots for problems [pb, pe) with
-// bn-column workgroups (bn / 2 slots each), one cluster per tile row.
-void add_tiles(std::vector<std::vector<Work>>& clusters, int pb, int pe, int64_t rows_tiled, int64_t slots, int bn,
+// Works covering rblocks x sblocks 32 x 32 blocks of C for problems [pb, pe)
+// (nch K blocks in all): panels of 8 tile columns, so that 32 neighbouring
+// works are 4 tile rows by 8 tile columns and read few distinct blocks.
+void add_tiles(std::vector<Work>& works, int tile, int pb, int pe, int nch, int rblocks, int sblocks,
                float* partial = nullptr, long long ldp = 0, int prows = 0, int pcols = 0) {
-  const int bs = slots_per_tile(bn);
-  const int tr = (int)(rows_tiled / BM), tc = (int)((slots + bs - 1) / bs);
-  for (int r = 0; r < tr; ++r) {
-    std::vector<Work> row;
-    for (int c = 0; c < tc; ++c) row.push_back(Work{pb, pe, r, c, partial, ldp, prows, pcols});
-    clusters.push_back(row);
+  const int tr = (rblocks + tile_rows(tile) - 1) / tile_rows(tile);
+  const int tc = (sblocks + tile_slots(tile) - 1) / tile_slots(tile);
+  for (int c0 = 0; c0 < tc; c0 += 8)
+    for (int r = 0; r < tr; ++r)
+      for (int c = c0; c < std::min(tc, c0 + 8); ++c)
+        works.push_back(Work{pb, pe, r, c, partial, ldp, prows, pcols, nch, 0});
+}
+
+int64_t blocks32(int64_t n) { return (n + 31) / 32; }
+
+constexpr int kCUs = 256;
+
+// Estimated time (us) of a launch whose work items each run `run` problems of
+// nkb K blocks on one tile of rblocks x sblocks blocks, `sets` such runs.
+// Fitted to kernel traces of single transforms (64^2 to 2048^2 -> 4096^2, every
+// tile forced) and of the broadband and segmented sweeps (every tile and run
+// length forced), within 20% of them; per K block a workgroup takes
+//   BIG    1.38 us, one per CU on a full chip (1.0 on up to half of the CUs),
+//   MID    0.95 us with two on the CU, 0.48 alone,
+//   SMALL  0.33 us with two on the CU, 0.27 alone (a wave runs a quarter),
+// and each problem adds its epilogue, each round of work items its start.
+double tile_cost(int tile, int64_t rblocks, int64_t sblocks, int64_t nkb, int64_t run, int64_t sets) {
+  struct Rate { double start, full, light, epilogue; };
+  const Rate r = tile == TILE_BIG ? Rate{6.0, 1.38, 1.0, 2.0}
+               : tile == TILE_SMALL ? Rate{1.0, 0.33, 0.27, 1.0} : Rate{1.5, 0.95, 0.48, 1.5};
+  const int64_t w = ((rblocks + tile_rows(tile) - 1) / tile_rows(tile)) *
+                    ((sblocks + tile_slots(tile) - 1) / tile_slots(tile)) * sets;
+  const int64_t per = tile == TILE_BIG ? kCUs : 2 * kCUs;
+  const int64_t rounds = w / per, rest = w % per;
+  const double full = r.start + run * (r.full * nkb + r.epilogue);
+  const double light = r.start + run * (r.light * nkb + r.epilogue);
+  return rounds * full + (rest == 0 ? 0.0 : 2 * rest > per ? full : light);
+}
+
+// Tile and run length (problems per work item, at most `most`) of a launch of
+// `count` problems of one shape that estimates fastest; a fixed tile is kept.
+// Ties go to the longer run (fewer partial images, a longer pipeline).
+struct Schedule {
+  int tile, run;
+};
+Schedule pick_schedule(int fixed, bool multi, int64_t rblocks, int64_t sblocks, int64_t nkb, int64_t count,
+                       int64_t most) {
+  Schedule best{TILE_MID, 1};
+  double cost = -1;
+  const int cand[3] = {TILE_BIG, multi ? TILE_MULTI : TILE_MID, TILE_SMALL};
+  for (int t : cand) {
+    if (multi && t == TILE_BIG) continue;
+    if (fixed >= 0 && t != fixed) continue;
+    for (int64_t g = std::min(most, count); g >= 1; --g) {
+      const double c = tile_cost(t, rblocks, sblocks, nkb, g, (count + g - 1) / g);
+      if (cost < 0 || c < 0.999 * cost) {
+        cost = c;
+        best = Schedule{t, (int)g};
+      }
+    }
   }
+  return best;
+}
+
+// Powers of two of the f16 form: the operand is scaled to at most 2^14 per
+// paired element (ScaleSrc), the tables by tw_scale, so stage 1's sums over K
+// pairs stay below K 2^14 tw_scale; stage 1 stores them times
+// 1 / (tw_scale 2^ceil(log2 K)), again at most 2^14, and stage 2 undoes all of it.
+double stage1_scale(int prec, int64_t k_pairs) {
+  if (prec != PREC_FP32) return 1.0;
+  int b = 0;
+  while ((1LL << b) < k_pairs) ++b;
+  return std::ldexp(1.0 / tw_scale(prec), -b);
+}
+double stage2_scale(int prec, int64_t k_pairs) {
+  return prec != PREC_FP32 ? 1.0 : 1.0 / (tw_scale(prec) * tw_scale(prec)) / stage1_scale(prec, k_pairs);
 }
 
 // Output grid of one MFT stage with N columns, signed twiddle scale alpha and
@@ -110,9 +176,48 @@ OutGrid make_grid(double alpha, double shift, int N) {
   return g;
 }
 
-void push_chunks(std::vector<double>& cx, int kpad, double x0) {
-  for (int c = 0; c < kpad / BK; ++c) cx.push_back(x0 + (double)(c * BK));
-}
+// Twiddle tables of a launch, shared by every problem with the same rate, slot
+// origin and sample parity (x' = k' + 1/2 for an even number of samples, k'
+// for an odd one).
+class Tables {
+ public:
+  // index of the table for `samples` input samples and `slots` output slots
+  int get(double alpha, double y0, int64_t samples, int64_t slots) {
+    const std::tuple<double, double, int> key{alpha, y0, (int)(samples & 1)};
+    auto it = index_.find(key);
+    if (it == index_.end()) {
+      it = index_.emplace(key, (int)ops.size()).first;
+      TableOp op = {};
+      op.alpha = alpha;
+      op.x0 = samples & 1 ? 0.0 : 0.5;
+      op.y0 = y0;
+      ops.push_back(op);
+    }
+    TableOp& op = ops[it->second];
+    op.nsb = std::max(op.nsb, (int)blocks32(slots));
+    op.nkb = std::max(op.nkb, pair_blocks(samples));
+    return it->second;
+  }
+  // thread ranges of the launch and offsets of the tables from `base`; the total bytes
+  size_t place(size_t base) {
+    off.clear();
+    threads = 0;
+    size_t at = base;
+    for (auto& op : ops) {
+      off.push_back(at);
+      at += table_bytes(op.nsb, op.nkb);
+      op.begin = group_begin(threads);
+      threads = op.begin + table_threads(op.nsb, op.nkb);
+    }
+    return at - base;
+  }
+  std::vector<TableOp> ops;
+  std::vector<size_t> off;
+  long long threads = 0;
+
+ private:
+  std::map<std::tuple<double, double, int>, int> index_;
+};
 
 }  // namespace
 
@@ -135,15 +240,18 @@ struct mftx_ctx {
 struct mftx_plan {
   mftx_ctx* ctx = nullptr;
   int prec = 0;
-  int bn = BN_DEFAULT;  // C columns per GEMM workgroup
+  int tile1 = 0, tile2 = 0, tile2c = 0, tile_f = 0;  // GEMM tiles of the launches below
   int64_t img_rows = 0, img_cols = 0;
   void* ws = nullptr;  // workspace: operands, intermediates, partial images, descriptors
   Work* works1 = nullptr;
   Work* works2 = nullptr;
   Problem* probs1 = nullptr;
   Problem* probs2 = nullptr;
-  double* chunk_x = nullptr;
-  PhasorWave* waves = nullptr;  // per phasor wavelength slot: 1/λ and the stage-1 fold
+  Seg* segs = nullptr;          // K segments of every problem list
+  PhasorWave* waves = nullptr;  // per phasor wavelength slot: 1/λ and both stages' folds
+  MaxOp* max_ops = nullptr;     // f16 form: the tiles' amplitude maxima
+  int n_max_ops = 0;
+  long long max_blocks = 0;
   int nwork1 = 0, nwork2 = 0;
   // stage 2 of the classes whose coherent group has several output grids:
   // their complex fields, summed by the fallbacks below (every other class
@@ -189,6 +297,9 @@ struct mftx_plan {
   Problem* probs_f = nullptr;
   int nwork_f = 0;
   std::vector<Problem> pf;       // host copy, pointers filled by set_fields
+  RowPhase* row_phases = nullptr;  // device: per class, the phase stage 1 left out
+  int max_rows = 0;                // the longest of them
+  std::vector<double> field_scale;  // what undoes the f16 form's scaling, per class
   std::vector<int> class_first;  // first member (problem index) of each class
   int fields_ready = 0;
 };
@@ -310,49 +421,18 @@ static int upload_desc(mftx_ctx* ctx, const void* src, size_t bytes, void** dev)
   return MFTX_OK;
 }
 
-// One GEMM launch of a single problem covering rows_tiled x p.cols of C with
-// bn-column workgroups (p.kpad a multiple of k_granule(bn)).
-static int run_single(mftx_ctx* ctx, int prec, int epi, int bn, Problem p, double x0, int64_t rows_tiled) {
-  std::vector<std::vector<Work>> clusters;
-  add_tiles(clusters, 0, 1, rows_tiled, p.cols, bn);
-  const std::vector<Work> works = xcd_order(clusters);
-  std::vector<double> cx;
-  push_chunks(cx, p.kpad, x0);
-  p.chunk_begin = 0;
-  const size_t off_cx = round_up(sizeof(Problem), 16);
-  const size_t off_w = round_up(off_cx + sizeof(double) * cx.size(), 16);
-  std::vector<char> host(off_w + sizeof(Work) * works.size());
-  std::memcpy(host.data(), &p, sizeof(Problem));
-  std::memcpy(host.data() + off_cx, cx.data(), sizeof(double) * cx.size());
-  std::memcpy(host.data() + off_w, works.data(), sizeof(Work) * works.size());
-  void* dev = nullptr;
-  int rc = upload_desc(ctx, host.data(), host.size(), &dev);
-  if (rc) return rc;
-  char* d = (char*)dev;
-  HIPCHK(ctx, launch_gemm(prec, epi, bn, (const Work*)(d + off_w), (int)works.size(), (const Problem*)d,
-                          (const double*)(d + off_cx), ctx->stream));
-  return MFTX_OK;
-}
-
 // Problem ranges [b, e) for work items: runs of g consecutive problems with
-// one tiling (rows tiled, output slots) and K length share a work item, so
-// the GEMM's staging pipeline runs across their K loops.  g is at most 8 and
-// keeps at least one work item per CU.  Grouping is used only when every run
-// has the same length g: a launch that mixed long and short work items would
-// finish on its long tail.
-static std::vector<std::pair<int, int>> group_runs(const std::vector<Problem>& ps, const std::vector<int64_t>& rows,
-                                                   int bn) {
+// one tiling and K length share a work item, so the GEMM's load pipeline runs
+// across their K loops.  Grouping is used only when every run has the same
+// length g: a launch that mixed long and short work items would finish on its
+// long tail.
+static std::vector<std::pair<int, int>> group_runs(const std::vector<Problem>& ps, const std::vector<int>& nkb, int g) {
   const int n = (int)ps.size();
-  int64_t single = 0;
-  for (int i = 0; i < n; ++i) single += (rows[i] / BM) * ((ps[i].cols + slots_per_tile(bn) - 1) / slots_per_tile(bn));
-  const int g = (int)std::max<int64_t>(1, std::min<int64_t>(8, single / 256));
   std::vector<std::pair<int, int>> runs;
   bool uniform = true;
   for (int i = 0; i < n;) {
     int e = i + 1;
-    while (e < n && e - i < g && rows[e] == rows[i] && ps[e].cols == ps[i].cols && ps[e].kpad == ps[i].kpad &&
-           ps[e].rows == ps[i].rows)
-      ++e;
+    while (e < n && e - i < g && ps[e].rblocks == ps[i].rblocks && ps[e].cols == ps[i].cols && nkb[e] == nkb[i]) ++e;
     uniform = uniform && e - i == g;
     runs.emplace_back(i, e);
     i = e;
@@ -364,218 +444,256 @@ static std::vector<std::pair<int, int>> group_runs(const std::vector<Problem>& p
   return runs;
 }
 
+// Schedule and works of a list of independent problems (one segment each,
+// nkb[i] K blocks): the tile is chosen for the whole launch by the summed
+// estimate of its shapes; runs of equal problems share work items.
+static int list_works(std::vector<Work>& works, const std::vector<Problem>& ps, const std::vector<int>& nkb, int fixed,
+                      int64_t most) {
+  struct Shape { int rb, sb, nkb; };
+  std::map<std::tuple<int, int, int>, int64_t> shapes;
+  for (size_t i = 0; i < ps.size(); ++i) ++shapes[{ps[i].rblocks, (int)blocks32(ps[i].cols), nkb[i]}];
+  // the shape with most work decides
+  std::tuple<int, int, int> top{};
+  double big = -1;
+  int64_t total = 0;
+  for (auto& kv : shapes) {
+    const double w = (double)std::get<0>(kv.first) * std::get<1>(kv.first) * std::get<2>(kv.first) * kv.second;
+    if (w > big) {
+      big = w;
+      top = kv.first;
+    }
+    total += kv.second;
+  }
+  const Schedule sch = pick_schedule(fixed, false, std::get<0>(top), std::get<1>(top), std::get<2>(top), total, most);
+  for (const auto& r : group_runs(ps, nkb, sch.run)) {
+    int nch = 0;
+    for (int i = r.first; i < r.second; ++i) nch += nkb[i];
+    add_tiles(works, sch.tile, r.first, r.second, nch, ps[r.first].rblocks, (int)blocks32(ps[r.first].cols));
+  }
+  return sch.tile;
+}
+
 // Geometry of one entry of mftx_dft2_many (the quantities mftx_dft2 derives).
 namespace {
-struct ManyGeo {
+struct MftGeo {
   bool col_first;
-  int64_t r1, c1, rows1, rows2;
+  int64_t r1, k1, c1, c2;  // stage-1 operand rows and K, stage-1 and stage-2 output columns
   double alpha1, alpha2, x01, x02;
   OutGrid g1, g2;
-  int kpad1, kpad2;
-  size_t off1, off2;  // workspace offsets of the packed stage-1 and stage-2 operands
+  double xc1() const { return x01 + 0.5 * (double)(k1 - 1); }  // midpoints of the two input axes
+  double xc2() const { return x02 + 0.5 * (double)(r1 - 1); }
+  size_t off1 = 0, off2 = 0;  // workspace offsets of the stage-1 and stage-2 operands
+  size_t off_max = 0;         // ... of the source's maxima, then its inverse scale (f16 form)
 };
+
+MftGeo mft_geometry(int64_t m, int64_t n, int64_t M, int64_t N, double alpha_r, double alpha_c, double shift_r,
+                    double shift_c, double offset_r, double offset_c, int conj) {
+  MftGeo g;
+  g.col_first = cost_col_first(m, n, M, N) < cost_row_first(m, n, M, N);
+  g.r1 = g.col_first ? n : m;
+  g.k1 = g.col_first ? m : n;
+  g.c1 = g.col_first ? M : N;
+  g.c2 = g.col_first ? N : M;
+  const double sgn = conj ? 1.0 : -1.0;
+  g.alpha1 = sgn * (g.col_first ? alpha_r : alpha_c);
+  g.alpha2 = sgn * (g.col_first ? alpha_c : alpha_r);
+  g.g1 = make_grid(g.alpha1, g.col_first ? shift_r : shift_c, (int)g.c1);
+  g.g2 = make_grid(g.alpha2, g.col_first ? shift_c : shift_r, (int)g.c2);
+  // twiddle coordinates: rows x = R + or against U - sr; columns x = S + oc
+  // against V - sc; each stage's output shift is folded into its A operand
+  const double xr0 = -centre(m) + offset_r, xc0 = -centre(n) + offset_c;
+  g.x01 = g.col_first ? xr0 : xc0;
+  g.x02 = g.col_first ? xc0 : xr0;
+  return g;
+}
+
+// The two GEMM problems of one transform (addresses filled by the caller).
+void mft_problems(const MftGeo& g, int prec, double scale, Problem& a, Problem& b) {
+  a = Problem{};
+  a.rblocks = pair_blocks(g.r1);
+  a.sblocks = (int)blocks32(g.g1.slots);
+  a.rows = 32 * a.rblocks;
+  a.cols = g.g1.slots;
+  a.ncols = (int)g.c1;
+  a.cp = g.g1.cp;
+  a.cm = g.g1.cm;
+  a.y0 = g.g1.y0;
+  a.xrot = g.alpha1 * g.xc1();
+  a.scale = (float)stage1_scale(prec, pairs(g.k1));
+  a.ldd = pair_blocks(g.r1);
+  b = Problem{};
+  b.rblocks = (int)blocks32(g.c1);
+  b.sblocks = (int)blocks32(g.g2.slots);
+  b.rows = (int)g.c1;
+  b.cols = g.g2.slots;
+  b.ncols = (int)g.c2;
+  b.cp = g.g2.cp;
+  b.cm = g.g2.cm;
+  b.y0 = g.g2.y0;
+  b.xrot = g.alpha2 * g.xc2();
+  b.scale = (float)(scale * stage2_scale(prec, pairs(g.k1)));
+  b.trans = g.col_first ? 0 : 1;  // C is F (column-first) or F^T (row-first)
+}
+
+// A transform whose output takes more tiles of 128 rows by 64 or 128 columns
+// than one descriptor block of kSlotBytes once held (40 bytes each behind 112
+// bytes and 8 per 16 K values) is refused, as it always was.
+bool too_large(const MftGeo& g) {
+  auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
+  const int64_t t1 = up(g.r1, BK * 8) / 128, t2 = up(g.c1, 128) / 128;
+  const int64_t wide = std::max(t1 * ((g.g1.slots + 63) / 64), t2 * ((g.g2.slots + 63) / 64));
+  const int64_t bs = wide >= 256 ? 64 : 32, kg = wide >= 256 ? 32 : 16;
+  auto bytes = [&](int64_t tr, int64_t slots, int64_t k) {
+    const int64_t tc = (slots + bs - 1) / bs, mx = (tr + 7) / 8 * tc;
+    const int64_t works = (mx - 1) * 8 + (tr % 8 ? tr % 8 : 8);
+    return up(112 + up(k, kg) / 16 * 8, 16) + 40 * works;
+  };
+  return bytes(t1, g.g1.slots, g.k1) > (int64_t)kSlotBytes || bytes(t2, g.g2.slots, g.r1) > (int64_t)kSlotBytes;
+}
 }  // namespace
 
-// The launches of a list of MFTs: all entries in one pack launch per input
+// The launches of a list of MFTs: all entries in one operand launch per input
 // kind and one GEMM launch per stage.  many_build derives the geometry and the
 // descriptors (workspace and descriptor addresses as offsets); many_place
 // rebases them onto a workspace and a device descriptor block and writes the
-// host copy of that block; many_launch issues the launches.
+// host copy of that block; many_tables and many_launch issue the launches.
 struct ManyBatch {
-  int bn = 64;
+  int tile1 = 0, tile2 = 0;
   size_t ws = 0, bytes = 0;  // workspace and descriptor block sizes
-  size_t o_wv = 0, o_ph = 0, o_pk = 0, o_p1 = 0, o_p2 = 0, o_cx = 0, o_w1 = 0, o_w2 = 0;
-  std::vector<ManyGeo> geo;
+  size_t o_wv = 0, o_ph = 0, o_pk = 0, o_mx = 0, o_tb = 0, o_p1 = 0, o_p2 = 0, o_s1 = 0, o_s2 = 0, o_w1 = 0, o_w2 = 0;
+  std::vector<MftGeo> geo;
   std::vector<PhasorWave> waves;
-  std::vector<PhasorOp> phops;
-  std::vector<PackOp> packs;
-  std::vector<int> wave_of;  // phasor wave of entry i, or -(pack index + 1)
+  std::vector<PhasorOp> phops, packs;  // phasor and complex sources
+  std::vector<MaxOp> maxes;
+  std::vector<int> op_of;  // phasor op of entry i, or -(pack index + 1)
+  Tables tables;
+  std::vector<int> tab1, tab2;
   std::vector<Problem> p1, p2;
-  std::vector<double> cx;
+  std::vector<Seg> s1, s2;
   std::vector<Work> w1, w2;
-  long long ph_total = 0, pk_total = 0;
+  long long ph_total = 0, pk_total = 0, mx_total = 0;
 };
 
-static void many_build(const mftx_mft* mfts, int32_t count, int prec, ManyBatch& mb) {
-  std::vector<ManyGeo>& geo = mb.geo;
-  geo.assign(count, ManyGeo{});
-  int64_t wide1 = 0, wide2 = 0;
+// `fixed`: the GEMM tile, or -1 to choose it.
+static void many_build(const mftx_mft* mfts, int32_t count, int prec, int fixed, ManyBatch& mb) {
+  std::vector<MftGeo>& geo = mb.geo;
+  geo.clear();
+  size_t ws = 0;
   for (int32_t i = 0; i < count; ++i) {
     const mftx_mft& q = mfts[i];
-    ManyGeo& g = geo[i];
-    g.col_first = cost_col_first(q.m, q.n, q.M, q.N) < cost_row_first(q.m, q.n, q.M, q.N);
-    g.r1 = g.col_first ? q.n : q.m;
-    g.c1 = g.col_first ? q.M : q.N;
-    const int64_t c2 = g.col_first ? q.N : q.M;
-    g.rows1 = round_up(g.r1, BM);
-    g.rows2 = round_up(g.c1, BM);
-    const double sgn = q.conj ? 1.0 : -1.0;
-    g.alpha1 = sgn * (g.col_first ? q.alpha_r : q.alpha_c);
-    g.alpha2 = sgn * (g.col_first ? q.alpha_c : q.alpha_r);
-    g.g1 = make_grid(g.alpha1, g.col_first ? q.shift_r : q.shift_c, (int)g.c1);
-    g.g2 = make_grid(g.alpha2, g.col_first ? q.shift_c : q.shift_r, (int)c2);
-    const double xr0 = -centre(q.m) + q.offset_r, xc0 = -centre(q.n) + q.offset_c;
-    g.x01 = g.col_first ? xr0 : xc0;
-    g.x02 = g.col_first ? xc0 : xr0;
-    wide1 += (g.rows1 / BM) * ((g.g1.slots + 63) / 64);
-    wide2 += (g.rows2 / BM) * ((g.g2.slots + 63) / 64);
+    geo.push_back(mft_geometry(q.m, q.n, q.M, q.N, q.alpha_r, q.alpha_c, q.shift_r, q.shift_c, q.offset_r, q.offset_c,
+                               q.conj));
+    geo[i].off1 = ws;
+    ws += folded_bytes(geo[i].r1, geo[i].k1);
   }
-  // 128-column tiles when the larger stage still gives every CU a workgroup
-  const int bn = mb.bn = std::max(wide1, wide2) >= 256 ? 128 : 64;
-  const int kg = k_granule(bn);
-  size_t& ws = mb.ws;
-  ws = 0;
-  for (int32_t i = 0; i < count; ++i) {
-    const mftx_mft& q = mfts[i];
-    ManyGeo& g = geo[i];
-    g.kpad1 = (int)round_up(g.col_first ? q.m : q.n, kg);
-    g.kpad2 = (int)round_up(g.r1, kg);
-    g.off1 = ws;
-    ws += round_up((int64_t)packed_bytes(prec, g.rows1, g.kpad1), 256);
+  for (auto& g : geo) {
+    g.off2 = ws;
+    ws += plain_bytes(g.c1, pair_blocks(g.r1));
   }
-  for (int32_t i = 0; i < count; ++i) {
-    geo[i].off2 = ws;
-    ws += round_up((int64_t)packed_bytes(prec, geo[i].rows2, geo[i].kpad2), 256);
+  for (auto& g : geo) {
+    mb.tab1.push_back(mb.tables.get(g.alpha1, g.g1.y0, g.k1, g.g1.slots));
+    mb.tab2.push_back(mb.tables.get(g.alpha2, g.g2.y0, g.r1, g.g2.slots));
   }
+  ws += mb.tables.place(ws);
 
-  // ---- descriptors -------------------------------------------------------------
-  std::vector<PhasorWave>& waves = mb.waves;
-  std::vector<PhasorOp>& phops = mb.phops;
-  std::vector<PackOp>& packs = mb.packs;
-  long long& ph_total = mb.ph_total;
-  long long& pk_total = mb.pk_total;
-  std::vector<int>& wave_of = mb.wave_of;
+  // ---- sources -----------------------------------------------------------------
+  auto source = [&](std::vector<PhasorOp>& ops, long long& total, const MftGeo& g, const mftx_mft& q) -> PhasorOp& {
+    PhasorOp op = {};
+    op.m = (int)q.m;
+    op.n = (int)q.n;
+    op.trans = g.col_first ? 1 : 0;
+    op.waves = (const PhasorWave*)(uintptr_t)mb.waves.size();  // index, rebased by many_place
+    op.dst = (void*)(uintptr_t)g.off1;                          // offset, rebased by many_place
+    op.wave_stride = (long long)folded_bytes(g.r1, g.k1);
+    op.begin = group_begin(total);
+    ops.push_back(op);
+    return ops.back();
+  };
   for (int32_t i = 0; i < count; ++i) {
     const mftx_mft& q = mfts[i];
-    const ManyGeo& g = geo[i];
-    if (q.f) {
-      PackOp op = {};
-      op.src = q.f;
-      op.dtype = q.f_dtype;
-      op.trans = g.col_first ? 1 : 0;
-      op.m = q.m;
-      op.n = q.n;
-      op.lds = q.ldf;
-      op.fold = g.g1.fold;
-      op.x0 = g.x01;
-      op.fold2 = g.g2.fold;
-      op.x02 = g.x02;
-      op.dst = nullptr;  // rebased below
-      op.rows_pad = g.rows1;
-      op.kpad = g.kpad1;
-      op.begin = group_begin(pk_total);
-      pk_total = op.begin + g.rows1 * (g.kpad1 / 2);  // one thread per (row, pair of K values)
-      packs.push_back(op);
-      wave_of.push_back(-(int)packs.size());  // -(pack index + 1)
-      continue;
-    }
+    const MftGeo& g = geo[i];
     // consecutive phasor entries of one pupil and geometry share an op
     // (their operands are one fixed stride apart in the workspace)
-    const size_t stride = round_up((int64_t)packed_bytes(prec, g.rows1, g.kpad1), 256);
     bool joined = false;
-    if (i > 0 && !mfts[i - 1].f && !phops.empty()) {
+    if (!q.f && i > 0 && !mfts[i - 1].f) {
       const mftx_mft& p = mfts[i - 1];
-      const ManyGeo& h = geo[i - 1];
-      PhasorOp& last = phops.back();
+      const MftGeo& h = geo[i - 1];
       joined = p.amp == q.amp && p.opd == q.opd && p.amp_dtype == q.amp_dtype && p.opd_dtype == q.opd_dtype &&
-               p.ld_amp == q.ld_amp && p.ld_opd == q.ld_opd && p.m == q.m && p.n == q.n &&
-               h.col_first == g.col_first && h.kpad1 == g.kpad1 && h.rows1 == g.rows1 &&
-               (long long)stride == last.wave_stride;
+               p.ld_amp == q.ld_amp && p.ld_opd == q.ld_opd && p.m == q.m && p.n == q.n && h.col_first == g.col_first;
     }
     if (!joined) {
-      if (!phops.empty())
-        ph_total = phops.back().begin + phasor_threads(phops.back().rows_pad, phops.back().kpad, phops.back().nwave);
-      PhasorOp op = {};
-      op.amp = q.amp;
-      op.opd = q.opd;
-      op.amp_dtype = q.amp_dtype;
-      op.opd_dtype = q.opd_dtype;
-      op.ld_amp = q.ld_amp;
-      op.ld_opd = q.ld_opd;
-      op.m = (int)q.m;
-      op.n = (int)q.n;
-      op.trans = g.col_first ? 1 : 0;
-      op.nwave = 0;
-      op.waves = (const PhasorWave*)(uintptr_t)waves.size();  // index, rebased below
-      op.dst = (void*)(uintptr_t)g.off1;                       // offset, rebased below
-      op.wave_stride = (long long)stride;
-      op.rows_pad = g.rows1;
-      op.kpad = g.kpad1;
-      op.begin = group_begin(ph_total);
-      phops.push_back(op);
+      PhasorOp& op = q.f ? source(mb.packs, mb.pk_total, g, q) : source(mb.phops, mb.ph_total, g, q);
+      op.amp = q.f ? q.f : q.amp;
+      op.amp_dtype = q.f ? q.f_dtype : q.amp_dtype;
+      op.ld_amp = q.f ? q.ldf : q.ld_amp;
+      op.opd = q.f ? nullptr : q.opd;
+      op.opd_dtype = q.f ? 0 : q.opd_dtype;
+      op.ld_opd = q.f ? 0 : q.ld_opd;
+      if (prec == PREC_FP32) {
+        MaxOp mx = {};
+        mx.src = op.amp;
+        mx.dtype = op.amp_dtype;
+        mx.m = q.m;
+        mx.n = q.n;
+        mx.ld = op.ld_amp;
+        mx.nblk = max_blocks(q.m, q.n);
+        mx.part = (float*)(uintptr_t)ws;
+        mx.begin = mb.mx_total;
+        mb.mx_total += mx.nblk;
+        op.sc = ScaleSrc{mx.part, (float*)(uintptr_t)(ws + sizeof(float) * mx.nblk), mx.nblk, 0};
+        ws += round_up((int64_t)(sizeof(float) * (mx.nblk + 1)), 256);
+        mb.maxes.push_back(mx);
+      }
     }
-    phops.back().nwave += 1;
-    waves.push_back(PhasorWave{q.inv_wl, g.g1.fold, g.x01, g.g2.fold, g.x02});
-    wave_of.push_back((int)waves.size() - 1);
+    PhasorOp& op = q.f ? mb.packs.back() : mb.phops.back();
+    op.nwave += 1;
+    mb.waves.push_back(PhasorWave{q.f ? 0.0 : q.inv_wl, g.g1.fold, g.x01, g.g2.fold, g.x02});
+    mb.op_of.push_back(q.f ? -(int)mb.packs.size() : (int)mb.phops.size() - 1);
+    (q.f ? mb.pk_total : mb.ph_total) = op.begin + phasor_threads(g.r1, g.k1, op.nwave);
   }
-  if (!phops.empty())
-    ph_total = phops.back().begin + phasor_threads(phops.back().rows_pad, phops.back().kpad, phops.back().nwave);
+  mb.ws = ws;
 
-  std::vector<Problem>& p1 = mb.p1;
-  std::vector<Problem>& p2 = mb.p2;
-  p1.assign(count, Problem{});
-  p2.assign(count, Problem{});
-  std::vector<double>& cx = mb.cx;
-  std::vector<std::vector<Work>> clus1, clus2;
+  // ---- problems and works ------------------------------------------------------
+  std::vector<int> nkb1, nkb2;
+  mb.p1.resize(count);
+  mb.p2.resize(count);
   for (int32_t i = 0; i < count; ++i) {
     const mftx_mft& q = mfts[i];
-    const ManyGeo& g = geo[i];
-    Problem& a = p1[i];
-    a.lda = packed_lda(prec, g.kpad1);
-    a.alpha = g.alpha1;
-    a.y0 = g.g1.y0;
-    a.rows = (int)g.r1;
-    a.cols = g.g1.slots;
-    a.ncols = (int)g.c1;
-    a.cp = g.g1.cp;
-    a.cm = g.g1.cm;
-    a.kpad = g.kpad1;
-    a.chunk_begin = (int)cx.size();
-    push_chunks(cx, g.kpad1, g.x01);
-    a.scale = 1.0f;
-    a.limit = g.kpad2;
-    a.ldd = packed_lda(prec, g.kpad2);
-
-    Problem& b = p2[i];
-    b.lda = packed_lda(prec, g.kpad2);
-    b.alpha = g.alpha2;
-    b.y0 = g.g2.y0;
-    b.rows = (int)g.c1;
-    b.cols = g.g2.slots;
-    b.ncols = (int)(g.col_first ? q.N : q.M);
-    b.cp = g.g2.cp;
-    b.cm = g.g2.cm;
-    b.kpad = g.kpad2;
-    b.chunk_begin = (int)cx.size();
-    push_chunks(cx, g.kpad2, g.x02);
-    b.scale = (float)q.scale;
+    const MftGeo& g = geo[i];
+    Problem& a = mb.p1[i];
+    Problem& b = mb.p2[i];
+    mft_problems(g, prec, q.scale, a, b);
+    a.sbeg = b.sbeg = i;
+    a.send = b.send = i + 1;
     b.dst = q.F;
     b.ldd = q.ldF;
-    b.trans = g.col_first ? 0 : 1;
     b.wmap = q.w;
     b.ldw = q.ldw;
     b.wdtype = q.w_dtype;
+    const int n1 = pair_blocks(g.k1), n2 = pair_blocks(g.r1);
+    mb.s1.push_back(Seg{nullptr, nullptr, 0.0, n1, n1, mb.tables.ops[mb.tab1[i]].nkb, 0});
+    mb.s2.push_back(Seg{nullptr, nullptr, 0.0, n2, n2, mb.tables.ops[mb.tab2[i]].nkb, 0});
+    nkb1.push_back(n1);
+    nkb2.push_back(n2);
   }
-  // works: runs of consecutive entries with one geometry share a work item
-  auto group_works = [&](std::vector<std::vector<Work>>& clus, const std::vector<Problem>& ps, bool first) {
-    std::vector<int64_t> rows(count);
-    for (int32_t i = 0; i < count; ++i) rows[i] = first ? geo[i].rows1 : geo[i].rows2;
-    for (const auto& r : group_runs(ps, rows, bn)) add_tiles(clus, r.first, r.second, rows[r.first], ps[r.first].cols, bn);
-  };
-  group_works(clus1, p1, true);
-  group_works(clus2, p2, false);
-  mb.w1 = xcd_order(clus1);
-  mb.w2 = xcd_order(clus2);
+  std::vector<Work> w1, w2;
+  mb.tile1 = list_works(w1, mb.p1, nkb1, fixed, 8);
+  mb.tile2 = list_works(w2, mb.p2, nkb2, fixed, 8);
+  mb.w1 = xcd_order(w1);
+  mb.w2 = xcd_order(w2);
 
-  // one descriptor block: waves, phasor ops, pack ops, problems, chunk origins, works
+  // one descriptor block: waves, source ops, tables, problems, segments, works
   size_t off = 0;
   auto take = [&](size_t b) { const size_t o = off; off = round_up((int64_t)(off + b), 16); return o; };
-  mb.o_wv = take(sizeof(PhasorWave) * waves.size());
-  mb.o_ph = take(sizeof(PhasorOp) * phops.size());
-  mb.o_pk = take(sizeof(PackOp) * packs.size());
-  mb.o_p1 = take(sizeof(Problem) * p1.size());
-  mb.o_p2 = take(sizeof(Problem) * p2.size());
-  mb.o_cx = take(sizeof(double) * cx.size());
+  mb.o_wv = take(sizeof(PhasorWave) * mb.waves.size());
+  mb.o_ph = take(sizeof(PhasorOp) * mb.phops.size());
+  mb.o_pk = take(sizeof(PhasorOp) * mb.packs.size());
+  mb.o_mx = take(sizeof(MaxOp) * mb.maxes.size());
+  mb.o_tb = take(sizeof(TableOp) * mb.tables.ops.size());
+  mb.o_p1 = take(sizeof(Problem) * mb.p1.size());
+  mb.o_p2 = take(sizeof(Problem) * mb.p2.size());
+  mb.o_s1 = take(sizeof(Seg) * mb.s1.size());
+  mb.o_s2 = take(sizeof(Seg) * mb.s2.size());
   mb.o_w1 = take(sizeof(Work) * mb.w1.size());
   mb.o_w2 = take(sizeof(Work) * mb.w2.size());
   mb.bytes = off;
@@ -584,69 +702,98 @@ static void many_build(const mftx_mft* mfts, int32_t count, int prec, ManyBatch&
 // Rebase the batch's descriptors onto workspace `base` and the device
 // descriptor block `d`, and write the block's contents to host memory `h`.
 static void many_place(ManyBatch& mb, char* base, char* d, char* h) {
-  for (auto& op : mb.phops) {
-    op.waves = (const PhasorWave*)(d + mb.o_wv) + (uintptr_t)op.waves;
-    op.dst = base + (uintptr_t)op.dst;
-  }
+  for (auto* ops : {&mb.phops, &mb.packs})
+    for (auto& op : *ops) {
+      op.waves = (const PhasorWave*)(d + mb.o_wv) + (uintptr_t)op.waves;
+      op.dst = base + (uintptr_t)op.dst;
+      if (op.sc.n) {
+        op.sc.part = (const float*)(base + (uintptr_t)op.sc.part);
+        op.sc.inv = (float*)(base + (uintptr_t)op.sc.inv);
+      }
+    }
+  for (auto& mx : mb.maxes) mx.part = (float*)(base + (uintptr_t)mx.part);
+  for (size_t t = 0; t < mb.tables.ops.size(); ++t) mb.tables.ops[t].dst = base + mb.tables.off[t];
   for (size_t i = 0; i < mb.geo.size(); ++i) {
-    mb.p1[i].a = base + mb.geo[i].off1;
+    mb.s1[i].a = base + mb.geo[i].off1;
+    mb.s1[i].b = base + mb.tables.off[mb.tab1[i]];
+    mb.s2[i].a = base + mb.geo[i].off2;
+    mb.s2[i].b = base + mb.tables.off[mb.tab2[i]];
     mb.p1[i].dst = base + mb.geo[i].off2;
-    mb.p2[i].a = base + mb.geo[i].off2;
-    if (mb.wave_of[i] < 0) mb.packs[-mb.wave_of[i] - 1].dst = base + mb.geo[i].off1;
+    const PhasorOp& op = mb.op_of[i] < 0 ? mb.packs[-mb.op_of[i] - 1] : mb.phops[mb.op_of[i]];
+    mb.p2[i].inv = op.sc.n ? op.sc.inv : nullptr;
   }
-  std::memcpy(h + mb.o_wv, mb.waves.data(), sizeof(PhasorWave) * mb.waves.size());
-  std::memcpy(h + mb.o_ph, mb.phops.data(), sizeof(PhasorOp) * mb.phops.size());
-  std::memcpy(h + mb.o_pk, mb.packs.data(), sizeof(PackOp) * mb.packs.size());
-  std::memcpy(h + mb.o_p1, mb.p1.data(), sizeof(Problem) * mb.p1.size());
-  std::memcpy(h + mb.o_p2, mb.p2.data(), sizeof(Problem) * mb.p2.size());
-  std::memcpy(h + mb.o_cx, mb.cx.data(), sizeof(double) * mb.cx.size());
-  std::memcpy(h + mb.o_w1, mb.w1.data(), sizeof(Work) * mb.w1.size());
-  std::memcpy(h + mb.o_w2, mb.w2.data(), sizeof(Work) * mb.w2.size());
+  auto put = [&](size_t o, const auto& v) {
+    if (!v.empty()) std::memcpy(h + o, v.data(), sizeof(v[0]) * v.size());
+  };
+  put(mb.o_wv, mb.waves);
+  put(mb.o_ph, mb.phops);
+  put(mb.o_pk, mb.packs);
+  put(mb.o_mx, mb.maxes);
+  put(mb.o_tb, mb.tables.ops);
+  put(mb.o_p1, mb.p1);
+  put(mb.o_p2, mb.p2);
+  put(mb.o_s1, mb.s1);
+  put(mb.o_s2, mb.s2);
+  put(mb.o_w1, mb.w1);
+  put(mb.o_w2, mb.w2);
 }
 
-// The launches of a placed batch (descriptors at device address d).
+// The twiddle tables of a placed batch (descriptors at device address d).
+static hipError_t many_tables(const ManyBatch& mb, int prec, const char* d, hipStream_t s) {
+  return launch_tables(prec, (const TableOp*)(d + mb.o_tb), (int)mb.tables.ops.size(), mb.tables.threads, s);
+}
+
+// The launches of a placed batch, its tables already made.
 static hipError_t many_launch(const ManyBatch& mb, int prec, const char* d, hipStream_t s) {
-  hipError_t e = hipSuccess;
-  if (!mb.phops.empty())
-    e = launch_phasor_group(prec, (const PhasorOp*)(d + mb.o_ph), (int)mb.phops.size(), mb.ph_total, s);
-  if (e == hipSuccess && !mb.packs.empty())
-    e = launch_pack_group(prec, (const PackOp*)(d + mb.o_pk), (int)mb.packs.size(), mb.pk_total, s);
+  hipError_t e = launch_absmax((const MaxOp*)(d + mb.o_mx), (int)mb.maxes.size(), mb.mx_total, s);
   if (e == hipSuccess)
-    e = launch_gemm(prec, EPI_STORE_PACKED_T, mb.bn, (const Work*)(d + mb.o_w1), (int)mb.w1.size(),
-                    (const Problem*)(d + mb.o_p1), (const double*)(d + mb.o_cx), s);
+    e = launch_operands(prec, false, (const PhasorOp*)(d + mb.o_ph), (int)mb.phops.size(), mb.ph_total, s);
   if (e == hipSuccess)
-    e = launch_gemm(prec, EPI_STORE_CPLX, mb.bn, (const Work*)(d + mb.o_w2), (int)mb.w2.size(),
-                    (const Problem*)(d + mb.o_p2), (const double*)(d + mb.o_cx), s);
+    e = launch_operands(prec, true, (const PhasorOp*)(d + mb.o_pk), (int)mb.packs.size(), mb.pk_total, s);
+  if (e == hipSuccess)
+    e = launch_gemm(prec, EPI_STORE_PACKED, mb.tile1, (const Work*)(d + mb.o_w1), (int)mb.w1.size(),
+                    (const Problem*)(d + mb.o_p1), (const Seg*)(d + mb.o_s1), s);
+  if (e == hipSuccess)
+    e = launch_gemm(prec, EPI_STORE_CPLX, mb.tile2, (const Work*)(d + mb.o_w2), (int)mb.w2.size(),
+                    (const Problem*)(d + mb.o_p2), (const Seg*)(d + mb.o_s2), s);
   return e;
 }
 
 // All entries [0, count) on the context stream with the context workspace and
 // one descriptor ring slot; a batch whose descriptors exceed a slot is split.
 static int dft2_many_run(mftx_ctx* ctx, const mftx_mft* mfts, int32_t count, int prec) {
-  ManyBatch mb;
-  many_build(mfts, count, prec, mb);
-  if (mb.bytes > kSlotBytes) {
-    if (count == 1) return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
-    const int32_t h = count / 2;
-    const int rc = dft2_many_run(ctx, mfts, h, prec);
-    return rc ? rc : dft2_many_run(ctx, mfts + h, count - h, prec);
+  std::unique_ptr<ManyBatch> mb(new ManyBatch());
+  many_build(mfts, count, prec, -1, *mb);
+  if (mb->bytes > kSlotBytes || (count == 1 && too_large(mb->geo[0]))) {
+    if (count == 1) {
+      // the widest tiles need the fewest descriptors
+      mb.reset(new ManyBatch());
+      many_build(mfts, count, prec, TILE_BIG, *mb);
+      if (mb->bytes > kSlotBytes || too_large(mb->geo[0]))
+        return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
+    } else {
+      const int32_t h = count / 2;
+      const int rc = dft2_many_run(ctx, mfts, h, prec);
+      return rc ? rc : dft2_many_run(ctx, mfts + h, count - h, prec);
+    }
   }
-  int rc = ensure_ws(ctx, mb.ws);
+  int rc = ensure_ws(ctx, mb->ws);
   if (rc) return rc;
   // the slot is reserved first: the descriptors hold device addresses inside it
   int slot;
   char *h, *d;
   rc = reserve_desc(ctx, &slot, &h, &d);
   if (rc) return rc;
-  many_place(mb, (char*)ctx->ws, d, h);
-  rc = commit_desc(ctx, slot, mb.bytes);
+  many_place(*mb, (char*)ctx->ws, d, h);
+  rc = commit_desc(ctx, slot, mb->bytes);
   if (rc) return rc;
-  HIPCHK(ctx, many_launch(mb, prec, d, ctx->stream));
+  HIPCHK(ctx, many_tables(*mb, prec, d, ctx->stream));
+  HIPCHK(ctx, many_launch(*mb, prec, d, ctx->stream));
   return MFTX_OK;
 }
 
 // A persistent list of MFTs (mftx_mft_plan_*): plan-owned workspace and
-// descriptors, built once.
+// descriptors, built once, the twiddle tables with them.
 struct mftx_mft_plan {
   mftx_ctx* ctx = nullptr;
   int prec = 0;
@@ -758,21 +905,29 @@ int mftx_dft2(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, i
               int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r, double shift_c,
               double offset_r, double offset_c, double scale, int conj, int precision) {
   return mftx::dft2_on_workspace(ctx, f, f_dtype, m, n, ldf, F, M, N, ldF, alpha_r, alpha_c, shift_r, shift_c,
-                                 offset_r, offset_c, scale, conj, precision, nullptr, 0);
+                                 offset_r, offset_c, scale, conj, precision, nullptr, 0, 0);
 }
 
 }  // extern "C"
 
-// mftx_dft2 on the caller's workspace `ws` of `cap` bytes, or on the
-// context's growable workspace when ws is null.  The operands are fully
-// written before they are read (the packed input with its zero padding,
-// then stage 1's output for every K the second stage reads), so the
-// workspace needs no clearing; its padding rows beyond the output only feed
-// output rows that are never stored.
+// mftx_dft2 on the caller's workspace `ws`, or on the context's growable
+// workspace when ws is null.  Three launches and nothing uploaded: the source's
+// maximum (f16 form, larger sources only), then operand, twiddle tables and
+// descriptors (launch_prepare_one), then the two GEMMs.  A table larger than
+// `table_cap` bytes is made and used in pieces of whole tile columns.
+//
+// `cap` bounds the transform as the no-allocation entry point documents it:
+// complex64-sized operands with rows padded to 128 and K to 16 or 32.  The
+// workspace then holds operands of up to twice that (K is padded to 32 and
+// paired), two tables of table_cap and the descriptors.  The operands are fully
+// written before they are read (the source's operand with its zero padding,
+// then stage 1's output for every K the second stage reads), so the workspace
+// needs no clearing; padding rows beyond the output only feed output rows that
+// are never stored.
 int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, int64_t ldf, void* F,
                             int64_t M, int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r,
                             double shift_c, double offset_r, double offset_c, double scale, int conj, int precision,
-                            void* ws, size_t cap) {
+                            void* ws, size_t cap, size_t table_cap) {
   if (!ctx) return MFTX_EHANDLE;
   if (!f || !F) return fail(ctx, MFTX_EINVAL, "null array pointer");
   if (m <= 0 || n <= 0 || M <= 0 || N <= 0) return fail(ctx, MFTX_EINVAL, "shapes must be positive");
@@ -783,82 +938,93 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
     return fail(ctx, MFTX_EINVAL, "dimension too large");
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const int prec = precision;
-  const bool col_first = cost_col_first(m, n, M, N) < cost_row_first(m, n, M, N);
-  // stage-1 operand: f (row-first) or f^T (column-first)
-  const int64_t r1 = col_first ? n : m, k1 = col_first ? m : n;  // rows and K of stage 1
-  const int64_t c1 = col_first ? M : N;                           // stage-1 output columns
-  const int64_t c2 = col_first ? N : M;                           // stage-2 output columns
-  const int64_t rows1 = round_up(r1, BM);
-  const int64_t rows2 = round_up(c1, BM);
-  const double sgn = conj ? 1.0 : -1.0;
-  const double alpha1 = sgn * (col_first ? alpha_r : alpha_c), alpha2 = sgn * (col_first ? alpha_c : alpha_r);
-  const OutGrid g1 = make_grid(alpha1, col_first ? shift_r : shift_c, (int)c1);
-  const OutGrid g2 = make_grid(alpha2, col_first ? shift_c : shift_r, (int)c2);
-  const int s1 = g1.slots, s2 = g2.slots;
-  // 128-column tiles when the larger stage still gives every CU a workgroup
-  const int64_t wide = std::max((rows1 / BM) * ((s1 + 63) / 64), (rows2 / BM) * ((s2 + 63) / 64));
-  const int bn = wide >= 256 ? 128 : 64;
-  const int kg = k_granule(bn);
-  const int kpad1 = (int)round_up(k1, kg);
-  const int kpad2 = (int)round_up(r1, kg);
-  const size_t b1 = packed_bytes(prec, rows1, kpad1);
-  const size_t b2 = packed_bytes(prec, rows2, kpad2);
-  const size_t need = (size_t)round_up((int64_t)b1, 256) + b2;
+  const MftGeo g = mft_geometry(m, n, M, N, alpha_r, alpha_c, shift_r, shift_c, offset_r, offset_c, conj);
+  if (ws) {
+    const int64_t rows1 = round_up(g.r1, 128), rows2 = round_up(g.c1, 128);
+    const int64_t wide = std::max(rows1 / 128 * ((g.g1.slots + 63) / 64), rows2 / 128 * ((g.g2.slots + 63) / 64));
+    const int64_t kg = wide >= 256 ? 32 : 16;
+    const int64_t need = round_up(rows1 * round_up(g.k1, kg) * 8, 256) + rows2 * round_up(g.r1, kg) * 8;
+    if (need > (int64_t)cap)
+      return fail(ctx, MFTX_EINVAL, "transform needs " + std::to_string(need) + " bytes of workspace, more than the " +
+                                        std::to_string(cap) + " available");
+  }
+  const int nkb1 = pair_blocks(g.k1), nkb2 = pair_blocks(g.r1);
+  OneMft one = {};
+  Problem& p1 = one.desc.prob[0];
+  Problem& p2 = one.desc.prob[1];
+  mft_problems(g, prec, scale, p1, p2);
+  const int tile[2] = {pick_schedule(-1, false, p1.rblocks, p1.sblocks, nkb1, 1, 1).tile,
+                       pick_schedule(-1, false, p2.rblocks, p2.sblocks, nkb2, 1, 1).tile};
+  // slot blocks of a stage whose table fits the cap (whole tiles)
+  if (!ws) table_cap = kTableCap;
+  auto piece = [&](int sblocks, int nkb, int t) {
+    const int64_t fit = (int64_t)(table_cap / table_bytes(1, nkb)) / tile_slots(t) * tile_slots(t);
+    return (int)std::min<int64_t>(sblocks, std::max<int64_t>(fit, tile_slots(t)));
+  };
+  const int piece1 = piece(p1.sblocks, nkb1, tile[0]), piece2 = piece(p2.sblocks, nkb2, tile[1]);
+  // workspace: descriptors, maxima and inverse scale, operands, tables
+  const size_t o_max = round_up(sizeof(OneDesc), 256), o_a1 = o_max + 512;
+  const size_t o_a2 = o_a1 + folded_bytes(g.r1, g.k1), o_t1 = o_a2 + plain_bytes(g.c1, nkb2);
+  const size_t o_t2 = o_t1 + table_bytes(piece1, nkb1), need = o_t2 + table_bytes(piece2, nkb2);
+  static_assert((kMaxBlocks + 1) * sizeof(float) <= 512, "maxima and inverse scale fit their space");
   int rc = MFTX_OK;
   if (!ws) {
     rc = ensure_ws(ctx, need);
     if (rc) return rc;
     ws = ctx->ws;
-  } else if (need > cap) {
-    return fail(ctx, MFTX_EINVAL, "transform needs " + std::to_string(need) + " bytes of workspace, more than the " +
-                                      std::to_string(cap) + " available");
   }
-  char* a1 = (char*)ws;
-  char* a2 = a1 + round_up((int64_t)b1, 256);
-  // twiddle coordinates: rows x = R + or against U - sr; columns x = S + oc
-  // against V - sc; each stage's output shift is folded into its A operand
-  const double xr0 = -centre(m) + offset_r, xc0 = -centre(n) + offset_c;
-  const double fold1 = g1.fold, fold2 = g2.fold;
-  const double x01 = col_first ? xr0 : xc0, x02 = col_first ? xc0 : xr0;
-  // the operand carries both folds: stage 1's along K, stage 2's along its
-  // rows (stage 1's output rows, stage 2's K)
-  HIPCHK(ctx, launch_pack(prec, f, f_dtype, m, n, ldf, col_first ? 1 : 0, fold1, x01, fold2, x02, a1, rows1,
-                          kpad1, ctx->stream));
+  if (too_large(g)) return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
+  char* base = (char*)ws;
+  float* part = (float*)(base + o_max);
+  float* inv = part + kMaxBlocks;
 
-  Problem p1 = {};
-  p1.a = a1;
-  p1.lda = packed_lda(prec, kpad1);
-  p1.alpha = alpha1;
-  p1.y0 = g1.y0;
-  p1.rows = (int)r1;
-  p1.cols = s1;
-  p1.ncols = (int)c1;
-  p1.cp = g1.cp;
-  p1.cm = g1.cm;
-  p1.kpad = kpad1;
-  p1.scale = 1.0f;
-  p1.limit = kpad2;
-  p1.dst = a2;
-  p1.ldd = packed_lda(prec, kpad2);
-  rc = run_single(ctx, prec, EPI_STORE_PACKED_T, bn, p1, x01, rows1);
-  if (rc) return rc;
-
-  Problem p2 = {};
-  p2.a = a2;
-  p2.lda = packed_lda(prec, kpad2);
-  p2.alpha = alpha2;
-  p2.y0 = g2.y0;
-  p2.rows = (int)c1;
-  p2.cols = s2;
-  p2.ncols = (int)c2;
-  p2.cp = g2.cp;
-  p2.cm = g2.cm;
-  p2.kpad = kpad2;
-  p2.scale = (float)scale;
+  one.op.amp = f;
+  one.op.amp_dtype = f_dtype;
+  one.op.ld_amp = ldf;
+  one.op.m = (int)m;
+  one.op.n = (int)n;
+  one.op.trans = g.col_first ? 1 : 0;
+  one.op.nwave = 1;
+  one.op.dst = base + o_a1;
+  MaxOp mx = {};
+  if (prec == PREC_FP32) {
+    mx.src = f;
+    mx.dtype = f_dtype;
+    mx.m = m;
+    mx.n = n;
+    mx.ld = ldf;
+    mx.nblk = max_blocks(m, n);
+    mx.part = part;
+    // a source of up to 8192 elements is read whole by every operand block
+    // instead: cheaper than a launch of its own
+    one.op.sc = ScaleSrc{part, inv, m * n <= 8192 ? 0 : mx.nblk, 0};
+    p2.inv = inv;
+  }
+  one.wave = PhasorWave{0.0, g.g1.fold, g.x01, g.g2.fold, g.x02};
+  one.tab[0] = TableOp{g.alpha1, g.k1 & 1 ? 0.0 : 0.5, g.g1.y0, piece1, nkb1, 0, 0, base + o_t1, 0};
+  one.tab[1] = TableOp{g.alpha2, g.r1 & 1 ? 0.0 : 0.5, g.g2.y0, piece2, nkb2, 0, 0, base + o_t2, 0};
+  one.desc.seg[0] = Seg{base + o_a1, base + o_t1, 0.0, nkb1, nkb1, nkb1, 0};
+  one.desc.seg[1] = Seg{base + o_a2, base + o_t2, 0.0, nkb2, nkb2, nkb2, 0};
+  p1.sbeg = p2.sbeg = 0;
+  p1.send = p2.send = 1;
+  p1.dst = base + o_a2;
   p2.dst = F;
   p2.ldd = ldF;
-  p2.trans = col_first ? 0 : 1;  // C is F (column-first) or F^T (row-first)
-  return run_single(ctx, prec, EPI_STORE_CPLX, bn, p2, x02, rows2);
+  one.desc_dev = (OneDesc*)base;
+  HIPCHK(ctx, launch_prepare_one(prec, one, mx, ctx->stream));
+  for (int st = 0; st < 2; ++st) {
+    const int sblocks = st ? p2.sblocks : p1.sblocks, step = st ? piece2 : piece1;
+    const int rblocks = st ? p2.rblocks : p1.rblocks, nkb = st ? nkb2 : nkb1;
+    for (int sb = 0; sb < sblocks; sb += step) {
+      TableOp t = one.tab[st];
+      t.sb0 = sb;
+      t.nsb = std::min(step, sblocks - sb);
+      if (sb) HIPCHK(ctx, launch_table_one(prec, t, ctx->stream));
+      HIPCHK(ctx, launch_gemm_one(prec, st ? EPI_STORE_CPLX : EPI_STORE_PACKED, tile[st], rblocks, sb, sb + t.nsb, nkb,
+                                  &one.desc_dev->prob[st], &one.desc_dev->seg[st], ctx->stream));
+    }
+  }
+  return MFTX_OK;
 }
 
 extern "C" {
@@ -989,7 +1155,7 @@ int mftx_mft_plan_create(mftx_ctx* ctx, const mftx_mft* mfts, int32_t count, int
   std::unique_ptr<mftx_mft_plan> plan(new mftx_mft_plan());  // frees its device block on every exit
   plan->ctx = ctx;
   plan->prec = precision;
-  many_build(mfts, count, precision, plan->mb);
+  many_build(mfts, count, precision, -1, plan->mb);
   const size_t wsb = (size_t)round_up((int64_t)plan->mb.ws, 256);
   if (!try_malloc(&plan->mem, wsb + plan->mb.bytes)) {
     plan->mem = nullptr;
@@ -1000,6 +1166,7 @@ int mftx_mft_plan_create(mftx_ctx* ctx, const mftx_mft* mfts, int32_t count, int
   many_place(plan->mb, (char*)plan->mem, plan->desc, host.data());
   if (hipMemcpy(plan->desc, host.data(), host.size(), hipMemcpyHostToDevice) != hipSuccess)
     return fail(ctx, MFTX_EDEVICE, "MFT plan upload failed");
+  HIPCHK(ctx, many_tables(plan->mb, precision, plan->desc, ctx->stream));
   *out = plan.release();
   return MFTX_OK;
   });
@@ -1299,10 +1466,10 @@ struct ClassInfo {
   std::vector<int> members;  // problem indices
   int group;
   bool col_first;
-  int64_t rows2;      // stage-2 A rows (tile-padded): N (row-first) or M (column-first)
-  int ktot;           // stage-2 K
-  std::vector<int> kbeg;
-  size_t abuf = 0;    // stage-2 A buffer
+  int rblocks2 = 0;         // stage-2 row blocks: of N (row-first) or M (column-first) rows
+  int64_t pairs1 = 0;       // K pairs of its longest stage-1 problem
+  std::vector<int> nkb;     // stage-2 K blocks per member
+  std::vector<size_t> abuf; // stage-2 operand per member
   size_t fbuf = 0;    // complex F (partial-overlap groups)
   int p2 = -1;        // index of its stage-2 problem
 };
@@ -1323,9 +1490,8 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   if (image_rows <= 0 || image_cols <= 0 || image_rows > (1 << 20) || image_cols > (1 << 20))
     return fail(ctx, MFTX_EINVAL, "bad image shape");
   if (lambda_group <= 0) lambda_group = 8;
-  if (tile_n == 0) tile_n = BN_DEFAULT;
-  if (!valid_bn(tile_n)) return fail(ctx, MFTX_EINVAL, "tile_n must be 0, 64 or 128");
-  const int kg = k_granule(tile_n);
+  if (tile_n != 0 && tile_n != 64 && tile_n != 128) return fail(ctx, MFTX_EINVAL, "tile_n must be 0, 64 or 128");
+  const int fixed_tile = tile_n == 64 ? TILE_MID : tile_n == 128 ? TILE_BIG : -1;
   for (int t = 0; t < ntiles; ++t) {
     const mftx_tile& T = tiles[t];
     if (!T.amp || !T.opd || T.m <= 0 || T.n <= 0 || T.m > (1 << 20) || T.n > (1 << 20) || T.ld_amp < T.n ||
@@ -1412,137 +1578,191 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   // ---- workspace layout ----------------------------------------------------------
   Layout lay;
   // phasor operands per (tile, orientation): every slot the pair is used with
-  std::map<std::pair<int, int>, std::vector<Slot>> tile_slots;
+  std::map<std::pair<int, int>, std::vector<Slot>> tile_slots_of;
   for (auto& c : cls)
-    for (int i : c.members) tile_slots[{problems[i].tile, c.col_first ? 1 : 0}].push_back(pslot[i]);
-  struct TileOp { int64_t rows; int kpad; size_t off; std::map<Slot, int> slot; int wave_off; int nslot; };
+    for (int i : c.members) tile_slots_of[{problems[i].tile, c.col_first ? 1 : 0}].push_back(pslot[i]);
+  struct TileOp { int64_t R, K; size_t off; std::map<Slot, int> slot; int wave_off; int nslot; };
   std::map<std::pair<int, int>, TileOp> tops;
   std::vector<Slot> wave_slots;  // every phasor slot, grouped by (tile, orientation)
-  for (auto& kv : tile_slots) {
+  for (auto& kv : tile_slots_of) {
     auto v = kv.second;
     std::sort(v.begin(), v.end());
     v.erase(std::unique(v.begin(), v.end()), v.end());
     const mftx_tile& T = tiles[kv.first.first];
     const bool tr = kv.first.second == 1;
     TileOp op;
-    op.rows = round_up(tr ? T.n : T.m, BM);
-    op.kpad = (int)round_up(tr ? T.m : T.n, kg);
+    op.R = tr ? T.n : T.m;
+    op.K = tr ? T.m : T.n;
     op.wave_off = (int)wave_slots.size();
     op.nslot = (int)v.size();
     for (size_t j = 0; j < v.size(); ++j) {
       op.slot[v[j]] = (int)j;
       wave_slots.push_back(v[j]);
     }
-    op.off = lay.take(packed_bytes(prec, op.rows, op.kpad) * v.size());
+    op.off = lay.take(folded_bytes(op.R, op.K) * v.size());
     tops[kv.first] = op;
   }
-  // stage-2 operands per class
+  // stage-2 operands per class and member
   for (auto& c : cls) {
-    c.rows2 = round_up(c.col_first ? c.key.M : c.key.N, BM);
-    int k = 0;
+    const int64_t rows2 = c.col_first ? c.key.M : c.key.N;
+    c.rblocks2 = (int)blocks32(rows2);
     for (int i : c.members) {
       const mftx_tile& T = tiles[problems[i].tile];
-      c.kbeg.push_back(k);
-      k += (int)round_up(c.col_first ? T.n : T.m, kg);
+      const int nkb = pair_blocks(c.col_first ? T.n : T.m);
+      c.nkb.push_back(nkb);
+      c.abuf.push_back(lay.take(plain_bytes(rows2, nkb)));
+      c.pairs1 = std::max<int64_t>(c.pairs1, pairs(c.col_first ? T.m : T.n));
     }
-    c.ktot = k;
-    c.abuf = lay.take(packed_bytes(prec, c.rows2, c.ktot));
     if (!cfast[&c - cls.data()]) c.fbuf = lay.take(sizeof(float2) * (size_t)c.key.M * c.key.N);
+  }
+  // f16 form: one scale for all tiles that meet in a coherent group (connected
+  // through classes), from the maxima of their amplitudes, which lie together
+  std::vector<int> comp(ntiles);
+  for (int t = 0; t < ntiles; ++t) comp[t] = t;
+  auto root = [&](int t) {
+    while (comp[t] != t) t = comp[t] = comp[comp[t]];
+    return t;
+  };
+  for (auto& kv : groups) {
+    const int t0 = problems[cls[kv.second[0]].members[0]].tile;
+    for (int c : kv.second)
+      for (int i : cls[c].members) comp[root(problems[i].tile)] = root(t0);
+  }
+  struct Comp { size_t part = 0, inv = 0; int n = 0; };  // workspace offsets of the maxima and the inverse scale
+  std::map<int, Comp> comps;
+  std::vector<MaxOp> maxes;
+  std::vector<size_t> max_part;  // workspace offset of each job's maxima
+  long long max_total = 0;
+  if (prec == PREC_FP32) {
+    for (int t = 0; t < ntiles; ++t) comps[root(t)].n += max_blocks(tiles[t].m, tiles[t].n);
+    for (auto& kv : comps) {
+      kv.second.part = lay.take(sizeof(float) * (kv.second.n + 1));
+      kv.second.inv = kv.second.part + sizeof(float) * kv.second.n;
+      size_t at = kv.second.part;
+      for (int t = 0; t < ntiles; ++t) {
+        if (root(t) != kv.first) continue;
+        const mftx_tile& T = tiles[t];
+        MaxOp mx = {};
+        mx.src = T.amp;
+        mx.dtype = T.amp_dtype;
+        mx.m = T.m;
+        mx.n = T.n;
+        mx.ld = T.ld_amp;
+        mx.nblk = max_blocks(T.m, T.n);
+        mx.begin = max_total;
+        max_total += mx.nblk;
+        maxes.push_back(mx);
+        max_part.push_back(at);
+        at += sizeof(float) * mx.nblk;
+      }
+    }
   }
 
   // ---- descriptors ---------------------------------------------------------------
-  std::vector<Problem> p1, p2;
-  std::vector<double> cx;
-  std::vector<std::vector<Work>> clus1, clus2;
-  struct Patch { int idx; size_t a, dst; };  // workspace offsets to rebase after allocation
+  // Segment addresses are workspace offsets (operand) and table indices until
+  // the workspace exists.
+  Tables tables;
+  struct SegRef { size_t a; int table; };
+  std::vector<Problem> p1, p2;  // stage 1 per (class, member); stage 2 per class
+  std::vector<Seg> segs;
+  std::vector<SegRef> refs;
+  struct Patch { size_t dst, inv; };  // workspace offsets of the destination and the inverse scale (0: none)
   std::vector<Patch> patch1, patch2;
-  std::vector<int64_t> s1rows;  // tiled rows of each stage-1 problem
-
-  for (auto& c : cls) {
+  std::vector<int> nkb1;              // K blocks of each stage-1 problem
+  std::vector<std::vector<std::pair<Seg, SegRef>>> seg2(cls.size());
+  std::vector<RowPhase> row_phases(cls.size(), RowPhase{});
+  size_t row_phase_rows = 0;
+  for (size_t ci = 0; ci < cls.size(); ++ci) {
+    ClassInfo& c = cls[ci];
     const ClassKey& K = c.key;
     const bool cf = c.col_first;
+    const bool single = cfast[ci] && c.members.size() == 1;
+    const double a1 = -(cf ? K.ar : K.ac), a2 = -(cf ? K.ac : K.ar);
+    const int n1 = cf ? K.M : K.N, n2 = cf ? K.N : K.M;  // output columns of the stages
+    const OutGrid g1 = make_grid(a1, cf ? K.sr : K.sc, n1);
+    const OutGrid g2 = make_grid(a2, cf ? K.sc : K.sr, n2);
+    double xc2 = 0;
     // stage 1, one problem per member
     for (size_t j = 0; j < c.members.size(); ++j) {
-      const mftx_problem& P = problems[c.members[j]];
-      const mftx_tile& T = tiles[P.tile];
-      const TileOp& op = tops[{P.tile, cf ? 1 : 0}];
-      const int kp2 = (int)round_up(cf ? T.n : T.m, kg);
-      const int n1 = cf ? K.M : K.N;  // output columns of stage 1
-      const Slot& sl = pslot[c.members[j]];
+      const int i = c.members[j];
+      const TileOp& op = tops[{problems[i].tile, cf ? 1 : 0}];
+      const double xc1 = std::get<2>(pslot[i]) + 0.5 * (double)(op.K - 1);
+      const double xc = std::get<4>(pslot[i]) + 0.5 * (double)(op.R - 1);
       Problem q = {};
-      q.lda = packed_lda(prec, op.kpad);
-      q.alpha = -(cf ? P.alpha_r : P.alpha_c);
-      const OutGrid g1 = make_grid(q.alpha, cf ? K.sr : K.sc, n1);
-      q.y0 = g1.y0;
-      q.rows = (int)(cf ? T.n : T.m);
+      q.sbeg = (int)segs.size();
+      q.send = q.sbeg + 1;
+      q.rblocks = pair_blocks(op.R);
+      q.sblocks = (int)blocks32(g1.slots);
+      q.rows = 32 * q.rblocks;
       q.cols = g1.slots;
       q.ncols = n1;
       q.cp = g1.cp;
       q.cm = g1.cm;
-      q.kpad = op.kpad;
-      q.chunk_begin = (int)cx.size();
-      push_chunks(cx, op.kpad, std::get<2>(sl));  // x01
-      q.scale = 1.0f;
-      q.limit = kp2;
-      q.ldd = packed_lda(prec, c.ktot);
-      // both folds are in the operand
-      const size_t elem = prec == PREC_FP32 ? sizeof(float2) : 4 * sizeof(uint16_t);
-      const int slot = op.slot.at(sl);
-      patch1.push_back(Patch{(int)p1.size(), op.off + (size_t)slot * packed_bytes(prec, op.rows, op.kpad),
-                             c.abuf + (size_t)c.kbeg[j] * elem});
-      s1rows.push_back(op.rows);
+      q.y0 = g1.y0;
+      // the phase of stage 1's input midpoint is a phase of stage 2's rows,
+      // which |F|^2 of a single segment does not see
+      q.xrot = single ? 0.0 : a1 * xc1;
+      q.scale = (float)stage1_scale(prec, c.pairs1);
+      q.ldd = c.nkb[j];
+      const int nkb = pair_blocks(op.K);
+      segs.push_back(Seg{nullptr, nullptr, 0.0, nkb, nkb, 0, 0});
+      refs.push_back(SegRef{op.off + (size_t)op.slot.at(pslot[i]) * folded_bytes(op.R, op.K),
+                            tables.get(a1, g1.y0, op.K, g1.slots)});
+      patch1.push_back(Patch{c.abuf[j], 0});
       p1.push_back(q);
+      nkb1.push_back(nkb);
+      // its stage-2 segment
+      Seg sg = {};
+      sg.nkb = sg.a_nkb = c.nkb[j];
+      sg.rot = j ? a2 * (xc2 - xc) : 0.0;
+      xc2 = xc;
+      seg2[ci].push_back({sg, SegRef{c.abuf[j], tables.get(a2, g2.y0, op.R, g2.slots)}});
+      if (single) {
+        row_phases[ci] = RowPhase{a1 * xc1, g1.cm + g1.y0, nullptr, n1, 0};
+        row_phase_rows += n1;
+      }
     }
-    // stage 2, one problem per class (K concatenated over members)
+    // stage 2, one problem per class
     Problem q = {};
-    const int n2 = cf ? K.N : K.M;
-    q.lda = packed_lda(prec, c.ktot);
-    q.alpha = -(cf ? K.ac : K.ar);
-    const OutGrid g2 = make_grid(q.alpha, cf ? K.sc : K.sr, n2);
-    q.y0 = g2.y0;
-    q.rows = cf ? K.M : K.N;
+    q.rblocks = c.rblocks2;
+    q.sblocks = (int)blocks32(g2.slots);
+    q.rows = n1;
     q.cols = g2.slots;
     q.ncols = n2;
     q.cp = g2.cp;
     q.cm = g2.cm;
-    q.kpad = c.ktot;
-    q.chunk_begin = (int)cx.size();
-    for (size_t j = 0; j < c.members.size(); ++j) {
-      const mftx_problem& P = problems[c.members[j]];
-      const mftx_tile& T = tiles[P.tile];
-      push_chunks(cx, (int)round_up(cf ? T.n : T.m, kg), cf ? -centre(T.n) + P.offset_c : -centre(T.m) + P.offset_r);
-    }
+    q.y0 = g2.y0;
+    q.xrot = a2 * xc2;
     q.trans = cf ? 0 : 1;
     const double unit = std::sqrt(std::fabs(K.ar * K.ac));  // unitary scale (fourier.py:100-101)
-    const bool cl_fast = cfast[&c - cls.data()];
-    if (cl_fast) {
-      q.scale = (float)(unit * unit * problems[c.members[0]].weight);
+    const bool cl_fast = cfast[ci];
+    if (cl_fast) {  // the scale is a power of two, so the weight is rounded once
+      q.scale = (float)stage2_scale(prec, c.pairs1);
+      q.weight = (float)(unit * unit * problems[c.members[0]].weight);
     } else {
-      q.scale = (float)unit;
+      q.scale = (float)(unit * stage2_scale(prec, c.pairs1));
       q.ldd = K.N;  // F[u][v]
     }
     c.p2 = (int)p2.size();
-    patch2.push_back(Patch{(int)p2.size(), c.abuf, cl_fast ? 0 : c.fbuf});
+    patch2.push_back(Patch{cl_fast ? 0 : c.fbuf, prec == PREC_FP32 ? comps[root(problems[c.members[0]].tile)].inv : 0});
     p2.push_back(q);
   }
+  bool multi = false;  // a class of several segments along K
+  for (auto& c : cls) multi = multi || c.members.size() > 1;
 
-  // stage-1 works: runs of g1 consecutive problems with one tiling and K
-  // length (the wavelengths of a tile) share a work item, so the staging
-  // pipeline runs on across their K loops instead of refilling for every
-  // short K loop; g1 keeps at least one work item per CU
-  {
-    std::vector<int64_t> rows(s1rows.begin(), s1rows.end());
-    for (const auto& r : group_runs(p1, rows, tile_n)) add_tiles(clus1, r.first, r.second, s1rows[r.first],
-                                                                 p1[r.first].cols, tile_n);
-  }
   // owned until returned: every failure or exception path frees the plan and its workspace
   std::unique_ptr<mftx_plan, int (*)(mftx_plan*)> owned(new mftx_plan(), mftx_plan_destroy);
   mftx_plan* plan = owned.get();
   plan->ctx = ctx;
   plan->prec = prec;
-  plan->bn = tile_n;
   plan->img_rows = image_rows;
   plan->img_cols = image_cols;
+
+  // stage-1 works: runs of consecutive problems with one tiling and K length
+  // (the wavelengths of a tile) share a work item, so the load pipeline runs
+  // on across their K loops instead of refilling for every short one
+  std::vector<Work> w1;
+  plan->tile1 = list_works(w1, p1, nkb1, fixed_tile, 8);
 
   // stage-2 works: λ-groups of classes with one output window and orientation
   // accumulate |F|^2 in registers (the intensity path); a class of a
@@ -1556,6 +1776,11 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   // that window's single reduction.
   struct GeoInfo { std::vector<std::vector<int>> lgroups; size_t partial; int64_t prow, pcol; };
   std::vector<GeoInfo> geos;
+  auto class_nkb = [&](int c) {
+    int n = 0;
+    for (int k : cls[c].nkb) n += k;
+    return n;
+  };
   {
     using Grid = std::tuple<int, int, int>;  // stage-2 (cp, cm, slots)
     std::map<std::tuple<int, int, int64_t, int64_t, int>, std::map<Grid, std::vector<int>>> geo;
@@ -1565,81 +1790,127 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
       geo[{cls[c].key.M, cls[c].key.N, cls[c].key.r0, cls[c].key.c0, cls[c].col_first ? 1 : 0}][{q.cp, q.cm, q.cols}]
           .push_back((int)c);
     }
+    // the tile and the λ-group length (lambda_group at most: shorter where
+    // that fills the chip better) follow the grid with most classes
+    const std::vector<int>* top = nullptr;
+    int64_t nfast = 0;
+    for (auto& kv : geo)
+      for (auto& sub : kv.second) {
+        nfast += sub.second.size();
+        if (!top || sub.second.size() > top->size()) top = &sub.second;
+      }
+    Schedule sch{multi ? TILE_MULTI : TILE_MID, lambda_group};
+    if (top) {
+      const Problem& q = p2[cls[(*top)[0]].p2];
+      sch = pick_schedule(multi && fixed_tile == TILE_BIG ? TILE_MULTI : fixed_tile == TILE_MID && multi ? TILE_MULTI : fixed_tile,
+                          multi, q.rblocks, q.sblocks, class_nkb((*top)[0]), nfast, lambda_group);
+    }
+    plan->tile2 = sch.tile;
     for (auto& kv : geo) {
       GeoInfo gi;
       for (auto& sub : kv.second) {
         const auto& cl = sub.second;
-        for (size_t s = 0; s < cl.size(); s += lambda_group)
-          gi.lgroups.emplace_back(cl.begin() + s, cl.begin() + std::min(cl.size(), s + (size_t)lambda_group));
+        // groups of nearly equal length, none longer than the schedule's
+        const size_t ng = (cl.size() + sch.run - 1) / sch.run;
+        for (size_t s = 0; s < ng; ++s)
+          gi.lgroups.emplace_back(cl.begin() + s * cl.size() / ng, cl.begin() + (s + 1) * cl.size() / ng);
       }
-      gi.prow = round_up(std::get<0>(kv.first), BM);  // partial[u][v]
-      gi.pcol = round_up(std::get<1>(kv.first), BM);
+      gi.prow = round_up(std::get<0>(kv.first), 128);  // partial[u][v]
+      gi.pcol = round_up(std::get<1>(kv.first), 128);
       gi.partial = lay.take(sizeof(float) * gi.prow * gi.pcol * gi.lgroups.size());
       geos.push_back(gi);
     }
   }
-  // stage-2 problem lists in launch order (λ-groups contiguous), intensity
-  // and complex-store
+  // stage-2 problem lists in launch order (λ-groups contiguous), intensity and
+  // complex-store, each problem followed by copies of its class's segments
   std::vector<Problem> p2_launch, p2c_launch;
   std::vector<Patch> patch2_launch, patch2c_launch;
-  std::vector<std::vector<Work>> clus2c;
-  {
-    for (auto& gi : geos) {
-      for (size_t g = 0; g < gi.lgroups.size(); ++g) {
-        const int pb = (int)p2_launch.size();
-        for (int c : gi.lgroups[g]) {
-          p2_launch.push_back(p2[cls[c].p2]);
-          patch2_launch.push_back(Patch{(int)p2_launch.size() - 1, patch2[cls[c].p2].a, 0});
-        }
-        const ClassInfo& c0 = cls[gi.lgroups[g][0]];
-        const size_t poff = gi.partial + sizeof(float) * gi.prow * gi.pcol * g;
-        // the partial image offset rides in the pointer field until the workspace exists
-        add_tiles(clus2, pb, (int)p2_launch.size(), c0.rows2, p2[c0.p2].cols, tile_n,
-                  (float*)(uintptr_t)poff, (long long)gi.pcol, c0.key.M, c0.key.N);
-      }
-    }
-    for (size_t ci = 0; ci < cls.size(); ++ci) {
-      if (cfast[ci]) continue;
-      const ClassInfo& c = cls[ci];
-      const int pb = (int)p2c_launch.size();
-      p2c_launch.push_back(p2[c.p2]);
-      patch2c_launch.push_back(Patch{pb, patch2[c.p2].a, patch2[c.p2].dst});
-      add_tiles(clus2c, pb, pb + 1, c.rows2, p2[c.p2].cols, tile_n);
-    }
-  }
-  std::vector<Work> w1 = xcd_order(clus1), w2 = xcd_order(clus2), w2c = xcd_order(clus2c);
-  // the complex-field set: each class's stage-2 problem, one work set per class
-  std::vector<std::vector<Work>> clusf;
-  for (size_t c = 0; c < cls.size(); ++c) {
+  std::vector<Work> w2, w2c, wf;
+  auto push2 = [&](std::vector<Problem>& list, std::vector<Patch>& patches, int c) {
     Problem q = p2[cls[c].p2];
-    q.dst = nullptr;
-    q.wmap = nullptr;
-    plan->pf.push_back(q);
-    plan->class_first.push_back(cls[c].members[0]);
-    add_tiles(clusf, (int)c, (int)c + 1, cls[c].rows2, q.cols, tile_n);
+    q.sbeg = (int)segs.size();
+    for (auto& sr : seg2[c]) {
+      segs.push_back(sr.first);
+      refs.push_back(sr.second);
+    }
+    q.send = (int)segs.size();
+    list.push_back(q);
+    patches.push_back(patch2[cls[c].p2]);
+  };
+  for (auto& gi : geos)
+    for (size_t g = 0; g < gi.lgroups.size(); ++g) {
+      const int pb = (int)p2_launch.size();
+      int nch = 0;
+      for (int c : gi.lgroups[g]) {
+        push2(p2_launch, patch2_launch, c);
+        nch += class_nkb(c);
+      }
+      const ClassInfo& c0 = cls[gi.lgroups[g][0]];
+      const size_t poff = gi.partial + sizeof(float) * gi.prow * gi.pcol * g;
+      // the partial image offset rides in the pointer field until the workspace exists
+      add_tiles(w2, plan->tile2, pb, (int)p2_launch.size(), nch, c0.rblocks2, p2[c0.p2].sblocks,
+                (float*)(uintptr_t)poff, (long long)gi.pcol, c0.key.M, c0.key.N);
+    }
+  {
+    // complex stores: one problem per work item
+    auto cplx_tile = [&](const std::vector<int>& cl) {
+      int rb = 0, sb = 0, nk = 0;
+      for (int c : cl) {
+        rb = std::max(rb, p2[cls[c].p2].rblocks);
+        sb = std::max(sb, p2[cls[c].p2].sblocks);
+        nk = std::max(nk, class_nkb(c));
+      }
+      const int fixed = multi && (fixed_tile == TILE_BIG || fixed_tile == TILE_MID) ? TILE_MULTI : fixed_tile;
+      return pick_schedule(fixed, multi, rb, sb, nk, cl.size(), 1).tile;
+    };
+    std::vector<int> slow, every;
+    for (size_t c = 0; c < cls.size(); ++c) {
+      every.push_back((int)c);
+      if (!cfast[c]) slow.push_back((int)c);
+    }
+    if (!slow.empty()) plan->tile2c = cplx_tile(slow);
+    if (!every.empty()) plan->tile_f = cplx_tile(every);
+    for (int c : slow) {
+      const int pb = (int)p2c_launch.size();
+      push2(p2c_launch, patch2c_launch, c);
+      add_tiles(w2c, plan->tile2c, pb, pb + 1, class_nkb(c), cls[c].rblocks2, p2[cls[c].p2].sblocks);
+    }
+    // the complex-field set: each class's stage-2 problem
+    std::vector<Patch> patch_f;
+    for (int c : every) {
+      push2(plan->pf, patch_f, c);
+      plan->class_first.push_back(cls[c].members[0]);
+      add_tiles(wf, plan->tile_f, c, c + 1, class_nkb(c), cls[c].rblocks2, p2[cls[c].p2].sblocks);
+    }
   }
-  std::vector<Work> wf = xcd_order(clusf);
-  // executed MFMA FLOPs of the two launches: per workgroup and problem, BM rows
-  // x slots x kpad x 4 real products (re/im x cos/sin) x 2, times the passes
-  const double passes = prec == PREC_BF16X3 ? 3.0 : 1.0;
-  const double per_slot_k = 8.0 * BM * slots_per_tile(tile_n) * passes;
-  double mf1 = 0, mf2 = 0;
-  for (auto& w : w1)
-    for (int i = w.pbeg; i < w.pend; ++i) mf1 += per_slot_k * p1[i].kpad;
-  for (auto& w : w2)
-    for (int i = w.pbeg; i < w.pend; ++i) mf2 += per_slot_k * p2_launch[i].kpad;
-  for (auto& w : w2c)
-    for (int i = w.pbeg; i < w.pend; ++i) mf2 += per_slot_k * p2c_launch[i].kpad;
+  // executed MFMA FLOPs of the two launches: 12 instructions of 32 x 32 x 16
+  // per 32 x 32 block and K block
+  auto mfma = [](const std::vector<Work>& ws, int tile) {
+    double f = 0;
+    for (auto& w : ws) f += (double)w.nch * tile_rows(tile) * tile_slots(tile) * 12.0 * 32768.0;
+    return f;
+  };
+  const double mf1 = mfma(w1, plan->tile1), mf2 = mfma(w2, plan->tile2) + mfma(w2c, plan->tile2c);
+  w1 = xcd_order(w1);
+  w2 = xcd_order(w2);
+  w2c = xcd_order(w2c);
+  wf = xcd_order(wf);
 
+  const size_t o_tab = lay.total;
+  lay.take(tables.place(o_tab));
+  const size_t o_rowph = lay.take(sizeof(float2) * std::max<size_t>(row_phase_rows, 1));
+  const size_t o_rpops = lay.take(sizeof(RowPhase) * std::max<size_t>(cls.size(), 1));
   const size_t o_w1 = lay.take(sizeof(Work) * std::max<size_t>(w1.size(), 1));
   const size_t o_w2 = lay.take(sizeof(Work) * std::max<size_t>(w2.size(), 1));
   const size_t o_p1 = lay.take(sizeof(Problem) * std::max<size_t>(p1.size(), 1));
   const size_t o_p2 = lay.take(sizeof(Problem) * std::max<size_t>(p2_launch.size(), 1));
   const size_t o_w2c = lay.take(sizeof(Work) * std::max<size_t>(w2c.size(), 1));
   const size_t o_p2c = lay.take(sizeof(Problem) * std::max<size_t>(p2c_launch.size(), 1));
-  const size_t o_cx = lay.take(sizeof(double) * std::max<size_t>(cx.size(), 1));
+  const size_t o_segs = lay.take(sizeof(Seg) * std::max<size_t>(segs.size(), 1));
   const size_t o_iw = lay.take(sizeof(PhasorWave) * std::max<size_t>(wave_slots.size(), 1));
   const size_t o_ops = lay.take(sizeof(PhasorOp) * std::max<size_t>(tops.size(), 1));
+  const size_t o_max = lay.take(sizeof(MaxOp) * std::max<size_t>(maxes.size(), 1));
+  const size_t o_top = lay.take(sizeof(TableOp) * std::max<size_t>(tables.ops.size(), 1));
   const size_t o_wf = lay.take(sizeof(Work) * std::max<size_t>(wf.size(), 1));
   const size_t o_pf = lay.take(sizeof(Problem) * std::max<size_t>(plan->pf.size(), 1));
   // partial-overlap groups: each group's union box on the image (its Fields'
@@ -1671,33 +1942,54 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     return fail(ctx, MFTX_ENOMEM, "plan workspace allocation of " + std::to_string(lay.total) + " bytes failed");
   }
   char* base = (char*)plan->ws;
-  for (auto& pt : patch1) {
-    p1[pt.idx].a = base + pt.a;
-    p1[pt.idx].dst = base + pt.dst;
+  for (size_t t = 0; t < tables.ops.size(); ++t) tables.ops[t].dst = base + tables.off[t];
+  for (size_t i = 0; i < segs.size(); ++i) {
+    segs[i].a = base + refs[i].a;
+    segs[i].b = base + tables.off[refs[i].table];
+    segs[i].b_nkb = tables.ops[refs[i].table].nkb;
   }
-  for (auto& pt : patch2_launch) {
-    p2_launch[pt.idx].a = base + pt.a;
-    p2_launch[pt.idx].dst = pt.dst ? (void*)(base + pt.dst) : nullptr;
-  }
-  for (auto& pt : patch2c_launch) {
-    p2c_launch[pt.idx].a = base + pt.a;
-    p2c_launch[pt.idx].dst = base + pt.dst;
-  }
+  auto rebase = [&](std::vector<Problem>& ps, const std::vector<Patch>& patches) {
+    for (size_t i = 0; i < ps.size(); ++i) {
+      ps[i].dst = patches[i].dst ? (void*)(base + patches[i].dst) : nullptr;
+      ps[i].inv = patches[i].inv ? (const float*)(base + patches[i].inv) : nullptr;
+    }
+  };
+  rebase(p1, patch1);
+  rebase(p2_launch, patch2_launch);
+  rebase(p2c_launch, patch2c_launch);
   for (auto& w : w2)
     if (w.partial) w.partial = (float*)(base + (size_t)(uintptr_t)w.partial);
-  for (size_t c = 0; c < cls.size(); ++c) plan->pf[c].a = base + patch2[cls[c].p2].a;
+  {
+    float2* rp = (float2*)(base + o_rowph);
+    for (size_t c = 0; c < cls.size(); ++c) {
+      Problem& q = plan->pf[c];
+      const Patch& pt = patch2[cls[c].p2];
+      q.dst = nullptr;
+      q.wmap = nullptr;
+      q.inv = pt.inv ? (const float*)(base + pt.inv) : nullptr;
+      plan->field_scale.push_back(stage2_scale(prec, cls[c].pairs1));
+      if (row_phases[c].rows) {
+        row_phases[c].table = rp;
+        q.rowph = rp;
+        rp += row_phases[c].rows;
+        plan->max_rows = std::max(plan->max_rows, row_phases[c].rows);
+      }
+    }
+    plan->row_phases = (RowPhase*)(base + o_rpops);
+  }
   std::vector<PhasorWave> iw(wave_slots.size());
   for (size_t i = 0; i < wave_slots.size(); ++i) {
     const Slot& sl = wave_slots[i];
     iw[i] = PhasorWave{1.0 / wavelengths[std::get<0>(sl)], std::get<1>(sl), std::get<2>(sl), std::get<3>(sl),
                        std::get<4>(sl)};
   }
+  for (size_t i = 0; i < maxes.size(); ++i) maxes[i].part = (float*)(base + max_part[i]);
 
   plan->works1 = (Work*)(base + o_w1);
   plan->works2 = (Work*)(base + o_w2);
   plan->probs1 = (Problem*)(base + o_p1);
   plan->probs2 = (Problem*)(base + o_p2);
-  plan->chunk_x = (double*)(base + o_cx);
+  plan->segs = (Seg*)(base + o_segs);
   plan->waves = (PhasorWave*)(base + o_iw);
   plan->nwork1 = (int)w1.size();
   plan->nwork2 = (int)w2.size();
@@ -1707,6 +1999,9 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   plan->works_f = (Work*)(base + o_wf);
   plan->probs_f = (Problem*)(base + o_pf);
   plan->nwork_f = (int)wf.size();
+  plan->max_ops = (MaxOp*)(base + o_max);
+  plan->n_max_ops = (int)maxes.size();
+  plan->max_blocks = max_total;
   hipError_t e = hipSuccess;
   auto up = [&](void* d, const void* s, size_t n) {
     if (e == hipSuccess && n) e = hipMemcpy(d, s, n, hipMemcpyHostToDevice);
@@ -1717,9 +2012,14 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   up(plan->probs2, p2_launch.data(), sizeof(Problem) * p2_launch.size());
   up(plan->works2c, w2c.data(), sizeof(Work) * w2c.size());
   up(plan->probs2c, p2c_launch.data(), sizeof(Problem) * p2c_launch.size());
-  up(plan->chunk_x, cx.data(), sizeof(double) * cx.size());
+  up(plan->segs, segs.data(), sizeof(Seg) * segs.size());
   up(plan->waves, iw.data(), sizeof(PhasorWave) * iw.size());
+  up(plan->row_phases, row_phases.data(), sizeof(RowPhase) * row_phases.size());
+  up(plan->max_ops, maxes.data(), sizeof(MaxOp) * maxes.size());
   up(plan->works_f, wf.data(), sizeof(Work) * wf.size());
+  up(base + o_top, tables.ops.data(), sizeof(TableOp) * tables.ops.size());
+  if (e == hipSuccess)  // the twiddle tables, once for the plan's life
+    e = launch_tables(prec, (const TableOp*)(base + o_top), (int)tables.ops.size(), tables.threads, ctx->stream);
   if (e != hipSuccess) {
     return hipfail(ctx, e, "plan descriptor upload");
   }
@@ -1742,11 +2042,13 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     ph.nwave = op.nslot;
     ph.waves = plan->waves + op.wave_off;
     ph.dst = base + op.off;
-    ph.wave_stride = (long long)packed_bytes(prec, op.rows, op.kpad);
-    ph.rows_pad = op.rows;
-    ph.kpad = op.kpad;
+    ph.wave_stride = (long long)folded_bytes(op.R, op.K);
+    if (prec == PREC_FP32) {
+      const Comp& cm = comps[root(kv.first.first)];
+      ph.sc = ScaleSrc{(const float*)(base + cm.part), (float*)(base + cm.inv), cm.n, 0};
+    }
     ph.begin = group_begin(pthreads);
-    pthreads = ph.begin + phasor_threads(ph.rows_pad, ph.kpad, ph.nwave);
+    pthreads = ph.begin + phasor_threads(op.R, op.K, ph.nwave);
     ops.push_back(ph);
   }
   plan->phasor_ops = (PhasorOp*)(base + o_ops);
@@ -1799,7 +2101,8 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   plan->info.mfma_flops[1] = mf2;
   double bytes = 0;
   for (auto& ph : ops) bytes += 2.0 * (double)ph.wave_stride * ph.nwave;  // write + read
-  for (auto& c : cls) bytes += 2.0 * packed_bytes(prec, c.rows2, c.ktot);
+  for (auto& c : cls)
+    for (int k : c.nkb) bytes += 2.0 * (double)c.rblocks2 * k * A_BLOCK;
   bytes += 4.0 * image_rows * image_cols;
   plan->info.bytes_hbm_min = bytes;
   double bph = 0, bre = 0;
@@ -1818,7 +2121,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   plan->info.n_stage2 = (int)cls.size();
   plan->info.n_work1 = plan->nwork1;
   plan->info.n_work2 = plan->nwork2 + plan->nwork2c;
-  int nl = (ops.empty() ? 0 : 1) + 1 + (w2.empty() ? 0 : 1) + (w2c.empty() ? 0 : 1) + (int)plan->reduces.size();
+  int nl = (maxes.empty() ? 0 : 1) + (ops.empty() ? 0 : 1) + 1 + (w2.empty() ? 0 : 1) + (w2c.empty() ? 0 : 1) + (int)plan->reduces.size();
   for (auto& fb : plan->fallbacks) nl += 2 + (int)fb.adds.size();  // clear, adds, |.|^2 into the image
   plan->info.n_launch = nl;
   *out = owned.release();
@@ -1829,7 +2132,9 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
 }  // extern "C"
 
 static hipError_t launch_phasors(const mftx_plan* plan, hipStream_t s) {
-  return launch_phasor_group(plan->prec, plan->phasor_ops, plan->n_phasor_ops, plan->phasor_threads, s);
+  const hipError_t e = launch_absmax(plan->max_ops, plan->n_max_ops, plan->max_blocks, s);
+  if (e != hipSuccess) return e;
+  return launch_operands(plan->prec, false, plan->phasor_ops, plan->n_phasor_ops, plan->phasor_threads, s);
 }
 
 static hipError_t launch_reduces(const mftx_plan* plan, void* image, int dtype, int64_t ldi, int accumulate,
@@ -1882,9 +2187,9 @@ static hipError_t launch_fallbacks(const mftx_plan* plan, void* image, int dtype
 static hipError_t launch_stage2(const mftx_plan* plan, hipStream_t s) {
   hipError_t e = hipSuccess;
   if (plan->nwork2)
-    e = launch_gemm(plan->prec, EPI_INTENSITY, plan->bn, plan->works2, plan->nwork2, plan->probs2, plan->chunk_x, s);
+    e = launch_gemm(plan->prec, EPI_INTENSITY, plan->tile2, plan->works2, plan->nwork2, plan->probs2, plan->segs, s);
   if (e == hipSuccess && plan->nwork2c)
-    e = launch_gemm(plan->prec, EPI_STORE_CPLX, plan->bn, plan->works2c, plan->nwork2c, plan->probs2c, plan->chunk_x,
+    e = launch_gemm(plan->prec, EPI_STORE_CPLX, plan->tile2c, plan->works2c, plan->nwork2c, plan->probs2c, plan->segs,
                     s);
   return e;
 }
@@ -1907,7 +2212,7 @@ static int plan_launch(mftx_plan* plan, void* image, int dtype, int64_t ldi, int
   mftx_ctx* ctx = plan->ctx;
   hipStream_t s = ctx->stream;
   HIPCHK(ctx, launch_phasors(plan, s));
-  HIPCHK(ctx, launch_gemm(plan->prec, EPI_STORE_PACKED_T, plan->bn, plan->works1, plan->nwork1, plan->probs1, plan->chunk_x, s));
+  HIPCHK(ctx, launch_gemm(plan->prec, EPI_STORE_PACKED, plan->tile1, plan->works1, plan->nwork1, plan->probs1, plan->segs, s));
   HIPCHK(ctx, launch_stage2(plan, s));
   HIPCHK(ctx, launch_finish(plan, image, dtype, ldi, accumulate, s));
   return MFTX_OK;
@@ -1968,7 +2273,7 @@ static hipError_t profile_launches(mftx_plan* plan, void* image, int dtype, int6
   for (int k = 0; k < upto && e == hipSuccess; ++k) {
     if (k == 0) e = launch_phasors(plan, s);
     if (k == 1)
-      e = launch_gemm(plan->prec, EPI_STORE_PACKED_T, plan->bn, plan->works1, plan->nwork1, plan->probs1, plan->chunk_x,
+      e = launch_gemm(plan->prec, EPI_STORE_PACKED, plan->tile1, plan->works1, plan->nwork1, plan->probs1, plan->segs,
                       s);
     if (k == 2) e = launch_stage2(plan, s);
     if (k == 3) e = launch_finish(plan, image, dtype, ldi, 0, s);
@@ -2095,12 +2400,14 @@ int mftx_plan_set_fields(mftx_plan* plan, void* const* dst, int64_t ldd, const v
       q.wmap = wmap ? wmap[i] : nullptr;
       q.wdtype = wmap_dtype;
       q.ldw = ldw;
-      q.scale = (float)scale[i];
+      q.scale = (float)(scale[i] * plan->field_scale[c]);
     }
     HIPCHK(ctx, hipSetDevice(ctx->device));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     if (!plan->pf.empty())
       HIPCHK(ctx, hipMemcpy(plan->probs_f, plan->pf.data(), sizeof(Problem) * plan->pf.size(), hipMemcpyHostToDevice));
+    if (!plan->fields_ready)  // once: the phases stage 1 leaves out
+      HIPCHK(ctx, launch_row_phases(plan->row_phases, (int)plan->pf.size(), plan->max_rows, ctx->stream));
     plan->fields_ready = 1;
     return MFTX_OK;
   });
@@ -2111,8 +2418,8 @@ int mftx_plan_execute_fields(mftx_plan* plan) {
   mftx_ctx* ctx = plan->ctx;
   if (!plan->fields_ready) return fail(ctx, MFTX_EINVAL, "mftx_plan_set_fields has not been called");
   HIPCHK(ctx, hipSetDevice(ctx->device));
-  HIPCHK(ctx, launch_gemm(plan->prec, EPI_STORE_CPLX, plan->bn, plan->works_f, plan->nwork_f, plan->probs_f,
-                          plan->chunk_x, ctx->stream));
+  HIPCHK(ctx, launch_gemm(plan->prec, EPI_STORE_CPLX, plan->tile_f, plan->works_f, plan->nwork_f, plan->probs_f,
+                          plan->segs, ctx->stream));
   return MFTX_OK;
 }
 

@@ -6,6 +6,8 @@ namespace mftx {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
 typedef float v4f32 __attribute__((ext_vector_type(4)));
@@ -71,14 +73,27 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
 }
 __device__ __forceinline__ float bf16_lo_to_f32(uint32_t u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float bf16_hi_to_f32(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
+__device__ __forceinline__ uint32_t pack_f16(float a, float b) {
+  f16x2_t v = {(_Float16)a, (_Float16)b};
+  return __builtin_bit_cast(uint32_t, v);
+}
 
-// Split two floats into (hi pair, lo pair) with x = hi + lo + O(2^-17 |x|).
-// (The empty asm keeps the compiler from looking through the pack, where it
-// would convert a to bf16 a second time instead of shifting the pair.)
+// Split two floats into (hi pair, lo pair): x = hi + lo + O(2^-17 |x|) for
+// bf16, O(2^-22 |x|) for f16.  (The empty asm keeps the compiler from looking
+// through the pack, where it would convert a a second time instead of
+// widening the pair.)
+template <int PREC>
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
-  hi = pack_bf16(a, b);
-  asm("" : "+v"(hi));
-  lo = pack_bf16(a - bf16_lo_to_f32(hi), b - bf16_hi_to_f32(hi));
+  if constexpr (PREC == PREC_BF16X3) {
+    hi = pack_bf16(a, b);
+    asm("" : "+v"(hi));
+    lo = pack_bf16(a - bf16_lo_to_f32(hi), b - bf16_hi_to_f32(hi));
+  } else {
+    hi = pack_f16(a, b);
+    asm("" : "+v"(hi));
+    const f16x2_t h = __builtin_bit_cast(f16x2_t, hi);
+    lo = pack_f16(a - (float)h.x, b - (float)h.y);
+  }
 }
 
 }  // namespace mftx

@@ -1,270 +1,63 @@
 // Complex x twiddle GEMM of the two MFT stages on gfx950 MFMA.
 //
-// A is data in HBM (packed, see mftx_internal.h); the twiddles
-// cis(alpha * x_k * Y_s) are generated on the fly into LDS:
-//     stage 1:  G   = f   . E2      (stored transposed, packed, as G^T)
+//     stage 1:  G   = f   . E2      (stored as the operand of stage 2, G^T)
 //     stage 2:  F^T = G^T . E1^T    (|F|^2 accumulated, or F stored)
 // which is the triple product of lentil fourier.py:97 with the twiddles of
-// fourier.py:108-109.
+// fourier.py:108-109, both coordinates paired (Problem in mftx_internal.h):
+// P = Ae cos, Q = Ao sin over K/2 pairs and N/2 slots, a quarter of the real
+// products of the direct complex product.  Ae and Ao (the operand's two
+// parts) and the cos and sin tables are split into hi and lo 16-bit planes and
+// stored as MFMA fragments; a real product is hi*hi + hi*lo + lo*hi on
+// v_mfma_f32_32x32x16 with FP32 accumulation.
 //
-// Centred output grid.  With the shift folded into A by its producer, each
-// stage is C[i][j] = sum_k A'[i][k] cis(alpha x_k Y_j) with Y symmetric about
-// 0, so one GEMM over the slots Y_s >= 0 with the real twiddle matrices
-// cos and sin gives P = A' cos, Q = A' sin and both output columns
-// C(+Y_s) = P + iQ and C(-Y_s) = P - iQ: half the MFMAs and half the
-// twiddles of the direct complex product.
+// One 32-row x 32-slot block of C and 16 pairs of K are 12 MFMAs: accumulators
+// P_re, P_im += (re, im of Ae) cos and Q_re, Q_im += (re, im of Ao) sin.
 //
-// Workgroup: 4 x WN waves, each wave a 32-row x 32-slot block (two output
-// columns per slot) with accumulators P_re, P_im, Q_re, Q_im; C tile 128 rows
-// x 32 WN slots.  K runs in chunks of 16 KS staged in double-buffered LDS, one
-// barrier per chunk.  Two configurations:
-//   WN = 1, KS = 1: 32 slots (64 output columns), 40 KiB LDS, two workgroups per CU;
-//   WN = 2, KS = 2: 64 slots (128 output columns), 32-wide K chunks, 96 KiB LDS,
-//                   one workgroup (8 waves) per CU.
-// Two chunks ahead, in one of two register sets that alternate by chunk, each
-// thread stages A items (32 bytes of one row: a BF16 plane or four complex64
-// values; global -> registers -> LDS) and generates 2 KS consecutive twiddles
-// of one slot, t_i = P * Q_i with P = cis(alpha * x * Y) (FP64 argument and
-// range reduction, FP32 sin/cos) per chunk and the per-problem table
-// Q_i = cis(alpha * i * Y).  The compiler schedules the loop (the twiddle VALU
-// work lands after the chunk's barrier, next to the LDS stores that use it;
-// scheduling hints and hand-threading it between the MFMAs measured no better).
+// TILE_BIG and TILE_MID (gemm_tile_kernel): workgroups of WR x WC waves, each
+// wave one 32-row block by S 32-slot blocks.  Operand and twiddle blocks of a
+// K block ("chunk") go straight from global memory into one of three LDS
+// stages (global_load_lds_dwordx4), two chunks ahead, one barrier per chunk:
+//   BIG: 4 x 2 waves, S = 2: 128 rows x 128 slots (256 output columns), 48 KiB
+//        per stage, one workgroup (two waves per SIMD) per CU;
+//   MID: 2 x 2 waves, S = 1: 64 rows x 64 slots, 24 KiB per stage, two
+//        workgroups per CU (TILE_MULTI: the same, for problems of several
+//        K segments).
+// What bounds them: the matrix pipe at the clock the power management allows
+// (a BIG chunk is 1536 MFMA cycles per SIMD against 128 KiB of fragment reads
+// and 48 KiB of LDS writes, 115 B per cycle of a 256 B/cycle read path).  S = 2
+// because a wave's operand fragments then feed two slot blocks: 16 fragment
+// reads per 24 MFMAs and 48 KiB of loads, where S = 1 takes 12 per 12 and 40.
 //
-// Precision forms
-//   PREC_FP32   : complex64 A, v_mfma_f32_32x32x2_f32: 4 real MFMAs per
-//                 (A element, twiddle) pair.
-//   PREC_BF16X3 : every FP32 operand x is split x = hi + lo (two BF16, round
-//                 to nearest even); a real product is hi*hi + hi*lo + lo*hi on
-//                 v_mfma_f32_32x32x16_bf16 with FP32 accumulation, 12 MFMAs per
-//                 32x32 slot block and 16-wide K step.
+// Measured on the 512^2 -> 1024^2 sweep of 64 wavelengths (bf16 pairs): stage 1
+// 128 us, stage 2 157 us = 1.31 PFLOP/s of executed products, the rate of a
+// large library GEMM on this card (1.28); 187 and 318 us when the sums ran over
+// all K samples with twiddles generated in the kernel.  Two workgroups per CU
+// of 64 rows x 128 slots were slower (157 and 176 us): the operand is then
+// loaded 1.33 times as often per product.
+//
+// TILE_SMALL (gemm_small_kernel): four waves split the K blocks of one 32 x 32
+// block between them, load fragments straight into registers and add their
+// sums through LDS.  For single transforms, whose few tiles would leave most
+// of the chip idle: the time is latency, and it is a quarter of the K loop.
 #include "mftx_device.h"
 
 namespace mftx {
 
-// Geometry of one tile configuration.
-template <int WN, int KS> struct Cfg {
-  static constexpr int BS = 32 * WN;               // slots per workgroup
-  static constexpr int BKC = 16 * KS;              // K per chunk
-  static constexpr int NT = 64 * WAVES_M * WN;     // threads per workgroup
-  static constexpr int A_ITEMS = 512 * KS / NT;    // A staging items per thread
-  static constexpr int TW = 2 * KS;                // twiddles per thread per chunk
-  static constexpr int WG_PER_CU = WN == 1 ? 2 : 1;
-  static_assert((512 * KS) % NT == 0, "A items must divide evenly");
-  static_assert(BS * BKC == NT * TW, "one twiddle item per thread");
+template <int PREC> struct Num;
+template <> struct Num<PREC_BF16X3> {
+  typedef bf16x8_t frag;
+  static __device__ __forceinline__ f32x16 mfma(frag a, frag b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+  }
+};
+template <> struct Num<PREC_FP32> {
+  typedef f16x8_t frag;
+  static __device__ __forceinline__ f32x16 mfma(frag a, frag b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+  }
 };
 
-template <int PREC, int WN, int KS> struct Lds;
-
-// bf16x3: 4 planes of [row][16 KS] bf16 (A: re_hi, re_lo, im_hi, im_lo; B:
-// cos_hi, cos_lo, sin_hi, sin_lo), made of 16-byte units of 8 K values.  Units
-// are swizzled per row, unit' = unit ^ swz_key(row).  For KS = 2 (64-byte
-// rows) the key ((row >> 1) ^ (row >> 2)) & 3 keeps the 16-byte accesses of
-// 8 consecutive rows on distinct banks of a 32-bank (128-byte) LDS line and
-// those of 16 consecutive rows on distinct banks of a 64-bank line, so the
-// fragment reads and the A staging stores are conflict-free whichever way the
-// hardware groups the lanes of a 16-byte access (checked on the CPU for 8 and
-// 16 lanes per cycle); (row >> 2) & 3 was conflict-free only for 16.
-template <int WN, int KS> struct Lds<PREC_BF16X3, WN, KS> {
-  __bf16 a[2][4][BM][16 * KS];
-  __bf16 b[2][4][Cfg<WN, KS>::BS][16 * KS];
-};
-template <int KS> __device__ __forceinline__ int swz_key(int row) {
-  return KS == 1 ? (row >> 3) & 1 : ((row >> 1) ^ (row >> 2)) & 3;
-}
-// element offset of logical unit u of a row
-template <int KS> __device__ __forceinline__ int swz(int row, int u) { return 8 * (u ^ swz_key<KS>(row)); }
-
-// fp32: complex64 [row][BKC + 2] (B: (cos, sin) pairs); the padded row stride
-// keeps the 16-byte stores of 16 consecutive rows and the 8-byte fragment
-// reads on distinct banks.
-template <int WN, int KS> struct Lds<PREC_FP32, WN, KS> {
-  static constexpr int RS = 16 * KS + 2;
-  float2 a[2][BM][RS];
-  float2 b[2][Cfg<WN, KS>::BS][RS];
-};
-
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(1))) const u32x4 gu32x4;  // global-memory view
-
-// A staging: 512 KS items of 32 bytes per chunk (128 rows x 4 parts x KS
-// 16-wide K steps; a part is a BF16 plane or four complex64 values).  Item i
-// is row (i & 15) + 16 ((i >> 6) & 7), part (i >> 4) & 3, K step i >> 9, so
-// 16 consecutive lanes store 16 consecutive rows of one part (conflict-free
-// LDS stores).  Thread t stages items t + j * NT.
-// B generation: BS x 8 items (slot, group of TW K values), one per thread.
-// KS = 1: slot (t & 15) + 16 (t >> 7), group (t >> 4) & 7.  KS = 2 (8-byte
-// stores of 4 K values): lane l of wave w takes slot (l & 7) + 8 ((l >> 4) & 1)
-// + 16 (w >> 1) and group ((l >> 3) & 1) + 2 ((l >> 5) & 1) + 4 (w & 1), so 16
-// consecutive lanes store 8 slots x the two halves of one 16-byte unit: 128
-// bytes on distinct banks (and 32 lanes 256 bytes), with the KS = 2 key.
-__device__ __forceinline__ int item_row(int i) { return (i & 15) + 16 * ((i >> 6) & 7); }
-__device__ __forceinline__ int item_part(int i) { return (i >> 4) & 3; }
-__device__ __forceinline__ int item_kstep(int i) { return i >> 9; }
-template <int KS> __device__ __forceinline__ int bitem_slot(int t) {
-  if (KS == 1) return (t & 15) + 16 * (t >> 7);
-  const int l = t & 63;
-  return (l & 7) + 8 * ((l >> 4) & 1) + 16 * (t >> 7);
-}
-template <int KS> __device__ __forceinline__ int bitem_group(int t) {
-  if (KS == 1) return (t >> 4) & 7;
-  const int l = t & 63;
-  return ((l >> 3) & 1) + 2 * ((l >> 5) & 1) + 4 * ((t >> 6) & 1);
-}
-
-// Staged chunk in registers: A prefetch and the generated twiddles.
-// bf16x3: b[p] holds plane p of the TW K values (TW / 2 words); fp32: the TW
-// (cos, sin) pairs, two per 16 bytes.  Native vector types keep these in VGPRs.
-template <int WN, int KS> struct Staged {
-  u32x4 a[Cfg<WN, KS>::A_ITEMS][2];
-  u32x4 b[4];
-};
-
-// Per-problem staging parameters (uniform) and the per-thread Q table.
-struct StageProb {
-  const char* a;
-  long long lda;
-  double alpha4;   // 4 * alpha: twiddle arguments in quarter turns
-  double y;        // Y of this thread's slot
-  int nch;         // chunks in the problem
-  int cb;          // chunk_begin (index of the problem's first 16-wide K block in chunk_x)
-};
-
-template <int KS, int NQ>
-__device__ __forceinline__ void set_stage(const Problem& P, int slot, StageProb& sp, float2 (&q)[NQ]) {
-  sp.a = (const char*)P.a;
-  sp.lda = P.lda;
-  sp.alpha4 = 4.0 * P.alpha;
-  sp.y = P.y0 + (double)slot;
-  sp.nch = P.kpad / (16 * KS);
-  sp.cb = P.chunk_begin;
-#pragma unroll
-  for (int i = 0; i < NQ; ++i) q[i] = cis_quarter(sp.alpha4 * ((double)i * sp.y));
-}
-
-// x of the first twiddle of group g of chunk c (chunk_x holds one origin per
-// 16-wide K block).  The block origins are read at a wave-uniform address
-// (scalar loads through the scalar cache) and selected per lane: a per-lane
-// index would make this a vector load whose latency sits on every chunk's
-// critical path.
-__device__ __forceinline__ double uniform_double(const double* p) {
-  const long long b = *(const long long*)p;
-  const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-template <int KS>
-__device__ __forceinline__ double twiddle_x(const double* __restrict__ chunk_x, const StageProb& sp, int c, int g) {
-  const int k = 2 * KS * g;
-  const double* px = chunk_x + __builtin_amdgcn_readfirstlane(sp.cb + KS * c);  // uniform by construction
-  const double x0 = uniform_double(px);
-  const double xb = KS == 2 ? ((k >> 4) ? uniform_double(px + 1) : x0) : x0;
-  return xb + (double)(k & 15);
-}
-
-template <int PREC, int WN, int KS>
-__device__ __forceinline__ void load_a(const StageProb& sp, long long row0, int tid, int chunk,
-                                       Staged<WN, KS>& st) {
-#pragma unroll
-  for (int j = 0; j < Cfg<WN, KS>::A_ITEMS; ++j) {
-    const int it = tid + j * Cfg<WN, KS>::NT;
-    const long long row = row0 + item_row(it);
-    const long long blk = (long long)chunk * KS + item_kstep(it);  // 16-wide K block
-    gu32x4* src;
-    if (PREC == PREC_BF16X3)
-      src = (gu32x4*)((const __bf16*)sp.a + row * sp.lda + blk * 64 + item_part(it) * 16);
-    else
-      src = (gu32x4*)((const float2*)sp.a + row * sp.lda + blk * 16 + item_part(it) * 4);
-    st.a[j][0] = src[0];
-    st.a[j][1] = src[1];
-  }
-}
-
-// TW consecutive twiddles from K origin x for this thread's slot.
-template <int PREC, int WN, int KS>
-__device__ __forceinline__ void gen_b(double x, const StageProb& sp, const float2 (&q)[2 * KS],
-                                      Staged<WN, KS>& st) {
-  constexpr int TW = 2 * KS;
-  const float2 pf = cis_quarter(sp.alpha4 * (x * sp.y));
-  float2 t[TW];
-#pragma unroll
-  for (int i = 0; i < TW; ++i) t[i] = cmul(pf, q[i]);
-  if (PREC == PREC_BF16X3) {
-    uint32_t ch[2] = {}, cl[2] = {}, sh[2] = {}, sl[2] = {};
-#pragma unroll
-    for (int i = 0; i < TW / 2; ++i) {
-      split2(t[2 * i].x, t[2 * i + 1].x, ch[i], cl[i]);
-      split2(t[2 * i].y, t[2 * i + 1].y, sh[i], sl[i]);
-    }
-    st.b[0] = u32x4{ch[0], ch[1], 0u, 0u};
-    st.b[1] = u32x4{cl[0], cl[1], 0u, 0u};
-    st.b[2] = u32x4{sh[0], sh[1], 0u, 0u};
-    st.b[3] = u32x4{sl[0], sl[1], 0u, 0u};
-  } else {
-    auto bits = [](float v) { return __float_as_uint(v); };
-#pragma unroll
-    for (int i = 0; i < TW / 2; ++i)
-      st.b[i] = u32x4{bits(t[2 * i].x), bits(t[2 * i].y), bits(t[2 * i + 1].x), bits(t[2 * i + 1].y)};
-  }
-}
-
-template <int PREC, int WN, int KS>
-__device__ __forceinline__ void write_b(Lds<PREC, WN, KS>& L, int buf, int slot, int g, const Staged<WN, KS>& st) {
-  constexpr int TW = 2 * KS;
-  if (PREC == PREC_BF16X3) {
-    auto& LB = reinterpret_cast<Lds<PREC_BF16X3, WN, KS>&>(L);
-    const int k = TW * g;  // first K of the group: unit k / 8, offset k % 8
-    const int e = swz<KS>(slot, k >> 3) + (k & 7);
-    if (KS == 1) {
-#pragma unroll
-      for (int p = 0; p < 4; ++p) *(uint32_t*)&LB.b[buf][p][slot][e] = st.b[p][0];
-    } else {
-#pragma unroll
-      for (int p = 0; p < 4; ++p) *(u32x2*)&LB.b[buf][p][slot][e] = u32x2{st.b[p][0], st.b[p][1]};
-    }
-  } else {
-    auto& LF = reinterpret_cast<Lds<PREC_FP32, WN, KS>&>(L);
-    u32x4* b = (u32x4*)&LF.b[buf][slot][g * TW];
-#pragma unroll
-    for (int i = 0; i < TW / 2; ++i) b[i] = st.b[i];
-  }
-}
-
-template <int PREC, int WN, int KS>
-__device__ __forceinline__ void write_a(Lds<PREC, WN, KS>& L, int buf, int tid, const Staged<WN, KS>& st) {
-#pragma unroll
-  for (int j = 0; j < Cfg<WN, KS>::A_ITEMS; ++j) {
-    const int it = tid + j * Cfg<WN, KS>::NT;
-    const int row = item_row(it), part = item_part(it), ks = item_kstep(it);
-    if (PREC == PREC_BF16X3) {
-      auto& LB = reinterpret_cast<Lds<PREC_BF16X3, WN, KS>&>(L);
-      *(u32x4*)&LB.a[buf][part][row][swz<KS>(row, 2 * ks)] = st.a[j][0];
-      *(u32x4*)&LB.a[buf][part][row][swz<KS>(row, 2 * ks + 1)] = st.a[j][1];
-    } else {
-      auto& LF = reinterpret_cast<Lds<PREC_FP32, WN, KS>&>(L);
-      u32x4* a = (u32x4*)&LF.a[buf][row][16 * ks + part * 4];
-      a[0] = st.a[j][0];
-      a[1] = st.a[j][1];
-    }
-  }
-}
-
-#define MFMA_BF16(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16((a), (b), (c), 0, 0, 0)
-
-// One 32x32 slot block, K = 16: P += A cos, Q += A sin for A = (re, im), each
-// real product as hi*hi + hi*lo + lo*hi.  a: planes (re_hi, re_lo, im_hi,
-// im_lo); b: planes (cos_hi, cos_lo, sin_hi, sin_lo).  acc: P_re, P_im, Q_re, Q_im.
-__device__ __forceinline__ void sblock_bf16(const bf16x8_t (&a)[4], const bf16x8_t (&b)[4], f32x16 (&acc)[4]) {
-#pragma unroll
-  for (int t = 0; t < 3; ++t) {
-    const int ia = t == 2 ? 1 : 0;   // hi, hi, lo  of A
-    const int ib = t == 1 ? 1 : 0;   // hi, lo, hi  of the twiddle
-    acc[0] = MFMA_BF16(a[ia], b[ib], acc[0]);
-    acc[1] = MFMA_BF16(a[2 + ia], b[ib], acc[1]);
-    acc[2] = MFMA_BF16(a[ia], b[2 + ib], acc[2]);
-    acc[3] = MFMA_BF16(a[2 + ia], b[2 + ib], acc[3]);
-  }
-}
+typedef __attribute__((address_space(3))) void lds_void;
 
 // Weight-map values at map offsets idx[0..n-1] (1 without a map).  No load
 // sits behind a branch, so they are in flight together.
@@ -282,764 +75,604 @@ __device__ __forceinline__ void load_weights(const Problem& P, const long long (
   }
 }
 
-// End of one problem.  Accumulator element e of a lane is C row
-// 8 (e / 4) + 4 (lane / 32) + e % 4 of its 32-row block and slot lane % 32;
-// the slot's two output columns are jp = cp + s (P + iQ) and jm = cm - s
-// (P - iQ).  Intensity accumulates w |C|^2 for both in registers; the store
-// forms write C * scale (complex, or packed transposed as the next stage's A';
-// the next stage's fold is already in C, from the phase of this stage's
-// operand rows).
+// A lane's (cos, sin) of the store's output phase for its slot: column cp + s
+// turns by (c, s), column cm - s by (c, -s).
+__device__ __forceinline__ float2 slot_phase(const Problem& P, int slot) {
+  return P.xrot != 0.0 ? cis_turns(P.xrot * (P.y0 + (double)slot)) : make_float2(1.0f, 0.0f);
+}
+// (a scalar load: a vector load's wait would drain the operand loads in flight)
+__device__ __forceinline__ float store_scale(const Problem& P) {
+  return P.inv ? P.scale * *(cptr<const float>)P.inv : P.scale;
+}
+
+// Store one side (0: column cp + s from P + iQ, 1: cm - s from P - iQ) of half
+// h of a 32 x 32 block: this lane's slot and the 8 rows 16 h + 8 g + 4 (lane /
+// 32) + e, g = 0, 1, e = 0 .. 3 of row block rb; re, im hold them unscaled.
+//
+// Lane l holds rows 0-3 and 8-11 of the 16, lane l + 32 rows 4-7 and 12-15.
+// One lane swap per word (v_permlane32_swap: the high half of the first
+// operand trades places with the low half of the second) gives lane l rows 0-7
+// and lane l + 32 rows 8-15, so a lane stores 16-byte pieces.
 template <int PREC, int EPI>
-__device__ __forceinline__ void problem_epilogue(const Problem& P, const Work& wk, int BS, int wr, int wc, int lane,
-                                                 const f32x16 (&acc)[4], f32x16 (&ip), f32x16 (&im)) {
-  const int s = wk.tc * BS + wc * 32 + (lane & 31);
-  const int N = P.ncols;
-  const int jp = P.cp + s, jm = P.cm - s;
-  if (EPI == EPI_INTENSITY) {
-    const float w = P.scale;
+__device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int side, int slot, int lane, float sc,
+                                           float2 ph, float (&re)[8], float (&im)[8]) {
+  const int j = side ? P.cm - slot : P.cp + slot;
+  const bool has = side ? (j >= 0 && j < P.ncols && j != P.cp + slot) : j < P.ncols;
+  if (P.xrot != 0.0) {
+    const float ps = side ? -ph.y : ph.y;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float pr = acc[0][e], pi = acc[1][e], qr = acc[2][e], qi = acc[3][e];
-      const float ar = pr - qi, ai = pi + qr;   // P + iQ
-      const float br = pr + qi, bi = pi - qr;   // P - iQ
-      ip[e] = __builtin_fmaf(w, __builtin_fmaf(ar, ar, ai * ai), ip[e]);
-      im[e] = __builtin_fmaf(w, __builtin_fmaf(br, br, bi * bi), im[e]);
+    for (int q = 0; q < 8; ++q) {
+      const float2 v = cmul(make_float2(re[q], im[q]), make_float2(ph.x, ps));
+      re[q] = v.x;
+      im[q] = v.y;
     }
-    return;
   }
-  const float sc = P.scale;
-  const bool has_p = jp < N, has_m = jm >= 0 && jm < N && jm != jp;
-  // the first C row of this wave's block, opaque to the compiler: the
-  // indices below then stay in the epilogue instead of being hoisted out of
-  // the K loop and spilled
-  int rblk = wk.tr * BM + wr * 32;
-  asm volatile("" : "+v"(rblk));
-  if (EPI == EPI_STORE_CPLX && P.trans) {
-    // Transposed complex store: C row r of output column j goes to
-    // dst[j * ldd + r].  As for the packed store, one lane swap per word
-    // gives lane l rows 0-7 and lane l+32 rows 8-15 of each 16-row block, so
-    // a lane stores 64 contiguous bytes as 16-byte pieces.
+  // the block's first C row, opaque to the compiler: the row indices below
+  // stay in the epilogue instead of being hoisted out of the K loop and spilled
+  int row0 = rb * 32 + 16 * h;
+  asm volatile("" : "+v"(row0));
+  if (EPI == EPI_STORE_CPLX) {
+    if (P.rowph) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int row = row0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
+        const v2f32 r = ((gptr<const v2f32>)P.rowph)[row < P.rows ? row : 0];
+        const float2 v = cmul(make_float2(re[q], im[q]), make_float2(r.x, r.y));
+        re[q] = v.x;
+        im[q] = v.y;
+      }
+    }
     float2* dst = (float2*)P.dst;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      float v[2][2][8];  // [side][group of the pair][re, im of rows e = 0..3]
-#pragma unroll
-      for (int gg = 0; gg < 2; ++gg) {
-        const int g = 2 * h + gg;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float pr = acc[0][4 * g + e], pi = acc[1][4 * g + e], qr = acc[2][4 * g + e], qi = acc[3][4 * g + e];
-          v[0][gg][2 * e] = (pr - qi) * sc;
-          v[0][gg][2 * e + 1] = (pi + qr) * sc;
-          v[1][gg][2 * e] = (pr + qi) * sc;
-          v[1][gg][2 * e + 1] = (pi - qr) * sc;
-        }
-      }
-      const int r0 = rblk + 16 * h + 8 * (lane >> 5);  // first of this lane's 8 rows
-#pragma unroll
-      for (int side = 0; side < 2; ++side) {
-        float o[16];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[side][0][q]),
-                                                          __float_as_uint(v[side][1][q]), false, false);
-          o[q] = __uint_as_float(r[0]);
-          o[8 + q] = __uint_as_float(r[1]);
-        }
-        if (!(side ? has_m : has_p)) continue;
-        const int j = side ? jm : jp;
-        // rows past P.rows (not stored) read the column's row 0
-        long long wi[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) wi[t] = (long long)j * P.ldw + (r0 + t < P.rows ? r0 + t : 0);
-        float wv[8];
-        load_weights(P, wi, wv);
-        float2* d = dst + (long long)j * P.ldd + r0;
-        if (r0 + 8 <= P.rows && (((uintptr_t)d) & 15) == 0) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t)
-            ((gptr<v4f32>)d)[t] = v4f32{o[4 * t] * wv[2 * t], o[4 * t + 1] * wv[2 * t], o[4 * t + 2] * wv[2 * t + 1],
-                                        o[4 * t + 3] * wv[2 * t + 1]};
-        } else {
-#pragma unroll
-          for (int t = 0; t < 8; ++t)
-            if (r0 + t < P.rows) ((gptr<v2f32>)d)[t] = v2f32{o[2 * t] * wv[t], o[2 * t + 1] * wv[t]};
-        }
-      }
-    }
-    return;
-  }
-  if (EPI == EPI_STORE_PACKED_T && PREC == PREC_BF16X3) {
-    // Lane l holds K 0-3 (group 2h) and 8-11 (group 2h+1) of a 16-K block of
-    // its output row, lane l+32 K 4-7 and 12-15.  One lane swap per word
-    // (v_permlane32_swap: the high half of the first operand trades places
-    // with the low half of the second) gives lane l K 0-7 and lane l+32 K
-    // 8-15, so each lane stores 16 bytes of every plane.
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int kb = wk.tr * BM + wr * 32 + 16 * h;  // first K of the block (wave-uniform)
-      if (kb >= P.limit) continue;
-      uint32_t w[2][2][4][2];  // [group of the pair][side][plane][word]
-#pragma unroll
-      for (int gg = 0; gg < 2; ++gg) {
-        const int g = 2 * h + gg;
-        float v[2][2][4];  // [side][re, im][e]
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float pr = acc[0][4 * g + e], pi = acc[1][4 * g + e], qr = acc[2][4 * g + e], qi = acc[3][4 * g + e];
-          v[0][0][e] = (pr - qi) * sc;
-          v[0][1][e] = (pi + qr) * sc;
-          v[1][0][e] = (pr + qi) * sc;
-          v[1][1][e] = (pi - qr) * sc;
-        }
-#pragma unroll
-        for (int side = 0; side < 2; ++side) {
-          split2(v[side][0][0], v[side][0][1], w[gg][side][0][0], w[gg][side][1][0]);
-          split2(v[side][0][2], v[side][0][3], w[gg][side][0][1], w[gg][side][1][1]);
-          split2(v[side][1][0], v[side][1][1], w[gg][side][2][0], w[gg][side][3][0]);
-          split2(v[side][1][2], v[side][1][3], w[gg][side][2][1], w[gg][side][3][1]);
-        }
-      }
-#pragma unroll
-      for (int side = 0; side < 2; ++side) {
-        uint32_t o[4][4];
-#pragma unroll
-        for (int pl = 0; pl < 4; ++pl) {
-#pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            const auto r = __builtin_amdgcn_permlane32_swap(w[0][side][pl][q], w[1][side][pl][q], false, false);
-            o[pl][q] = r[0];
-            o[pl][2 + q] = r[1];
-          }
-        }
-        if (side ? has_m : has_p) {
-          __bf16* d = (__bf16*)P.dst + (long long)(side ? jm : jp) * P.ldd + (long long)(kb >> 4) * 64 + 8 * (lane >> 5);
-#pragma unroll
-          for (int pl = 0; pl < 4; ++pl)
-            *(gptr<v4u32>)(d + 16 * pl) = v4u32{o[pl][0], o[pl][1], o[pl][2], o[pl][3]};
-        }
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    // rows row0 .. row0+3 of C in this lane
-    const int row0 = rblk + 8 * g + 4 * (lane >> 5);
-    float pre[4], pim[4], mre[4], mim[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float pr = acc[0][4 * g + e], pi = acc[1][4 * g + e], qr = acc[2][4 * g + e], qi = acc[3][4 * g + e];
-      pre[e] = (pr - qi) * sc;
-      pim[e] = (pi + qr) * sc;
-      mre[e] = (pr + qi) * sc;
-      mim[e] = (pi - qr) * sc;
-    }
-    if (EPI == EPI_STORE_CPLX) {
-      float2* dst = (float2*)P.dst;
-      // optional real weight map, indexed like the destination; an element
-      // that is not stored reads the map's first value
+    if (!P.trans) {
       long long wi[8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = row0 + e;
-        const bool in = row < P.rows;
-        wi[e] = in && has_p ? (P.trans ? (long long)jp * P.ldw + row : (long long)row * P.ldw + jp) : 0;
-        wi[4 + e] = in && has_m ? (P.trans ? (long long)jm * P.ldw + row : (long long)row * P.ldw + jm) : 0;
+      for (int q = 0; q < 8; ++q) {
+        const int row = row0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
+        wi[q] = has && row < P.rows ? (long long)row * P.ldw + j : 0;
       }
       float wv[8];
       load_weights(P, wi, wv);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = row0 + e;
-        if (row < P.rows) {
-          if (has_p) {
-            const long long o = P.trans ? (long long)jp * P.ldd + row : (long long)row * P.ldd + jp;
-            ((gptr<v2f32>)dst)[o] = v2f32{pre[e] * wv[e], pim[e] * wv[e]};
-          }
-          if (has_m) {
-            const long long o = P.trans ? (long long)jm * P.ldd + row : (long long)row * P.ldd + jm;
-            ((gptr<v2f32>)dst)[o] = v2f32{mre[e] * wv[4 + e], mim[e] * wv[4 + e]};
-          }
-        }
+      for (int q = 0; q < 8; ++q) {
+        const int row = row0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
+        if (has && row < P.rows)
+          ((gptr<v2f32>)dst)[(long long)row * P.ldd + j] = v2f32{re[q] * sc * wv[q], im[q] * sc * wv[q]};
       }
-    } else if (row0 < P.limit) {  // EPI_STORE_PACKED_T: destination row = output column, K = C row
-#pragma unroll
-      for (int side = 0; side < 2; ++side) {
-        const int j = side ? jm : jp;
-        if (side ? !has_m : !has_p) continue;
-        const float* re = side ? mre : pre;
-        const float* imv = side ? mim : pim;
-        if (PREC == PREC_BF16X3) {
-          uint32_t rh0, rl0, rh1, rl1, ih0, il0, ih1, il1;
-          split2(re[0], re[1], rh0, rl0);
-          split2(re[2], re[3], rh1, rl1);
-          split2(imv[0], imv[1], ih0, il0);
-          split2(imv[2], imv[3], ih1, il1);
-          __bf16* d = (__bf16*)P.dst + (long long)j * P.ldd + (long long)(row0 >> 4) * 64 + (row0 & 15);
-          *(gptr<v2u32>)(d + 0) = v2u32{rh0, rh1};
-          *(gptr<v2u32>)(d + 16) = v2u32{rl0, rl1};
-          *(gptr<v2u32>)(d + 32) = v2u32{ih0, ih1};
-          *(gptr<v2u32>)(d + 48) = v2u32{il0, il1};
-        } else {
-          gptr<v4f32> d = (gptr<v4f32>)((float2*)P.dst + (long long)j * P.ldd + row0);
-          d[0] = v4f32{re[0], imv[0], re[1], imv[1]};
-          d[1] = v4f32{re[2], imv[2], re[3], imv[3]};
-        }
-      }
+      return;
     }
-  }
-}
-
-// The workgroup's summed intensity into its partial image (transposed like
-// the problems' trans flag), clipped to the partial extent.
-__device__ __forceinline__ void store_partial(const Work& wk, const Problem& P, int BS, int wr, int wc, int lane,
-                                              const f32x16& ip, const f32x16& im) {
-  const int s = wk.tc * BS + wc * 32 + (lane & 31);
-  const int jp = P.cp + s, jm = P.cm - s;
-  const bool has_p = jp < P.ncols, has_m = jm >= 0 && jm < P.ncols && jm != jp;
-  const int trans = P.trans;
-  if (trans) {
-    // C rows run along the partial's rows, and a lane's elements 4g .. 4g+3
-    // are 4 consecutive C rows: one aligned 16-byte store each (the partial
-    // and its row stride are multiples of 128 floats).  Rows past pcols
-    // land in the partial's padding columns, inside its allocation, which
-    // the reduction never reads.
+    float o[16];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int row = wk.tr * BM + wr * 32 + 8 * g + 4 * (lane >> 5);
-      if (has_p && jp < wk.prows)
-        *(gptr<v4f32>)&((gptr<float>)wk.partial)[(long long)jp * wk.ldp + row] =
-            v4f32{ip[4 * g], ip[4 * g + 1], ip[4 * g + 2], ip[4 * g + 3]};
-      if (has_m && jm < wk.prows)
-        *(gptr<v4f32>)&((gptr<float>)wk.partial)[(long long)jm * wk.ldp + row] =
-            v4f32{im[4 * g], im[4 * g + 1], im[4 * g + 2], im[4 * g + 3]};
+    for (int q = 0; q < 4; ++q) {
+      const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(re[q] * sc), __float_as_uint(re[4 + q] * sc),
+                                                      false, false);
+      const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(im[q] * sc), __float_as_uint(im[4 + q] * sc),
+                                                      false, false);
+      o[2 * q] = __uint_as_float(a[0]);
+      o[2 * q + 1] = __uint_as_float(b[0]);
+      o[8 + 2 * q] = __uint_as_float(a[1]);
+      o[9 + 2 * q] = __uint_as_float(b[1]);
+    }
+    if (!has) return;
+    const int r0 = row0 + 8 * (lane >> 5);  // first of this lane's 8 rows
+    long long wi[8];  // rows past P.rows (not stored) read the column's row 0
+#pragma unroll
+    for (int t = 0; t < 8; ++t) wi[t] = (long long)j * P.ldw + (r0 + t < P.rows ? r0 + t : 0);
+    float wv[8];
+    load_weights(P, wi, wv);
+    float2* d = dst + (long long)j * P.ldd + r0;
+    if (r0 + 8 <= P.rows && (((uintptr_t)d) & 15) == 0) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        ((gptr<v4f32>)d)[t] = v4f32{o[4 * t] * wv[2 * t], o[4 * t + 1] * wv[2 * t], o[4 * t + 2] * wv[2 * t + 1],
+                                    o[4 * t + 3] * wv[2 * t + 1]};
+    } else {
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        if (r0 + t < P.rows) ((gptr<v2f32>)d)[t] = v2f32{o[2 * t] * wv[t], o[2 * t + 1] * wv[t]};
     }
     return;
   }
+  // EPI_STORE_PACKED: row j of the next operand, K block rb, part h (the
+  // operand's rows come as 16 even and 16 odd rows per block)
+  uint32_t w[4][4];  // [plane][word]
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int row = wk.tr * BM + wr * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-    if (has_p) {
-      const int pr = trans ? jp : row, pc = trans ? row : jp;
-      if (pr < wk.prows && pc < wk.pcols) ((gptr<float>)wk.partial)[(long long)pr * wk.ldp + pc] = ip[e];
-    }
-    if (has_m) {
-      const int pr = trans ? jm : row, pc = trans ? row : jm;
-      if (pr < wk.prows && pc < wk.pcols) ((gptr<float>)wk.partial)[(long long)pr * wk.ldp + pc] = im[e];
+  for (int q = 0; q < 2; ++q) {
+    uint32_t rh0, rl0, rh1, rl1, ih0, il0, ih1, il1;
+    split2<PREC>(re[2 * q] * sc, re[2 * q + 1] * sc, rh0, rl0);
+    split2<PREC>(re[4 + 2 * q] * sc, re[5 + 2 * q] * sc, rh1, rl1);
+    split2<PREC>(im[2 * q] * sc, im[2 * q + 1] * sc, ih0, il0);
+    split2<PREC>(im[4 + 2 * q] * sc, im[5 + 2 * q] * sc, ih1, il1);
+    const auto a = __builtin_amdgcn_permlane32_swap(rh0, rh1, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(rl0, rl1, false, false);
+    const auto c = __builtin_amdgcn_permlane32_swap(ih0, ih1, false, false);
+    const auto d = __builtin_amdgcn_permlane32_swap(il0, il1, false, false);
+    w[0][q] = a[0];
+    w[0][2 + q] = a[1];
+    w[1][q] = b[0];
+    w[1][2 + q] = b[1];
+    w[2][q] = c[0];
+    w[2][2 + q] = c[1];
+    w[3][q] = d[0];
+    w[3][2 + q] = d[1];
+  }
+  if (!has) return;
+  char* d = (char*)P.dst + ((long long)(j >> 5) * P.ldd + (row0 >> 5)) * A_BLOCK + h * 4 * FRAG +
+            16 * ((j & 31) + 32 * (lane >> 5));
+#pragma unroll
+  for (int pl = 0; pl < 4; ++pl)
+    *(gptr<v4u32>)(d + pl * FRAG) = v4u32{w[pl][0], w[pl][1], w[pl][2], w[pl][3]};
+}
+
+// The summed intensity of one 32 x 32 block into the work item's partial image
+// (transposed like the problems' trans flag), clipped to the partial extent:
+// this lane's slot and C rows row0 + 8 g + 4 (lane / 32) + e for its NG groups.
+template <int NG>
+__device__ __forceinline__ void store_partial(const Work& wk, const Problem& P, int row0, int side, int slot, int lane,
+                                              const float (&v)[4 * NG]) {
+  const int j = side ? P.cm - slot : P.cp + slot;
+  const bool has = side ? (j >= 0 && j < P.ncols && j != P.cp + slot) : j < P.ncols;
+  if (!has) return;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    const int row = row0 + 8 * g + 4 * (lane >> 5);
+    if (P.trans) {
+      // C rows run along the partial's rows, so a lane's 4 consecutive C rows
+      // are one aligned 16-byte store (the partial and its row stride are
+      // multiples of 128 floats).  Rows past pcols land in the partial's
+      // padding columns, inside its allocation, which the reduction never reads.
+      if (j < wk.prows)
+        *(gptr<v4f32>)&((gptr<float>)wk.partial)[(long long)j * wk.ldp + row] =
+            v4f32{v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
+    } else if (j < wk.pcols) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (row + e < wk.prows) ((gptr<float>)wk.partial)[(long long)(row + e) * wk.ldp + j] = v[4 * g + e];
     }
   }
 }
 
-// The work item's loop.  MF = false for a wave whose 32 rows all lie past
-// the problems' last row (the ragged last row tile of a small tile): it
-// stages its share of the operands and keeps the barriers but issues no
-// fragment reads or MFMAs, and its zero accumulators give the same zero rows
-// the padding would, so the wave sharing its SIMD runs alone.
-template <int PREC, int EPI, int WN, int KS, bool MF>
-__device__ __forceinline__ void gemm_body(const Work& wk, const Problem* __restrict__ probs,
-                                          const double* __restrict__ chunk_x, Lds<PREC, WN, KS>& lds) {
-  using C = Cfg<WN, KS>;
-  constexpr int BS = C::BS;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int wr = wid / WN, wc = wid % WN;
-
-  // staging coordinates: A rows from a_row0, one slot / K group of twiddles
-  const long long a_row0 = (long long)wk.tr * BM;
-  const int st_slot = bitem_slot<KS>(tid);
-  const int st_g = bitem_group<KS>(tid);
-  const int b_slot = wk.tc * BS + st_slot;
-
-  f32x16 acc[4], ip, im;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = f32x16{};
-  ip = f32x16{};
-  im = f32x16{};
-
-  // ---- prologue: chunk 0 into LDS buffer 0, chunks 1 and 2 staged in the two
-  // register sets (chunk k in set k & 1), so each global load has two chunks
-  // of work to arrive in ----
-  int sp = wk.pbeg, ss = 0;  // staging cursor: next (problem, chunk) to stage
-  StageProb sgp;
-  float2 q[C::TW];
-  Staged<WN, KS> st0, st1;
-  set_stage<KS>(probs[sp], b_slot, sgp, q);
-  double sx = twiddle_x<KS>(chunk_x, sgp, 0, st_g);
-  auto advance = [&]() {
-    if (++ss == sgp.nch) {
-      ss = 0;
-      if (++sp < wk.pend) set_stage<KS>(probs[sp], b_slot, sgp, q);
-    }
-    sx = twiddle_x<KS>(chunk_x, sgp, sp < wk.pend ? ss : 0, st_g);
-  };
-  // stage the cursor's chunk (past the last chunk: a valid chunk restaged, never read)
-  auto stage = [&](Staged<WN, KS>& X) {
-    const bool more = sp < wk.pend;
-    load_a<PREC, WN, KS>(sgp, a_row0, tid, more ? ss : 0, X);
-    gen_b<PREC, WN, KS>(sx, sgp, q, X);
-    if (more) advance();
-  };
-  stage(st0);
-  write_b<PREC, WN, KS>(lds, 0, st_slot, st_g, st0);
-  write_a<PREC, WN, KS>(lds, 0, tid, st0);
-  stage(st1);
-  stage(st0);
-  __syncthreads();
-
-  int cur = 0;
-  int pc = wk.pbeg, cs = 0, cn = probs[pc].kpad / C::BKC;  // compute cursor: problem, chunk, chunks
-  // Chunk s: store chunk s+1 from its register set X into the idle buffer (its
-  // LDS stores then overlap this chunk's MFMAs), stage chunk s+3 into X,
-  // compute chunk s, and close the problem after its last chunk.
-  auto chunk = [&](Staged<WN, KS>& X) {
-    write_b<PREC, WN, KS>(lds, cur ^ 1, st_slot, st_g, X);
-    write_a<PREC, WN, KS>(lds, cur ^ 1, tid, X);
-    stage(X);
-
-    if (!MF) {
-      // no fragment reads or MFMAs for this wave
-    } else if (PREC == PREC_BF16X3) {
-      auto& L = reinterpret_cast<Lds<PREC_BF16X3, WN, KS>&>(lds);
-      const int r0 = wr * 32 + (lane & 31), c0 = wc * 32 + (lane & 31);
-#pragma unroll
-      for (int j = 0; j < KS; ++j) {
-        // fragment rows are 16-aligned + (lane & 31): one swizzle key per lane
-        const int koff = swz<KS>(lane & 31, 2 * j + (lane >> 5));
-        bf16x8_t a[4], b[4];
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-          a[p] = *(const bf16x8_t*)&L.a[cur][p][r0][koff];
-          b[p] = *(const bf16x8_t*)&L.b[cur][p][c0][koff];
-        }
-        sblock_bf16(a, b, acc);
-      }
-    } else {
-      auto& L = reinterpret_cast<Lds<PREC_FP32, WN, KS>&>(lds);
-#pragma unroll
-      for (int ks = 0; ks < C::BKC / 2; ++ks) {
-        const int kk = 2 * ks + (lane >> 5);
-        const float2 a = L.a[cur][wr * 32 + (lane & 31)][kk];
-        const float2 b = L.b[cur][wc * 32 + (lane & 31)][kk];
-        acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc[0], 0, 0, 0);
-        acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.x, acc[1], 0, 0, 0);
-        acc[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.y, acc[2], 0, 0, 0);
-        acc[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc[3], 0, 0, 0);
-      }
-    }
-
-    __syncthreads();
-    cur ^= 1;
-    if (++cs == cn) {
-      problem_epilogue<PREC, EPI>(probs[pc], wk, BS, wr, wc, lane, acc, ip, im);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = f32x16{};
-      if (++pc < wk.pend) {
-        cs = 0;
-        cn = probs[pc].kpad / C::BKC;
-      }
-    }
-  };
-  // two chunks per trip, so each register set has a fixed name
-  while (true) {
-    chunk(st1);
-    if (pc >= wk.pend) break;
-    chunk(st0);
-    if (pc >= wk.pend) break;
-  }
-  if (EPI == EPI_INTENSITY)
-    store_partial(wk, probs[wk.pbeg], BS, wr, wc, lane, ip, im);
-}
-
-template <int PREC, int EPI, int WN, int KS>
-__global__ __launch_bounds__((Cfg<WN, KS>::NT), (Cfg<WN, KS>::WG_PER_CU)) void gemm_kernel(
-    const Work* __restrict__ works, const Problem* __restrict__ probs, const double* __restrict__ chunk_x) {
-  __shared__ Lds<PREC, WN, KS> lds;
-  const Work wk = works[blockIdx.x];
-  if (wk.pbeg >= wk.pend) return;
-  int rows = 0;
-  for (int p = wk.pbeg; p < wk.pend; ++p) rows = max(rows, probs[p].rows);
-  const int wr = (threadIdx.x >> 6) / WN;
-  if (wk.tr * BM + wr * 32 < rows)  // wave-uniform
-    gemm_body<PREC, EPI, WN, KS, true>(wk, probs, chunk_x, lds);
-  else
-    gemm_body<PREC, EPI, WN, KS, false>(wk, probs, chunk_x, lds);
+// Work item of a launch without a work list: workgroup b is tile (b / ntc,
+// tc0 + b % ntc) of problem 0.
+// The twiddle table holds the slot blocks from sb0 on.
+struct OneWork {
+  int ntc, tc0, nch, sb0;
+};
+__device__ __forceinline__ Work get_work(const Work* __restrict__ works, const OneWork& one) {
+  if (works) return works[blockIdx.x];
+  Work wk = {};
+  wk.pend = 1;
+  wk.tr = (int)blockIdx.x / one.ntc;
+  wk.tc = one.tc0 + (int)blockIdx.x % one.ntc;
+  wk.nch = one.nch;
+  return wk;
 }
 
 // ---------------------------------------------------------------------------
-// Warp-specialised form of the 128-row x 64-slot, 32-wide-K configuration
-// (BF16x3).  Twelve waves per workgroup, three per SIMD:
-//   consumers (waves 0-7): a 4 x 2 grid of 32-row x 32-slot blocks; each
-//     issues the direct-to-LDS loads (global_load_lds_dwordx4, 16 bytes per
-//     lane at M0 + 16 lane) of 16 rows of the A tile two chunks ahead, reads
-//     its fragments from LDS and issues the 24 MFMAs of a chunk, and runs the
-//     problem epilogues;
-//   producers (waves 8-11): producer wave p generates the twiddles of K
-//     group p (8 consecutive K values for each of the 64 slots) one chunk
-//     ahead into LDS.
-// The twiddle VALU work thus runs on a wave of its own on each SIMD while
-// that SIMD's two consumer waves keep the MFMA pipe busy.  The A operand
-// never passes through VGPRs, and its loads, which stall the issuing wave
-// while the vector memory path is backed up, sit with the MFMA waves (the
-// SIMD's other consumer keeps the pipe busy) rather than in series with the
-// twiddle VALU.  LDS: A in three buffers (chunk s in s % 3), B in two
-// (s % 2), 128 KiB.  An A buffer is row-major, a row's 256 bytes of the
-// chunk (two 16-wide K blocks of 4 planes) in 16-byte units swizzled as
-// unit ^ (row & 15): one load moves 4 whole rows (8 cache lines, every byte
-// used), and the fragment reads of 16 (or 8) consecutive rows fall on
-// distinct banks.  One barrier per chunk (in stage 2 before the chunk's last
-// product group, so the next chunk's first fragment reads run under that
-// group).  Consumers wait for their previous
-// chunk's loads (vmcnt(4): the 4 loads just issued may stay in flight; loads
-// complete in issue order, so epilogue stores in between do not weaken this)
-// and their fragment reads, producers for their twiddle stores.  The barrier
-// and waits are written out: an LDS fence would make the compiler drain every
-// load, direct-to-LDS ones included, at each barrier.
-namespace ws {
-constexpr int NCONS = 8, NPROD = 4;
-constexpr int NT = 64 * (NCONS + NPROD);
-constexpr int BS = 64, BKC = 32;
-constexpr int NA = 3, NB = 2;
-// 16-byte alignment stated: the fragment reads are 16-byte LDS reads
-// (ds_read_b128), which the compiler emits only where it can prove it.
-struct alignas(16) Lds {
-  __bf16 a[NA][BM][128];   // [row][16-byte unit ^ (row & 15)][8 K values]
-  __bf16 b[NB][4][BS][32];
-};
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void gvoid;
-}  // namespace ws
-
-// A consumer's A cursor: the chunk its next direct-to-LDS loads fetch.
-// Consumer wave w loads rows 16 w .. 16 w + 15 of the tile, 4 rows per load:
-// lane l takes row 16 w + 4 j + (l >> 4) of load j and LDS unit l & 15, which
-// holds the row's logical unit (l & 15) ^ (row & 15) (row & 15 = 4 j + (l >> 4)).
-struct WsACursor {
-  int p, c, nch;              // problem, chunk in it, chunks in it
-  const char* base;           // wave-uniform: the wave's first row (16 w) at chunk 0
-  int voff[4];                // this lane's byte offset from base (at chunk 0) for load j
+// LDS-staged tiles
+// ---------------------------------------------------------------------------
+template <int WR, int WC, int S> struct Cfg {
+  static constexpr int NW = WR * WC;            // waves
+  static constexpr int NT = 64 * NW;            // threads
+  static constexpr int RB = WR, SB = WC * S;    // row and slot blocks per workgroup
+  static constexpr int ABYTES = RB * A_BLOCK, STAGE = ABYTES + SB * B_BLOCK;
+  static constexpr int NSTAGE = 3;
+  static constexpr int WG_PER_CU = 163840 / (NSTAGE * STAGE);
+  // every wave loads one part (4 fragments) of an operand block and one half
+  // (2 fragments: cos or sin) of a twiddle block per chunk
+  static_assert(2 * RB == NW && 2 * SB == NW, "loads divide evenly over the waves");
 };
 
-// The base is wave-uniform (row0 and w are), so it lives in SGPRs and each
-// load adds only the chunk offset to it there; a lane's offset within the
-// wave's 16 rows fits 32 bits (15 rows of a row stride below 128 MiB).
-__device__ __forceinline__ void ws_a_set(WsACursor& ac, const Problem& P, long long row0, int lane, int w) {
-  const long long ldb = P.lda * 2;  // bytes per A row
-  const int rr = lane >> 4, pu = lane & 15;
-  ac.nch = P.kpad / ws::BKC;
-  ac.base = (const char*)P.a + (row0 + 16 * w) * ldb;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) ac.voff[j] = (int)((4 * j + rr) * ldb) + 16 * (pu ^ (4 * j + rr));
-}
+// A wave's load cursor: the chunk its next six direct-to-LDS loads fetch.
+// Everything is wave-uniform and lives in SGPRs; a lane adds 16 bytes times
+// its index plus the fragment's offset.
+struct Cursor {
+  int seg, kb, nkb;
+  const char *a, *b;
+};
 
-// Direct-to-LDS load j (rows 16 w + 4 j .. + 3) of the cursor's chunk into A
-// buffer ab: lane l's 16 bytes land at M0 + 16 l.  Written out rather than
-// through the builtin: the compiler counts a builtin LDS DMA on the LDS/scalar
-// counter too, and then waits for every fragment read at once (lgkmcnt(0))
-// where a count would do; the load has no register result, and the waits for
-// it (vmcnt) are explicit.  SALU writes of M0 need one wait state before an
-// LDS DMA reads it.  The compiler reserves M0 and warns that it will not
-// restore it across the statement; these loads are the only M0 readers and
-// writers in the GEMM kernels (nothing else here uses M0), so nothing needs it
-// restored.
+// One direct-to-LDS load: lane l's 16 bytes at src + voff land at LDS byte dst
+// + 16 l.  Written out rather than through the builtin: the compiler counts a
+// builtin LDS DMA on the LDS/scalar counter too, and then waits for every
+// fragment read at once (lgkmcnt(0)) where a count would do; the load has no
+// register result, and the waits for it (vmcnt) are explicit.  SALU writes of
+// M0 need one wait state before an LDS DMA reads it.  The compiler reserves M0
+// and warns that it will not restore it across the statement; these loads are
+// the only M0 readers and writers here, so nothing needs it restored.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void ws_a_load1(ws::Lds& L, int ab, int w, const WsACursor& ac, int j) {
-  const char* src = ac.base + (long long)ac.c * 256;  // wave-uniform
-  const unsigned dst = (unsigned)(size_t)(ws::lds_void*)&L.a[ab][16 * w + 4 * j][0];
+__device__ __forceinline__ void lds_load(const char* src, int voff, unsigned dst) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :: "v"(ac.voff[j]), "s"(src), "s"(dst) : "memory", "m0");
+               :: "v"(voff), "s"(src), "s"(dst) : "memory", "m0");
 }
 #pragma clang diagnostic pop
 
-// All 4 loads of this wave's 16 rows of the cursor's chunk into A buffer ab.
-__device__ __forceinline__ void ws_a_load(ws::Lds& L, int ab, int w, const WsACursor& ac) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) ws_a_load1(L, ab, w, ac, j);
+__device__ __forceinline__ const char* uniform_ptr(const char* p) {
+  const uint64_t v = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+  return (const char*)(((uint64_t)hi << 32) | lo);
 }
 
-// The producer's twiddle state for one problem: 8 consecutive K values of one
-// slot per chunk, t_i = cis(alpha x Y) cis(alpha i Y), i = 0..7.
-struct WsB {
-  int p, c, nch, cb;
-  double alpha4, y;
-  float2 q[8];
-};
+// MULTI: problems may have several segments (the turn between them costs the
+// registers of a second set of accumulators, so only MID is built with it).
+template <int PREC, int EPI, int WR, int WC, int S, bool MULTI>
+__global__ __launch_bounds__((Cfg<WR, WC, S>::NT), (Cfg<WR, WC, S>::WG_PER_CU)) void gemm_tile_kernel(
+    const Work* __restrict__ works, const Problem* __restrict__ probs, const Seg* __restrict__ segs, OneWork one) {
+  using C = Cfg<WR, WC, S>;
+  using N = Num<PREC>;
+  typedef typename N::frag frag;
+  __shared__ alignas(16) char lds[C::NSTAGE * C::STAGE];
+  const Work wk = get_work(works, one);
+  if (wk.pbeg >= wk.pend) return;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int wr = wid / WC, wc = wid % WC;
 
-// Per problem: the slot's phase rate and q[i] = cis(4 alpha i y), i = 0..7,
-// from one FP64-phase evaluation and a product tree of depth 3 (about 3 ulp):
-// eight full evaluations at every problem start made the twiddle waves late
-// for that chunk's barrier.
-__device__ __forceinline__ void ws_b_set(WsB& b, const Problem& P, int slot) {
-  b.alpha4 = 4.0 * P.alpha;
-  b.y = P.y0 + (double)slot;
-  b.nch = P.kpad / ws::BKC;
-  b.cb = P.chunk_begin;
-  const float2 q1 = cis_quarter(b.alpha4 * b.y);
-  const float2 q2 = cmul(q1, q1), q4 = cmul(q2, q2);
-  b.q[0] = make_float2(1.0f, 0.0f);
-  b.q[1] = q1;
-  b.q[2] = q2;
-  b.q[3] = cmul(q2, q1);
-  b.q[4] = q4;
-  b.q[5] = cmul(q4, q1);
-  b.q[6] = cmul(q4, q2);
-  b.q[7] = cmul(q4, b.q[3]);
-}
-
-// Twiddles of K group g (K 8g .. 8g+7 of the chunk) of this thread's slot into B buffer bb.
-__device__ __forceinline__ void ws_b_write(ws::Lds& L, int bb, int slot, int g, const WsB& b,
-                                           const double* __restrict__ chunk_x) {
-  // chunk_x holds one origin per 16-wide K block; this group lies in block g >> 1
-  const double* px = chunk_x + __builtin_amdgcn_readfirstlane(b.cb + 2 * b.c + (g >> 1));
-  const double x = uniform_double(px) + (double)(8 * (g & 1));
-  const float2 pf = cis_quarter(b.alpha4 * (x * b.y));
-  uint32_t ch[4], cl[4], sh[4], sl[4];
+  // ---- loads ----
+  const int lrow = wid >> 1, lhalf = wid & 1;  // the block this wave loads, and its part / half
+  int voff[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float2 t0 = cmul(pf, b.q[2 * i]), t1 = cmul(pf, b.q[2 * i + 1]);
-    split2(t0.x, t1.x, ch[i], cl[i]);
-    split2(t0.y, t1.y, sh[i], sl[i]);
-  }
-  const int e = swz<2>(slot, g);
-  *(u32x4*)&L.b[bb][0][slot][e] = u32x4{ch[0], ch[1], ch[2], ch[3]};
-  *(u32x4*)&L.b[bb][1][slot][e] = u32x4{cl[0], cl[1], cl[2], cl[3]};
-  *(u32x4*)&L.b[bb][2][slot][e] = u32x4{sh[0], sh[1], sh[2], sh[3]};
-  *(u32x4*)&L.b[bb][3][slot][e] = u32x4{sl[0], sl[1], sl[2], sl[3]};
-}
-
-template <int EPI>
-__device__ __forceinline__ void gemm_ws_body(const Work& wk, const Problem* __restrict__ probs,
-                                             const double* __restrict__ chunk_x, ws::Lds& L) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, in an SGPR
-  int nchunks = 0;  // every problem's K loop back to back (uniform)
-  for (int p = wk.pbeg; p < wk.pend; ++p) nchunks += probs[p].kpad / ws::BKC;
-
-  if (wid >= ws::NCONS) {
-    // ---------------- producer ----------------
-    const int pw = wid - ws::NCONS;           // K group of the twiddles
-    const int slot = lane;                    // this thread's twiddle slot in the tile
-    WsB b;
-    b.p = wk.pbeg;
-    b.c = 0;
-    ws_b_set(b, probs[b.p], wk.tc * ws::BS + slot);
-    auto b_next = [&]() {
-      if (++b.c == b.nch) {
-        b.c = 0;
-        if (++b.p < wk.pend) ws_b_set(b, probs[b.p], wk.tc * ws::BS + slot);
-      }
-    };
-    ws_b_write(L, 0, slot, pw, b, chunk_x);
-    b_next();
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    for (int s = 0; s < nchunks; ++s) {
-      if (s + 1 < nchunks) {
-        ws_b_write(L, (s + 1) & 1, slot, pw, b, chunk_x);
-        b_next();
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    }
-    return;
-  }
-
-  // ---------------- consumer ----------------
-  const int wr = wid >> 1, wc = wid & 1;
-  int rows = 0;
-  for (int p = wk.pbeg; p < wk.pend; ++p) rows = max(rows, probs[p].rows);
-  const bool mf = wk.tr * BM + wr * 32 < rows;  // wave-uniform: past the last row a wave issues no MFMAs
-  f32x16 acc[4], ip, im;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = f32x16{};
-  ip = f32x16{};
-  im = f32x16{};
-  const int r0 = wr * 32 + (lane & 31), c0 = wc * 32 + (lane & 31);
-  const long long row0 = (long long)wk.tr * BM;
-  WsACursor ac;
-  ac.p = wk.pbeg;
-  ac.c = 0;
-  ws_a_set(ac, probs[ac.p], row0, lane, wid);
+  for (int f = 0; f < 4; ++f) voff[f] = 16 * lane + f * FRAG;
+  const unsigned lds0 = (unsigned)(size_t)(lds_void*)&lds[0];
+  const unsigned dst_a = lds0 + lrow * A_BLOCK + lhalf * 4 * FRAG;
+  const unsigned dst_b = lds0 + C::ABYTES + lrow * B_BLOCK + lhalf * 2 * FRAG;
+  const int seg_end = probs[wk.pend - 1].send;
+  // blocks past the operand's or table's last one reload it: valid memory
+  // whose results nobody stores
+  const int lrb = min(wk.tr * C::RB + lrow, probs[wk.pbeg].rblocks - 1);
+  const int lsb = min(wk.tc * C::SB + lrow, probs[wk.pbeg].sblocks - 1) - one.sb0;
+  Cursor cur;
+  auto cursor_set = [&](int seg) {
+    const Seg& sg = segs[seg];
+    cur.seg = seg;
+    cur.kb = 0;
+    cur.nkb = sg.nkb;
+    cur.a = uniform_ptr((const char*)sg.a + (long long)lrb * sg.a_nkb * A_BLOCK + lhalf * 4 * FRAG);
+    cur.b = uniform_ptr((const char*)sg.b + (long long)lsb * sg.b_nkb * B_BLOCK + lhalf * 2 * FRAG);
+  };
   // past the work's last chunk the cursor stays on it: the loads stay valid and nobody reads them
-  auto a_next = [&]() {
-    if (ac.c + 1 < ac.nch) {
-      ++ac.c;
-    } else if (ac.p + 1 < wk.pend) {
-      ++ac.p;
-      ac.c = 0;
-      ws_a_set(ac, probs[ac.p], row0, lane, wid);
+  auto cursor_next = [&]() {
+    if (cur.kb + 1 < cur.nkb) {
+      ++cur.kb;
+      cur.a += A_BLOCK;
+      cur.b += B_BLOCK;
+    } else if (cur.seg + 1 < seg_end) {
+      cursor_set(cur.seg + 1);
     }
   };
-  ws_a_load(L, 0, wid, ac);
-  a_next();
-  ws_a_load(L, 1, wid, ac);
-  a_next();
-  asm volatile("s_waitcnt vmcnt(4)\n\ts_barrier" ::: "memory");
-  int pc = wk.pbeg, cs = 0, cn = probs[pc].kpad / ws::BKC;
-  int ab = 0, an = 2;  // A buffers of chunks s and s + 2
-  // Operands of a 16-wide K block: A planes hi (re, im) and lo, twiddle
-  // planes hi (cos, sin) and lo.
-  const int ua = (lane >> 5) ^ (r0 & 15);  // A unit of (block 0, plane 0); block j, plane p: ua ^ (8 j + 2 p)
-  auto rd_a = [&](int buf, int j, int p) { return *(const bf16x8_t*)&L.a[buf][r0][8 * (ua ^ (8 * j + 2 * p))]; };
-  auto rd_b = [&](int buf, int j, int p) {
-    return *(const bf16x8_t*)&L.b[buf][p][c0][swz<2>(lane & 31, 2 * j + (lane >> 5))];
+  auto load = [&](int stage, int i) {  // i = 0..3: operand fragments, 4, 5: twiddle fragments
+    const unsigned st = (unsigned)(stage * C::STAGE);
+    if (i < 4) lds_load(cur.a, voff[i], dst_a + st + i * FRAG);
+    else lds_load(cur.b, voff[i - 4], dst_b + st + (i - 4) * FRAG);
   };
-  auto mf4 = [&](const bf16x8_t (&x)[2], const bf16x8_t (&y)[2]) {
-    acc[0] = MFMA_BF16(x[0], y[0], acc[0]);   // re cos
-    acc[1] = MFMA_BF16(x[1], y[0], acc[1]);   // im cos
-    acc[2] = MFMA_BF16(x[0], y[1], acc[2]);   // re sin
-    acc[3] = MFMA_BF16(x[1], y[1], acc[3]);   // im sin
+  cursor_set(probs[wk.pbeg].sbeg);
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+#pragma unroll
+    for (int i = 0; i < 6; ++i) load(st, i);
+    cursor_next();
+  }
+  asm volatile("s_waitcnt vmcnt(6)\n\ts_barrier" ::: "memory");
+
+  // ---- accumulators ----
+  f32x16 acc[S][4];  // P_re, P_im, Q_re, Q_im of each slot block
+  float ip[EPI == EPI_INTENSITY ? S : 1][16] = {}, im[EPI == EPI_INTENSITY ? S : 1][16] = {};
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[s][i] = f32x16{};
+  const int rb = wk.tr * C::RB + wr;  // this wave's row block
+  const bool mf = rb < probs[wk.pbeg].rblocks;  // wave-uniform: past the last row block a wave issues no MFMAs
+
+  // fragment reads: operand part p fragment f (re hi, re lo, im hi, im lo),
+  // twiddle slot block s, half p (cos, sin), fragment f (hi, lo)
+  const char* la = lds + wr * A_BLOCK + 16 * lane;
+  const char* lb = lds + C::ABYTES + wc * S * B_BLOCK + 16 * lane;
+  auto rd_a = [&](int stage, int p, int f) { return *(const frag*)(la + stage * C::STAGE + (4 * p + f) * FRAG); };
+  auto rd_b = [&](int stage, int s, int p, int f) {
+    return *(const frag*)(lb + stage * C::STAGE + s * B_BLOCK + (2 * p + f) * FRAG);
   };
-  auto load = [&](int j) {
-    __builtin_amdgcn_sched_barrier(0);
-    ws_a_load1(L, an, wid, ac, j);
-    __builtin_amdgcn_sched_barrier(0);
+  auto group = [&](int p, const frag (&x)[2], const frag (&y)[S]) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      acc[s][2 * p] = N::mfma(x[0], y[s], acc[s][2 * p]);
+      acc[s][2 * p + 1] = N::mfma(x[1], y[s], acc[s][2 * p + 1]);
+    }
   };
-  // Chunk s + 1's first fragments are read under chunk s's last product
-  // group, across the chunk's barrier (the complex store, whose epilogue
-  // needs those 16 registers at problem ends, reads them at the chunk's top).
-  constexpr bool kAhead = EPI != EPI_STORE_CPLX;
-  // Block 0's A hi and twiddle lo fragments of chunk s.
-  bf16x8_t ah[2] = {}, bl[2] = {};
+  auto fence = [&]() { __builtin_amdgcn_sched_barrier(0); };
+  auto loads = [&](int stage, int i0, int i1) {
+    fence();
+#pragma unroll
+    for (int i = i0; i < i1; ++i) load(stage, i);
+    fence();
+  };
   // Nothing is outstanding on the LDS/scalar counter after this wait; the
   // compiler sees it (the barrier's own waits are in asm it cannot read), so
   // it waits for each fragment read below by count, not for all at once.
   auto drained = [&]() { __builtin_amdgcn_s_waitcnt(0xc07f); };  // lgkmcnt(0); vmcnt, expcnt unrestricted
   auto barrier = [&]() {
-    // Wait for this wave's chunk s + 1 loads (the 4 just issued for chunk
+    // Wait for this wave's chunk s + 1 loads (the 6 just issued for chunk
     // s + 2 may stay in flight: loads complete in issue order, so epilogue
     // stores in between do not weaken this) and its fragment reads.
-    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     drained();
   };
-  auto first_reads = [&](int abuf, int bbuf) {
-    ah[0] = rd_a(abuf, 0, 0);
-    ah[1] = rd_a(abuf, 0, 2);
-    bl[0] = rd_b(bbuf, 0, 1);
-    bl[1] = rd_b(bbuf, 0, 3);
+  frag ah[2] = {}, bl[S] = {};
+  auto first_reads = [&](int stage) {
+    ah[0] = rd_a(stage, 0, 0);
+    ah[1] = rd_a(stage, 0, 2);
+#pragma unroll
+    for (int s = 0; s < S; ++s) bl[s] = rd_b(stage, s, 0, 1);
   };
+
+  int pc = wk.pbeg, sc = probs[pc].sbeg, left = segs[sc].nkb;  // compute cursor: problem, segment, chunks left in it
+  int st = 0, ld = 2;                                          // LDS stages of chunks s and s + 2
   drained();
-  if (kAhead && mf) first_reads(0, 0);
-  for (int s = 0; s < nchunks; ++s) {
-    const int b0 = s & 1;
+  if (mf) first_reads(0);
+  for (int n = 0; n < wk.nch; ++n) {
+    const int nx = st == 2 ? 0 : st + 1;
     if (mf) {
-      if (!kAhead) first_reads(ab, b0);
-      // The block's three products run in the order hi*lo, hi*hi, lo*hi, so
-      // each operand pair is dead as early as possible and the next
-      // fragments are read into its registers right after the MFMAs that
-      // last read it: block 1's reads are in flight while block 0
-      // multiplies, and the next chunk's first reads while the last group
-      // multiplies, without extra registers.  The 4 direct-to-LDS loads of
-      // chunk s + 2 sit between product groups, so the address unit works
-      // through the workgroup's 32 loads while the MFMAs issue.  Reading
-      // ahead, the chunk's barrier comes before its last group: by then
-      // every fragment read of chunk s and every load of chunk s + 2 is
-      // issued, and after it chunk s + 1 is complete in LDS.  Scheduling
-      // barriers pin this order.
-      bf16x8_t al[2] = {rd_a(ab, 0, 1), rd_a(ab, 0, 3)};
-      bf16x8_t bh[2] = {rd_b(b0, 0, 0), rd_b(b0, 0, 2)};
-      mf4(ah, bl);
-      load(0);
-      bl[0] = rd_b(b0, 1, 1);
-      bl[1] = rd_b(b0, 1, 3);
-      mf4(ah, bh);
-      load(1);
-      ah[0] = rd_a(ab, 1, 0);
-      ah[1] = rd_a(ab, 1, 2);
-      mf4(al, bh);
-      __builtin_amdgcn_sched_barrier(0);
-      bh[0] = rd_b(b0, 1, 0);
-      bh[1] = rd_b(b0, 1, 2);
-      al[0] = rd_a(ab, 1, 1);
-      al[1] = rd_a(ab, 1, 3);
-      __builtin_amdgcn_sched_barrier(0);
-      mf4(ah, bl);
-      load(2);
-      mf4(ah, bh);
-      load(3);
-      if (kAhead) {
-        barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        // chunk s + 1's first fragments (past the last chunk: a buffer
-        // nobody writes any more, read and unused)
-        first_reads(ab == 2 ? 0 : ab + 1, b0 ^ 1);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      mf4(al, bh);
-      if (!kAhead) barrier();
+      // The three products run in the order hi*lo, hi*hi, lo*hi, so each
+      // operand pair is dead as early as possible and the next fragments are
+      // read into its registers while the current group multiplies.  The
+      // chunk's barrier comes before its last group: by then every fragment
+      // read of chunk s and every load of chunk s + 2 is issued, and after it
+      // chunk s + 1 is complete in LDS and its first fragments are read under
+      // that group.  Scheduling barriers pin this order.
+      frag al[2] = {rd_a(st, 0, 1), rd_a(st, 0, 3)};
+      frag bh[S];
+#pragma unroll
+      for (int s = 0; s < S; ++s) bh[s] = rd_b(st, s, 0, 0);
+      group(0, ah, bl);
+      loads(ld, 0, 1);
+#pragma unroll
+      for (int s = 0; s < S; ++s) bl[s] = rd_b(st, s, 1, 1);
+      group(0, ah, bh);
+      loads(ld, 1, 2);
+      ah[0] = rd_a(st, 1, 0);
+      ah[1] = rd_a(st, 1, 2);
+      group(0, al, bh);
+      loads(ld, 2, 3);
+#pragma unroll
+      for (int s = 0; s < S; ++s) bh[s] = rd_b(st, s, 1, 0);
+      al[0] = rd_a(st, 1, 1);
+      al[1] = rd_a(st, 1, 3);
+      fence();
+      group(1, ah, bl);
+      loads(ld, 3, 5);
+      group(1, ah, bh);
+      loads(ld, 5, 6);
+      barrier();
+      fence();
+      first_reads(nx);  // past the last chunk: a stage nobody writes any more, read and unused
+      fence();
+      group(1, al, bh);
     } else {
-      ws_a_load(L, an, wid, ac);
+      loads(ld, 0, 6);
       barrier();
     }
-    a_next();
-    an = an == 2 ? 0 : an + 1;
-    ab = ab == 2 ? 0 : ab + 1;
-    if (++cs == cn) {
-      problem_epilogue<PREC_BF16X3, EPI>(probs[pc], wk, ws::BS, wr, wc, lane, acc, ip, im);
+    cursor_next();
+    st = nx;
+    ld = ld == 2 ? 0 : ld + 1;
+    if (--left > 0) continue;
+    const Problem& P = probs[pc];
+    ++sc;
+    if (MULTI && sc < P.send) {
+      // the next segment's midpoint: turn (P, Q) by its rotation
+      const Seg& sg = segs[sc];
+      left = sg.nkb;
+      if (mf) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = f32x16{};
-      if (++pc < wk.pend) {
-        cs = 0;
-        cn = probs[pc].kpad / ws::BKC;
+        for (int s = 0; s < S; ++s) {
+          const float2 r = cis_turns(sg.rot * (P.y0 + (double)((wk.tc * C::SB + wc * S + s) * 32 + (lane & 31))));
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+              const float p = acc[s][i][e], q = acc[s][2 + i][e];
+              acc[s][i][e] = r.x * p - r.y * q;
+              acc[s][2 + i][e] = r.y * p + r.x * q;
+            }
+        }
+      }
+      continue;
+    }
+    if (mf) {
+      const float scale = store_scale(P);
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const int slot = (wk.tc * C::SB + wc * S + s) * 32 + (lane & 31);
+        if (EPI == EPI_INTENSITY) {
+          const float w = P.weight * scale * scale;
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const float pr = acc[s][0][e], pi = acc[s][1][e], qr = acc[s][2][e], qi = acc[s][3][e];
+            const float ar = pr - qi, ai = pi + qr;   // P + iQ
+            const float br = pr + qi, bi = pi - qr;   // P - iQ
+            ip[s][e] = __builtin_fmaf(w, __builtin_fmaf(ar, ar, ai * ai), ip[s][e]);
+            im[s][e] = __builtin_fmaf(w, __builtin_fmaf(br, br, bi * bi), im[s][e]);
+          }
+        } else {
+          const float2 ph = slot_phase(P, slot);
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int side = 0; side < 2; ++side) {
+              float re[8], imv[8];
+#pragma unroll
+              for (int q = 0; q < 8; ++q) {
+                const int e = 8 * h + q;
+                const float pr = acc[s][0][e], pi = acc[s][1][e], qr = acc[s][2][e], qi = acc[s][3][e];
+                re[q] = side ? pr + qi : pr - qi;
+                imv[q] = side ? pi - qr : pi + qr;
+              }
+              store_half<PREC, EPI>(P, rb, h, side, slot, lane, scale, ph, re, imv);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[s][i] = f32x16{};
       }
     }
+    if (++pc < wk.pend) left = segs[sc].nkb;  // its first segment follows the last one
   }
   // no load may still be writing LDS when the workgroup ends
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if (EPI == EPI_INTENSITY) store_partial(wk, probs[wk.pbeg], ws::BS, wr, wc, lane, ip, im);
+  if (EPI == EPI_INTENSITY && mf) {
+    const Problem& P = probs[wk.pbeg];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int slot = (wk.tc * C::SB + wc * S + s) * 32 + (lane & 31);
+      store_partial<4>(wk, P, rb * 32, 0, slot, lane, ip[s]);
+      store_partial<4>(wk, P, rb * 32, 1, slot, lane, im[s]);
+    }
+  }
 }
 
-template <int EPI>
-__global__ __launch_bounds__(ws::NT, 1) void gemm_ws_kernel(const Work* __restrict__ works,
+// ---------------------------------------------------------------------------
+// One 32 x 32 block per workgroup, K split over its four waves
+// ---------------------------------------------------------------------------
+template <int PREC, int EPI>
+__global__ __launch_bounds__(256, 2) void gemm_small_kernel(const Work* __restrict__ works,
                                                             const Problem* __restrict__ probs,
-                                                            const double* __restrict__ chunk_x) {
-  __shared__ ws::Lds lds;
-  const Work wk = works[blockIdx.x];
+                                                            const Seg* __restrict__ segs, OneWork one) {
+  using N = Num<PREC>;
+  typedef typename N::frag frag;
+  __shared__ alignas(16) float red[4][4][4][64][4];  // [wave][accumulator][row group][lane][element]
+  const Work wk = get_work(works, one);
   if (wk.pbeg >= wk.pend) return;
-  gemm_ws_body<EPI>(wk, probs, chunk_x, lds);
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int h = wid & 1, side = wid >> 1;  // the rows and columns this wave stores
+  const int slot = wk.tc * 32 + (lane & 31);
+  float isum[8] = {};
+  for (int pc = wk.pbeg; pc < wk.pend; ++pc) {
+    const Problem& P = probs[pc];
+    f32x16 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = f32x16{};
+    for (int sg = P.sbeg; sg < P.send; ++sg) {
+      const Seg& sgm = segs[sg];
+      if (sg > P.sbeg) {
+        const float2 r = cis_turns(sgm.rot * (P.y0 + (double)slot));
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const float p = acc[i][e], q = acc[2 + i][e];
+            acc[i][e] = r.x * p - r.y * q;
+            acc[2 + i][e] = r.y * p + r.x * q;
+          }
+      }
+      gptr<const char> a = (gptr<const char>)sgm.a + (long long)wk.tr * sgm.a_nkb * A_BLOCK + 16 * lane;
+      gptr<const char> b = (gptr<const char>)sgm.b + (long long)(wk.tc - one.sb0) * sgm.b_nkb * B_BLOCK + 16 * lane;
+      frag af[2][8], bf[2][4];
+      auto get = [&](int buf, int kb) {
+#pragma unroll
+        for (int f = 0; f < 8; ++f) af[buf][f] = *(gptr<const frag>)(a + (long long)kb * A_BLOCK + f * FRAG);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) bf[buf][f] = *(gptr<const frag>)(b + (long long)kb * B_BLOCK + f * FRAG);
+      };
+      auto mul = [&](int buf) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          const int ia = t == 2 ? 1 : 0, ib = t == 0 ? 1 : 0;  // hi*lo, hi*hi, lo*hi
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            acc[2 * p] = N::mfma(af[buf][4 * p + ia], bf[buf][2 * p + ib], acc[2 * p]);
+            acc[2 * p + 1] = N::mfma(af[buf][4 * p + 2 + ia], bf[buf][2 * p + ib], acc[2 * p + 1]);
+          }
+        }
+      };
+      // the next block's fragments are loaded while the current one multiplies
+      int kb = wid;
+      if (kb < sgm.nkb) get(0, kb);
+      while (kb < sgm.nkb) {
+        if (kb + 4 < sgm.nkb) get(1, kb + 4);
+        mul(0);
+        kb += 4;
+        if (kb >= sgm.nkb) break;
+        if (kb + 4 < sgm.nkb) get(0, kb + 4);
+        mul(1);
+        kb += 4;
+      }
+    }
+    if (pc > wk.pbeg) __syncthreads();  // the last problem's sums have been read
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *(v4f32*)red[wid][i][g][lane] = v4f32{acc[i][4 * g], acc[i][4 * g + 1], acc[i][4 * g + 2], acc[i][4 * g + 3]};
+    __syncthreads();
+    float t[4][8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        v4f32 v = *(const v4f32*)red[0][i][2 * h + g][lane];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) v += *(const v4f32*)red[w][i][2 * h + g][lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[i][4 * g + e] = v[e];
+      }
+    float re[8], imv[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      re[q] = side ? t[0][q] + t[3][q] : t[0][q] - t[3][q];
+      imv[q] = side ? t[1][q] - t[2][q] : t[1][q] + t[2][q];
+    }
+    const float scale = store_scale(P);
+    if (EPI == EPI_INTENSITY) {
+      const float w = P.weight * scale * scale;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) isum[q] = __builtin_fmaf(w, __builtin_fmaf(re[q], re[q], imv[q] * imv[q]), isum[q]);
+    } else {
+      store_half<PREC, EPI>(P, wk.tr, h, side, slot, lane, scale, slot_phase(P, slot), re, imv);
+    }
+  }
+  if (EPI == EPI_INTENSITY) store_partial<2>(wk, probs[wk.pbeg], wk.tr * 32 + 16 * h, side, slot, lane, isum);
 }
 
-static hipError_t launch_ws(int epi, const Work* work, int nwork, const Problem* probs, const double* chunk_x,
-                            hipStream_t s) {
-  dim3 grid(nwork), block(ws::NT);
-  if (epi == EPI_STORE_CPLX)
-    hipLaunchKernelGGL((gemm_ws_kernel<EPI_STORE_CPLX>), grid, block, 0, s, work, probs, chunk_x);
-  else if (epi == EPI_STORE_PACKED_T)
-    hipLaunchKernelGGL((gemm_ws_kernel<EPI_STORE_PACKED_T>), grid, block, 0, s, work, probs, chunk_x);
+template <int PREC, int EPI>
+static hipError_t launch_epi(int tile, const Work* work, int nwork, const Problem* probs, const Seg* segs,
+                             const OneWork& one, hipStream_t s) {
+  if (tile == TILE_BIG)
+    hipLaunchKernelGGL((gemm_tile_kernel<PREC, EPI, 4, 2, 2, false>), dim3(nwork), dim3(Cfg<4, 2, 2>::NT), 0, s, work, probs,
+                       segs, one);
+  else if (tile == TILE_MID)
+    hipLaunchKernelGGL((gemm_tile_kernel<PREC, EPI, 2, 2, 1, false>), dim3(nwork), dim3(Cfg<2, 2, 1>::NT), 0, s, work,
+                       probs, segs, one);
+  else if (tile == TILE_MULTI)
+    hipLaunchKernelGGL((gemm_tile_kernel<PREC, EPI, 2, 2, 1, true>), dim3(nwork), dim3(Cfg<2, 2, 1>::NT), 0, s, work,
+                       probs, segs, one);
   else
-    hipLaunchKernelGGL((gemm_ws_kernel<EPI_INTENSITY>), grid, block, 0, s, work, probs, chunk_x);
+    hipLaunchKernelGGL((gemm_small_kernel<PREC, EPI>), dim3(nwork), dim3(256), 0, s, work, probs, segs, one);
   return hipGetLastError();
 }
 
-template <int WN, int KS>
-static hipError_t launch_cfg(int prec, int epi, const Work* work, int nwork, const Problem* probs,
-                             const double* chunk_x, hipStream_t s) {
-  dim3 grid(nwork), block(Cfg<WN, KS>::NT);
-#define MFTX_LAUNCH(P, E) \
-  hipLaunchKernelGGL((gemm_kernel<P, E, WN, KS>), grid, block, 0, s, work, probs, chunk_x)
-  if (prec == PREC_BF16X3) {
-    if (epi == EPI_STORE_CPLX) MFTX_LAUNCH(PREC_BF16X3, EPI_STORE_CPLX);
-    else if (epi == EPI_STORE_PACKED_T) MFTX_LAUNCH(PREC_BF16X3, EPI_STORE_PACKED_T);
-    else MFTX_LAUNCH(PREC_BF16X3, EPI_INTENSITY);
-  } else {
-    if (epi == EPI_STORE_CPLX) MFTX_LAUNCH(PREC_FP32, EPI_STORE_CPLX);
-    else if (epi == EPI_STORE_PACKED_T) MFTX_LAUNCH(PREC_FP32, EPI_STORE_PACKED_T);
-    else MFTX_LAUNCH(PREC_FP32, EPI_INTENSITY);
-  }
-#undef MFTX_LAUNCH
-  return hipGetLastError();
+template <int PREC>
+static hipError_t launch_prec(int epi, int tile, const Work* work, int nwork, const Problem* probs, const Seg* segs,
+                              const OneWork& one, hipStream_t s) {
+  if (epi == EPI_STORE_CPLX) return launch_epi<PREC, EPI_STORE_CPLX>(tile, work, nwork, probs, segs, one, s);
+  if (epi == EPI_STORE_PACKED) return launch_epi<PREC, EPI_STORE_PACKED>(tile, work, nwork, probs, segs, one, s);
+  return launch_epi<PREC, EPI_INTENSITY>(tile, work, nwork, probs, segs, one, s);
 }
 
-hipError_t launch_gemm(int prec, int epi, int bn, const Work* work, int nwork, const Problem* probs,
-                       const double* chunk_x, hipStream_t s) {
+static hipError_t launch_any(int prec, int epi, int tile, const Work* work, int nwork, const Problem* probs,
+                             const Seg* segs, const OneWork& one, hipStream_t s) {
   if (nwork <= 0) return hipSuccess;
-  if (bn == 64) return launch_cfg<1, 1>(prec, epi, work, nwork, probs, chunk_x, s);
-  if (bn == 128) {
-    if (prec == PREC_BF16X3) return launch_ws(epi, work, nwork, probs, chunk_x, s);
-    return launch_cfg<2, 2>(prec, epi, work, nwork, probs, chunk_x, s);
-  }
-  return hipErrorInvalidValue;
+  return prec == PREC_BF16X3 ? launch_prec<PREC_BF16X3>(epi, tile, work, nwork, probs, segs, one, s)
+                             : launch_prec<PREC_FP32>(epi, tile, work, nwork, probs, segs, one, s);
+}
+
+hipError_t launch_gemm(int prec, int epi, int tile, const Work* work, int nwork, const Problem* probs, const Seg* segs,
+                       hipStream_t s) {
+  return launch_any(prec, epi, tile, work, nwork, probs, segs, OneWork{}, s);
+}
+
+hipError_t launch_gemm_one(int prec, int epi, int tile, int rblocks, int sb0, int sb1, int nch, const Problem* prob,
+                           const Seg* seg, hipStream_t s) {
+  const int tr = (rblocks + tile_rows(tile) - 1) / tile_rows(tile);
+  const int tc0 = sb0 / tile_slots(tile), ntc = (sb1 + tile_slots(tile) - 1) / tile_slots(tile) - tc0;
+  return launch_any(prec, epi, tile, nullptr, tr * ntc, prob, seg, OneWork{ntc, tc0, nch, sb0}, s);
 }
 
 }  // namespace mftx

@@ -7,28 +7,45 @@ struct mftx_ctx;
 
 namespace mftx {
 
-// Tile geometry of the complex GEMM: WAVES_M x WN waves per workgroup, each
-// wave a 32-row x 32-slot block (64 output columns, see Problem); BM rows and
-// 32 WN slots per workgroup.
-constexpr int WAVES_M = 4;
-constexpr int BM = 32 * WAVES_M;   // C rows per workgroup (A rows)
-constexpr int BK = 16;             // K block: granule of the packed layout and of chunk_x
-constexpr int BN_DEFAULT = 128;    // output columns per workgroup unless a plan picks another
-// output columns per workgroup: 64 (32 slots, 16-wide K steps) or 128 (64 slots, 32-wide K steps)
-inline bool valid_bn(int bn) { return bn == 64 || bn == 128; }
-// K per GEMM pipeline stage for a tile width; every GEMM problem's kpad is a multiple of it.
-inline int k_granule(int bn) { return bn == 128 ? 32 : 16; }
-// slots per workgroup for a tile width
-inline int slots_per_tile(int bn) { return bn / 2; }
-static_assert(BM == 128, "staging assumes 128 A rows per workgroup");
+// Every GEMM operand lives in HBM as MFMA fragments: 1 KiB blocks, one per
+// 32 rows (or slots) x 16 K values of one 16-bit plane, holding lane l's eight
+// K values 8 (l / 32) .. + 7 of row l % 32 at byte 16 l.  A block is loaded
+// into LDS or registers by one 16-byte-per-lane access, whole cache lines,
+// and read from LDS without bank conflicts.
+constexpr int BK = 16;                 // K values per block
+constexpr int FRAG = 1024;             // bytes of one fragment
+constexpr int A_BLOCK = 8 * FRAG;      // operand bytes per (32 rows, K block): two parts x four planes
+constexpr int B_BLOCK = 4 * FRAG;      // twiddle bytes per (32 slots, K block): cos hi, cos lo, sin hi, sin lo
 
+// Number formats of the split operands: every value is hi + lo of one 16-bit
+// type, a real product is hi*hi + hi*lo + lo*hi with FP32 accumulation.
+//   PREC_FP32   : f16 pairs (22 bits).  The operand is scaled by a power of two
+//                 per launch so its largest value fits f16 (see ScaleSrc); the
+//                 result's error is below that of FP32 MFMAs, whose rounding
+//                 grows with the K / 2 accumulations of a K = 2 instruction.
+//   PREC_BF16X3 : bf16 pairs (16 bits), no scaling.
 enum Precision { PREC_FP32 = 0, PREC_BF16X3 = 1 };
 
 // Epilogues of the GEMM.
 enum Epilogue {
-  EPI_STORE_CPLX = 0,   // dst complex64, (r, c) -> dst[c*ld + r] if trans else dst[r*ld + c]; * scale; bounds
-  EPI_STORE_PACKED_T = 1,  // dst packed A-operand layout (precision dependent) of C^T, rows r < limit
-  EPI_INTENSITY = 2,    // accumulate w*|C|^2 over the workgroup's problems into a partial image
+  EPI_STORE_CPLX = 0,    // dst complex64, (r, j) -> dst[j*ld + r] if trans else dst[r*ld + j]; * scale; bounds
+  EPI_STORE_PACKED = 1,  // dst is the next stage's operand: rows = output columns j, K = C rows
+  EPI_INTENSITY = 2,     // accumulate w*|C|^2 over the work item's problems into a partial image
+};
+
+// Workgroup tiles of the GEMM (see mftx_gemm.hip).
+enum Tile { TILE_SMALL = 0, TILE_MID = 1, TILE_BIG = 2, TILE_MULTI = 3 };
+inline int tile_rows(int t) { return t == TILE_BIG ? 4 : t == TILE_SMALL ? 1 : 2; }  // 32-row blocks
+inline int tile_slots(int t) { return tile_rows(t); }                               // 32-slot blocks
+
+// One K segment of a GEMM problem.
+struct Seg {
+  const void* a;        // operand: [row block][a_nkb][A_BLOCK]
+  const void* b;        // twiddles: [slot block][b_nkb][B_BLOCK]
+  double rot;           // turns per unit Y the accumulators turn by before this segment (0: none)
+  int nkb;              // K blocks
+  int a_nkb, b_nkb;     // K blocks per row block of a / per slot block of b
+  int pad_;
 };
 
 // One complex GEMM problem: one MFT stage,
@@ -38,44 +55,109 @@ enum Epilogue {
 // j = N/2 + shift or at the grid centre next to it).  The producer of A has
 // multiplied A[i][k] by the fold cis(-alpha (shift + N/2 - c) x_k), so that
 // with Y = j - c
-//   C[i][j] = sum_k A'[i][k] cis(alpha x_k Y),
-// whose cosine part is even and sine part odd in Y.  The GEMM runs over slots
-// s = 0 .. cols-1 with Y_s = y0 + s (y0 = 0 for integer c, 1/2 otherwise):
-// P = sum_k A' cos, Q = sum_k A' sin, and
-//   C[i][cp + s] = P + i Q,    C[i][cm - s] = P - i Q
+//   C[i][j] = sum_k A'[i][k] cis(alpha x_k Y).
+// Both coordinates are paired.  x runs symmetrically about its midpoint xc,
+// x = xc +- x' with x' = k' + 1/2 (even length) or k' (odd), and the operand
+// holds the even and odd parts Ae = A'(+x') + A'(-x'), Ao = A'(+x') - A'(-x'):
+//   C[i][j] = cis(alpha xc Y) (P + iQ),  P = sum_k' Ae cos(2 pi alpha x' Y),
+//                                        Q = sum_k' Ao sin(2 pi alpha x' Y),
+// half the K of the plain product.  P is even and Q odd in Y, so the GEMM runs
+// over slots s = 0 .. cols-1 with Y_s = y0 + s only (y0 = 0 for integer c, 1/2
+// otherwise) and gives both output columns cp + s (P + iQ) and cm - s (P - iQ)
 // (cp = ceil(c), cm = floor(c); outputs outside [0, N) are dropped, and the
-// second is dropped where it equals the first).  c = 0 is the direct product
-// (one output per slot).  Twiddle B[k][s] = cis(alpha * x_k * Y_s) with
-// x_k = chunk_x[chunk_begin + k/BK] + (k % BK): x advances by one per K index
-// inside each BK-wide block, and each block carries its own starting x (so
-// several K segments with their own coordinate origins can be concatenated).
+// second where it equals the first).  c = 0 is the direct product (one output
+// per slot).  The phase cis(alpha xc Y) is left out where only |C|^2 of one
+// segment matters, and applied by the store otherwise (xrot).  Segments with
+// their own xc follow each other along K: turning (P, Q) by alpha (xc - xc')
+// re-expresses the sum so far about the next segment's midpoint.
 struct Problem {
-  const void* a;        // packed A' operand (row-major, K-blocked)
-  long long lda;        // A row stride in scalar elements (float2 for fp32, bf16 for bf16x3)
-  double alpha;         // signed twiddle scale in turns per unit of x*y
-  double y0;            // Y of slot 0
-  int rows;             // valid C rows
+  int sbeg, send;       // K segments
+  int rblocks, sblocks; // 32-row blocks of the operand, 32-slot blocks of the twiddle table
+  int rows;             // valid C rows (EPI_STORE_CPLX)
   int cols;             // slots
   int ncols;            // N: output columns
   int cp, cm;           // output columns of slot 0 (P + iQ, P - iQ)
-  int kpad;             // K (multiple of the launch's k_granule); A is zero beyond the valid K
-  int chunk_begin;      // index of this problem's first entry in chunk_x
-  float scale;          // store: C *= scale; intensity: weight applied to |C|^2
-  int limit;            // EPI_STORE_PACKED_T: C rows written (K extent of the destination)
   int trans;            // EPI_STORE_CPLX / EPI_INTENSITY: write C transposed
+  double y0;            // Y of slot 0
+  double xrot;          // stores: turns per unit Y of the phase applied to the output (0: none)
+  const float* inv;     // optional device factor of the scale (undoes the operand's scaling)
+  float scale;          // store: C *= scale; intensity: C *= scale before |C|^2
+  float weight;         // intensity: weight of |C|^2
   void* dst;            // store destination (EPI_STORE_*)
-  long long ldd;        // destination row stride (elements of its type)
+  long long ldd;        // EPI_STORE_CPLX: row stride; EPI_STORE_PACKED: K blocks per row block of dst
   const void* wmap;     // EPI_STORE_CPLX: optional real map multiplied into each stored value,
   long long ldw;        //   indexed like the destination (row stride ldw)
   int wdtype;           //   1 float32, 3 float64
   int pad2_;
+  const float2* rowph;  // EPI_STORE_CPLX: optional phase per C row
 };
+
+// A workgroup's unit of work: problems [pbeg, pend) on tile (tr, tc) of C.
+// For EPI_INTENSITY the problems' |C|^2 are summed into partial[r][c]
+// (row-major, stride ldp, transposed like the problems' trans flag).  nch is
+// the K blocks of all its problems together.
+struct Work {
+  int pbeg, pend;
+  int tr, tc;
+  float* partial;
+  long long ldp;
+  int prows, pcols;     // partial image extent (bounds for the store)
+  int nch, pad_;
+};
+
+// Extents of a paired operand axis of n samples: pairs, and 16-pair blocks.
+__host__ __device__ inline long long pairs(long long n) { return (n + 1) / 2; }
+__host__ __device__ inline int pair_blocks(long long n) { return (int)((pairs(n) + BK - 1) / BK); }
+// Bytes of the operand of an r x k array (row pairs in blocks of 16: the 16
+// even rows, then the 16 odd rows, of each block), and of a plain-row operand
+// (stage 2: rows are output columns) with nkb K blocks.
+inline size_t folded_bytes(long long r, long long k) { return (size_t)pair_blocks(r) * pair_blocks(k) * A_BLOCK; }
+inline size_t plain_bytes(long long rows, int nkb) { return (size_t)((rows + 31) / 32) * nkb * A_BLOCK; }
+
+// Scaling of a PREC_FP32 operand: `part` holds absolute maxima of the source
+// (written by launch_absmax); the consumers scale by the power of two that
+// takes four times their maximum (the sum of a pixel and its three mirror
+// images) to at most 2^14, and *inv receives its reciprocal.  n = 0: no scaling.
+struct ScaleSrc {
+  const float* part;
+  float* inv;
+  int n, pad_;
+};
+// One absolute-maximum job: blocks [begin, begin + nblk) of the launch write
+// part[0 .. nblk).
+struct MaxOp {
+  const void* src;
+  int dtype;            // 0..3 (see load_elem)
+  int nblk;
+  long long m, n, ld;
+  float* part;
+  long long begin;
+};
+constexpr int kMaxBlocks = 64;  // blocks (and part entries) of one absolute-maximum job, at most
+inline int max_blocks(long long m, long long n) {
+  const long long b = (m * n + 4095) / 4096;
+  return (int)(b < 1 ? 1 : b > kMaxBlocks ? kMaxBlocks : b);
+}
+
+// One twiddle table: cos and sin of 2 pi alpha x' (y0 + s), x' = k' + x0,
+// times tw_scale(prec), for nsb blocks of 32 slots from slot block sb0 and nkb
+// blocks of 16 k'.
+struct TableOp {
+  double alpha, x0, y0;
+  int nsb, nkb, sb0, pad_;
+  void* dst;
+  long long begin;      // first thread: one per (slot, 8 k')
+};
+__host__ __device__ inline long long table_threads(int nsb, int nkb) { return 64LL * nsb * nkb; }
+inline size_t table_bytes(int nsb, int nkb) { return (size_t)nsb * nkb * B_BLOCK; }
+// Twiddles of the f16 form are scaled so the lo parts of small ones stay normal.
+__host__ __device__ inline float tw_scale(int prec) { return prec == PREC_FP32 ? 256.0f : 1.0f; }
 
 // Per-wavelength parameters of a phasor launch: the phase opd * inv_wl, the
 // stage-1 fold cis(fold * (x0 + k)) along the operand's K index k, and the
 // stage-2 fold cis(fold2 * (x02 + r)) along its row index r (stage 1's C row r
 // is the operand's row r times the row's phase, so the stage-1 output comes
-// out folded for stage 2).
+// out folded for stage 2).  k and r index the source before pairing.
 struct PhasorWave {
   double inv_wl;
   double fold;
@@ -84,80 +166,75 @@ struct PhasorWave {
   double x02;
 };
 
-// A workgroup's unit of work: problems [pbeg, pend) on tile (tr, tc) of C.
-// For EPI_INTENSITY the problems' |C|^2 are summed into partial[r][c]
-// (row-major, stride ldp, transposed like the problems' trans flag).
-struct Work {
-  int pbeg, pend;
-  int tr, tc;
-  float* partial;
-  long long ldp;
-  int prows, pcols;     // partial image extent (bounds for the store)
-};
-
-// Packed A-operand layouts.
-//  fp32   : complex64 row-major, element (r, k) at r*lda + k.
-//  bf16x3 : per row, K in blocks of 16; each block holds 4 planes of 16 bf16
-//           (re_hi, re_lo, im_hi, im_lo): element (r, k, p) at
-//           r*lda + (k/16)*64 + p*16 + (k%16), lda = 4*kpad.
-__host__ __device__ inline long long packed_lda(int prec, int kpad) { return prec == PREC_FP32 ? kpad : 4LL * kpad; }
-__host__ __device__ inline size_t packed_bytes(int prec, long long rows, int kpad) {
-  return (size_t)rows * (size_t)kpad * (prec == PREC_FP32 ? 8 : 8);
-}
-
-// One phasor operand of a plan: the packed (transposed when trans) operand
-// of an m x n tile for nwave wavelengths, written wave_stride bytes apart.
-// `begin` is the op's first thread in the grouped launch.
-constexpr int PH_WAVES = 8;  // wavelengths per phasor thread
+// One operand source (a pupil phasor at nwave wavelengths, or complex data:
+// nwave = 1): the folded, paired operand of the m x n source (rows are the
+// source's columns when trans) for every wavelength, written wave_stride bytes
+// apart.  `begin` is the op's first thread in the grouped launch.
+constexpr int PH_WAVES = 4;  // wavelengths per phasor thread
 struct PhasorOp {
-  const void* amp;
-  const void* opd;
+  const void* amp;      // amplitude, or the complex source
+  const void* opd;      // OPD; null for a complex source
   int amp_dtype, opd_dtype;
   long long ld_amp, ld_opd;
   int m, n, trans, nwave;
   const PhasorWave* waves;
   void* dst;
-  long long wave_stride, rows_pad;
-  int kpad, pad_;
+  long long wave_stride;
+  ScaleSrc sc;
   long long begin;
 };
-__host__ __device__ inline long long phasor_threads(long long rows_pad, int kpad, int nwave) {
-  return rows_pad * (kpad / 8) * ((nwave + PH_WAVES - 1) / PH_WAVES);
+// threads of one wavelength group of an r x k operand (whole waves)
+__host__ __device__ inline long long group_threads(long long r, long long k) {
+  return 64LL * (((long long)pair_blocks(r) * pair_blocks(k) + 1) / 2);
+}
+__host__ __device__ inline long long phasor_threads(long long r, long long k, int nwave) {
+  return group_threads(r, k) * ((nwave + PH_WAVES - 1) / PH_WAVES);
 }
 
-// Grouped launches (phasor and pack ops): blocks of kGroupBlock threads, and
+// Grouped launches (phasor, table, maximum ops): blocks of kGroupBlock threads, and
 // every op's first thread is a multiple of kGroupBlock, so a block belongs to
 // one op and finds it with a block-uniform search.
 constexpr int kGroupBlock = 256;
 inline long long group_begin(long long total) { return (total + kGroupBlock - 1) / kGroupBlock * kGroupBlock; }
 
-// One packed operand from complex data (mftx_dft2_many): src (or src^T) times
-// the fold cis(fold * (x0 + k)) along K; rows_pad * kpad / 2 threads from `begin`.
-struct PackOp {
-  const void* src;
-  int dtype, trans;
-  long long m, n, lds;
-  double fold, x0;      // stage-1 fold along K
-  double fold2, x02;    // stage-2 fold along the packed rows (see PhasorWave)
-  void* dst;
-  long long rows_pad;
-  int kpad, pad_;
-  long long begin;
-};
-
 // launchers (mftx_gemm.hip, mftx_kernels.hip)
-// bn: output columns per workgroup (64 or 128, see valid_bn).
-hipError_t launch_gemm(int prec, int epi, int bn, const Work* work, int nwork, const Problem* probs,
-                       const double* chunk_x, hipStream_t s);
-// packed A' = src (or src^T) times the folds cis(fold * (x0 + k)) along K and
-// cis(fold2 * (x02 + row)) along the packed rows
-hipError_t launch_pack(int prec, const void* src, int src_dtype, long long m, long long n,
-                       long long lds, int trans, double fold, double x0, double fold2, double x02, void* dst,
-                       long long rows_pad, int kpad, hipStream_t s);
-// every op of a plan in one launch (ops_dev on the device, sorted by begin)
-hipError_t launch_phasor_group(int prec, const PhasorOp* ops_dev, int nops, long long total_threads, hipStream_t s);
-// every complex pack op in one launch (ops_dev on the device, sorted by begin)
-hipError_t launch_pack_group(int prec, const PackOp* ops_dev, int nops, long long total_threads, hipStream_t s);
+hipError_t launch_gemm(int prec, int epi, int tile, const Work* work, int nwork, const Problem* probs,
+                       const Seg* segs, hipStream_t s);
+// one problem (on the device, with its one segment of nch K blocks) over row
+// blocks [0, rblocks) and slot blocks [sb0, sb1), sb0 on a tile boundary
+hipError_t launch_gemm_one(int prec, int epi, int tile, int rblocks, int sb0, int sb1, int nch, const Problem* prob,
+                           const Seg* seg, hipStream_t s);
+// every operand source of a plan in one launch (ops_dev on the device, sorted
+// by begin): pupil phasors, or (cplx) complex arrays
+hipError_t launch_operands(int prec, bool cplx, const PhasorOp* ops_dev, int nops, long long total_threads,
+                           hipStream_t s);
+// every twiddle table / absolute maximum in one launch (sorted by begin)
+hipError_t launch_tables(int prec, const TableOp* ops_dev, int nops, long long total_threads, hipStream_t s);
+hipError_t launch_absmax(const MaxOp* ops_dev, int nops, long long total_blocks, hipStream_t s);
+// One transform's operand, twiddle tables and descriptors (prepare_one_kernel),
+// passed by value: nothing is uploaded.  With op.sc.n == 0 the f16 form's
+// maximum is taken inside the launch.
+struct OneDesc {
+  Problem prob[2];
+  Seg seg[2];
+};
+struct OneMft {
+  PhasorOp op;
+  PhasorWave wave;
+  TableOp tab[2];
+  OneDesc desc;
+  OneDesc* desc_dev;    // device copy for the GEMM launches
+};
+hipError_t launch_prepare_one(int prec, const OneMft& one, const MaxOp& mx, hipStream_t s);
+hipError_t launch_table_one(int prec, const TableOp& op, hipStream_t s);
+// table[r] = cis(rate * (r - centre)) for every op (rows 0: none)
+struct RowPhase {
+  double rate, centre;
+  float2* table;
+  int rows, pad_;
+};
+hipError_t launch_row_phases(const RowPhase* ops_dev, int nops, int most_rows, hipStream_t s);
+// launchers (mftx_gemm.hip, mftx_kernels.hip)
 hipError_t launch_phasor_field(const void* amp, int amp_dtype, long long ld_amp, const void* opd,
                                int opd_dtype, long long ld_opd, int m, int n, double inv_wavelength,
                                void* dst, hipStream_t s);
@@ -229,12 +306,13 @@ hipError_t launch_zernike(const double* rho, const double* theta, const void* ma
                           double* out, hipStream_t s);
 
 // host side of the C ABI (mftx_api.cpp)
-// mftx_dft2 on the caller's workspace ws (cap bytes), or on the context's own
-// growable workspace when ws is null
+// mftx_dft2 on the caller's workspace ws (for transforms of up to cap bytes,
+// see the definition, with table_cap bytes per twiddle table), or on the
+// context's own growable workspace when ws is null
 int dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, int64_t ldf, void* F,
                       int64_t M, int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r,
                       double shift_c, double offset_r, double offset_c, double scale, int conj, int precision,
-                      void* ws, size_t cap);
+                      void* ws, size_t cap, size_t table_cap);
 // record msg as the context's last error and return code
 int set_error(mftx_ctx* ctx, int code, const char* msg);
 // the device a context was created on

@@ -1,12 +1,11 @@
-// MI355X (gfx950) element-wise kernels of the MFT path: operand packing,
-// pupil phasors, detector accumulation, Field products and fills.
+// MI355X (gfx950) element-wise kernels of the MFT path: GEMM operands (pupil
+// phasors or complex data), twiddle tables, detector accumulation, Field
+// products and fills.
 #include "mftx_device.h"
 
-namespace mftx {
+#include <algorithm>
 
-// --------------------------------------------------------------------------
-// operand packing
-// --------------------------------------------------------------------------
+namespace mftx {
 
 // dtype codes: 0 complex64, 1 float32, 2 complex128, 3 float64
 __device__ __forceinline__ float2 load_elem(const void* p, int dtype, long long idx) {
@@ -19,72 +18,6 @@ __device__ __forceinline__ float2 load_elem(const void* p, int dtype, long long 
     }
     default: return make_float2((float)((const double*)p)[idx], 0.f);
   }
-}
-
-__device__ __forceinline__ void store_packed16(int prec, void* dst, long long lda, long long row, int kb,
-                                               const float2 (&v)[16]) {
-  if (prec == PREC_BF16X3) {
-    uint32_t rh[8], rl[8], ih[8], il[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      split2(v[2 * i].x, v[2 * i + 1].x, rh[i], rl[i]);
-      split2(v[2 * i].y, v[2 * i + 1].y, ih[i], il[i]);
-    }
-    uint4* d = (uint4*)((__bf16*)dst + row * lda + (long long)kb * 64);
-    d[0] = make_uint4(rh[0], rh[1], rh[2], rh[3]);
-    d[1] = make_uint4(rh[4], rh[5], rh[6], rh[7]);
-    d[2] = make_uint4(rl[0], rl[1], rl[2], rl[3]);
-    d[3] = make_uint4(rl[4], rl[5], rl[6], rl[7]);
-    d[4] = make_uint4(ih[0], ih[1], ih[2], ih[3]);
-    d[5] = make_uint4(ih[4], ih[5], ih[6], ih[7]);
-    d[6] = make_uint4(il[0], il[1], il[2], il[3]);
-    d[7] = make_uint4(il[4], il[5], il[6], il[7]);
-  } else {
-    float4* d = (float4*)((float2*)dst + row * lda + (long long)kb * 16);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) d[i] = make_float4(v[2 * i].x, v[2 * i].y, v[2 * i + 1].x, v[2 * i + 1].y);
-  }
-}
-
-// One thread per (row, 16-wide K block) of the packed destination.  The
-// source is m x n with row stride lds; packed element (row, k) is source
-// (row, k), or source (k, row) when trans (the packed operand is then n x m),
-// times the folds cis(fold * (x0 + k) + fold2 * (x02 + row)).  Everything
-// outside the source is zero.
-__global__ void pack_kernel(int prec, const void* __restrict__ src, int dtype, long long m, long long n,
-                            long long lds, int trans, double fold, double x0, double fold2, double x02,
-                            void* __restrict__ dst, long long rows_pad, int kpad) {
-  const int kblocks = kpad / 16;
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= rows_pad * kblocks) return;
-  const long long row = t / kblocks;
-  const int kb = (int)(t % kblocks);
-  const bool folded = fold != 0.0 || fold2 != 0.0;
-  const double row_phase = fold2 * (x02 + (double)row);
-  float2 v[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const long long k = (long long)kb * 16 + i;
-    const long long r = trans ? k : row, c = trans ? row : k;
-    if (r < m && c < n) {
-      const float2 e = load_elem(src, dtype, r * lds + c);
-      v[i] = folded ? cmul(e, cis_turns(__builtin_fma(fold, x0 + (double)k, row_phase))) : e;
-    } else {
-      v[i] = make_float2(0.f, 0.f);
-    }
-  }
-  store_packed16(prec, dst, packed_lda(prec, kpad), row, kb, v);
-}
-
-hipError_t launch_pack(int prec, const void* src, int src_dtype, long long m, long long n, long long lds,
-                       int trans, double fold, double x0, double fold2, double x02, void* dst, long long rows_pad,
-                       int kpad, hipStream_t s) {
-  const long long total = rows_pad * (kpad / 16);
-  if (total <= 0) return hipSuccess;
-  const int bs = 256;
-  hipLaunchKernelGGL(pack_kernel, dim3((unsigned)((total + bs - 1) / bs)), dim3(bs), 0, s, prec, src,
-                     src_dtype, m, n, lds, trans, fold, x0, fold2, x02, dst, rows_pad, kpad);
-  return hipGetLastError();
 }
 
 // Index of the op that block b0 (its first thread) belongs to: ops start on
@@ -100,62 +33,91 @@ __device__ __forceinline__ int block_op(const Op* __restrict__ ops, int nops, lo
   return lo;
 }
 
-// Grouped form of pack_kernel with one thread per (op, row, pair of K
-// values): lanes run along K (along the packed row) for a row-major source and
-// along the packed rows (along the source row) for a transposed one, so the
-// source reads of a wave are contiguous; each thread writes 4 bytes of every
-// BF16 plane (or one 16-byte complex64 pair).
-__global__ void pack_group_kernel(int prec, const PackOp* __restrict__ ops, int nops, long long total) {
-  const long long b0 = (long long)blockIdx.x * kGroupBlock;
-  const PackOp& op = ops[block_op(ops, nops, b0)];
-  const long long u = b0 + threadIdx.x - op.begin;
-  const int npairs = op.kpad / 2;
-  if (u >= op.rows_pad * npairs) return;
-  const long long row = op.trans ? u % op.rows_pad : u / npairs;
-  const int kp = (int)(op.trans ? u / op.rows_pad : u % npairs);
-  const bool folded = op.fold != 0.0 || op.fold2 != 0.0;
-  const double row_phase = op.fold2 * (op.x02 + (double)row);
-  float2 v[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const long long k = 2LL * kp + i;
-    const long long r = op.trans ? k : row, c = op.trans ? row : k;
-    if (r < op.m && c < op.n) {
-      const float2 e = load_elem(op.src, op.dtype, r * op.lds + c);
-      v[i] = folded ? cmul(e, cis_turns(__builtin_fma(op.fold, op.x0 + (double)k, row_phase))) : e;
-    } else {
-      v[i] = make_float2(0.f, 0.f);
-    }
-  }
-  const long long lda = packed_lda(prec, op.kpad);
-  const int k0 = 2 * kp;
-  if (prec == PREC_BF16X3) {
-    uint32_t rh, rl, ih, il;
-    split2(v[0].x, v[1].x, rh, rl);
-    split2(v[0].y, v[1].y, ih, il);
-    uint32_t* d = (uint32_t*)((__bf16*)op.dst + row * lda + (long long)(k0 / 16) * 64 + (k0 % 16));
-    d[0] = rh;    // plane 0 (re hi) at +0, plane p at + p * 16 bf16 = 8 words
-    d[8] = rl;
-    d[16] = ih;
-    d[24] = il;
-  } else {
-    *(float4*)((float2*)op.dst + row * lda + k0) = make_float4(v[0].x, v[0].y, v[1].x, v[1].y);
-  }
+__device__ __forceinline__ double load_real(const void* p, int dtype, long long idx) {
+  return dtype == 3 ? ((const double*)p)[idx] : (double)((const float*)p)[idx];
 }
 
-hipError_t launch_pack_group(int prec, const PackOp* ops, int nops, long long total, hipStream_t s) {
-  if (total <= 0 || nops <= 0) return hipSuccess;
-  hipLaunchKernelGGL(pack_group_kernel, dim3((unsigned)((total + kGroupBlock - 1) / kGroupBlock)), dim3(kGroupBlock),
-                     0, s, prec, ops, nops, total);
+// Largest value of the block's threads, in every thread (all of them call it).
+__device__ __forceinline__ float block_max(float v) {
+  __shared__ float w[kGroupBlock / 64];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = w[0];
+#pragma unroll
+  for (int i = 1; i < kGroupBlock / 64; ++i) v = fmaxf(v, w[i]);
+  return v;
+}
+
+// Bound of an element's modulus (0 where it is not finite: such an element
+// makes its results non-finite whatever the scale).
+__device__ __forceinline__ float elem_bound(const void* src, int dtype, long long i) {
+  const float2 e = load_elem(src, dtype, i);
+  const float v = fabsf(e.x) + fabsf(e.y);
+  return v <= 3.4028234e38f ? v : 0.f;
+}
+
+// Bound over elements [first, m * n) in steps of `step` of an m x n array.
+__device__ __forceinline__ float array_bound(const void* src, int dtype, long long m, long long n, long long ld,
+                                             long long first, long long step) {
+  float v = 0.f;
+  const long long total = m * n;
+  if (ld == n) {
+    for (long long i = first; i < total; i += step) v = fmaxf(v, elem_bound(src, dtype, i));
+  } else if (total < (1LL << 31)) {
+    for (unsigned i = (unsigned)first; i < (unsigned)total; i += (unsigned)step)
+      v = fmaxf(v, elem_bound(src, dtype, (long long)(i / (unsigned)n) * ld + i % (unsigned)n));
+  } else {
+    for (long long i = first; i < total; i += step) v = fmaxf(v, elem_bound(src, dtype, i / n * ld + i % n));
+  }
+  return v;
+}
+
+__global__ void absmax_kernel(const MaxOp* __restrict__ ops, int nops) {
+  const MaxOp& op = ops[block_op(ops, nops, (long long)blockIdx.x)];
+  const int b = (int)((long long)blockIdx.x - op.begin);
+  const float v = block_max(array_bound(op.src, op.dtype, op.m, op.n, op.ld, (long long)b * kGroupBlock + threadIdx.x,
+                                        (long long)op.nblk * kGroupBlock));
+  if (threadIdx.x == 0) op.part[b] = v;
+}
+
+hipError_t launch_absmax(const MaxOp* ops, int nops, long long total_blocks, hipStream_t s) {
+  if (total_blocks <= 0 || nops <= 0) return hipSuccess;
+  hipLaunchKernelGGL(absmax_kernel, dim3((unsigned)total_blocks), dim3(kGroupBlock), 0, s, ops, nops);
   return hipGetLastError();
 }
 
+// Power of two that takes 4 * bound to at most 2^14 (1 for bound 0).
+__device__ __forceinline__ float operand_scale(float bound) {
+  if (!(bound > 0.f)) return 1.0f;
+  const int e = 12 - __builtin_amdgcn_frexp_expf(bound);  // bound < 2^frexp_exp
+  return __uint_as_float((uint32_t)(127 + min(max(e, -126), 126)) << 23);
+}
+
+// The scale of an operand source (every thread of the block calls it).
+__device__ __forceinline__ float block_scale(const ScaleSrc& sc, bool first) {
+  if (sc.n == 0) return 1.0f;
+  float v = 0.f;
+  for (int i = threadIdx.x; i < sc.n; i += kGroupBlock) v = fmaxf(v, sc.part[i]);
+  const float s = operand_scale(block_max(v));
+  if (first && threadIdx.x == 0) *sc.inv = 1.0f / s;
+  return s;
+}
+
 // --------------------------------------------------------------------------
-// pupil phasor  f = amp * exp(2*pi*i*opd/lambda)   (plane.py:507)
+// GEMM operands: pupil phasors  f = amp * exp(2*pi*i*opd/lambda)  (plane.py:507)
+// or complex data, times both stages' folds, paired along both axes
 // --------------------------------------------------------------------------
 
-__device__ __forceinline__ double load_real(const void* p, int dtype, long long idx) {
-  return dtype == 3 ? ((const double*)p)[idx] : (double)((const float*)p)[idx];
+// Sample pair i of an n-sample axis: indices midpoint + x' and midpoint - x'
+// (x' = i + 1/2 for even n, i for odd; -1 where there is none: past the end,
+// or the middle sample's partner).
+__device__ __forceinline__ void pair_index(int n, int i, int& plus, int& minus) {
+  const int h = n >> 1;
+  plus = h + i < n ? h + i : -1;
+  minus = n & 1 ? (i > 0 ? h - i : -1) : h - 1 - i;
+  if (minus < 0) minus = -1;
 }
 
 __device__ __forceinline__ PhasorWave load_wave(cptr<const PhasorWave> p) {
@@ -168,117 +130,355 @@ __device__ __forceinline__ PhasorWave load_wave(cptr<const PhasorWave> p) {
   return w;
 }
 
-// One thread per (op, row, half of a 16-wide K block, group of PH_WAVES
-// wavelengths), every phasor operand of a plan in one launch (the op is found
-// by a block-uniform search).  The 8 amp/opd values are read once and the
-// packed operand of the m x n tile (n x m when trans) is written for each
-// wavelength of the group, with that wavelength's stage-1 fold along K and
-// stage-2 fold along the rows r in the same phase:
-// amp * cis(opd * inv_wl + fold * (x0 + k) + fold2 * (x02 + r)).  Consecutive threads
-// take consecutive source columns (half blocks when not trans, rows of the
-// transposed operand when trans), so the source reads of a wave are
-// contiguous; the two halves of a block store one 32-byte plane together.
-__global__ void phasor_group_kernel(int prec, const PhasorOp* __restrict__ ops, int nops, long long total) {
-  const long long b0 = (long long)blockIdx.x * kGroupBlock;
-  const PhasorOp& op = ops[block_op(ops, nops, b0)];
-  const long long u = b0 + threadIdx.x - op.begin;
-  if (u >= phasor_threads(op.rows_pad, op.kpad, op.nwave)) return;
-  const int khalves = op.kpad / 8;
-  const long long per_group = op.rows_pad * khalves;
-  // the wavelength group is wave-uniform: rows_pad is a multiple of 128 and
-  // op.begin of kGroupBlock, so a group spans whole waves; its descriptors
-  // are then scalar loads
+// One thread per (op, 16-pair row block, K block of 16 pairs, row pair of the
+// block, half of the K block, group of PH_WAVES wavelengths): 8 K pairs of one
+// row pair, 32 source samples, read once; for each wavelength the four
+// samples of a (row, K) quad, each with its phase
+//     opd * inv_wl + fold * (x0 + k) + fold2 * (x02 + r),
+// are combined into the even and odd rows' even and odd parts, split and
+// stored as 16 16-byte pieces.  32 consecutive threads write one K block, so
+// a store covers whole 256-byte runs.
+template <int PREC, bool CPLX, typename Waves>
+__device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave, long long u, float scale) {
+  const int R = op.trans ? op.n : op.m, K = op.trans ? op.m : op.n;
+  const int nrb = pair_blocks(R), nkb = pair_blocks(K);
+  // a wavelength group spans whole waves, so its descriptors are scalar loads
+  const long long per_group = group_threads(R, K);
   const int g = __builtin_amdgcn_readfirstlane((int)(u / per_group));
-  const long long r = u % per_group;
-  const long long row = op.trans ? r % op.rows_pad : r / khalves;
-  const int kh = (int)(op.trans ? r / op.rows_pad : r % khalves);
-  const int kb = kh >> 1, i0 = (kh & 1) * 8;
-  // Every load is issued before any math and none sits behind a branch, so
-  // they are in flight together: an element outside the m x n tile reads
-  // element 0 and is zeroed afterwards, the dtypes are tested once, and the
-  // thread's wavelength descriptors are read up front.
-  long long ia[8], io[8];
-  bool in[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const long long k = (long long)kb * 16 + i0 + i;
-    const long long sr = op.trans ? k : row, sc = op.trans ? row : k;
-    in[i] = sr < op.m && sc < op.n;
-    ia[i] = in[i] ? sr * op.ld_amp + sc : 0;
-    io[i] = in[i] ? sr * op.ld_opd + sc : 0;
-  }
-  float a[8];
-  double o[8];
-  if (op.amp_dtype == 3) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) a[i] = (float)((gptr<const double>)op.amp)[ia[i]];
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) a[i] = ((gptr<const float>)op.amp)[ia[i]];
-  }
-  if (op.opd_dtype == 3) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = ((gptr<const double>)op.opd)[io[i]];
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = (double)((gptr<const float>)op.opd)[io[i]];
-  }
+  const int v = (int)(u % per_group);
+  if (v >= 32 * nrb * nkb) return;
+  const int lr = v & 15, kh = (v >> 4) & 1, blk = v >> 5;
+  const int kb = blk % nkb, rb = blk / nkb;
+  int r2[2];
+  pair_index(R, rb * 16 + lr, r2[0], r2[1]);
+  const int kp0 = kb * 16 + kh * 8;
+  const bool even_k = !(K & 1);
+  const int kh2 = K >> 1;
+  // K index of pair kp0 + i: plus side kh2 + kp0 + i, minus side kminus0 - i
+  const int kplus0 = kh2 + kp0, kminus0 = even_k ? kh2 - 1 - kp0 : kh2 - kp0;
   const int w0 = g * PH_WAVES, nw = min(op.nwave - w0, PH_WAVES);
-  PhasorWave pws[PH_WAVES];
+  char* out = (char*)op.dst + ((long long)rb * nkb + kb) * A_BLOCK + 16 * (lr + 32 * kh);
+
+  // every load is issued before any math and none sits behind a branch: a
+  // sample outside the array reads element 0 and is zeroed afterwards
+  float a[2][2][8];                          // amplitude [row side][k side][pair]
+  double o[CPLX ? 1 : 2][CPLX ? 1 : 2][CPLX ? 1 : 8];
+  float ci[CPLX ? 2 : 1][CPLX ? 2 : 1][CPLX ? 8 : 1];
 #pragma unroll
-  for (int j = 0; j < PH_WAVES; ++j) pws[j] = load_wave((cptr<const PhasorWave>)op.waves + w0 + min(j, nw - 1));
+  for (int rs = 0; rs < 2; ++rs)
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    a[i] = in[i] ? a[i] : 0.f;
-    o[i] = in[i] ? o[i] : 0.0;
-  }
-  const long long lda = packed_lda(prec, op.kpad);
-  // The precision is tested once, outside the wavelength loop, so each
-  // loop is straight-line code whose stores are never waited for.
-  auto store_all = [&](auto bf16x3) {
-#pragma unroll
-    for (int j = 0; j < PH_WAVES; ++j) {
-      if (j >= nw) break;
-      const PhasorWave pw = pws[j];
-      // both folds' phase at K = 16 kb of this row: the stage-1 fold along
-      // K, the stage-2 fold along the rows
-      const double f0 = __builtin_fma(pw.fold, pw.x0 + (double)kb * 16, pw.fold2 * (pw.x02 + (double)row));
-      float2 v[8];
+    for (int ks = 0; ks < 2; ++ks) {
+      long long ia[8];
+      bool in[8];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float2 c = cis_turns(__builtin_fma(o[i], pw.inv_wl, __builtin_fma(pw.fold, (double)(i0 + i), f0)));
-        v[i] = make_float2(a[i] * c.x, a[i] * c.y);
+        const int k = ks ? kminus0 - i : kplus0 + i;
+        in[i] = r2[rs] >= 0 && k >= 0 && k < K && !(ks && !even_k && kp0 + i == 0);
+        const long long r = r2[rs], kk = k;
+        ia[i] = in[i] ? (op.trans ? kk * op.ld_amp + r : r * op.ld_amp + kk) : 0;
       }
-      char* dst = (char*)op.dst + (long long)(w0 + j) * op.wave_stride;
-      if constexpr (decltype(bf16x3)::value) {
-        uint32_t rh[4], rl[4], ih[4], il[4];
+      if constexpr (CPLX) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          split2(v[2 * i].x, v[2 * i + 1].x, rh[i], rl[i]);
-          split2(v[2 * i].y, v[2 * i + 1].y, ih[i], il[i]);
+        for (int i = 0; i < 8; ++i) {
+          const float2 e = load_elem(op.amp, op.amp_dtype, ia[i]);
+          a[rs][ks][i] = in[i] ? e.x : 0.f;
+          ci[rs][ks][i] = in[i] ? e.y : 0.f;
         }
-        gptr<v4u32> d = (gptr<v4u32>)((__bf16*)dst + row * lda + (long long)kb * 64 + i0);  // plane p at + 16 p bf16
-        d[0] = v4u32{rh[0], rh[1], rh[2], rh[3]};
-        d[2] = v4u32{rl[0], rl[1], rl[2], rl[3]};
-        d[4] = v4u32{ih[0], ih[1], ih[2], ih[3]};
-        d[6] = v4u32{il[0], il[1], il[2], il[3]};
       } else {
-        gptr<v4f32> d = (gptr<v4f32>)((float2*)dst + row * lda + (long long)kb * 16 + i0);
+        if (op.amp_dtype == 3) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) d[i] = v4f32{v[2 * i].x, v[2 * i].y, v[2 * i + 1].x, v[2 * i + 1].y};
+          for (int i = 0; i < 8; ++i) a[rs][ks][i] = (float)((gptr<const double>)op.amp)[ia[i]];
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) a[rs][ks][i] = ((gptr<const float>)op.amp)[ia[i]];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int k = ks ? kminus0 - i : kplus0 + i;
+          const long long r = r2[rs], kk = k;
+          ia[i] = in[i] ? (op.trans ? kk * op.ld_opd + r : r * op.ld_opd + kk) : 0;
+        }
+        if (op.opd_dtype == 3) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) o[rs][ks][i] = ((gptr<const double>)op.opd)[ia[i]];
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) o[rs][ks][i] = (double)((gptr<const float>)op.opd)[ia[i]];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          a[rs][ks][i] = in[i] ? a[rs][ks][i] * scale : 0.f;
+          o[rs][ks][i] = in[i] ? o[rs][ks][i] : 0.0;
+        }
       }
     }
-  };
-  if (prec == PREC_BF16X3)
-    store_all(std::true_type{});
-  else
-    store_all(std::false_type{});
+#pragma unroll 1
+  for (int j = 0; j < nw; ++j) {
+    const PhasorWave pw = wave(w0 + j);
+    const bool folded = pw.fold != 0.0 || pw.fold2 != 0.0;
+    // phase of pair 0 of each quadrant; K advances by +-1 per pair
+    double base[2][2];
+#pragma unroll
+    for (int rs = 0; rs < 2; ++rs)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        base[rs][ks] = __builtin_fma(pw.fold, pw.x0 + (double)(ks ? kminus0 : kplus0),
+                                     pw.fold2 * (pw.x02 + (double)r2[rs]));
+    uint32_t w[2][2][4][4];  // [row parity][part][plane][word]
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float2 p[2][2][2];  // [row parity][part][pair]
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int i = 2 * t + q;
+        float2 e[2][2];
+#pragma unroll
+        for (int rs = 0; rs < 2; ++rs)
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks) {
+            const double ph = __builtin_fma(ks ? -pw.fold : pw.fold, (double)i, base[rs][ks]);
+            if constexpr (CPLX) {
+              const float2 z = make_float2(a[rs][ks][i] * scale, ci[rs][ks][i] * scale);
+              e[rs][ks] = folded ? cmul(z, cis_turns(ph)) : z;
+            } else {
+              const float2 c = cis_turns(__builtin_fma(o[rs][ks][i], pw.inv_wl, ph));
+              e[rs][ks] = make_float2(a[rs][ks][i] * c.x, a[rs][ks][i] * c.y);
+            }
+          }
+#pragma unroll
+        for (int par = 0; par < 2; ++par) {
+          const float sg = par ? -1.f : 1.f;
+          const float2 kp = make_float2(__builtin_fmaf(sg, e[1][0].x, e[0][0].x), __builtin_fmaf(sg, e[1][0].y, e[0][0].y));
+          const float2 km = make_float2(__builtin_fmaf(sg, e[1][1].x, e[0][1].x), __builtin_fmaf(sg, e[1][1].y, e[0][1].y));
+          p[par][0][q] = make_float2(kp.x + km.x, kp.y + km.y);
+          p[par][1][q] = make_float2(kp.x - km.x, kp.y - km.y);
+        }
+      }
+#pragma unroll
+      for (int par = 0; par < 2; ++par)
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+          split2<PREC>(p[par][part][0].x, p[par][part][1].x, w[par][part][0][t], w[par][part][1][t]);
+          split2<PREC>(p[par][part][0].y, p[par][part][1].y, w[par][part][2][t], w[par][part][3][t]);
+        }
+    }
+    char* d = out + (long long)(w0 + j) * op.wave_stride;
+#pragma unroll
+    for (int par = 0; par < 2; ++par)
+#pragma unroll
+      for (int part = 0; part < 2; ++part)
+#pragma unroll
+        for (int pl = 0; pl < 4; ++pl) {
+          const uint32_t (&x)[4] = w[par][part][pl];
+          *(gptr<v4u32>)(d + (part * 4 + pl) * FRAG + par * 256) = v4u32{x[0], x[1], x[2], x[3]};
+        }
+  }
 }
 
-hipError_t launch_phasor_group(int prec, const PhasorOp* ops, int nops, long long total, hipStream_t s) {
+// Every operand source of a plan in one launch (the op is found by a
+// block-uniform search).
+template <int PREC, bool CPLX>
+__global__ __launch_bounds__(kGroupBlock, 2) void operand_group_kernel(const PhasorOp* __restrict__ ops, int nops) {
+  const long long b0 = (long long)blockIdx.x * kGroupBlock;
+  const PhasorOp& op = ops[block_op(ops, nops, b0)];
+  const float scale = block_scale(op.sc, b0 == op.begin);
+  const long long u = b0 + threadIdx.x - op.begin;
+  if (u >= phasor_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, op.nwave)) return;
+  operand_thread<PREC, CPLX>(op, [&](int w) { return load_wave((cptr<const PhasorWave>)op.waves + w); }, u, scale);
+}
+
+hipError_t launch_operands(int prec, bool cplx, const PhasorOp* ops, int nops, long long total, hipStream_t s) {
   if (total <= 0 || nops <= 0) return hipSuccess;
-  hipLaunchKernelGGL(phasor_group_kernel, dim3((unsigned)((total + kGroupBlock - 1) / kGroupBlock)),
-                     dim3(kGroupBlock), 0, s, prec, ops, nops, total);
+  const dim3 grid((unsigned)((total + kGroupBlock - 1) / kGroupBlock)), block(kGroupBlock);
+  if (prec == PREC_BF16X3) {
+    if (cplx) hipLaunchKernelGGL((operand_group_kernel<PREC_BF16X3, true>), grid, block, 0, s, ops, nops);
+    else hipLaunchKernelGGL((operand_group_kernel<PREC_BF16X3, false>), grid, block, 0, s, ops, nops);
+  } else {
+    if (cplx) hipLaunchKernelGGL((operand_group_kernel<PREC_FP32, true>), grid, block, 0, s, ops, nops);
+    else hipLaunchKernelGGL((operand_group_kernel<PREC_FP32, false>), grid, block, 0, s, ops, nops);
+  }
+  return hipGetLastError();
+}
+
+// --------------------------------------------------------------------------
+// twiddle tables
+// --------------------------------------------------------------------------
+
+// (cos, sin)(2 pi t) in FP64 for t in turns: t is reduced to a quarter-turn
+// index and a remainder |a| <= pi/4, whose Taylor series to degree 13 (sin)
+// and 14 (cos) are below 1e-13 off there.
+__device__ __forceinline__ double2 cis_turns64(double t) {
+  const double q = t * 4.0;
+  const double n = __builtin_rint(q);
+  const int quad = (int)(long long)n;
+  const double a = (q - n) * 1.57079632679489661923, a2 = a * a;
+  double s = 1.0 / 6227020800.0;
+  s = __builtin_fma(s, a2, -1.0 / 39916800.0);
+  s = __builtin_fma(s, a2, 1.0 / 362880.0);
+  s = __builtin_fma(s, a2, -1.0 / 5040.0);
+  s = __builtin_fma(s, a2, 1.0 / 120.0);
+  s = __builtin_fma(s, a2, -1.0 / 6.0);
+  s = __builtin_fma(a * a2, s, a);
+  double c = -1.0 / 87178291200.0;
+  c = __builtin_fma(c, a2, 1.0 / 479001600.0);
+  c = __builtin_fma(c, a2, -1.0 / 3628800.0);
+  c = __builtin_fma(c, a2, 1.0 / 40320.0);
+  c = __builtin_fma(c, a2, -1.0 / 720.0);
+  c = __builtin_fma(c, a2, 1.0 / 24.0);
+  c = __builtin_fma(c, a2, -0.5);
+  c = __builtin_fma(c, a2, 1.0);
+  const double re = quad & 1 ? s : c, im = quad & 1 ? c : s;
+  return make_double2((quad + 1) & 2 ? -re : re, quad & 2 ? -im : im);
+}
+
+// One thread per (slot, 8 k').  The values are correctly rounded to the
+// format's hi + lo but for 1e-13, tighter than FP32 twiddles.
+template <int PREC>
+__device__ __forceinline__ void table_thread(const TableOp& op, long long u) {
+  const int l = (int)(u & 63);
+  const long long blk = u >> 6;
+  const int kb = (int)(blk % op.nkb), sb = (int)(blk / op.nkb);
+  const double y = op.y0 + (double)((op.sb0 + sb) * 32 + (l & 31));
+  const double x0 = op.x0 + (double)(kb * 16 + 8 * (l >> 5));
+  const float ts = tw_scale(PREC);
+  uint32_t w[4][4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    float c[2], s[2], cl[2], sl[2];
+    uint32_t ch, sh;
+    double2 v[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      v[q] = cis_turns64(op.alpha * ((x0 + (double)(2 * t + q)) * y));
+      v[q].x *= ts;
+      v[q].y *= ts;
+      c[q] = (float)v[q].x;
+      s[q] = (float)v[q].y;
+    }
+    auto widen = [](uint32_t h, int q) -> double {
+      if constexpr (PREC == PREC_BF16X3) return q ? bf16_hi_to_f32(h) : bf16_lo_to_f32(h);
+      else return (double)(float)(__builtin_bit_cast(f16x2_t, h)[q]);
+    };
+    auto pk = [](float x, float y2) { return PREC == PREC_BF16X3 ? pack_bf16(x, y2) : pack_f16(x, y2); };
+    ch = pk(c[0], c[1]);
+    sh = pk(s[0], s[1]);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      cl[q] = (float)(v[q].x - widen(ch, q));
+      sl[q] = (float)(v[q].y - widen(sh, q));
+    }
+    w[0][t] = ch;
+    w[1][t] = pk(cl[0], cl[1]);
+    w[2][t] = sh;
+    w[3][t] = pk(sl[0], sl[1]);
+  }
+  char* d = (char*)op.dst + ((long long)sb * op.nkb + kb) * B_BLOCK + 16 * l;
+#pragma unroll
+  for (int pl = 0; pl < 4; ++pl)
+    *(gptr<v4u32>)(d + pl * FRAG) = v4u32{w[pl][0], w[pl][1], w[pl][2], w[pl][3]};
+}
+
+template <int PREC>
+__global__ void table_group_kernel(const TableOp* __restrict__ ops, int nops) {
+  const long long b0 = (long long)blockIdx.x * kGroupBlock;
+  const TableOp& op = ops[block_op(ops, nops, b0)];
+  const long long u = b0 + threadIdx.x - op.begin;
+  if (u < table_threads(op.nsb, op.nkb)) table_thread<PREC>(op, u);
+}
+
+hipError_t launch_tables(int prec, const TableOp* ops, int nops, long long total, hipStream_t s) {
+  if (total <= 0 || nops <= 0) return hipSuccess;
+  const dim3 grid((unsigned)((total + kGroupBlock - 1) / kGroupBlock)), block(kGroupBlock);
+  if (prec == PREC_BF16X3) hipLaunchKernelGGL((table_group_kernel<PREC_BF16X3>), grid, block, 0, s, ops, nops);
+  else hipLaunchKernelGGL((table_group_kernel<PREC_FP32>), grid, block, 0, s, ops, nops);
+  return hipGetLastError();
+}
+
+__global__ void row_phase_kernel(const RowPhase* __restrict__ ops) {
+  const RowPhase op = ops[blockIdx.y];
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= op.rows) return;
+  const double2 v = cis_turns64(op.rate * ((double)t - op.centre));
+  op.table[t] = make_float2((float)v.x, (float)v.y);
+}
+
+hipError_t launch_row_phases(const RowPhase* ops, int nops, int most_rows, hipStream_t s) {
+  for (int b = 0; b < nops && most_rows > 0; b += 65535)
+    hipLaunchKernelGGL(row_phase_kernel, dim3((unsigned)((most_rows + 255) / 256), std::min(nops - b, 65535)), dim3(256),
+                       0, s, ops + b);
+  return hipGetLastError();
+}
+
+// --------------------------------------------------------------------------
+// one transform: absolute maximum, then operand, both tables and the GEMMs'
+// descriptors in one launch, everything passed by value
+// --------------------------------------------------------------------------
+template <int PREC>
+__global__ __launch_bounds__(kGroupBlock, 2) void prepare_one_kernel(PhasorOp op, PhasorWave wave, TableOp tab0,
+                                                                     TableOp tab1, OneDesc desc, OneDesc* out,
+                                                                     int op_blocks, int tab_blocks) {
+  const int b = (int)blockIdx.x;
+  if (b < op_blocks) {
+    float scale = 1.0f;
+    if (PREC == PREC_FP32) {
+      if (op.sc.n == 0) {  // a small source: every block takes its maximum
+        scale = operand_scale(block_max(array_bound(op.amp, op.amp_dtype, op.m, op.n, op.ld_amp, threadIdx.x,
+                                                    kGroupBlock)));
+        if (b == 0 && threadIdx.x == 0) *op.sc.inv = 1.0f / scale;
+      } else {
+        scale = block_scale(op.sc, b == 0);
+      }
+    }
+    if (b == 0 && threadIdx.x == 0) *out = desc;
+    const long long u = (long long)b * kGroupBlock + threadIdx.x;
+    if (u < phasor_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, 1))
+      operand_thread<PREC, true>(op, [=](int) { return wave; }, u, scale);
+    return;
+  }
+  long long u = (long long)(b - op_blocks) * kGroupBlock + threadIdx.x;
+  if (b - op_blocks < tab_blocks) {
+    if (u < table_threads(tab0.nsb, tab0.nkb)) table_thread<PREC>(tab0, u);
+    return;
+  }
+  u -= (long long)tab_blocks * kGroupBlock;
+  if (u < table_threads(tab1.nsb, tab1.nkb)) table_thread<PREC>(tab1, u);
+}
+
+template <int PREC>
+__global__ void table_one_kernel(TableOp op) {
+  const long long u = (long long)blockIdx.x * kGroupBlock + threadIdx.x;
+  if (u < table_threads(op.nsb, op.nkb)) table_thread<PREC>(op, u);
+}
+
+__global__ void absmax_one_kernel(MaxOp op) {
+  const float v = block_max(array_bound(op.src, op.dtype, op.m, op.n, op.ld,
+                                        (long long)blockIdx.x * kGroupBlock + threadIdx.x,
+                                        (long long)op.nblk * kGroupBlock));
+  if (threadIdx.x == 0) op.part[blockIdx.x] = v;
+}
+
+hipError_t launch_prepare_one(int prec, const OneMft& one, const MaxOp& mx, hipStream_t s) {
+  if (prec == PREC_FP32 && one.op.sc.n > 0) hipLaunchKernelGGL(absmax_one_kernel, dim3(mx.nblk), dim3(kGroupBlock), 0, s, mx);
+  const PhasorOp& op = one.op;
+  const int op_blocks =
+      (int)((phasor_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, 1) + kGroupBlock - 1) / kGroupBlock);
+  int blocks[2];
+  for (int t = 0; t < 2; ++t)
+    blocks[t] = (int)((table_threads(one.tab[t].nsb, one.tab[t].nkb) + kGroupBlock - 1) / kGroupBlock);
+  const dim3 grid(op_blocks + blocks[0] + blocks[1]), block(kGroupBlock);
+  if (prec == PREC_BF16X3)
+    hipLaunchKernelGGL((prepare_one_kernel<PREC_BF16X3>), grid, block, 0, s, op, one.wave, one.tab[0], one.tab[1],
+                       one.desc, one.desc_dev, op_blocks, blocks[0]);
+  else
+    hipLaunchKernelGGL((prepare_one_kernel<PREC_FP32>), grid, block, 0, s, op, one.wave, one.tab[0], one.tab[1],
+                       one.desc, one.desc_dev, op_blocks, blocks[0]);
+  return hipGetLastError();
+}
+
+hipError_t launch_table_one(int prec, const TableOp& op, hipStream_t s) {
+  const dim3 grid((unsigned)((table_threads(op.nsb, op.nkb) + kGroupBlock - 1) / kGroupBlock)), block(kGroupBlock);
+  if (prec == PREC_BF16X3) hipLaunchKernelGGL((table_one_kernel<PREC_BF16X3>), grid, block, 0, s, op);
+  else hipLaunchKernelGGL((table_one_kernel<PREC_FP32>), grid, block, 0, s, op);
   return hipGetLastError();
 }
 

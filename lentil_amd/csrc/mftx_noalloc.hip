@@ -21,10 +21,14 @@
 
 namespace mftx {
 
+// The documented limit counts complex64-sized operands; what the kernels lay
+// out for a transform within it takes at most twice that (K padded to pairs of
+// 32), two twiddle tables and the descriptors (dft2_on_workspace).
 constexpr size_t kScratchBytes = MFTX_NOALLOC_SCRATCH_BYTES;
+constexpr size_t kTableBytes = 16u << 20;
 constexpr int kMaxDevices = 64;
 
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[2 * kScratchBytes + 2 * kTableBytes + 4096];
 
 // Device address of this device's `scratch`, looked up on the first call for
 // the device (mftx_create makes that call with the device current).
@@ -58,5 +62,5 @@ extern "C" int mftx_dft2_noalloc(mftx_ctx* ctx, const void* f, int f_dtype, int6
     return mftx::set_error(ctx, MFTX_EDEVICE,
                            (std::string("scratch address lookup: ") + hipGetErrorString(e)).c_str());
   return mftx::dft2_on_workspace(ctx, f, f_dtype, m, n, ldf, F, M, N, ldF, alpha_r, alpha_c, shift_r, shift_c,
-                                 offset_r, offset_c, scale, conj, precision, ws, mftx::kScratchBytes);
+                                 offset_r, offset_c, scale, conj, precision, ws, mftx::kScratchBytes, mftx::kTableBytes);
 }
