@@ -13,7 +13,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -254,7 +253,7 @@ struct mftx_plan {
   long long max_blocks = 0;
   int nwork1 = 0, nwork2 = 0;
   // stage 2 of the classes whose coherent group has several output grids:
-  // their complex fields, summed by the fallbacks below (every other class
+  // their complex fields, summed by the coherent launch (every other class
   // runs the intensity launch above)
   Work* works2c = nullptr;
   Problem* probs2c = nullptr;
@@ -269,21 +268,11 @@ struct mftx_plan {
     long long r0, c0;
   };
   std::vector<Reduce> reduces;
-  // coherent groups whose Fields overlap only partially: complex outputs
-  // summed into an image-sized accumulator, then |.|^2 (field.py:331-346)
-  struct Add {
-    const float2* F;
-    int M, N;
-    int64_t r0, c0;
-  };
-  struct Fallback {
-    float2* acc;            // the plan's one accumulator, shared by the groups in launch order
-    int64_t br0, bc0;       // the group's union box on the image (clipped)
-    int64_t brows, bcols;
-    std::vector<Add> adds;
-    double weight;
-  };
-  std::vector<Fallback> fallbacks;
+  // coherent groups whose Fields have several output grids: complex outputs,
+  // summed and squared into the image by one launch (field.py:331-346)
+  CoherentGroup* cgroups = nullptr;
+  CoherentAdd* cadds = nullptr;
+  int n_cgroups = 0;
   mftx_plan_info info = {};
   int use_graph = 0;
   hipGraphExec_t gexec = nullptr;
@@ -1913,29 +1902,17 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   const size_t o_top = lay.take(sizeof(TableOp) * std::max<size_t>(tables.ops.size(), 1));
   const size_t o_wf = lay.take(sizeof(Work) * std::max<size_t>(wf.size(), 1));
   const size_t o_pf = lay.take(sizeof(Problem) * std::max<size_t>(plan->pf.size(), 1));
-  // partial-overlap groups: each group's union box on the image (its Fields'
-  // placements clipped to the image, field.py:282-296); one accumulator of
-  // the largest box serves every group in turn (same stream, in order)
-  std::vector<std::array<int64_t, 4>> fb_box;  // r0, c0, rows, cols per several-class group (map order)
-  size_t fb_acc = 0;
-  if (!fast) {
-    int64_t most = 0;
-    for (auto& kv : groups) {
-      if (kv.second.size() < 2) continue;
-      int64_t r0 = image_rows, c0 = image_cols, r1 = 0, c1 = 0;
-      for (int c : kv.second) {
-        const ClassKey& K = cls[c].key;
-        r0 = std::min(r0, std::max<int64_t>(K.r0, 0));
-        c0 = std::min(c0, std::max<int64_t>(K.c0, 0));
-        r1 = std::max(r1, std::min<int64_t>(K.r0 + K.M, image_rows));
-        c1 = std::max(c1, std::min<int64_t>(K.c0 + K.N, image_cols));
-      }
-      const int64_t rows = std::max<int64_t>(r1 - r0, 0), cols = std::max<int64_t>(c1 - c0, 0);
-      fb_box.push_back({r0, c0, rows, cols});
-      most = std::max(most, rows * cols);
-    }
-    fb_acc = lay.take(sizeof(float2) * (size_t)std::max<int64_t>(most, 1));
+  // groups with several output grids: their classes' fields in map order
+  std::vector<CoherentGroup> cgroups;
+  std::vector<int> cadd_class;
+  for (auto& kv : groups) {
+    if (kv.second.size() < 2) continue;
+    cgroups.push_back(CoherentGroup{(int)cadd_class.size(), (int)kv.second.size(),
+                                    problems[cls[kv.second[0]].members[0]].weight});
+    cadd_class.insert(cadd_class.end(), kv.second.begin(), kv.second.end());
   }
+  const size_t o_cg = lay.take(sizeof(CoherentGroup) * std::max<size_t>(cgroups.size(), 1));
+  const size_t o_ca = lay.take(sizeof(CoherentAdd) * std::max<size_t>(cadd_class.size(), 1));
 
   if (!try_malloc(&plan->ws, lay.total)) {
     plan->ws = nullptr;
@@ -2014,6 +1991,15 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   up(plan->probs2c, p2c_launch.data(), sizeof(Problem) * p2c_launch.size());
   up(plan->segs, segs.data(), sizeof(Seg) * segs.size());
   up(plan->waves, iw.data(), sizeof(PhasorWave) * iw.size());
+  std::vector<CoherentAdd> cadds;
+  for (int c : cadd_class)
+    cadds.push_back(CoherentAdd{(const float2*)(base + cls[c].fbuf), cls[c].key.M, cls[c].key.N, (int)cls[c].key.r0,
+                                (int)cls[c].key.c0});
+  plan->cgroups = (CoherentGroup*)(base + o_cg);
+  plan->cadds = (CoherentAdd*)(base + o_ca);
+  plan->n_cgroups = (int)cgroups.size();
+  up(plan->cgroups, cgroups.data(), sizeof(CoherentGroup) * cgroups.size());
+  up(plan->cadds, cadds.data(), sizeof(CoherentAdd) * cadds.size());
   up(plan->row_phases, row_phases.data(), sizeof(RowPhase) * row_phases.size());
   up(plan->max_ops, maxes.data(), sizeof(MaxOp) * maxes.size());
   up(plan->works_f, wf.data(), sizeof(Work) * wf.size());
@@ -2064,26 +2050,6 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
                                               (long long)gi.pcol, (int)gi.lgroups.size(), c0.key.M, c0.key.N,
                                               c0.key.r0, c0.key.c0});
   }
-  {
-    size_t g = 0;
-    for (auto& kv : groups) {
-      if (kv.second.size() < 2) continue;
-      mftx_plan::Fallback fb;
-      fb.acc = (float2*)(base + fb_acc);
-      fb.br0 = fb_box[g][0];
-      fb.bc0 = fb_box[g][1];
-      fb.brows = fb_box[g][2];
-      fb.bcols = fb_box[g][3];
-      ++g;
-      fb.weight = problems[cls[kv.second[0]].members[0]].weight;
-      for (int c : kv.second) {
-        const ClassKey& K = cls[c].key;
-        fb.adds.push_back(mftx_plan::Add{(const float2*)(base + cls[c].fbuf), K.M, K.N, K.r0, K.c0});
-      }
-      plan->fallbacks.push_back(fb);
-    }
-  }
-
   // ---- info: algorithmic FLOPs are 8 per complex MAC of the cheaper order -------
   double fl = 0, g1 = 0, g2 = 0;
   for (auto& c : cls)
@@ -2122,7 +2088,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   plan->info.n_work1 = plan->nwork1;
   plan->info.n_work2 = plan->nwork2 + plan->nwork2c;
   int nl = (maxes.empty() ? 0 : 1) + (ops.empty() ? 0 : 1) + 1 + (w2.empty() ? 0 : 1) + (w2c.empty() ? 0 : 1) + (int)plan->reduces.size();
-  for (auto& fb : plan->fallbacks) nl += 2 + (int)fb.adds.size();  // clear, adds, |.|^2 into the image
+  nl += plan->n_cgroups ? 1 : 0;
   plan->info.n_launch = nl;
   *out = owned.release();
   return MFTX_OK;
@@ -2159,29 +2125,6 @@ static hipError_t launch_reduces(const mftx_plan* plan, void* image, int dtype, 
   return hipSuccess;
 }
 
-static hipError_t launch_fallbacks(const mftx_plan* plan, void* image, int dtype, int64_t ldi, int accumulate,
-                                   hipStream_t s) {
-  const size_t esz = dtype == 3 ? 8 : 4;
-  hipError_t e = hipSuccess;
-  if (!accumulate) e = launch_zero_rows(image, (int)esz, plan->img_rows, plan->img_cols, ldi, s);
-  for (auto& fb : plan->fallbacks) {
-    if (fb.brows <= 0 || fb.bcols <= 0) continue;  // every Field of the group lies off the image
-    if (e == hipSuccess) e = launch_zero(fb.acc, sizeof(float2) * fb.brows * fb.bcols, s);
-    for (auto& a : fb.adds) {
-      // clip F's placement to the image (field.py:282-296); acc holds the group's union box
-      const int64_t or0 = std::max<int64_t>(a.r0, 0), oc0 = std::max<int64_t>(a.c0, 0);
-      const int64_t or1 = std::min<int64_t>(a.r0 + a.M, plan->img_rows), oc1 = std::min<int64_t>(a.c0 + a.N, plan->img_cols);
-      if (or1 <= or0 || oc1 <= oc0 || e != hipSuccess) continue;
-      e = launch_insert(a.F, a.N, (int)(or0 - a.r0), (int)(oc0 - a.c0), (int)(or1 - or0), (int)(oc1 - oc0), fb.acc, 0,
-                        fb.bcols, (int)(or0 - fb.br0), (int)(oc0 - fb.bc0), 0, 1.0, s);
-    }
-    if (e == hipSuccess)
-      e = launch_insert(fb.acc, fb.bcols, 0, 0, (int)fb.brows, (int)fb.bcols, image, dtype, ldi, (int)fb.br0,
-                        (int)fb.bc0, 1, fb.weight, s);
-  }
-  return e;
-}
-
 // Stage 2: the intensity launch (classes alone in their coherent group) and
 // the complex-store launch (the classes of several-class groups).
 static hipError_t launch_stage2(const mftx_plan* plan, hipStream_t s) {
@@ -2198,14 +2141,14 @@ static hipError_t launch_stage2(const mftx_plan* plan, hipStream_t s) {
 // several-class groups add their |sum of fields|^2.
 static hipError_t launch_finish(const mftx_plan* plan, void* image, int dtype, int64_t ldi, int accumulate,
                                 hipStream_t s) {
-  if (plan->fallbacks.empty()) return launch_reduces(plan, image, dtype, ldi, accumulate, s);
-  hipError_t e = hipSuccess;
+  if (!plan->n_cgroups) return launch_reduces(plan, image, dtype, ldi, accumulate, s);
   if (!plan->reduces.empty()) {
-    e = launch_reduces(plan, image, dtype, ldi, accumulate, s);
+    const hipError_t e = launch_reduces(plan, image, dtype, ldi, accumulate, s);
+    if (e != hipSuccess) return e;
     accumulate = 1;
   }
-  if (e == hipSuccess) e = launch_fallbacks(plan, image, dtype, ldi, accumulate, s);
-  return e;
+  return launch_coherent(plan->cgroups, plan->n_cgroups, plan->cadds, image, dtype, ldi, (int)plan->img_rows,
+                         (int)plan->img_cols, accumulate, s);
 }
 
 static int plan_launch(mftx_plan* plan, void* image, int dtype, int64_t ldi, int accumulate) {
@@ -2265,7 +2208,7 @@ int mftx_plan_execute(mftx_plan* plan, void* image, int32_t image_dtype, int64_t
 // One execute's launch groups with a timing event before, between and after
 // them (ev[0..4]) on stream s.
 // The plan's launch groups in execute order (phasors, stage-1 GEMM, stage-2
-// GEMM, reduction or fallback), the first `upto` of them; with `ev`, an event
+// GEMM, reduction), the first `upto` of them; with `ev`, an event
 // is recorded before the first and after each.
 static hipError_t profile_launches(mftx_plan* plan, void* image, int dtype, int64_t ldi, hipStream_t s, int upto,
                                    const hipEvent_t* ev) {

@@ -242,6 +242,20 @@ hipError_t launch_reduce_partials(const float* partial, long long group_stride, 
                                   int rows, int cols, long long ldp, void* out, int out_dtype,
                                   long long ldo, int out_rows, int out_cols, int r0, int c0,
                                   int accumulate, hipStream_t s);
+// Coherent groups of a plan whose Fields have several output grids: group g's
+// Fields are adds[first .. first + count) of the launch.
+struct CoherentAdd {
+  const float2* F;      // M x N, row stride N
+  int M, N;
+  int r0, c0;           // image pixel of F[0][0] (may lie outside the image)
+};
+struct CoherentGroup {
+  int first, count;
+  double weight;
+};
+// image (+)= sum_g weight_g |sum of the group's Fields|^2
+hipError_t launch_coherent(const CoherentGroup* groups_dev, int ngroups, const CoherentAdd* adds_dev, void* image,
+                           int dtype, long long ldi, int rows, int cols, int accumulate, hipStream_t s);
 hipError_t launch_insert(const void* field, long long ldf, int fr0, int fc0, int h, int w,
                          void* out, int out_dtype, long long ldo, int or0, int oc0,
                          int intensity, double weight, hipStream_t s);
