@@ -260,6 +260,7 @@ struct mftx_plan {
   int nwork2c = 0;
   PhasorOp* phasor_ops = nullptr;  // device descriptors of the grouped phasor launch
   int n_phasor_ops = 0;
+  OperandSplit split{2, 1};
   long long phasor_threads = 0;
   struct Reduce {
     float* partial;
@@ -560,6 +561,7 @@ struct ManyBatch {
   std::vector<Problem> p1, p2;
   std::vector<Seg> s1, s2;
   std::vector<Work> w1, w2;
+  OperandSplit ph_split{2, 1}, pk_split{2, 1};
   long long ph_total = 0, pk_total = 0, mx_total = 0;
 };
 
@@ -586,6 +588,10 @@ static void many_build(const mftx_mft* mfts, int32_t count, int prec, int fixed,
   ws += mb.tables.place(ws);
 
   // ---- sources -----------------------------------------------------------------
+  long long ph_quads = 0, pk_quads = 0;
+  for (int32_t i = 0; i < count; ++i) (mfts[i].f ? pk_quads : ph_quads) += operand_quads(geo[i].r1, geo[i].k1, 1);
+  mb.ph_split = operand_split(ph_quads);
+  mb.pk_split = operand_split(pk_quads);
   auto source = [&](std::vector<PhasorOp>& ops, long long& total, const MftGeo& g, const mftx_mft& q) -> PhasorOp& {
     PhasorOp op = {};
     op.m = (int)q.m;
@@ -636,9 +642,9 @@ static void many_build(const mftx_mft* mfts, int32_t count, int prec, int fixed,
     }
     PhasorOp& op = q.f ? mb.packs.back() : mb.phops.back();
     op.nwave += 1;
-    mb.waves.push_back(PhasorWave{q.f ? 0.0 : q.inv_wl, g.g1.fold, g.x01, g.g2.fold, g.x02});
+    mb.waves.push_back(PhasorWave{q.f ? 0.0 : 4.0 * q.inv_wl, 4.0 * g.g1.fold, g.x01, 4.0 * g.g2.fold, g.x02});
     mb.op_of.push_back(q.f ? -(int)mb.packs.size() : (int)mb.phops.size() - 1);
-    (q.f ? mb.pk_total : mb.ph_total) = op.begin + phasor_threads(g.r1, g.k1, op.nwave);
+    (q.f ? mb.pk_total : mb.ph_total) = op.begin + operand_threads(g.r1, g.k1, op.nwave, q.f ? mb.pk_split : mb.ph_split);
   }
   mb.ws = ws;
 
@@ -736,9 +742,9 @@ static hipError_t many_tables(const ManyBatch& mb, int prec, const char* d, hipS
 static hipError_t many_launch(const ManyBatch& mb, int prec, const char* d, hipStream_t s) {
   hipError_t e = launch_absmax((const MaxOp*)(d + mb.o_mx), (int)mb.maxes.size(), mb.mx_total, s);
   if (e == hipSuccess)
-    e = launch_operands(prec, false, (const PhasorOp*)(d + mb.o_ph), (int)mb.phops.size(), mb.ph_total, s);
+    e = launch_operands(prec, false, mb.ph_split, (const PhasorOp*)(d + mb.o_ph), (int)mb.phops.size(), mb.ph_total, s);
   if (e == hipSuccess)
-    e = launch_operands(prec, true, (const PhasorOp*)(d + mb.o_pk), (int)mb.packs.size(), mb.pk_total, s);
+    e = launch_operands(prec, true, mb.pk_split, (const PhasorOp*)(d + mb.o_pk), (int)mb.packs.size(), mb.pk_total, s);
   if (e == hipSuccess)
     e = launch_gemm(prec, EPI_STORE_PACKED, mb.tile1, (const Work*)(d + mb.o_w1), (int)mb.w1.size(),
                     (const Problem*)(d + mb.o_p1), (const Seg*)(d + mb.o_s1), s);
@@ -952,10 +958,10 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
   };
   const int piece1 = piece(p1.sblocks, nkb1, tile[0]), piece2 = piece(p2.sblocks, nkb2, tile[1]);
   // workspace: descriptors, maxima and inverse scale, operands, tables
-  const size_t o_max = round_up(sizeof(OneDesc), 256), o_a1 = o_max + 512;
+  const size_t o_max = round_up(sizeof(OneDesc), 256), o_a1 = o_max + 2048;
   const size_t o_a2 = o_a1 + folded_bytes(g.r1, g.k1), o_t1 = o_a2 + plain_bytes(g.c1, nkb2);
   const size_t o_t2 = o_t1 + table_bytes(piece1, nkb1), need = o_t2 + table_bytes(piece2, nkb2);
-  static_assert((kMaxBlocks + 1) * sizeof(float) <= 512, "maxima and inverse scale fit their space");
+  static_assert((kMaxBlocks + 1) * sizeof(float) <= 2048, "maxima and inverse scale fit their space");
   int rc = MFTX_OK;
   if (!ws) {
     rc = ensure_ws(ctx, need);
@@ -989,7 +995,7 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
     one.op.sc = ScaleSrc{part, inv, m * n <= 8192 ? 0 : mx.nblk, 0};
     p2.inv = inv;
   }
-  one.wave = PhasorWave{0.0, g.g1.fold, g.x01, g.g2.fold, g.x02};
+  one.wave = PhasorWave{0.0, 4.0 * g.g1.fold, g.x01, 4.0 * g.g2.fold, g.x02};
   one.tab[0] = TableOp{g.alpha1, g.k1 & 1 ? 0.0 : 0.5, g.g1.y0, piece1, nkb1, 0, 0, base + o_t1, 0};
   one.tab[1] = TableOp{g.alpha2, g.r1 & 1 ? 0.0 : 0.5, g.g2.y0, piece2, nkb2, 0, 0, base + o_t2, 0};
   one.desc.seg[0] = Seg{base + o_a1, base + o_t1, 0.0, nkb1, nkb1, nkb1, 0};
@@ -1957,8 +1963,8 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   std::vector<PhasorWave> iw(wave_slots.size());
   for (size_t i = 0; i < wave_slots.size(); ++i) {
     const Slot& sl = wave_slots[i];
-    iw[i] = PhasorWave{1.0 / wavelengths[std::get<0>(sl)], std::get<1>(sl), std::get<2>(sl), std::get<3>(sl),
-                       std::get<4>(sl)};
+    iw[i] = PhasorWave{4.0 / wavelengths[std::get<0>(sl)], 4.0 * std::get<1>(sl), std::get<2>(sl),
+                       4.0 * std::get<3>(sl), std::get<4>(sl)};
   }
   for (size_t i = 0; i < maxes.size(); ++i) maxes[i].part = (float*)(base + max_part[i]);
 
@@ -2011,7 +2017,9 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   }
 
   std::vector<PhasorOp> ops;
-  long long pthreads = 0;
+  long long pthreads = 0, quads = 0;
+  for (auto& kv : tops) quads += operand_quads(kv.second.R, kv.second.K, kv.second.nslot);
+  plan->split = operand_split(quads);
   for (auto& kv : tops) {
     const TileOp& op = kv.second;
     const mftx_tile& T = tiles[kv.first.first];
@@ -2034,7 +2042,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
       ph.sc = ScaleSrc{(const float*)(base + cm.part), (float*)(base + cm.inv), cm.n, 0};
     }
     ph.begin = group_begin(pthreads);
-    pthreads = ph.begin + phasor_threads(op.R, op.K, ph.nwave);
+    pthreads = ph.begin + operand_threads(op.R, op.K, ph.nwave, plan->split);
     ops.push_back(ph);
   }
   plan->phasor_ops = (PhasorOp*)(base + o_ops);
@@ -2100,7 +2108,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
 static hipError_t launch_phasors(const mftx_plan* plan, hipStream_t s) {
   const hipError_t e = launch_absmax(plan->max_ops, plan->n_max_ops, plan->max_blocks, s);
   if (e != hipSuccess) return e;
-  return launch_operands(plan->prec, false, plan->phasor_ops, plan->n_phasor_ops, plan->phasor_threads, s);
+  return launch_operands(plan->prec, false, plan->split, plan->phasor_ops, plan->n_phasor_ops, plan->phasor_threads, s);
 }
 
 static hipError_t launch_reduces(const mftx_plan* plan, void* image, int dtype, int64_t ldi, int accumulate,

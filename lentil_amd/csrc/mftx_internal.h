@@ -133,9 +133,9 @@ struct MaxOp {
   float* part;
   long long begin;
 };
-constexpr int kMaxBlocks = 64;  // blocks (and part entries) of one absolute-maximum job, at most
+constexpr int kMaxBlocks = 256;  // blocks (and part entries) of one absolute-maximum job, at most
 inline int max_blocks(long long m, long long n) {
-  const long long b = (m * n + 4095) / 4096;
+  const long long b = (m * n + 1023) / 1024;
   return (int)(b < 1 ? 1 : b > kMaxBlocks ? kMaxBlocks : b);
 }
 
@@ -153,7 +153,8 @@ inline size_t table_bytes(int nsb, int nkb) { return (size_t)nsb * nkb * B_BLOCK
 // Twiddles of the f16 form are scaled so the lo parts of small ones stay normal.
 __host__ __device__ inline float tw_scale(int prec) { return prec == PREC_FP32 ? 256.0f : 1.0f; }
 
-// Per-wavelength parameters of a phasor launch: the phase opd * inv_wl, the
+// Per-wavelength parameters of a phasor launch, in quarter turns (rates times
+// 4, so the kernels reduce the phase without a product): the phase opd * inv_wl, the
 // stage-1 fold cis(fold * (x0 + k)) along the operand's K index k, and the
 // stage-2 fold cis(fold2 * (x02 + r)) along its row index r (stage 1's C row r
 // is the operand's row r times the row's phase, so the stage-1 output comes
@@ -170,7 +171,6 @@ struct PhasorWave {
 // nwave = 1): the folded, paired operand of the m x n source (rows are the
 // source's columns when trans) for every wavelength, written wave_stride bytes
 // apart.  `begin` is the op's first thread in the grouped launch.
-constexpr int PH_WAVES = 4;  // wavelengths per phasor thread
 struct PhasorOp {
   const void* amp;      // amplitude, or the complex source
   const void* opd;      // OPD; null for a complex source
@@ -183,12 +183,28 @@ struct PhasorOp {
   ScaleSrc sc;
   long long begin;
 };
+// How an operand launch splits its work: K pairs (2, 4 or 8) and wavelengths
+// per thread.
+struct OperandSplit {
+  int np, waves;
+};
 // threads of one wavelength group of an r x k operand (whole waves)
-__host__ __device__ inline long long group_threads(long long r, long long k) {
-  return 64LL * (((long long)pair_blocks(r) * pair_blocks(k) + 1) / 2);
+__host__ __device__ inline long long group_threads(long long r, long long k, int np) {
+  return ((long long)pair_blocks(r) * pair_blocks(k) * (256 / np) + 63) / 64 * 64;
 }
-__host__ __device__ inline long long phasor_threads(long long r, long long k, int nwave) {
-  return group_threads(r, k) * ((nwave + PH_WAVES - 1) / PH_WAVES);
+__host__ __device__ inline long long operand_threads(long long r, long long k, int nwave, OperandSplit sp) {
+  return group_threads(r, k, sp.np) * ((nwave + sp.waves - 1) / sp.waves);
+}
+// The split of a launch of `quads` (row pair, K pair) quads over all its
+// sources and wavelengths.  Large launches: 4 pairs and 4 wavelengths per
+// thread, so a source is read once per 4 wavelengths.  Where that would leave
+// fewer than two waves per SIMD (131072 threads), one wavelength and 2 pairs:
+// the launch then takes the latency of 8 samples instead of 64.
+inline OperandSplit operand_split(long long quads) {
+  return quads / 16 >= 131072 ? OperandSplit{4, 4} : OperandSplit{2, 1};
+}
+inline long long operand_quads(long long r, long long k, int nwave) {
+  return 256LL * pair_blocks(r) * pair_blocks(k) * nwave;
 }
 
 // Grouped launches (phasor, table, maximum ops): blocks of kGroupBlock threads, and
@@ -206,8 +222,8 @@ hipError_t launch_gemm_one(int prec, int epi, int tile, int rblocks, int sb0, in
                            const Seg* seg, hipStream_t s);
 // every operand source of a plan in one launch (ops_dev on the device, sorted
 // by begin): pupil phasors, or (cplx) complex arrays
-hipError_t launch_operands(int prec, bool cplx, const PhasorOp* ops_dev, int nops, long long total_threads,
-                           hipStream_t s);
+hipError_t launch_operands(int prec, bool cplx, OperandSplit sp, const PhasorOp* ops_dev, int nops,
+                           long long total_threads, hipStream_t s);
 // every twiddle table / absolute maximum in one launch (sorted by begin)
 hipError_t launch_tables(int prec, const TableOp* ops_dev, int nops, long long total_threads, hipStream_t s);
 hipError_t launch_absmax(const MaxOp* ops_dev, int nops, long long total_blocks, hipStream_t s);

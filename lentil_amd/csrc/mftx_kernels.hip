@@ -131,47 +131,55 @@ __device__ __forceinline__ PhasorWave load_wave(cptr<const PhasorWave> p) {
 }
 
 // One thread per (op, 16-pair row block, K block of 16 pairs, row pair of the
-// block, half of the K block, group of PH_WAVES wavelengths): 8 K pairs of one
-// row pair, 32 source samples, read once; for each wavelength the four
+// block, NP of the K block's pairs, group of sp.waves wavelengths): NP K pairs
+// of one row pair, 4 NP source samples, read once; for each wavelength the four
 // samples of a (row, K) quad, each with its phase
 //     opd * inv_wl + fold * (x0 + k) + fold2 * (x02 + r),
 // are combined into the even and odd rows' even and odd parts, split and
-// stored as 16 16-byte pieces.  32 consecutive threads write one K block, so
-// a store covers whole 256-byte runs.
-template <int PREC, bool CPLX, typename Waves>
-__device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave, long long u, float scale) {
+// stored as 16 pieces of 2 NP bytes.  Threads run along K within a row's 8
+// pairs, then along the rows, so a store covers whole 256-byte runs.
+//
+// Bound by the arithmetic of the phases (about 40 instructions per sample and
+// wavelength, several FP64) beside the stores.  NP = 4 holds 48 registers of
+// source and 32 of result, four waves per SIMD; NP = 8 left room for two.
+// Where every sample of a wave is outside the aperture (amplitude 0) the
+// phases are skipped.
+template <int PREC, bool CPLX, int NP, typename Waves>
+__device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave, int waves, long long u, float scale) {
+  static_assert(NP == 2 || NP == 4 || NP == 8, "a thread's pairs lie in one half of a K block");
+  constexpr int SUB = 8 / NP;  // threads per (row pair, half K block)
   const int R = op.trans ? op.n : op.m, K = op.trans ? op.m : op.n;
   const int nrb = pair_blocks(R), nkb = pair_blocks(K);
   // a wavelength group spans whole waves, so its descriptors are scalar loads
-  const long long per_group = group_threads(R, K);
+  const long long per_group = group_threads(R, K, NP);
   const int g = __builtin_amdgcn_readfirstlane((int)(u / per_group));
   const int v = (int)(u % per_group);
-  if (v >= 32 * nrb * nkb) return;
-  const int lr = v & 15, kh = (v >> 4) & 1, blk = v >> 5;
+  if (v >= 32 * SUB * nrb * nkb) return;
+  const int sub = v & (SUB - 1), lr = (v / SUB) & 15, kh = (v / (16 * SUB)) & 1, blk = v / (32 * SUB);
   const int kb = blk % nkb, rb = blk / nkb;
   int r2[2];
   pair_index(R, rb * 16 + lr, r2[0], r2[1]);
-  const int kp0 = kb * 16 + kh * 8;
+  const int kp0 = kb * 16 + kh * 8 + sub * NP;
   const bool even_k = !(K & 1);
   const int kh2 = K >> 1;
-  // K index of pair kp0 + i: plus side kh2 + kp0 + i, minus side kminus0 - i
+  // K index of pair kp0 + i: plus side kplus0 + i, minus side kminus0 - i
   const int kplus0 = kh2 + kp0, kminus0 = even_k ? kh2 - 1 - kp0 : kh2 - kp0;
-  const int w0 = g * PH_WAVES, nw = min(op.nwave - w0, PH_WAVES);
-  char* out = (char*)op.dst + ((long long)rb * nkb + kb) * A_BLOCK + 16 * (lr + 32 * kh);
+  const int w0 = g * waves, nw = min(op.nwave - w0, waves);
+  char* out = (char*)op.dst + ((long long)rb * nkb + kb) * A_BLOCK + 16 * (lr + 32 * kh) + 2 * NP * sub;
 
   // every load is issued before any math and none sits behind a branch: a
   // sample outside the array reads element 0 and is zeroed afterwards
-  float a[2][2][8];                          // amplitude [row side][k side][pair]
-  double o[CPLX ? 1 : 2][CPLX ? 1 : 2][CPLX ? 1 : 8];
-  float ci[CPLX ? 2 : 1][CPLX ? 2 : 1][CPLX ? 8 : 1];
+  float a[2][2][NP];                          // amplitude [row side][k side][pair]
+  double o[CPLX ? 1 : 2][CPLX ? 1 : 2][CPLX ? 1 : NP];
+  float ci[CPLX ? 2 : 1][CPLX ? 2 : 1][CPLX ? NP : 1];
 #pragma unroll
   for (int rs = 0; rs < 2; ++rs)
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
-      long long ia[8];
-      bool in[8];
+      long long ia[NP];
+      bool in[NP];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < NP; ++i) {
         const int k = ks ? kminus0 - i : kplus0 + i;
         in[i] = r2[rs] >= 0 && k >= 0 && k < K && !(ks && !even_k && kp0 + i == 0);
         const long long r = r2[rs], kk = k;
@@ -179,88 +187,106 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
       }
       if constexpr (CPLX) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < NP; ++i) {
           const float2 e = load_elem(op.amp, op.amp_dtype, ia[i]);
-          a[rs][ks][i] = in[i] ? e.x : 0.f;
-          ci[rs][ks][i] = in[i] ? e.y : 0.f;
+          a[rs][ks][i] = in[i] ? e.x * scale : 0.f;
+          ci[rs][ks][i] = in[i] ? e.y * scale : 0.f;
         }
       } else {
         if (op.amp_dtype == 3) {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) a[rs][ks][i] = (float)((gptr<const double>)op.amp)[ia[i]];
+          for (int i = 0; i < NP; ++i) a[rs][ks][i] = (float)((gptr<const double>)op.amp)[ia[i]];
         } else {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) a[rs][ks][i] = ((gptr<const float>)op.amp)[ia[i]];
+          for (int i = 0; i < NP; ++i) a[rs][ks][i] = ((gptr<const float>)op.amp)[ia[i]];
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < NP; ++i) {
           const int k = ks ? kminus0 - i : kplus0 + i;
           const long long r = r2[rs], kk = k;
           ia[i] = in[i] ? (op.trans ? kk * op.ld_opd + r : r * op.ld_opd + kk) : 0;
         }
         if (op.opd_dtype == 3) {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) o[rs][ks][i] = ((gptr<const double>)op.opd)[ia[i]];
+          for (int i = 0; i < NP; ++i) o[rs][ks][i] = ((gptr<const double>)op.opd)[ia[i]];
         } else {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) o[rs][ks][i] = (double)((gptr<const float>)op.opd)[ia[i]];
+          for (int i = 0; i < NP; ++i) o[rs][ks][i] = (double)((gptr<const float>)op.opd)[ia[i]];
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < NP; ++i) {
           a[rs][ks][i] = in[i] ? a[rs][ks][i] * scale : 0.f;
           o[rs][ks][i] = in[i] ? o[rs][ks][i] : 0.0;
         }
       }
     }
+  bool lit = true;
+  if constexpr (!CPLX) {
+    // a phase that is not finite makes even a dark sample's phasor NaN
+    lit = false;
+#pragma unroll
+    for (int i = 0; i < 4 * NP; ++i) {
+      const float x = a[i / (2 * NP)][i / NP % 2][i % NP];
+      const double y = o[i / (2 * NP)][i / NP % 2][i % NP];
+      lit = lit || x != 0.f || !(__builtin_fabs(y) < 1e300);
+    }
+    lit = __any(lit);
+  }
 #pragma unroll 1
   for (int j = 0; j < nw; ++j) {
     const PhasorWave pw = wave(w0 + j);
     const bool folded = pw.fold != 0.0 || pw.fold2 != 0.0;
-    // phase of pair 0 of each quadrant; K advances by +-1 per pair
-    double base[2][2];
+    uint32_t w[2][2][4][NP / 2];  // [row parity][part][plane][word]
+    if (!lit) {
 #pragma unroll
-    for (int rs = 0; rs < 2; ++rs)
+      for (int i = 0; i < 16 * (NP / 2); ++i) w[i / (8 * NP / 2)][i / (4 * NP / 2) % 2][i / (NP / 2) % 4][i % (NP / 2)] = 0u;
+    } else {
+      // phase of pair 0 of each quadrant; K advances by +-1 per pair
+      double base[2][2];
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        base[rs][ks] = __builtin_fma(pw.fold, pw.x0 + (double)(ks ? kminus0 : kplus0),
-                                     pw.fold2 * (pw.x02 + (double)r2[rs]));
-    uint32_t w[2][2][4][4];  // [row parity][part][plane][word]
+      for (int rs = 0; rs < 2; ++rs)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float2 p[2][2][2];  // [row parity][part][pair]
+        for (int ks = 0; ks < 2; ++ks)
+          base[rs][ks] = __builtin_fma(pw.fold, pw.x0 + (double)(ks ? kminus0 : kplus0),
+                                       pw.fold2 * (pw.x02 + (double)r2[rs]));
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int i = 2 * t + q;
-        float2 e[2][2];
+      for (int t = 0; t < NP / 2; ++t) {
+        float2 p[2][2][2];  // [row parity][part][pair]
 #pragma unroll
-        for (int rs = 0; rs < 2; ++rs)
+        for (int q = 0; q < 2; ++q) {
+          const int i = 2 * t + q;
+          float2 e[2][2];
 #pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            const double ph = __builtin_fma(ks ? -pw.fold : pw.fold, (double)i, base[rs][ks]);
-            if constexpr (CPLX) {
-              const float2 z = make_float2(a[rs][ks][i] * scale, ci[rs][ks][i] * scale);
-              e[rs][ks] = folded ? cmul(z, cis_turns(ph)) : z;
-            } else {
-              const float2 c = cis_turns(__builtin_fma(o[rs][ks][i], pw.inv_wl, ph));
-              e[rs][ks] = make_float2(a[rs][ks][i] * c.x, a[rs][ks][i] * c.y);
+          for (int rs = 0; rs < 2; ++rs)
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+              const double ph = __builtin_fma(ks ? -pw.fold : pw.fold, (double)i, base[rs][ks]);
+              if constexpr (CPLX) {
+                const float2 z = make_float2(a[rs][ks][i], ci[rs][ks][i]);
+                e[rs][ks] = folded ? cmul(z, cis_quarter(ph)) : z;
+              } else {
+                const float2 c = cis_quarter(__builtin_fma(o[rs][ks][i], pw.inv_wl, ph));
+                e[rs][ks] = make_float2(a[rs][ks][i] * c.x, a[rs][ks][i] * c.y);
+              }
             }
+#pragma unroll
+          for (int par = 0; par < 2; ++par) {
+            const float2 kp = par ? make_float2(e[0][0].x - e[1][0].x, e[0][0].y - e[1][0].y)
+                                  : make_float2(e[0][0].x + e[1][0].x, e[0][0].y + e[1][0].y);
+            const float2 km = par ? make_float2(e[0][1].x - e[1][1].x, e[0][1].y - e[1][1].y)
+                                  : make_float2(e[0][1].x + e[1][1].x, e[0][1].y + e[1][1].y);
+            p[par][0][q] = make_float2(kp.x + km.x, kp.y + km.y);
+            p[par][1][q] = make_float2(kp.x - km.x, kp.y - km.y);
           }
-#pragma unroll
-        for (int par = 0; par < 2; ++par) {
-          const float sg = par ? -1.f : 1.f;
-          const float2 kp = make_float2(__builtin_fmaf(sg, e[1][0].x, e[0][0].x), __builtin_fmaf(sg, e[1][0].y, e[0][0].y));
-          const float2 km = make_float2(__builtin_fmaf(sg, e[1][1].x, e[0][1].x), __builtin_fmaf(sg, e[1][1].y, e[0][1].y));
-          p[par][0][q] = make_float2(kp.x + km.x, kp.y + km.y);
-          p[par][1][q] = make_float2(kp.x - km.x, kp.y - km.y);
         }
+#pragma unroll
+        for (int par = 0; par < 2; ++par)
+#pragma unroll
+          for (int part = 0; part < 2; ++part) {
+            split2<PREC>(p[par][part][0].x, p[par][part][1].x, w[par][part][0][t], w[par][part][1][t]);
+            split2<PREC>(p[par][part][0].y, p[par][part][1].y, w[par][part][2][t], w[par][part][3][t]);
+          }
       }
-#pragma unroll
-      for (int par = 0; par < 2; ++par)
-#pragma unroll
-        for (int part = 0; part < 2; ++part) {
-          split2<PREC>(p[par][part][0].x, p[par][part][1].x, w[par][part][0][t], w[par][part][1][t]);
-          split2<PREC>(p[par][part][0].y, p[par][part][1].y, w[par][part][2][t], w[par][part][3][t]);
-        }
     }
     char* d = out + (long long)(w0 + j) * op.wave_stride;
 #pragma unroll
@@ -269,33 +295,47 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
       for (int part = 0; part < 2; ++part)
 #pragma unroll
         for (int pl = 0; pl < 4; ++pl) {
-          const uint32_t (&x)[4] = w[par][part][pl];
-          *(gptr<v4u32>)(d + (part * 4 + pl) * FRAG + par * 256) = v4u32{x[0], x[1], x[2], x[3]};
+          const uint32_t (&x)[NP / 2] = w[par][part][pl];
+          char* dp = d + (part * 4 + pl) * FRAG + par * 256;
+          if constexpr (NP == 8) *(gptr<v4u32>)dp = v4u32{x[0], x[1], x[2], x[3]};
+          else if constexpr (NP == 4) *(gptr<v2u32>)dp = v2u32{x[0], x[1]};
+          else *(gptr<uint32_t>)dp = x[0];
         }
   }
 }
 
 // Every operand source of a plan in one launch (the op is found by a
 // block-uniform search).
-template <int PREC, bool CPLX>
-__global__ __launch_bounds__(kGroupBlock, 2) void operand_group_kernel(const PhasorOp* __restrict__ ops, int nops) {
+template <int PREC, bool CPLX, int NP>
+__global__ __launch_bounds__(kGroupBlock, 4) void operand_group_kernel(const PhasorOp* __restrict__ ops, int nops,
+                                                                       int waves) {
   const long long b0 = (long long)blockIdx.x * kGroupBlock;
   const PhasorOp& op = ops[block_op(ops, nops, b0)];
   const float scale = block_scale(op.sc, b0 == op.begin);
   const long long u = b0 + threadIdx.x - op.begin;
-  if (u >= phasor_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, op.nwave)) return;
-  operand_thread<PREC, CPLX>(op, [&](int w) { return load_wave((cptr<const PhasorWave>)op.waves + w); }, u, scale);
+  if (u >= operand_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, op.nwave, OperandSplit{NP, waves})) return;
+  operand_thread<PREC, CPLX, NP>(op, [&](int w) { return load_wave((cptr<const PhasorWave>)op.waves + w); }, waves, u,
+                                 scale);
 }
 
-hipError_t launch_operands(int prec, bool cplx, const PhasorOp* ops, int nops, long long total, hipStream_t s) {
+template <int PREC, bool CPLX>
+static void launch_operands_of(OperandSplit sp, dim3 grid, const PhasorOp* ops, int nops, hipStream_t s) {
+  if (sp.np == 2)
+    hipLaunchKernelGGL((operand_group_kernel<PREC, CPLX, 2>), grid, dim3(kGroupBlock), 0, s, ops, nops, sp.waves);
+  else
+    hipLaunchKernelGGL((operand_group_kernel<PREC, CPLX, 4>), grid, dim3(kGroupBlock), 0, s, ops, nops, sp.waves);
+}
+
+hipError_t launch_operands(int prec, bool cplx, OperandSplit sp, const PhasorOp* ops, int nops, long long total,
+                           hipStream_t s) {
   if (total <= 0 || nops <= 0) return hipSuccess;
-  const dim3 grid((unsigned)((total + kGroupBlock - 1) / kGroupBlock)), block(kGroupBlock);
+  const dim3 grid((unsigned)((total + kGroupBlock - 1) / kGroupBlock));
   if (prec == PREC_BF16X3) {
-    if (cplx) hipLaunchKernelGGL((operand_group_kernel<PREC_BF16X3, true>), grid, block, 0, s, ops, nops);
-    else hipLaunchKernelGGL((operand_group_kernel<PREC_BF16X3, false>), grid, block, 0, s, ops, nops);
+    if (cplx) launch_operands_of<PREC_BF16X3, true>(sp, grid, ops, nops, s);
+    else launch_operands_of<PREC_BF16X3, false>(sp, grid, ops, nops, s);
   } else {
-    if (cplx) hipLaunchKernelGGL((operand_group_kernel<PREC_FP32, true>), grid, block, 0, s, ops, nops);
-    else hipLaunchKernelGGL((operand_group_kernel<PREC_FP32, false>), grid, block, 0, s, ops, nops);
+    if (cplx) launch_operands_of<PREC_FP32, true>(sp, grid, ops, nops, s);
+    else launch_operands_of<PREC_FP32, false>(sp, grid, ops, nops, s);
   }
   return hipGetLastError();
 }
@@ -414,7 +454,7 @@ hipError_t launch_row_phases(const RowPhase* ops, int nops, int most_rows, hipSt
 // descriptors in one launch, everything passed by value
 // --------------------------------------------------------------------------
 template <int PREC>
-__global__ __launch_bounds__(kGroupBlock, 2) void prepare_one_kernel(PhasorOp op, PhasorWave wave, TableOp tab0,
+__global__ __launch_bounds__(kGroupBlock, 4) void prepare_one_kernel(PhasorOp op, PhasorWave wave, TableOp tab0,
                                                                      TableOp tab1, OneDesc desc, OneDesc* out,
                                                                      int op_blocks, int tab_blocks) {
   const int b = (int)blockIdx.x;
@@ -431,8 +471,8 @@ __global__ __launch_bounds__(kGroupBlock, 2) void prepare_one_kernel(PhasorOp op
     }
     if (b == 0 && threadIdx.x == 0) *out = desc;
     const long long u = (long long)b * kGroupBlock + threadIdx.x;
-    if (u < phasor_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, 1))
-      operand_thread<PREC, true>(op, [=](int) { return wave; }, u, scale);
+    if (u < operand_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, 1, OperandSplit{2, 1}))
+      operand_thread<PREC, true, 2>(op, [=](int) { return wave; }, 1, u, scale);
     return;
   }
   long long u = (long long)(b - op_blocks) * kGroupBlock + threadIdx.x;
@@ -461,7 +501,8 @@ hipError_t launch_prepare_one(int prec, const OneMft& one, const MaxOp& mx, hipS
   if (prec == PREC_FP32 && one.op.sc.n > 0) hipLaunchKernelGGL(absmax_one_kernel, dim3(mx.nblk), dim3(kGroupBlock), 0, s, mx);
   const PhasorOp& op = one.op;
   const int op_blocks =
-      (int)((phasor_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, 1) + kGroupBlock - 1) / kGroupBlock);
+      (int)((operand_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, 1, OperandSplit{2, 1}) + kGroupBlock - 1) /
+            kGroupBlock);
   int blocks[2];
   for (int t = 0; t < 2; ++t)
     blocks[t] = (int)((table_threads(one.tab[t].nsb, one.tab[t].nkb) + kGroupBlock - 1) / kGroupBlock);
