@@ -1220,16 +1220,13 @@ int mftx_fft_filter(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int
     return fail(ctx, MFTX_EINVAL, "bad filter shape");
   if (precision != MFTX_PREC_FP32 && precision != MFTX_PREC_BF16X3) return fail(ctx, MFTX_EINVAL, "unknown precision");
   HIPCHK(ctx, hipSetDevice(ctx->device));
-  const int64_t n = rows * cols;
-  const int64_t nb = (n + 255) / 256;
-  const size_t fbytes = (size_t)round_up(n * (int64_t)sizeof(float2), 256);
-  int rc = ensure_aux(ctx, 2 * fbytes + sizeof(double) * (size_t)(2 * nb + 2));
+  const size_t fbytes = (size_t)round_up(rows * cols * (int64_t)sizeof(float2), 256);
+  int rc = ensure_aux(ctx, 2 * fbytes + sizeof(double) * 2 * kMaxPart);
   if (rc) return rc;
   char* a = (char*)ctx->aux;
   float2* F = (float2*)a;
   float2* Y = (float2*)(a + fbytes);
   double* part = (double*)(a + 2 * fbytes);
-  double* sums = part + 2 * nb;
   // fft2 then ifft2 as MFTs with alpha = 1/N: input coordinate r and output
   // coordinate u (uncentred) are r - N//2 + N//2 and (u - N//2) + N//2,
   // offsets taken modulo N
@@ -1265,10 +1262,10 @@ int mftx_fft_filter(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int
   b.w = nullptr;
   rc = dft2_many_run(ctx, &b, 1, precision);
   if (rc) return rc;
-  HIPCHK(ctx, launch_magnitude(Y, cols, rows, cols, out, out_dtype, ldo, part, sums + 1, ctx->stream));
+  HIPCHK(ctx, launch_magnitude(Y, cols, rows, cols, out, out_dtype, ldo, part, ctx->stream));
   if (normalize) {
-    HIPCHK(ctx, launch_sum(img, dtype, rows, cols, ld, part + nb, sums, ctx->stream));
-    HIPCHK(ctx, launch_scale_ratio(out, out_dtype, rows, cols, ldo, sums, sums + 1, ctx->stream));
+    HIPCHK(ctx, launch_sum(img, dtype, rows, cols, ld, part + kMaxPart, ctx->stream));
+    HIPCHK(ctx, launch_scale_ratio(out, out_dtype, rows, cols, ldo, part + kMaxPart, part, ctx->stream));
   }
   return MFTX_OK;
 }
@@ -1292,9 +1289,8 @@ int mftx_rescale(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int64_
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const int npad = 12;  // the most any mode pads
   const int64_t np_ = (rows + 2 * npad) * (cols + 2 * npad), no = out_rows * out_cols;
-  const int64_t nb = (std::max(np_, no) + 255) / 256;
   const size_t b_pad = (size_t)round_up(np_ * 8, 256), b_out = (size_t)round_up(no * 8, 256);
-  int rc = ensure_aux(ctx, 2 * b_pad + 3 * b_out + sizeof(double) * (size_t)(nb + 4));
+  int rc = ensure_aux(ctx, 2 * b_pad + 3 * b_out + sizeof(double) * 4 * kMaxPart);
   if (rc) return rc;
   char* a = (char*)ctx->aux;
   double* P = (double*)a;
@@ -1303,7 +1299,6 @@ int mftx_rescale(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int64_
   double* raw_im = (double*)(a + 2 * b_pad + b_out);
   double* mval = (double*)(a + 2 * b_pad + 2 * b_out);
   double* part = (double*)(a + 2 * b_pad + 3 * b_out);
-  double* sums = part + nb;
   // the mask's dtype sets the threshold (util.py:338-339, numpy finfo eps of
   // the mask, or of the image's real dtype when the mask is derived from it)
   const int mdt = mask ? mask_dtype : dtype;
@@ -1311,7 +1306,7 @@ int mftx_rescale(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int64_
   const double eps = single ? 1.1920928955078125e-07 : 2.220446049250313e-16;
   HIPCHK(ctx, launch_rescale(img, dtype, rows, cols, ld, mask ? mask : img, mask ? 2 : 1, mdt, mask ? ldm : ld, eps,
                              scale, out_rows, out_cols, order, mode, unitary, out, out_dtype, ldo, P, T, raw, raw_im,
-                             mval, part, sums, ctx->stream));
+                             mval, part, ctx->stream));
   return MFTX_OK;
 }
 

@@ -21,23 +21,43 @@ __device__ __forceinline__ double load_real(const void* p, int dtype, long long 
   return dtype == 3 ? ((const double*)p)[i] : (double)((const float*)p)[i];
 }
 
+// component `comp` (0 real, 1 imaginary) of element i of a real or complex array
+__device__ __forceinline__ double load_component(const void* p, int dtype, long long i, int comp) {
+  switch (dtype) {
+    case 0: return comp ? ((const float2*)p)[i].y : ((const float2*)p)[i].x;
+    case 2: return comp ? ((const double2*)p)[i].y : ((const double2*)p)[i].x;
+    default: return comp ? 0.0 : load_real(p, dtype, i);
+  }
+}
+
 __device__ __forceinline__ void store_real(void* p, int dtype, long long i, double v) {
   if (dtype == 3) ((double*)p)[i] = v;
   else ((float*)p)[i] = (float)v;
 }
 
-// Sum of v over the block into part[blockIdx.x] (fixed order: deterministic).
-__device__ void block_partial(double v, double* part) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+// Sum of v over the block, in every thread (fixed order: deterministic).
+__device__ double block_sum(double v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   __shared__ double w[kBlock / 64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) w[wave] = v;
+  __syncthreads();  // an earlier sum's readers are done
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < kBlock / 64; ++i) s += w[i];
-    part[blockIdx.x] = s;
-  }
+  double s = 0.0;
+  for (int i = 0; i < kBlock / 64; ++i) s += w[i];
+  return s;
+}
+
+// Reductions leave one partial sum per block, at most kMaxPart of them, and
+// whoever needs the total adds them itself: a launch to finish the sum took
+// longer (5 us) than reading 1024 doubles in every block of the consumer.
+__device__ double total(const double* __restrict__ part, int n) {
+  double v = 0.0;
+  for (int i = threadIdx.x; i < n; i += kBlock) v += part[i];
+  return block_sum(v);
+}
+int part_blocks(long long n) {
+  const long long b = (n + kBlock - 1) / kBlock;
+  return (int)(b < 1 ? 1 : b > kMaxPart ? kMaxPart : b);
 }
 
 unsigned blocks_for(long long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -74,77 +94,71 @@ hipError_t launch_rebin(const void* src, int dtype, long long nimg, long long ro
 // reductions and the weight-preserving rescale of the filters
 // --------------------------------------------------------------------------
 
-// part[b] = sum of a real rows x cols array over block b's elements
-__global__ void sum_kernel(const void* __restrict__ x, int dtype, long long rows, long long cols, long long ld,
-                           double* __restrict__ part) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+// part[b] = sum of component comp (0 real, 1 imaginary) of a rows x cols array
+// over block b's elements (every gridDim-th run of 256)
+__global__ void sum_kernel(const void* __restrict__ x, int dtype, int comp, long long rows, long long cols,
+                           long long ld, double* __restrict__ part) {
+  const long long n = rows * cols, step = (long long)gridDim.x * kBlock;
   double v = 0.0;
-  if (t < rows * cols) v = load_real(x, dtype, (t / cols) * ld + t % cols);
-  block_partial(v, part);
+#pragma unroll 4
+  for (long long t = (long long)blockIdx.x * kBlock + threadIdx.x; t < n; t += step)
+    v += load_component(x, dtype, ld == cols ? t : t / cols * ld + t % cols, comp);
+  v = block_sum(v);
+  if (threadIdx.x == 0) part[blockIdx.x] = v;
 }
 
 // out = |F| (F complex64), part[b] = block sums of out
 __global__ void magnitude_kernel(const float2* __restrict__ F, long long ldF, long long rows, long long cols,
                                  void* __restrict__ out, int odt, long long ldo, double* __restrict__ part) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  double v = 0.0;
-  if (t < rows * cols) {
+  const long long n = rows * cols, step = (long long)gridDim.x * kBlock;
+  double sum = 0.0;
+#pragma unroll 4
+  for (long long t = (long long)blockIdx.x * kBlock + threadIdx.x; t < n; t += step) {
     const long long r = t / cols, c = t % cols;
     const float2 f = F[r * ldF + c];
-    v = sqrt((double)f.x * f.x + (double)f.y * f.y);
+    const double v = sqrt((double)f.x * f.x + (double)f.y * f.y);
     store_real(out, odt, r * ldo + c, v);
-    if (odt != 3) v = (double)(float)v;  // sum what was stored
+    sum += odt != 3 ? (double)(float)v : v;  // sum what was stored
   }
-  block_partial(v, part);
+  sum = block_sum(sum);
+  if (threadIdx.x == 0) part[blockIdx.x] = sum;
 }
 
-// *out = sum of part[0 .. n) (one block, fixed order)
-__global__ void finalize_sum_kernel(const double* __restrict__ part, long long n, double* __restrict__ out) {
-  double v = 0.0;
-  for (long long i = threadIdx.x; i < n; i += blockDim.x) v += part[i];
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  __shared__ double w[kBlock / 64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) w[wave] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < kBlock / 64; ++i) s += w[i];
-    *out = s;
-  }
-}
-
-// x *= num / den  (device scalars)
+// x *= sum(num) / sum(den)  (partial sums)
 __global__ void scale_ratio_kernel(void* __restrict__ x, int dtype, long long rows, long long cols, long long ld,
-                                   const double* __restrict__ num, const double* __restrict__ den) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= rows * cols) return;
-  const long long i = (t / cols) * ld + t % cols;
-  store_real(x, dtype, i, load_real(x, dtype, i) * (*num / *den));
+                                   const double* __restrict__ num, const double* __restrict__ den, int nparts) {
+  const double ratio = total(num, nparts) / total(den, nparts);
+  const long long n = rows * cols, step = (long long)gridDim.x * kBlock;
+  for (long long t = (long long)blockIdx.x * kBlock + threadIdx.x; t < n; t += step) {
+    const long long i = (t / cols) * ld + t % cols;
+    store_real(x, dtype, i, load_real(x, dtype, i) * ratio);
+  }
 }
 
-hipError_t launch_sum(const void* x, int dtype, long long rows, long long cols, long long ld, double* part,
-                      double* out, hipStream_t s) {
-  const unsigned nb = blocks_for(rows * cols);
-  hipLaunchKernelGGL(sum_kernel, dim3(nb), dim3(kBlock), 0, s, x, dtype, rows, cols, ld, part);
-  hipLaunchKernelGGL(finalize_sum_kernel, dim3(1), dim3(kBlock), 0, s, (const double*)part, (long long)nb, out);
+static hipError_t launch_component_sum(const void* x, int dtype, int comp, long long rows, long long cols,
+                                       long long ld, double* part, hipStream_t s) {
+  hipLaunchKernelGGL(sum_kernel, dim3(part_blocks(rows * cols)), dim3(kBlock), 0, s, x, dtype, comp, rows, cols, ld,
+                     part);
   return hipGetLastError();
 }
 
+hipError_t launch_sum(const void* x, int dtype, long long rows, long long cols, long long ld, double* part,
+                      hipStream_t s) {
+  return launch_component_sum(x, dtype, 0, rows, cols, ld, part, s);
+}
+
 hipError_t launch_magnitude(const void* F, long long ldF, long long rows, long long cols, void* out, int odt,
-                            long long ldo, double* part, double* sum, hipStream_t s) {
-  const unsigned nb = blocks_for(rows * cols);
-  hipLaunchKernelGGL(magnitude_kernel, dim3(nb), dim3(kBlock), 0, s, (const float2*)F, ldF, rows, cols, out, odt, ldo,
-                     part);
-  hipLaunchKernelGGL(finalize_sum_kernel, dim3(1), dim3(kBlock), 0, s, (const double*)part, (long long)nb, sum);
+                            long long ldo, double* part, hipStream_t s) {
+  hipLaunchKernelGGL(magnitude_kernel, dim3(part_blocks(rows * cols)), dim3(kBlock), 0, s, (const float2*)F, ldF, rows,
+                     cols, out, odt, ldo, part);
   return hipGetLastError();
 }
 
 hipError_t launch_scale_ratio(void* x, int dtype, long long rows, long long cols, long long ld, const double* num,
                               const double* den, hipStream_t s) {
   if (rows * cols <= 0) return hipSuccess;
-  hipLaunchKernelGGL(scale_ratio_kernel, dim3(blocks_for(rows * cols)), dim3(kBlock), 0, s, x, dtype, rows, cols, ld,
-                     num, den);
+  const int nb = part_blocks(rows * cols);
+  hipLaunchKernelGGL(scale_ratio_kernel, dim3(nb), dim3(kBlock), 0, s, x, dtype, rows, cols, ld, num, den, nb);
   return hipGetLastError();
 }
 
@@ -279,14 +293,6 @@ __device__ __forceinline__ long long first_tap(double c, int order) {
   return order & 1 ? (long long)floor(c) - (order - 1) / 2 : (long long)floor(c + 0.5) - order / 2;
 }
 
-// component `comp` (0 real, 1 imaginary) of element i of a real or complex array
-__device__ __forceinline__ double load_component(const void* p, int dtype, long long i, int comp) {
-  switch (dtype) {
-    case 0: return comp ? ((const float2*)p)[i].y : ((const float2*)p)[i].x;
-    case 2: return comp ? ((const double2*)p)[i].y : ((const double2*)p)[i].x;
-    default: return comp ? 0.0 : load_real(p, dtype, i);
-  }
-}
 __device__ __forceinline__ bool nonzero(const void* p, int dtype, long long i) {
   return load_component(p, dtype, i, 0) != 0.0 || ((dtype == 0 || dtype == 2) && load_component(p, dtype, i, 1) != 0.0);
 }
@@ -309,23 +315,117 @@ __global__ void rescale_load_kernel(const void* __restrict__ img, int dtype, int
   P[t] = load_component(img, dtype, r * ld + c, comp);
 }
 
-// One axis of the B-spline prefilter as its two-sided impulse response,
-// dst[i] = sum_{|k| <= taps} h[|k|] src[extend(i + k)], along axis 0
-// (columns) or 1 (rows) of a P0 x P1 array.  h is the product over the
-// order's poles z of (1 - z) / (1 + z) z^|k|, truncated where it falls
-// below double rounding; the boundary rule is the mode's.
-__global__ void spline_fir_kernel(const double* __restrict__ src, double* __restrict__ dst, long long P0, long long P1,
-                                  int axis, int rule, PrefilterTaps taps) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= P0 * P1) return;
-  const long long i = t / P1, j = t % P1;
-  const long long n = axis == 0 ? P0 : P1, pos = axis == 0 ? i : j;
-  const long long stride = axis == 0 ? P1 : 1;
-  const double* line = src + (axis == 0 ? j : i * P1);
-  double s = taps.h[0] * line[pos * stride];
-  for (int k = 1; k <= taps.n; ++k)
-    s += taps.h[k] * (line[extend_index(pos - k, n, rule) * stride] + line[extend_index(pos + k, n, rule) * stride]);
-  dst[t] = s;
+// The B-spline prefilter, one axis at a time, as its two-sided impulse response
+//     dst[i] = sum_{|k| <= taps} h[|k|] src[extend(i + k)].
+// h is the product over the order's poles z of (1 - z) / (1 + z) z^|k|,
+// truncated where it falls below double rounding; the boundary rule is the
+// mode's.  Each block stages its samples and their halo in LDS once, the
+// extension rule applied there (the loads in batches, so their latency is paid
+// a few times); a thread computes NQ consecutive outputs from two windows that
+// slide by one sample per tap, two LDS reads per tap for all of them.  The sum
+// runs in the order k = 0, 1, ...  Every output reading its neighbours through
+// the caches and extending every index itself took 95 us per axis for 1048^2.
+//
+// window(d): this thread's sample at distance d from its first output.
+template <int NQ, typename Window>
+__device__ __forceinline__ void fir_outputs(const PrefilterTaps& taps, Window&& window, double (&s)[NQ]) {
+  double l[NQ], r[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    l[q] = r[q] = window(q);
+    s[q] = taps.h[0] * l[q];
+  }
+  auto step = [&](int k) {
+    const double h = taps.h[k];
+#pragma unroll
+    for (int q = NQ - 1; q > 0; --q) l[q] = l[q - 1];
+    l[0] = window(-k);
+#pragma unroll
+    for (int q = 0; q < NQ - 1; ++q) r[q] = r[q + 1];
+    r[NQ - 1] = window(NQ - 1 + k);
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) s[q] += h * (l[q] + r[q]);
+  };
+  int k = 1;
+  for (; k + NQ - 1 <= taps.n; k += NQ)  // whole turns of the windows: the shifts are renames
+#pragma unroll
+    for (int u = 0; u < NQ; ++u) step(k + u);
+  for (; k <= taps.n; ++k) step(k);
+}
+
+// Columns (axis 0), straight from the image: component comp with npad samples
+// of edge values (or zeros) around it.  256 threads: 32 columns x 64 rows, 8
+// rows per thread.  The dtype is a template parameter (a test per load would
+// wait for each); HALO is the LDS reserved for the taps, at most that many:
+// orders 2 and 3 fit 32, so five blocks fit a CU.
+constexpr int kFirRows = 64, kFirCols = 32;
+template <int DT, int HALO>
+__global__ __launch_bounds__(256) void fir_columns_kernel(const void* __restrict__ img, int comp,
+                                                          long long rows, long long cols, long long ld, int npad,
+                                                          int pad_zero, int rule, PrefilterTaps taps,
+                                                          double* __restrict__ dst) {
+  __shared__ double L[kFirRows + 2 * HALO][kFirCols];
+  const long long P0 = rows + 2 * npad, P1 = cols + 2 * npad;
+  const unsigned nbc = (unsigned)((P1 + kFirCols - 1) / kFirCols);
+  const int lc = threadIdx.x & 31, group = threadIdx.x >> 5;
+  const long long c = (long long)(blockIdx.x % nbc) * kFirCols + lc, r0 = (long long)(blockIdx.x / nbc) * kFirRows;
+  const long long ic = min(max(c - npad, 0LL), cols - 1);
+  const bool zc = pad_zero && (c - npad < 0 || c - npad >= cols);
+  const int nload = (int)min((long long)kFirRows, P0 - r0) + 2 * taps.n;
+  for (int i0 = group; i0 < nload; i0 += 64) {
+    double v[8];
+    bool z[8];
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const long long r = extend_index(r0 + min(i0 + 8 * b, nload - 1) - taps.n, P0, rule) - npad;
+      z[b] = zc || (pad_zero && (r < 0 || r >= rows));
+      v[b] = load_component(img, DT, min(max(r, 0LL), rows - 1) * ld + ic, comp);
+    }
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+      if (i0 + 8 * b < nload) L[i0 + 8 * b][lc] = z[b] ? 0.0 : v[b];
+  }
+  __syncthreads();
+  double s[8];
+  // rows past the last are computed from whatever LDS holds and not stored
+  fir_outputs<8>(taps, [&](int d) { return L[group * 8 + taps.n + d][lc]; }, s);
+  if (c >= P1) return;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const long long r = r0 + group * 8 + q;
+    if (r < P0) dst[r * P1 + c] = s[q];
+  }
+}
+
+// Rows (axis 1) of a P0 x P1 array.  256 threads: 4 rows x 256 columns, a
+// thread 4 adjacent columns; column c of a row lies at [c & 3][c >> 2], so
+// lanes 4 columns apart read neighbouring LDS words.
+constexpr int kFirSpan = 256;
+__global__ __launch_bounds__(256) void fir_rows_kernel(const double* __restrict__ src, long long P0, long long P1,
+                                                       int rule, PrefilterTaps taps, double* __restrict__ dst) {
+  constexpr int W = (kFirSpan + 2 * kPrefilterTaps) / 4;
+  __shared__ double L[4][4][W];
+  const long long nbc = (P1 + kFirSpan - 1) / kFirSpan;
+  const long long c0 = blockIdx.x % nbc * kFirSpan, r0 = blockIdx.x / nbc * 4;
+  const int nrow = (int)min(4LL, P0 - r0);
+  const int nload = (int)min((long long)kFirSpan, P1 - c0) + 2 * taps.n;
+  for (int i = threadIdx.x; i < nload; i += 256) {
+    const long long c = extend_index(c0 + i - taps.n, P1, rule);
+    double v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = src[(r0 + min(q, nrow - 1)) * P1 + c];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) L[q][i & 3][i >> 2] = v[q];
+  }
+  __syncthreads();
+  const int row = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double s[4];
+  fir_outputs<4>(taps, [&](int d) { return L[row][(taps.n + d) & 3][lane + ((taps.n + d) >> 2)]; }, s);
+  if (row >= nrow) return;
+  const long long c = c0 + 4 * (threadIdx.x & 63);
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (c + q < P1) dst[(r0 + row) * P1 + c + q] = s[q];
 }
 
 // Resample at the coordinates of util.py:333-336,
@@ -340,9 +440,10 @@ __global__ void resample_kernel(const double* __restrict__ C, long long P0, long
                                 long long ocols, const void* __restrict__ msrc, int mask_mode, int mdt, long long ldm,
                                 double eps, double* __restrict__ raw, double* __restrict__ mval,
                                 double* __restrict__ part) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  double v = 0.0;
-  if (t < orows * ocols) {
+  double sum = 0.0;
+  const long long n = orows * ocols, step = (long long)gridDim.x * kBlock;
+  for (long long t = (long long)blockIdx.x * kBlock + threadIdx.x; t < n; t += step) {
+    double v = 0.0;
     const long long r = t / ocols, c = t % ocols;
     const double y = ((double)r - (double)orows / 2.0) / scale + (double)rows / 2.0;
     const double x = ((double)c - (double)ocols / 2.0) / scale + (double)cols / 2.0;
@@ -353,18 +454,29 @@ __global__ void resample_kernel(const double* __restrict__ C, long long P0, long
       const double cx = (npad ? x : map_coordinate(x, cols, mode)) + npad;
       const int rule = tap_rule(mode);
       const long long sy = first_tap(cy, order), sx = first_tap(cx, order);
+      // the columns' taps and weights once, every load of a row before its sum
+      long long cc[6];
+      double wx[6];
+#pragma unroll
+      for (int b = 0; b < 6; ++b) {
+        cc[b] = b <= order ? extend_index(sx + b, P1, rule) : -1;
+        wx[b] = cc[b] >= 0 ? bspline(order, cx - (double)(sx + b)) : 0.0;
+        cc[b] = max(cc[b], 0LL);
+      }
       for (int a = 0; a <= order; ++a) {
         const long long rr = extend_index(sy + a, P0, rule);
         if (rr < 0) continue;
-        double row = 0.0;
-        for (int b = 0; b <= order; ++b) {
-          const long long cc = extend_index(sx + b, P1, rule);
-          if (cc >= 0) row += bspline(order, cx - (double)(sx + b)) * C[rr * P1 + cc];
-        }
+        double e[6], row = 0.0;
+#pragma unroll
+        for (int b = 0; b < 6; ++b) e[b] = C[rr * P1 + cc[b]];
+#pragma unroll
+        for (int b = 0; b < 6; ++b)
+          if (b <= order) row += wx[b] * e[b];
         v += bspline(order, cy - (double)(sy + a)) * row;
       }
     }
     raw[t] = v;
+    sum += v;
     if (mval) {
       const double my = fmin(fmax(y, 0.0), (double)(rows - 1)), mx = fmin(fmax(x, 0.0), (double)(cols - 1));
       const long long fy = (long long)floor(my), fx = (long long)floor(mx);
@@ -379,15 +491,22 @@ __global__ void resample_kernel(const double* __restrict__ C, long long P0, long
       mval[t] = mv;
     }
   }
-  block_partial(v, part);
+  sum = block_sum(sum);
+  if (threadIdx.x == 0) part[blockIdx.x] = sum;
 }
 
 // out = raw * (unitary ? sum(img) / sum(raw) : 1) * mval   (util.py:340-347);
-// with raw_im, complex: the ratio of the complex sums, sums = (img_re,
-// img_im, raw_re, raw_im), out complex64 (odt 0) or complex128 (odt 2).
+// with raw_im, complex: the ratio of the complex sums, out complex64 (odt 0)
+// or complex128 (odt 2).  The partial sums of (img_re, img_im, raw_re, raw_im)
+// lie kMaxPart apart, ni of each image sum and nr of each resampled one.
 __global__ void rescale_finish_kernel(const double* __restrict__ raw, const double* __restrict__ raw_im,
                                       const double* __restrict__ mval, long long orows, long long ocols, int unitary,
-                                      const double* __restrict__ sums, void* __restrict__ out, int odt, long long ldo) {
+                                      const double* __restrict__ part, int ni, int nr, void* __restrict__ out,
+                                      int odt, long long ldo) {
+  double sums[4] = {};
+  if (unitary)
+    for (int q = 0; q < 4; ++q)
+      if (raw_im || !(q & 1)) sums[q] = total(part + q * kMaxPart, q < 2 ? ni : nr);
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= orows * ocols) return;
   const long long o = (t / ocols) * ldo + t % ocols;
@@ -444,8 +563,10 @@ static PrefilterTaps make_prefilter_taps(int order) {
     }
     cur.swap(nxt);
   }
-  h.n = kPrefilterTaps;
   for (int k = 0; k <= kPrefilterTaps; ++k) h.h[k] = cur[W + k];
+  // the last tap that is not lost in the rounding of the first (2^-56 of it:
+  // 23 taps for order 2, 30, 39 and 46 for orders 3 to 5)
+  while (h.n < kPrefilterTaps && std::fabs(h.h[h.n + 1]) > std::ldexp(h.h[0], -56)) ++h.n;
   return h;
 }
 
@@ -458,36 +579,41 @@ PrefilterTaps prefilter_taps(int order) {
 hipError_t launch_rescale(const void* img, int dtype, long long rows, long long cols, long long ld, const void* msrc,
                           int mask_mode, int mdt, long long ldm, double eps, double scale, long long orows,
                           long long ocols, int order, int mode, int unitary, void* out, int odt, long long ldo,
-                          double* P, double* T, double* raw, double* raw_im, double* mval, double* part, double* sums,
+                          double* P, double* T, double* raw, double* raw_im, double* mval, double* part,
                           hipStream_t s) {
   const bool cplx = dtype == 0 || dtype == 2;
   const int npad = order > 1 && (mode == MFTX_MODE_NEAREST || mode == MFTX_MODE_GRID_CONSTANT) ? 12 : 0;
+  const int zero = mode == MFTX_MODE_GRID_CONSTANT ? 1 : 0;
   const long long P0 = rows + 2 * npad, P1 = cols + 2 * npad;
-  const unsigned nbp = blocks_for(P0 * P1);
-  const unsigned nbo = blocks_for(orows * ocols);
+  const int ni = part_blocks(rows * cols), nr = part_blocks(orows * ocols);
   const PrefilterTaps taps = prefilter_taps(order);
   for (int comp = 0; comp < (cplx ? 2 : 1); ++comp) {
-    hipLaunchKernelGGL(rescale_load_kernel, dim3(nbp), dim3(kBlock), 0, s, img, dtype, comp, rows, cols, ld, npad,
-                       mode == MFTX_MODE_GRID_CONSTANT ? 1 : 0, P);
-    if (unitary) {  // sum of the image component: the interior of P
-      hipError_t e = launch_sum(P + npad * P1 + npad, 3, rows, cols, P1, part, sums + comp, s);
+    if (unitary) {
+      const hipError_t e = launch_component_sum(img, dtype, comp, rows, cols, ld, part + comp * kMaxPart, s);
       if (e != hipSuccess) return e;
     }
     if (order > 1) {
-      hipLaunchKernelGGL(spline_fir_kernel, dim3(nbp), dim3(kBlock), 0, s, (const double*)P, T, P0, P1, 0,
-                         filter_rule(mode), taps);
-      hipLaunchKernelGGL(spline_fir_kernel, dim3(nbp), dim3(kBlock), 0, s, (const double*)T, P, P0, P1, 1,
-                         filter_rule(mode), taps);
+      const auto columns = taps.n <= 32 ? (dtype == 0 ? fir_columns_kernel<0, 32> : dtype == 1 ? fir_columns_kernel<1, 32>
+                                           : dtype == 2 ? fir_columns_kernel<2, 32> : fir_columns_kernel<3, 32>)
+                                        : (dtype == 0 ? fir_columns_kernel<0, kPrefilterTaps>
+                                           : dtype == 1 ? fir_columns_kernel<1, kPrefilterTaps>
+                                           : dtype == 2 ? fir_columns_kernel<2, kPrefilterTaps>
+                                                        : fir_columns_kernel<3, kPrefilterTaps>);
+      hipLaunchKernelGGL(columns, dim3((unsigned)((P1 + kFirCols - 1) / kFirCols * ((P0 + kFirRows - 1) / kFirRows))),
+                         dim3(256), 0, s, img, comp, rows, cols, ld, npad, zero, filter_rule(mode), taps, T);
+      hipLaunchKernelGGL(fir_rows_kernel, dim3((unsigned)((P1 + 255) / 256 * ((P0 + 3) / 4))), dim3(256), 0, s,
+                         (const double*)T, P0, P1, filter_rule(mode), taps, P);
+    } else {
+      hipLaunchKernelGGL(rescale_load_kernel, dim3(blocks_for(P0 * P1)), dim3(kBlock), 0, s, img, dtype, comp, rows,
+                         cols, ld, npad, zero, P);
     }
-    hipLaunchKernelGGL(resample_kernel, dim3(nbo), dim3(kBlock), 0, s, (const double*)P, P0, P1, npad, order, mode,
+    hipLaunchKernelGGL(resample_kernel, dim3(nr), dim3(kBlock), 0, s, (const double*)P, P0, P1, npad, order, mode,
                        rows, cols, scale, orows, ocols, msrc, mask_mode, mdt, ldm, eps, comp ? raw_im : raw,
-                       comp ? (double*)nullptr : mval, part);
-    hipLaunchKernelGGL(finalize_sum_kernel, dim3(1), dim3(kBlock), 0, s, (const double*)part, (long long)nbo,
-                       sums + 2 + comp);
+                       comp ? (double*)nullptr : mval, part + (2 + comp) * kMaxPart);
   }
-  hipLaunchKernelGGL(rescale_finish_kernel, dim3(nbo), dim3(kBlock), 0, s, (const double*)raw,
+  hipLaunchKernelGGL(rescale_finish_kernel, dim3(blocks_for(orows * ocols)), dim3(kBlock), 0, s, (const double*)raw,
                      cplx ? (const double*)raw_im : nullptr, (const double*)mval, orows, ocols, unitary,
-                     (const double*)sums, out, odt, ldo);
+                     (const double*)part, ni, nr, out, odt, ldo);
   return hipGetLastError();
 }
 

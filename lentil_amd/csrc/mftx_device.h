@@ -13,6 +13,7 @@ typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
 typedef float v4f32 __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u32 __attribute__((ext_vector_type(2)));
 typedef float v2f32 __attribute__((ext_vector_type(2)));
+typedef double v2f64 __attribute__((ext_vector_type(2)));
 
 // Global-memory views: pointers that arrive inside descriptors are generic,
 // and generic (flat) accesses also count on the LDS/scalar counter, so every

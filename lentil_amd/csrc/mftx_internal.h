@@ -146,9 +146,9 @@ struct TableOp {
   double alpha, x0, y0;
   int nsb, nkb, sb0, pad_;
   void* dst;
-  long long begin;      // first thread: one per (slot, 8 k')
+  long long begin;      // first thread: one per (slot, 2 k')
 };
-__host__ __device__ inline long long table_threads(int nsb, int nkb) { return 64LL * nsb * nkb; }
+__host__ __device__ inline long long table_threads(int nsb, int nkb) { return 256LL * nsb * nkb; }
 inline size_t table_bytes(int nsb, int nkb) { return (size_t)nsb * nkb * B_BLOCK; }
 // Twiddles of the f16 form are scaled so the lo parts of small ones stay normal.
 __host__ __device__ inline float tw_scale(int prec) { return prec == PREC_FP32 ? 256.0f : 1.0f; }
@@ -291,19 +291,18 @@ hipError_t launch_phase_grad(const void* amp, int amp_dtype, long long ld_amp, c
 // detector-grid post-processing (mftx_detector.hip)
 hipError_t launch_rebin(const void* src, int dtype, long long nimg, long long rows, long long cols, long long ld,
                         int factor, void* dst, int odt, hipStream_t s);
-// *out = sum of a real array (part: one double per 256 elements)
+// Reductions leave at most kMaxPart partial sums, the same number for arrays of
+// one size; their users add them up.
+constexpr int kMaxPart = 1024;
+// part = partial sums of a real array
 hipError_t launch_sum(const void* x, int dtype, long long rows, long long cols, long long ld, double* part,
-                      double* out, hipStream_t s);
-// out = |F| (F complex64), *sum = sum of out (part as for launch_sum)
+                      hipStream_t s);
+// out = |F| (F complex64), part = partial sums of out
 hipError_t launch_magnitude(const void* F, long long ldF, long long rows, long long cols, void* out, int odt,
-                            long long ldo, double* part, double* sum, hipStream_t s);
-// x *= *num / *den
+                            long long ldo, double* part, hipStream_t s);
+// x *= sum(num) / sum(den), partial sums of arrays of its size
 hipError_t launch_scale_ratio(void* x, int dtype, long long rows, long long cols, long long ld, const double* num,
                               const double* den, hipStream_t s);
-// map_coordinates(order 0/1/3, mode 'nearest') resampling with the mask and
-// unitary scaling of rescale; P, T: (rows + 24) x (cols + 24) doubles; raw,
-// mval: orows x ocols doubles; part: one double per 256 elements of the
-// larger of the input and output; sums: 2 doubles
 // The B-spline prefilter of a spline order as its two-sided impulse response
 // h[|k|], |k| <= n (n = 0 for orders 0 and 1).
 constexpr int kPrefilterTaps = 48;
@@ -315,11 +314,11 @@ PrefilterTaps prefilter_taps(int order);
 // rescale (util.py:262-349): map_coordinates(order 0..5, mode MFTX_MODE_*)
 // of a real or complex (dtype 0 / 2) image, mask, unitary ratio; P and T hold
 // the padded image (rows + 24) x (cols + 24) doubles each, raw / raw_im / mval
-// the output size, part ceil(max(padded, output) / 256) doubles, sums 4.
+// the output size, part 4 kMaxPart doubles.
 hipError_t launch_rescale(const void* img, int dtype, long long rows, long long cols, long long ld, const void* msrc,
                           int mask_mode, int mdt, long long ldm, double eps, double scale, long long orows,
                           long long ocols, int order, int mode, int unitary, void* out, int odt, long long ldo,
-                          double* P, double* T, double* raw, double* raw_im, double* mval, double* part, double* sums,
+                          double* P, double* T, double* raw, double* raw_im, double* mval, double* part,
                           hipStream_t s);
 
 // modal OPD operations (mftx_modal.hip)

@@ -10,13 +10,16 @@ namespace mftx {
 // dtype codes: 0 complex64, 1 float32, 2 complex128, 3 float64
 __device__ __forceinline__ float2 load_elem(const void* p, int dtype, long long idx) {
   switch (dtype) {
-    case 0: return ((const float2*)p)[idx];
-    case 1: return make_float2(((const float*)p)[idx], 0.f);
+    case 0: {
+      const v2f32 v = ((gptr<const v2f32>)p)[idx];
+      return make_float2(v.x, v.y);
+    }
+    case 1: return make_float2(((gptr<const float>)p)[idx], 0.f);
     case 2: {
-      const double2 v = ((const double2*)p)[idx];
+      const v2f64 v = ((gptr<const v2f64>)p)[idx];
       return make_float2((float)v.x, (float)v.y);
     }
-    default: return make_float2((float)((const double*)p)[idx], 0.f);
+    default: return make_float2((float)((gptr<const double>)p)[idx], 0.f);
   }
 }
 
@@ -37,6 +40,17 @@ __device__ __forceinline__ double load_real(const void* p, int dtype, long long 
   return dtype == 3 ? ((const double*)p)[idx] : (double)((const float*)p)[idx];
 }
 
+// u / d and u % d; the 64-bit division is a long instruction sequence
+__device__ __forceinline__ void div_mod(long long u, long long d, long long& q, int& r) {
+  if (((u | d) >> 32) == 0) {
+    q = (unsigned)u / (unsigned)d;
+    r = (int)((unsigned)u - (unsigned)q * (unsigned)d);
+  } else {
+    q = u / d;
+    r = (int)(u - q * d);
+  }
+}
+
 // Largest value of the block's threads, in every thread (all of them call it).
 __device__ __forceinline__ float block_max(float v) {
   __shared__ float w[kGroupBlock / 64];
@@ -50,28 +64,44 @@ __device__ __forceinline__ float block_max(float v) {
   return v;
 }
 
-// Bound of an element's modulus (0 where it is not finite: such an element
-// makes its results non-finite whatever the scale).
-__device__ __forceinline__ float elem_bound(const void* src, int dtype, long long i) {
-  const float2 e = load_elem(src, dtype, i);
-  const float v = fabsf(e.x) + fabsf(e.y);
-  return v <= 3.4028234e38f ? v : 0.f;
-}
-
-// Bound over elements [first, m * n) in steps of `step` of an m x n array.
-__device__ __forceinline__ float array_bound(const void* src, int dtype, long long m, long long n, long long ld,
-                                             long long first, long long step) {
+// Bound over elements [first, m * n) in steps of `step` of an m x n array:
+// |re| + |im|, 0 for an element that is not finite (it makes its results
+// non-finite whatever the scale).  The dtype is tested outside the loop, so
+// the loads of 8 elements are in flight together.
+template <typename Get>
+__device__ __forceinline__ float bound_of(long long m, long long n, long long ld, long long first, long long step,
+                                          Get&& get) {
   float v = 0.f;
   const long long total = m * n;
-  if (ld == n) {
-    for (long long i = first; i < total; i += step) v = fmaxf(v, elem_bound(src, dtype, i));
-  } else if (total < (1LL << 31)) {
-    for (unsigned i = (unsigned)first; i < (unsigned)total; i += (unsigned)step)
-      v = fmaxf(v, elem_bound(src, dtype, (long long)(i / (unsigned)n) * ld + i % (unsigned)n));
-  } else {
-    for (long long i = first; i < total; i += step) v = fmaxf(v, elem_bound(src, dtype, i / n * ld + i % n));
+  auto one = [&](long long i) {
+    const float2 e = get(ld == n ? i : total < (1LL << 31) ? (long long)((unsigned)i / (unsigned)n) * ld + (unsigned)i % (unsigned)n
+                                                           : i / n * ld + i % n);
+    const float b = fabsf(e.x) + fabsf(e.y);
+    return b <= 3.4028234e38f ? b : 0.f;
+  };
+  long long i = first;
+  for (; i + 7 * step < total; i += 8 * step) {
+    float b[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) b[q] = one(i + q * step);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v = fmaxf(v, b[q]);
   }
+  for (; i < total; i += step) v = fmaxf(v, one(i));
   return v;
+}
+__device__ __forceinline__ float array_bound(const void* src, int dtype, long long m, long long n, long long ld,
+                                             long long first, long long step) {
+  switch (dtype) {
+    case 0:
+      return bound_of(m, n, ld, first, step, [&](long long i) {
+        const v2f32 e = ((gptr<const v2f32>)src)[i];
+        return make_float2(e.x, e.y);
+      });
+    case 1: return bound_of(m, n, ld, first, step, [&](long long i) { return make_float2(((gptr<const float>)src)[i], 0.f); });
+    case 2: return bound_of(m, n, ld, first, step, [&](long long i) { return load_elem(src, 2, i); });
+    default: return bound_of(m, n, ld, first, step, [&](long long i) { return load_elem(src, 3, i); });
+  }
 }
 
 __global__ void absmax_kernel(const MaxOp* __restrict__ ops, int nops) {
@@ -144,7 +174,8 @@ __device__ __forceinline__ PhasorWave load_wave(cptr<const PhasorWave> p) {
 // source and 32 of result, four waves per SIMD; NP = 8 left room for two.
 // Where every sample of a wave is outside the aperture (amplitude 0) the
 // phases are skipped.
-template <int PREC, bool CPLX, int NP, typename Waves>
+// DT: the dtype of a complex source.
+template <int PREC, bool CPLX, int NP, int DT, typename Waves>
 __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave, int waves, long long u, float scale) {
   static_assert(NP == 2 || NP == 4 || NP == 8, "a thread's pairs lie in one half of a K block");
   constexpr int SUB = 8 / NP;  // threads per (row pair, half K block)
@@ -152,11 +183,13 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
   const int nrb = pair_blocks(R), nkb = pair_blocks(K);
   // a wavelength group spans whole waves, so its descriptors are scalar loads
   const long long per_group = group_threads(R, K, NP);
-  const int g = __builtin_amdgcn_readfirstlane((int)(u / per_group));
-  const int v = (int)(u % per_group);
+  long long group;
+  int v;
+  div_mod(u, per_group, group, v);
+  const int g = __builtin_amdgcn_readfirstlane((int)group);
   if (v >= 32 * SUB * nrb * nkb) return;
   const int sub = v & (SUB - 1), lr = (v / SUB) & 15, kh = (v / (16 * SUB)) & 1, blk = v / (32 * SUB);
-  const int kb = blk % nkb, rb = blk / nkb;
+  const int kb = (unsigned)blk % (unsigned)nkb, rb = (unsigned)blk / (unsigned)nkb;
   int r2[2];
   pair_index(R, rb * 16 + lr, r2[0], r2[1]);
   const int kp0 = kb * 16 + kh * 8 + sub * NP;
@@ -188,7 +221,7 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
       if constexpr (CPLX) {
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
-          const float2 e = load_elem(op.amp, op.amp_dtype, ia[i]);
+          const float2 e = load_elem(op.amp, DT, ia[i]);
           a[rs][ks][i] = in[i] ? e.x * scale : 0.f;
           ci[rs][ks][i] = in[i] ? e.y * scale : 0.f;
         }
@@ -304,6 +337,22 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
   }
 }
 
+// operand_thread for the op's source dtype (tested once per thread: a test per
+// load would wait for each)
+template <int PREC, bool CPLX, int NP, typename Waves>
+__device__ __forceinline__ void operand_source(const PhasorOp& op, Waves&& wave, int waves, long long u, float scale) {
+  if constexpr (!CPLX) {
+    operand_thread<PREC, false, NP, 0>(op, wave, waves, u, scale);
+  } else {
+    switch (op.amp_dtype) {
+      case 0: operand_thread<PREC, true, NP, 0>(op, wave, waves, u, scale); break;
+      case 1: operand_thread<PREC, true, NP, 1>(op, wave, waves, u, scale); break;
+      case 2: operand_thread<PREC, true, NP, 2>(op, wave, waves, u, scale); break;
+      default: operand_thread<PREC, true, NP, 3>(op, wave, waves, u, scale);
+    }
+  }
+}
+
 // Every operand source of a plan in one launch (the op is found by a
 // block-uniform search).
 template <int PREC, bool CPLX, int NP>
@@ -314,7 +363,7 @@ __global__ __launch_bounds__(kGroupBlock, 4) void operand_group_kernel(const Pha
   const float scale = block_scale(op.sc, b0 == op.begin);
   const long long u = b0 + threadIdx.x - op.begin;
   if (u >= operand_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, op.nwave, OperandSplit{NP, waves})) return;
-  operand_thread<PREC, CPLX, NP>(op, [&](int w) { return load_wave((cptr<const PhasorWave>)op.waves + w); }, waves, u,
+  operand_source<PREC, CPLX, NP>(op, [&](int w) { return load_wave((cptr<const PhasorWave>)op.waves + w); }, waves, u,
                                  scale);
 }
 
@@ -350,7 +399,7 @@ hipError_t launch_operands(int prec, bool cplx, OperandSplit sp, const PhasorOp*
 __device__ __forceinline__ double2 cis_turns64(double t) {
   const double q = t * 4.0;
   const double n = __builtin_rint(q);
-  const int quad = (int)(long long)n;
+  const int quad = (int)n;  // |q| below 2^31, as for cis_quarter
   const double a = (q - n) * 1.57079632679489661923, a2 = a * a;
   double s = 1.0 / 6227020800.0;
   s = __builtin_fma(s, a2, -1.0 / 39916800.0);
@@ -371,51 +420,37 @@ __device__ __forceinline__ double2 cis_turns64(double t) {
   return make_double2((quad + 1) & 2 ? -re : re, quad & 2 ? -im : im);
 }
 
-// One thread per (slot, 8 k').  The values are correctly rounded to the
+// One thread per (slot, 2 k').  The values are correctly rounded to the
 // format's hi + lo but for 1e-13, tighter than FP32 twiddles.
 template <int PREC>
 __device__ __forceinline__ void table_thread(const TableOp& op, long long u) {
-  const int l = (int)(u & 63);
-  const long long blk = u >> 6;
-  const int kb = (int)(blk % op.nkb), sb = (int)(blk / op.nkb);
-  const double y = op.y0 + (double)((op.sb0 + sb) * 32 + (l & 31));
-  const double x0 = op.x0 + (double)(kb * 16 + 8 * (l >> 5));
+  const int t = (int)(u & 3), l = (int)(u >> 2) & 63;
+  long long sb;
+  int kb;
+  div_mod(u >> 8, op.nkb, sb, kb);
+  const double y = op.y0 + (double)((op.sb0 + (int)sb) * 32 + (l & 31));
+  const double x0 = op.x0 + (double)(kb * 16 + 8 * (l >> 5) + 2 * t);
   const float ts = tw_scale(PREC);
-  uint32_t w[4][4];
+  double2 v[2];
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    float c[2], s[2], cl[2], sl[2];
-    uint32_t ch, sh;
-    double2 v[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      v[q] = cis_turns64(op.alpha * ((x0 + (double)(2 * t + q)) * y));
-      v[q].x *= ts;
-      v[q].y *= ts;
-      c[q] = (float)v[q].x;
-      s[q] = (float)v[q].y;
-    }
-    auto widen = [](uint32_t h, int q) -> double {
-      if constexpr (PREC == PREC_BF16X3) return q ? bf16_hi_to_f32(h) : bf16_lo_to_f32(h);
-      else return (double)(float)(__builtin_bit_cast(f16x2_t, h)[q]);
-    };
-    auto pk = [](float x, float y2) { return PREC == PREC_BF16X3 ? pack_bf16(x, y2) : pack_f16(x, y2); };
-    ch = pk(c[0], c[1]);
-    sh = pk(s[0], s[1]);
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      cl[q] = (float)(v[q].x - widen(ch, q));
-      sl[q] = (float)(v[q].y - widen(sh, q));
-    }
-    w[0][t] = ch;
-    w[1][t] = pk(cl[0], cl[1]);
-    w[2][t] = sh;
-    w[3][t] = pk(sl[0], sl[1]);
+  for (int q = 0; q < 2; ++q) {
+    v[q] = cis_turns64(op.alpha * ((x0 + (double)q) * y));
+    v[q].x *= ts;
+    v[q].y *= ts;
   }
-  char* d = (char*)op.dst + ((long long)sb * op.nkb + kb) * B_BLOCK + 16 * l;
-#pragma unroll
-  for (int pl = 0; pl < 4; ++pl)
-    *(gptr<v4u32>)(d + pl * FRAG) = v4u32{w[pl][0], w[pl][1], w[pl][2], w[pl][3]};
+  auto pk = [](float x, float z) { return PREC == PREC_BF16X3 ? pack_bf16(x, z) : pack_f16(x, z); };
+  auto widen = [](uint32_t h, int q) -> double {
+    if constexpr (PREC == PREC_BF16X3) return q ? bf16_hi_to_f32(h) : bf16_lo_to_f32(h);
+    else return (double)(float)(__builtin_bit_cast(f16x2_t, h)[q]);
+  };
+  const uint32_t ch = pk((float)v[0].x, (float)v[1].x), sh = pk((float)v[0].y, (float)v[1].y);
+  const uint32_t cl = pk((float)(v[0].x - widen(ch, 0)), (float)(v[1].x - widen(ch, 1)));
+  const uint32_t sl = pk((float)(v[0].y - widen(sh, 0)), (float)(v[1].y - widen(sh, 1)));
+  char* d = (char*)op.dst + (sb * op.nkb + kb) * B_BLOCK + 16 * l + 4 * t;
+  *(gptr<uint32_t>)d = ch;
+  *(gptr<uint32_t>)(d + FRAG) = cl;
+  *(gptr<uint32_t>)(d + 2 * FRAG) = sh;
+  *(gptr<uint32_t>)(d + 3 * FRAG) = sl;
 }
 
 template <int PREC>
@@ -472,7 +507,7 @@ __global__ __launch_bounds__(kGroupBlock, 4) void prepare_one_kernel(PhasorOp op
     if (b == 0 && threadIdx.x == 0) *out = desc;
     const long long u = (long long)b * kGroupBlock + threadIdx.x;
     if (u < operand_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, 1, OperandSplit{2, 1}))
-      operand_thread<PREC, true, 2>(op, [=](int) { return wave; }, 1, u, scale);
+      operand_source<PREC, true, 2>(op, [=](int) { return wave; }, 1, u, scale);
     return;
   }
   long long u = (long long)(b - op_blocks) * kGroupBlock + threadIdx.x;
