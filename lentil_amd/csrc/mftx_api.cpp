@@ -523,14 +523,17 @@ void mft_problems(const MftGeo& g, int prec, double scale, Problem& a, Problem& 
   b.xrot = g.alpha2 * g.xc2();
   b.scale = (float)(scale * stage2_scale(prec, pairs(g.k1)));
   b.trans = g.col_first ? 0 : 1;  // C is F (column-first) or F^T (row-first)
+  b.wrows = (int)(g.col_first ? g.c1 : g.c2);
+  b.wcols = (int)(g.col_first ? g.c2 : g.c1);
 }
 
 // A transform whose output takes more tiles of 128 rows by 64 or 128 columns
-// than one descriptor block of kSlotBytes once held (40 bytes each behind 112
-// bytes and 8 per 16 K values) is refused, as it always was.
-bool too_large(const MftGeo& g) {
+// than a descriptor block of kSlotBytes once held (40 bytes each behind 112
+// bytes and 8 per 16 K values; a list entry's two stages together, with 104
+// bytes of source) is refused, as it always was.
+bool too_large(const MftGeo& g, bool list_entry) {
   auto up = [](int64_t v, int64_t q) { return (v + q - 1) / q * q; };
-  const int64_t t1 = up(g.r1, BK * 8) / 128, t2 = up(g.c1, 128) / 128;
+  const int64_t t1 = up(g.r1, 128) / 128, t2 = up(g.c1, 128) / 128;
   const int64_t wide = std::max(t1 * ((g.g1.slots + 63) / 64), t2 * ((g.g2.slots + 63) / 64));
   const int64_t bs = wide >= 256 ? 64 : 32, kg = wide >= 256 ? 32 : 16;
   auto bytes = [&](int64_t tr, int64_t slots, int64_t k) {
@@ -538,7 +541,8 @@ bool too_large(const MftGeo& g) {
     const int64_t works = (mx - 1) * 8 + (tr % 8 ? tr % 8 : 8);
     return up(112 + up(k, kg) / 16 * 8, 16) + 40 * works;
   };
-  return bytes(t1, g.g1.slots, g.k1) > (int64_t)kSlotBytes || bytes(t2, g.g2.slots, g.r1) > (int64_t)kSlotBytes;
+  const int64_t b1 = bytes(t1, g.g1.slots, g.k1), b2 = bytes(t2, g.g2.slots, g.r1);
+  return list_entry ? 112 + b1 + b2 > (int64_t)kSlotBytes : std::max(b1, b2) > (int64_t)kSlotBytes;
 }
 }  // namespace
 
@@ -759,12 +763,12 @@ static hipError_t many_launch(const ManyBatch& mb, int prec, const char* d, hipS
 static int dft2_many_run(mftx_ctx* ctx, const mftx_mft* mfts, int32_t count, int prec) {
   std::unique_ptr<ManyBatch> mb(new ManyBatch());
   many_build(mfts, count, prec, -1, *mb);
-  if (mb->bytes > kSlotBytes || (count == 1 && too_large(mb->geo[0]))) {
+  if (mb->bytes > kSlotBytes || (count == 1 && too_large(mb->geo[0], true))) {
     if (count == 1) {
       // the widest tiles need the fewest descriptors
       mb.reset(new ManyBatch());
       many_build(mfts, count, prec, TILE_BIG, *mb);
-      if (mb->bytes > kSlotBytes || too_large(mb->geo[0]))
+      if (mb->bytes > kSlotBytes || too_large(mb->geo[0], true))
         return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
     } else {
       const int32_t h = count / 2;
@@ -905,7 +909,28 @@ int mftx_dft2(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, i
 
 }  // extern "C"
 
-// mftx_dft2 on the caller's workspace `ws`, or on the context's growable
+// One transform (the arguments of mftx_dft2, checked) with a real weight map on
+// the output, wrapped by (wrow, wcol), or a conjugated input.  reuse_tables:
+// the last transform on this workspace had the same geometry but for offsets,
+// and its twiddle tables are still there.
+namespace {
+struct OneSpec {
+  const void* f;
+  int f_dtype;
+  int64_t m, n, ldf;
+  void* F;
+  int64_t M, N, ldF;
+  double alpha_r, alpha_c, shift_r, shift_c, offset_r, offset_c, scale;
+  int conj, precision;
+  const void* w = nullptr;
+  int w_dtype = 0;
+  int64_t ldw = 0;
+  int wrow = 0, wcol = 0;
+  bool conj_input = false, reuse_tables = false;
+};
+}  // namespace
+
+// One transform on the caller's workspace `ws`, or on the context's growable
 // workspace when ws is null.  Three launches and nothing uploaded: the source's
 // maximum (f16 form, larger sources only), then operand, twiddle tables and
 // descriptors (launch_prepare_one), then the two GEMMs.  A table larger than
@@ -919,21 +944,12 @@ int mftx_dft2(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, i
 // then stage 1's output for every K the second stage reads), so the workspace
 // needs no clearing; padding rows beyond the output only feed output rows that
 // are never stored.
-int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, int64_t ldf, void* F,
-                            int64_t M, int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r,
-                            double shift_c, double offset_r, double offset_c, double scale, int conj, int precision,
-                            void* ws, size_t cap, size_t table_cap) {
-  if (!ctx) return MFTX_EHANDLE;
-  if (!f || !F) return fail(ctx, MFTX_EINVAL, "null array pointer");
-  if (m <= 0 || n <= 0 || M <= 0 || N <= 0) return fail(ctx, MFTX_EINVAL, "shapes must be positive");
-  if (ldf < n || ldF < N) return fail(ctx, MFTX_EINVAL, "row stride smaller than row length");
-  if (f_dtype < 0 || f_dtype > 3) return fail(ctx, MFTX_EINVAL, "unknown input dtype");
-  if (precision != MFTX_PREC_FP32 && precision != MFTX_PREC_BF16X3) return fail(ctx, MFTX_EINVAL, "unknown precision");
-  if (m > (1 << 20) || n > (1 << 20) || M > (1 << 20) || N > (1 << 20))
-    return fail(ctx, MFTX_EINVAL, "dimension too large");
+static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t cap, size_t table_cap) {
   HIPCHK(ctx, hipSetDevice(ctx->device));
-  const int prec = precision;
-  const MftGeo g = mft_geometry(m, n, M, N, alpha_r, alpha_c, shift_r, shift_c, offset_r, offset_c, conj);
+  const int prec = q.precision;
+  const int64_t m = q.m, n = q.n;
+  const MftGeo g = mft_geometry(m, n, q.M, q.N, q.alpha_r, q.alpha_c, q.shift_r, q.shift_c, q.offset_r, q.offset_c,
+                                q.conj);
   if (ws) {
     const int64_t rows1 = round_up(g.r1, 128), rows2 = round_up(g.c1, 128);
     const int64_t wide = std::max(rows1 / 128 * ((g.g1.slots + 63) / 64), rows2 / 128 * ((g.g2.slots + 63) / 64));
@@ -947,7 +963,7 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
   OneMft one = {};
   Problem& p1 = one.desc.prob[0];
   Problem& p2 = one.desc.prob[1];
-  mft_problems(g, prec, scale, p1, p2);
+  mft_problems(g, prec, q.scale, p1, p2);
   const int tile[2] = {pick_schedule(-1, false, p1.rblocks, p1.sblocks, nkb1, 1, 1).tile,
                        pick_schedule(-1, false, p2.rblocks, p2.sblocks, nkb2, 1, 1).tile};
   // slot blocks of a stage whose table fits the cap (whole tiles)
@@ -968,14 +984,15 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
     if (rc) return rc;
     ws = ctx->ws;
   }
-  if (too_large(g)) return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
+  if (too_large(g, false)) return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
   char* base = (char*)ws;
   float* part = (float*)(base + o_max);
   float* inv = part + kMaxBlocks;
 
-  one.op.amp = f;
-  one.op.amp_dtype = f_dtype;
-  one.op.ld_amp = ldf;
+  one.op.amp = q.f;
+  one.op.amp_dtype = q.f_dtype;
+  one.op.ld_amp = q.ldf;
+  one.op.conj = q.conj_input ? 1 : 0;
   one.op.m = (int)m;
   one.op.n = (int)n;
   one.op.trans = g.col_first ? 1 : 0;
@@ -983,11 +1000,11 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
   one.op.dst = base + o_a1;
   MaxOp mx = {};
   if (prec == PREC_FP32) {
-    mx.src = f;
-    mx.dtype = f_dtype;
+    mx.src = q.f;
+    mx.dtype = q.f_dtype;
     mx.m = m;
     mx.n = n;
-    mx.ld = ldf;
+    mx.ld = q.ldf;
     mx.nblk = max_blocks(m, n);
     mx.part = part;
     // a source of up to 8192 elements is read whole by every operand block
@@ -1003,10 +1020,21 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
   p1.sbeg = p2.sbeg = 0;
   p1.send = p2.send = 1;
   p1.dst = base + o_a2;
-  p2.dst = F;
-  p2.ldd = ldF;
+  p2.dst = q.F;
+  p2.ldd = q.ldF;
+  p2.wmap = q.w;
+  p2.wdtype = q.w_dtype;
+  p2.ldw = q.ldw;
+  p2.wrow = q.wrow;
+  p2.wcol = q.wcol;
   one.desc_dev = (OneDesc*)base;
-  HIPCHK(ctx, launch_prepare_one(prec, one, mx, ctx->stream));
+  {
+    OneMft first = one;
+    // a table used in pieces is always made again
+    if (q.reuse_tables && piece1 == p1.sblocks) first.tab[0].nsb = 0;
+    if (q.reuse_tables && piece2 == p2.sblocks) first.tab[1].nsb = 0;
+    HIPCHK(ctx, launch_prepare_one(prec, first, mx, ctx->stream));
+  }
   for (int st = 0; st < 2; ++st) {
     const int sblocks = st ? p2.sblocks : p1.sblocks, step = st ? piece2 : piece1;
     const int rblocks = st ? p2.rblocks : p1.rblocks, nkb = st ? nkb2 : nkb1;
@@ -1020,6 +1048,23 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
     }
   }
   return MFTX_OK;
+}
+
+int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, int64_t ldf, void* F,
+                            int64_t M, int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r,
+                            double shift_c, double offset_r, double offset_c, double scale, int conj, int precision,
+                            void* ws, size_t cap, size_t table_cap) {
+  if (!ctx) return MFTX_EHANDLE;
+  if (!f || !F) return fail(ctx, MFTX_EINVAL, "null array pointer");
+  if (m <= 0 || n <= 0 || M <= 0 || N <= 0) return fail(ctx, MFTX_EINVAL, "shapes must be positive");
+  if (ldf < n || ldF < N) return fail(ctx, MFTX_EINVAL, "row stride smaller than row length");
+  if (f_dtype < 0 || f_dtype > 3) return fail(ctx, MFTX_EINVAL, "unknown input dtype");
+  if (precision != MFTX_PREC_FP32 && precision != MFTX_PREC_BF16X3) return fail(ctx, MFTX_EINVAL, "unknown precision");
+  if (m > (1 << 20) || n > (1 << 20) || M > (1 << 20) || N > (1 << 20))
+    return fail(ctx, MFTX_EINVAL, "dimension too large");
+  OneSpec q{f, f_dtype, m, n, ldf, F, M, N, ldF, alpha_r, alpha_c, shift_r, shift_c, offset_r, offset_c, scale, conj,
+            precision};
+  return run_one(ctx, q, ws, cap, table_cap);
 }
 
 extern "C" {
@@ -1227,42 +1272,39 @@ int mftx_fft_filter(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int
   float2* F = (float2*)a;
   float2* Y = (float2*)(a + fbytes);
   double* part = (double*)(a + 2 * fbytes);
-  // fft2 then ifft2 as MFTs with alpha = 1/N: input coordinate r and output
-  // coordinate u (uncentred) are r - N//2 + N//2 and (u - N//2) + N//2,
-  // offsets taken modulo N
-  mftx_mft e = {};
-  e.f = img;
-  e.f_dtype = dtype;
-  e.m = rows;
-  e.n = cols;
-  e.ldf = ld;
-  e.F = F;
-  e.M = rows;
-  e.N = cols;
-  e.ldF = cols;
-  e.alpha_r = 1.0 / (double)rows;
-  e.alpha_c = 1.0 / (double)cols;
-  e.offset_r = wrap_coord(rows / 2, rows);
-  e.offset_c = wrap_coord(cols / 2, cols);
-  e.shift_r = wrap_coord(-(rows / 2), rows);
-  e.shift_c = wrap_coord(-(cols / 2), cols);
-  e.scale = 1.0;
-  e.w = kernel;  // the MTF multiplies the spectrum in the store
-  e.w_dtype = kernel_dtype;
-  e.ldw = ldk;
-  rc = dft2_many_run(ctx, &e, 1, precision);
+  // fft2, the MTF, then |ifft2|, as two MFTs with alpha = 1/N.  Both outputs
+  // are computed about their centre, where columns pair (the coordinates are
+  // integers modulo N, so the order of the outputs is free): the spectrum is
+  // held centred, with the MTF (in numpy's fftfreq order) read wrapped, and
+  // the magnitude is taken from the wrapped result.  |ifft2(G)| is |fft2(conj
+  // G)| / n, so the second transform uses the first one's twiddle tables.
+  const int64_t hr = rows / 2, hc = cols / 2;
+  // the size limit is that of the uncentred transform
+  if (too_large(mft_geometry(rows, cols, rows, cols, 1.0 / (double)rows, 1.0 / (double)cols, wrap_coord(-hr, rows),
+                             wrap_coord(-hc, cols), wrap_coord(hr, rows), wrap_coord(hc, cols), 0), true))
+    return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
+  OneSpec q{img, dtype, rows, cols, ld, F, rows, cols, cols, 1.0 / (double)rows, 1.0 / (double)cols, 0.0, 0.0,
+            wrap_coord(hr, rows), wrap_coord(hc, cols), 1.0, 0, precision};
+  q.w = kernel;
+  q.w_dtype = kernel_dtype;
+  q.ldw = ldk;
+  q.wrow = (int)((rows - hr) % rows);
+  q.wcol = (int)((cols - hc) % cols);
+  rc = run_one(ctx, q, nullptr, 0, 0);
   if (rc) return rc;
-  mftx_mft b = e;
+  OneSpec b = q;
   b.f = F;
   b.f_dtype = 0;
   b.ldf = cols;
   b.F = Y;
-  b.conj = 1;
+  b.offset_r = b.offset_c = 0.0;
   b.scale = 1.0 / ((double)rows * (double)cols);
   b.w = nullptr;
-  rc = dft2_many_run(ctx, &b, 1, precision);
+  b.conj_input = true;
+  b.reuse_tables = true;
+  rc = run_one(ctx, b, nullptr, 0, 0);
   if (rc) return rc;
-  HIPCHK(ctx, launch_magnitude(Y, cols, rows, cols, out, out_dtype, ldo, part, ctx->stream));
+  HIPCHK(ctx, launch_magnitude(Y, cols, rows, cols, hr, hc, out, out_dtype, ldo, part, ctx->stream));
   if (normalize) {
     HIPCHK(ctx, launch_sum(img, dtype, rows, cols, ld, part + kMaxPart, ctx->stream));
     HIPCHK(ctx, launch_scale_ratio(out, out_dtype, rows, cols, ldo, part + kMaxPart, part, ctx->stream));
@@ -1724,6 +1766,8 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     q.y0 = g2.y0;
     q.xrot = a2 * xc2;
     q.trans = cf ? 0 : 1;
+    q.wrows = K.M;
+    q.wcols = K.N;
     const double unit = std::sqrt(std::fabs(K.ar * K.ac));  // unitary scale (fourier.py:100-101)
     const bool cl_fast = cfast[ci];
     if (cl_fast) {  // the scale is a power of two, so the weight is rounded once

@@ -107,15 +107,18 @@ __global__ void sum_kernel(const void* __restrict__ x, int dtype, int comp, long
   if (threadIdx.x == 0) part[blockIdx.x] = v;
 }
 
-// out = |F| (F complex64), part[b] = block sums of out
+// out[r][c] = |F[(r + r0) % rows][(c + c0) % cols]| (F complex64, 0 <= r0 < rows,
+// 0 <= c0 < cols), part[b] = block sums of out
 __global__ void magnitude_kernel(const float2* __restrict__ F, long long ldF, long long rows, long long cols,
-                                 void* __restrict__ out, int odt, long long ldo, double* __restrict__ part) {
+                                 long long r0, long long c0, void* __restrict__ out, int odt, long long ldo,
+                                 double* __restrict__ part) {
   const long long n = rows * cols, step = (long long)gridDim.x * kBlock;
   double sum = 0.0;
 #pragma unroll 4
   for (long long t = (long long)blockIdx.x * kBlock + threadIdx.x; t < n; t += step) {
     const long long r = t / cols, c = t % cols;
-    const float2 f = F[r * ldF + c];
+    const long long fr = r + r0 < rows ? r + r0 : r + r0 - rows, fc = c + c0 < cols ? c + c0 : c + c0 - cols;
+    const float2 f = F[fr * ldF + fc];
     const double v = sqrt((double)f.x * f.x + (double)f.y * f.y);
     store_real(out, odt, r * ldo + c, v);
     sum += odt != 3 ? (double)(float)v : v;  // sum what was stored
@@ -147,10 +150,10 @@ hipError_t launch_sum(const void* x, int dtype, long long rows, long long cols, 
   return launch_component_sum(x, dtype, 0, rows, cols, ld, part, s);
 }
 
-hipError_t launch_magnitude(const void* F, long long ldF, long long rows, long long cols, void* out, int odt,
-                            long long ldo, double* part, hipStream_t s) {
+hipError_t launch_magnitude(const void* F, long long ldF, long long rows, long long cols, long long r0, long long c0,
+                            void* out, int odt, long long ldo, double* part, hipStream_t s) {
   hipLaunchKernelGGL(magnitude_kernel, dim3(part_blocks(rows * cols)), dim3(kBlock), 0, s, (const float2*)F, ldF, rows,
-                     cols, out, odt, ldo, part);
+                     cols, r0, c0, out, odt, ldo, part);
   return hipGetLastError();
 }
 

@@ -75,6 +75,15 @@ __device__ __forceinline__ void load_weights(const Problem& P, const long long (
   }
 }
 
+// Map offset of F's element (u, v).
+__device__ __forceinline__ long long weight_index(const Problem& P, int u, int v) {
+  u += P.wrow;
+  v += P.wcol;
+  if (u >= P.wrows) u -= P.wrows;
+  if (v >= P.wcols) v -= P.wcols;
+  return (long long)u * P.ldw + v;
+}
+
 // A lane's (cos, sin) of the store's output phase for its slot: column cp + s
 // turns by (c, s), column cm - s by (c, -s).
 __device__ __forceinline__ float2 slot_phase(const Problem& P, int slot) {
@@ -128,7 +137,7 @@ __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int 
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int row = row0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-        wi[q] = has && row < P.rows ? (long long)row * P.ldw + j : 0;
+        wi[q] = has && row < P.rows ? weight_index(P, row, j) : 0;
       }
       float wv[8];
       load_weights(P, wi, wv);
@@ -156,7 +165,7 @@ __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int 
     const int r0 = row0 + 8 * (lane >> 5);  // first of this lane's 8 rows
     long long wi[8];  // rows past P.rows (not stored) read the column's row 0
 #pragma unroll
-    for (int t = 0; t < 8; ++t) wi[t] = (long long)j * P.ldw + (r0 + t < P.rows ? r0 + t : 0);
+    for (int t = 0; t < 8; ++t) wi[t] = weight_index(P, j, r0 + t < P.rows ? r0 + t : 0);
     float wv[8];
     load_weights(P, wi, wv);
     float2* d = dst + (long long)j * P.ldd + r0;

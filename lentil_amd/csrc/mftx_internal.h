@@ -88,6 +88,8 @@ struct Problem {
   const void* wmap;     // EPI_STORE_CPLX: optional real map multiplied into each stored value,
   long long ldw;        //   indexed like the destination (row stride ldw)
   int wdtype;           //   1 float32, 3 float64
+  int wrow, wcol;       //   added to F's row and column index, modulo wrows and wcols
+  int wrows, wcols;
   int pad2_;
   const float2* rowph;  // EPI_STORE_CPLX: optional phase per C row
 };
@@ -177,6 +179,7 @@ struct PhasorOp {
   int amp_dtype, opd_dtype;
   long long ld_amp, ld_opd;
   int m, n, trans, nwave;
+  int conj, pad_;       // complex source: conjugate it
   const PhasorWave* waves;
   void* dst;
   long long wave_stride;
@@ -229,7 +232,7 @@ hipError_t launch_tables(int prec, const TableOp* ops_dev, int nops, long long t
 hipError_t launch_absmax(const MaxOp* ops_dev, int nops, long long total_blocks, hipStream_t s);
 // One transform's operand, twiddle tables and descriptors (prepare_one_kernel),
 // passed by value: nothing is uploaded.  With op.sc.n == 0 the f16 form's
-// maximum is taken inside the launch.
+// maximum is taken inside the launch; tables with nsb = 0 are there already.
 struct OneDesc {
   Problem prob[2];
   Seg seg[2];
@@ -297,9 +300,9 @@ constexpr int kMaxPart = 1024;
 // part = partial sums of a real array
 hipError_t launch_sum(const void* x, int dtype, long long rows, long long cols, long long ld, double* part,
                       hipStream_t s);
-// out = |F| (F complex64), part = partial sums of out
-hipError_t launch_magnitude(const void* F, long long ldF, long long rows, long long cols, void* out, int odt,
-                            long long ldo, double* part, hipStream_t s);
+// out[r][c] = |F[(r + r0) % rows][(c + c0) % cols]| (F complex64), part = partial sums of out
+hipError_t launch_magnitude(const void* F, long long ldF, long long rows, long long cols, long long r0, long long c0,
+                            void* out, int odt, long long ldo, double* part, hipStream_t s);
 // x *= sum(num) / sum(den), partial sums of arrays of its size
 hipError_t launch_scale_ratio(void* x, int dtype, long long rows, long long cols, long long ld, const double* num,
                               const double* den, hipStream_t s);

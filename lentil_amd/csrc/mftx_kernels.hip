@@ -223,7 +223,7 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
         for (int i = 0; i < NP; ++i) {
           const float2 e = load_elem(op.amp, DT, ia[i]);
           a[rs][ks][i] = in[i] ? e.x * scale : 0.f;
-          ci[rs][ks][i] = in[i] ? e.y * scale : 0.f;
+          ci[rs][ks][i] = in[i] ? e.y * (op.conj ? -scale : scale) : 0.f;
         }
       } else {
         if (op.amp_dtype == 3) {

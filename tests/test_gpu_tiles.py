@@ -123,3 +123,20 @@ def test_fields_of_a_single_segment(L, precision, shape_in):
         ref = sc * w.double().cpu().numpy() * mft.dft2(amp * np.exp(2j * np.pi * opd / wl[p['wave']]), p['alpha'],
                                                        (p['M'], p['N']), p['shift'], p['offset'], unitary=False)
         assert rel_l2(f.cpu().numpy(), ref) < TOL[precision]
+
+
+@pytest.mark.parametrize('precision, tol', [('fp32', 2e-6), ('bf16x3', 2e-5)])
+@pytest.mark.parametrize('shape', [(1, 1), (2, 3), (31, 64), (97, 65), (200, 131)])
+def test_filter_grids(L, precision, tol, shape):
+    """The FFT filter's centred transforms: even, odd and ragged grids, a kernel
+    that is symmetric in neither axis, negative pixels, against numpy's FFT.
+    Two transforms at the fields' gates, relative to the filtered image."""
+    rng = np.random.default_rng(shape[0])
+    img = rng.standard_normal(shape)
+    k = rng.uniform(-1, 1, shape)
+    ref = np.abs(np.fft.ifft2(np.fft.fft2(img) * k))
+    t = torch.from_numpy(img).cuda()
+    got = L.detector.fft_filter(t, torch.from_numpy(k).cuda(), False, precision)
+    assert rel_l2(got.cpu().numpy(), ref) < 3 * tol
+    got = L.detector.fft_filter(t.float(), torch.from_numpy(k).cuda().float(), True, precision)
+    assert rel_l2(got.cpu().numpy(), ref * img.sum() / ref.sum()) < 5 * tol * max(1, abs(np.abs(img).sum() / img.sum()))
