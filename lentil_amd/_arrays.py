@@ -16,11 +16,11 @@ def is_dev(x):
     arrays, CPU tensors, tensors on another device) is host-side data that is
     copied to the device where a kernel reads it, so no kernel is ever handed
     a pointer it cannot dereference."""
-    return isinstance(x, torch.Tensor) and x.is_cuda and x.device == _lib.device()
+    return isinstance(x, torch.Tensor) and x.is_cuda and x.get_device() == _lib.device_index()
 
 
 def shape_of(x):
-    return tuple(x.shape)
+    return x.shape if type(x) is np.ndarray else tuple(x.shape)
 
 
 def size_of(x):
@@ -29,9 +29,8 @@ def size_of(x):
 
 def to_dev(x, real=False):
     """Device tensor of x: complex128/float64 stay exact; the kernels read them directly."""
-    dev = _lib.device()
     if isinstance(x, torch.Tensor):
-        t = x.to(dev)
+        t = x if x.is_cuda and x.get_device() == _lib.device_index() else x.to(_lib.device())
     else:
         a = np.asarray(x)
         if np.iscomplexobj(a):
@@ -41,12 +40,19 @@ def to_dev(x, real=False):
         a = np.ascontiguousarray(a)
         if not a.flags.writeable:
             a = a.copy()
-        t = torch.from_numpy(a).to(dev)
+        t = torch.from_numpy(a).to(_lib.device())
     if real and t.is_complex():
         raise TypeError('expected a real array')
     if t.dim() == 2 and t.stride(1) != 1:
         t = t.contiguous()
     return t
+
+
+def two(x):
+    """x as a read-only pair; one that already is comes back as it is."""
+    if type(x) is np.ndarray and x.shape == (2,) and not x.flags.writeable:
+        return x
+    return np.broadcast_to(x, (2,))
 
 
 def write_back(dst, src):

@@ -12,6 +12,7 @@ import ctypes
 import os
 import threading
 
+import numpy as np
 import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -145,18 +146,37 @@ def check(rc, ctx=None, what=''):
     raise RuntimeError(f'mftx error {rc}: {msg}')
 
 
+_devices = {}     # torch.device by index, filled once a HIP device has been seen
+
+
+def device_index():
+    """Index of the current HIP device."""
+    if not _devices:
+        # asked once: torch reads the environment and the driver on every call
+        if not torch.cuda.is_available():
+            raise RuntimeError('lentil_amd needs a HIP device; none is visible')
+        torch.cuda.init()
+        _devices.update((i, torch.device('cuda', i)) for i in range(torch.cuda.device_count()))
+    return _current_device()
+
+
+# torch's own accessors, where it has them: without the lazy initialisation
+# that device_index has done already, and without building a Stream object
+_current_device = getattr(torch._C, '_cuda_getDevice', torch.cuda.current_device)
+_raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream',
+                      lambda idx: torch.cuda.current_stream(idx).cuda_stream)
+
+
 def device():
     """The HIP device the path runs on (torch 'cuda' is HIP on ROCm)."""
-    if not torch.cuda.is_available():
-        raise RuntimeError('lentil_amd needs a HIP device; none is visible')
-    return torch.device('cuda', torch.cuda.current_device())
+    idx = device_index()
+    return _devices.get(idx) or torch.device('cuda', idx)
 
 
 def context(dev=None):
     """Per-device mftx context bound to torch's current stream."""
-    lib = load()
-    dev = dev or device()
-    idx = dev.index if dev.index is not None else torch.cuda.current_device()
+    lib = _lib or load()
+    idx = device_index() if dev is None or dev.index is None else dev.index
     ctx = _ctx.get(idx)
     if ctx is None:
         with _lock:  # one context per device, also when threads race here
@@ -166,9 +186,21 @@ def context(dev=None):
                 check(lib.mftx_create(idx, ctypes.byref(h)), None, 'mftx_create')
                 ctx = h.value
                 _ctx[idx] = ctx
-    stream = torch.cuda.current_stream(idx).cuda_stream
-    check(lib.mftx_set_stream(ctx, c_vp(stream)), ctx, 'mftx_set_stream')
+    rc = lib.mftx_set_stream(ctx, _raw_stream(idx))
+    if rc != OK:
+        check(rc, ctx, 'mftx_set_stream')
     return ctx
+
+
+def pair(value):
+    """(float, float) of a scalar or a pair, as numpy broadcasts it to (2,)."""
+    if isinstance(value, (float, int)):
+        return float(value), float(value)
+    if type(value) is tuple and len(value) == 2 and isinstance(value[0], (float, int)) \
+            and isinstance(value[1], (float, int)):
+        return float(value[0]), float(value[1])
+    a, b = np.broadcast_to(value, (2,))
+    return float(a), float(b)
 
 
 DTYPE_CODE = {torch.complex64: DT_C64, torch.float32: DT_F32, torch.complex128: DT_C128, torch.float64: DT_F64}

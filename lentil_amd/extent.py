@@ -8,12 +8,11 @@ import numpy as np
 
 def array_extent(shape, shift, parent_shape=None):
     """extent.py:5-40; fewer than two dimensions count as (1, 1)."""
-    if len(shape) < 2:
-        shape = (1, 1)
-    rmin = int(-(shape[0] // 2) + shift[0])
-    cmin = int(-(shape[1] // 2) + shift[1])
-    rmax = int(rmin + shape[0] - 1)
-    cmax = int(cmin + shape[1] - 1)
+    nr, nc = (shape[0], shape[1]) if len(shape) >= 2 else (1, 1)
+    rmin = int(-(nr // 2) + shift[0])
+    cmin = int(-(nc // 2) + shift[1])
+    rmax = int(rmin + nr - 1)
+    cmax = int(cmin + nc - 1)
     if parent_shape is not None:
         pr, pc = (np.asarray(parent_shape) // 2)
         rmin, rmax, cmin, cmax = rmin + pr, rmax + pr, cmin + pc, cmax + pc

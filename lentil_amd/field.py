@@ -30,7 +30,7 @@ class Field:
         self.pixelscale = pixelscale
         self.offset = offset if offset is not None else [0, 0]
         self.tilt = tilt if tilt else []
-        self.extent = _ext.array_extent(self.shape, self.offset)
+        self.extent = _ext.array_extent(shape_of(self.data), self.offset)
 
     @property
     def shape(self):
@@ -43,6 +43,10 @@ class Field:
     def __mul__(self, other):
         """Product over the intersection of extents (field.py:80-147)."""
         tilt = self.tilt + other.tilt
+        for unit, fld in ((self, other), (other, self)):
+            if _is_unit(unit.data) and is_dev(fld.data) and fld.data.dim() == 2 and fld.data.numel() > 1:
+                # the plane wave a Wavefront starts from, times an array: the array where it lies
+                return Field(data=fld.data, offset=_ext.array_center(fld.extent), tilt=tilt)
         if self.size == 1 and other.size == 1:
             if np.array_equal(self.offset, other.offset):
                 data, offset = _scalar_product(self.data, other.data), self.offset
@@ -74,7 +78,7 @@ def tilt_shift(tilts, z, wavelength, pixelscale, oversample, indexing='ij'):
     x, y = 0, 0
     for t in tilts:
         x, y = t.__shift__(xs=x, ys=y, z=z, wavelength=wavelength)
-    ps = np.broadcast_to(pixelscale, (2,))
+    ps = pixelscale if type(pixelscale) is np.ndarray and pixelscale.shape == (2,) else np.broadcast_to(pixelscale, (2,))
     out = x / ps[0] * oversample, y / ps[1] * oversample
     if indexing == 'ij':
         out = -out[1], out[0]
@@ -115,6 +119,10 @@ def _c64(x):
     else:
         t = to_dev(np.ascontiguousarray(x)).to(torch.complex64)
     return t.contiguous()
+
+
+def _is_unit(x):
+    return type(x) is np.ndarray and x.ndim == 0 and x == 1
 
 
 def _is_broadcast_one(x):
@@ -167,7 +175,7 @@ def insert_slices(field_shape, field_offset, out_shape):
     Returns (out_r0, out_c0, field_r0, field_c0, h, w); h or w <= 0 means
     the Field misses the output entirely.
     """
-    if tuple(field_shape) == tuple(out_shape) and np.array_equal(field_offset, [0, 0]):
+    if tuple(field_shape) == tuple(out_shape) and field_offset[0] == 0 and field_offset[1] == 0:
         return 0, 0, 0, 0, int(out_shape[0]), int(out_shape[1])
     oh, ow = int(out_shape[0]), int(out_shape[1])
     fh, fw = int(field_shape[0]), int(field_shape[1])
@@ -230,7 +238,6 @@ def insert(field, out, intensity=False, weight=1):
 
 
 def _device_insert(data, fr0, fc0, h, w, out, or0, oc0, intensity, weight):
-    lib = _lib.load()
     src = data if is_dev(data) and data.dtype == torch.complex64 else to_dev(data).to(torch.complex64)
     src = src.contiguous()
     code = _lib.dtype_code(out)
@@ -239,10 +246,11 @@ def _device_insert(data, fr0, fc0, h, w, out, or0, oc0, intensity, weight):
     if not intensity and code not in (_lib.DT_C64, _lib.DT_C128):
         raise TypeError(f'cannot accumulate a complex field into dtype {out.dtype}')
     ctx = _lib.context()
-    rc = lib.mftx_insert(ctx, ctypes.c_void_p(src.data_ptr()), src.stride(0), fr0, fc0, h, w,
-                         ctypes.c_void_p(out.data_ptr()), code, row_stride(out), or0, oc0,
-                         1 if intensity else 0, float(np.real(weight)))
-    _lib.check(rc, ctx, 'mftx_insert')
+    rc = _lib.load().mftx_insert(ctx, src.data_ptr(), src.stride(0), fr0, fc0, h, w, out.data_ptr(), code,
+                                 row_stride(out), or0, oc0, 1 if intensity else 0,
+                                 weight if type(weight) is float else float(np.real(weight)))
+    if rc != _lib.OK:
+        _lib.check(rc, ctx, 'mftx_insert')
 
 
 def merge(a, b, enforce_overlap=True):

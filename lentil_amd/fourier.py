@@ -9,7 +9,7 @@ tensor.  ``out`` may be either kind and is returned.
 
 The extra keyword-only ``precision`` selects 'fp32' (default) or 'bf16x3'.
 """
-import ctypes
+import math
 
 import numpy as np
 import torch
@@ -32,38 +32,42 @@ def get_precision():
 
 
 def _mft(f, alpha, shape, shift, offset, scale, conj, out, precision):
-    alpha_r, alpha_c = (float(v) for v in np.broadcast_to(alpha, (2,)))
+    alpha_r, alpha_c = _lib.pair(alpha)
     host_input = not is_dev(f)
     if host_input:
         f = np.asarray(f)
     if f.ndim != 2:
         raise ValueError(f'f must be 2-dimensional, got shape {tuple(f.shape)}')
-    m, n = (int(v) for v in f.shape)
+    m, n = f.shape
     if shape is None:
-        shape = (m, n)
-    M, N = (int(v) for v in np.broadcast_to(shape, (2,)))
-    shift_r, shift_c = (float(v) for v in np.broadcast_to(shift, (2,)))
-    off_r, off_c = (float(v) for v in np.broadcast_to(offset, (2,)))
+        M, N = m, n
+    elif type(shape) is tuple and len(shape) == 2:
+        M, N = int(shape[0]), int(shape[1])
+    else:
+        M, N = (int(v) for v in np.broadcast_to(shape, (2,)))
+    shift_r, shift_c = _lib.pair(shift)
+    off_r, off_c = _lib.pair(offset)
     if out is not None:
         odt = out.dtype
         ok = odt.is_complex if isinstance(out, torch.Tensor) else np.can_cast(complex, odt)
         if not ok:
             raise TypeError(f"Cannot cast complex output to dtype('{odt}')")
     prec = _lib.precision_code(precision or _default_precision)
-    src = to_dev(f)
-    if src.dtype not in (torch.complex64, torch.float32, torch.complex128, torch.float64):
+    src = f if not host_input else to_dev(f)
+    if src.dtype not in _lib.DTYPE_CODE:
         src = src.to(torch.complex128 if src.is_complex() else torch.float64)
     src = src.contiguous()
-    if is_dev(out) and out.dtype == torch.complex64 and out.dim() == 2 and out.stride(1) == 1 \
+    if out is not None and is_dev(out) and out.dtype == torch.complex64 and out.dim() == 2 and out.stride(1) == 1 \
             and tuple(out.shape) == (M, N) and out.data_ptr() != src.data_ptr():
         F = out
     else:
         F = torch.empty((M, N), dtype=torch.complex64, device=src.device)
     ctx = _lib.context()
-    rc = _lib.load().mftx_dft2(ctx, ctypes.c_void_p(src.data_ptr()), _lib.dtype_code(src), m, n, src.stride(0),
-                               ctypes.c_void_p(F.data_ptr()), M, N, F.stride(0), alpha_r, alpha_c,
-                               shift_r, shift_c, off_r, off_c, float(scale), 1 if conj else 0, prec)
-    _lib.check(rc, ctx, 'mftx_dft2')
+    rc = _lib.load().mftx_dft2(ctx, src.data_ptr(), _lib.DTYPE_CODE[src.dtype], m, n, src.stride(0), F.data_ptr(), M, N,
+                               F.stride(0), alpha_r, alpha_c, shift_r, shift_c, off_r, off_c, float(scale),
+                               1 if conj else 0, prec)
+    if rc != _lib.OK:
+        _lib.check(rc, ctx, 'mftx_dft2')
     if out is None:
         return F.cpu().numpy().astype(complex) if host_input else F
     if F is out:
@@ -82,9 +86,9 @@ def dft2(f, alpha, shape=None, shift=(0, 0), offset=(0, 0), unitary=True, out=No
     with centred coordinates R = arange(m) - floor(m/2) (fourier.py:113-121)
     and c = sqrt(|ar ac|) when ``unitary``.
     """
-    ar, ac = np.broadcast_to(alpha, (2,))
-    scale = np.sqrt(np.abs(ar * ac)) if unitary else 1.0
-    return _mft(f, alpha, shape, shift, offset, scale, False, out, precision)
+    ar, ac = _lib.pair(alpha)
+    scale = math.sqrt(abs(ar * ac)) if unitary else 1.0
+    return _mft(f, (ar, ac), shape, shift, offset, scale, False, out, precision)
 
 
 def idft2(F, alpha, shape=None, shift=(0, 0), unitary=True, out=None, *, precision=None):
@@ -94,9 +98,9 @@ def idft2(F, alpha, shape=None, shift=(0, 0), unitary=True, out=None, *, precisi
     as in the reference.  Implemented as conjugated twiddles on F directly.
     """
     size = int(F.numel()) if is_dev(F) else int(np.size(F))
-    ar, ac = np.broadcast_to(alpha, (2,))
-    scale = (np.sqrt(np.abs(ar * ac)) if unitary else 1.0) / size
-    return _mft(F, alpha, shape, shift, (0, 0), scale, True, out, precision)
+    ar, ac = _lib.pair(alpha)
+    scale = (np.sqrt(abs(ar * ac)) if unitary else 1.0) / size
+    return _mft(F, (ar, ac), shape, shift, (0, 0), scale, True, out, precision)
 
 
 def dft2_adjoint(G, alpha, in_shape, shift=(0, 0), offset=(0, 0), unitary=True, *, precision=None):

@@ -31,6 +31,5 @@ def slice_offset(slc, shape):
         if slice(None, None, None) in slc:
             return (0, 0)
         raise ValueError(f"Can't compute offset from slice {slc}")
-    size = np.array((slc[0].stop - slc[0].start, slc[1].stop - slc[1].start))
-    off = np.array((slc[0].start + size[0] // 2, slc[1].start + size[1] // 2)) - np.asarray(shape) // 2
-    return (0, 0) if np.all(off == 0) else tuple(off)
+    r, c = slc[0], slc[1]
+    return (r.start + (r.stop - r.start) // 2 - shape[0] // 2, c.start + (c.stop - c.start) // 2 - shape[1] // 2)

@@ -17,7 +17,7 @@ import torch
 from . import _lib, helper
 from .ptype import ptype as as_ptype, none as PT_NONE, pupil as PT_PUPIL, image as PT_IMAGE, tilt as PT_TILT, \
     transform as PT_TRANSFORM
-from ._arrays import to_dev
+from ._arrays import to_dev, two
 from .field import Field
 from .util import boundary
 
@@ -351,17 +351,17 @@ def device_phasor(amp, opd, wavelength):
     m, n = amp.shape
     out = torch.empty((m, n), dtype=torch.complex64, device=amp.device)
     ctx = _lib.context()
-    rc = _lib.load().mftx_phasor(ctx, ctypes.c_void_p(amp.data_ptr()), _lib.dtype_code(amp), amp.stride(0),
-                                 ctypes.c_void_p(opd.data_ptr()), _lib.dtype_code(opd), opd.stride(0), m, n,
-                                 float(wavelength), ctypes.c_void_p(out.data_ptr()))
-    _lib.check(rc, ctx, 'mftx_phasor')
+    rc = _lib.load().mftx_phasor(ctx, amp.data_ptr(), _lib.dtype_code(amp), amp.stride(0), opd.data_ptr(),
+                                 _lib.dtype_code(opd), opd.stride(0), m, n, float(wavelength), out.data_ptr())
+    if rc != _lib.OK:
+        _lib.check(rc, ctx, 'mftx_phasor')
     return out
 
 
 def _mul_pixelscale(a, b):
     """plane.py:614-629."""
-    a = None if a is None else np.broadcast_to(a, (2,))
-    b = None if b is None else np.broadcast_to(b, (2,))
+    a = None if a is None else two(a)
+    b = None if b is None else two(b)
     if a is None and b is None:
         return None
     if a is None:

@@ -10,6 +10,8 @@ with alpha = 1/N on the unpadded field: the zero padding drops out of the
 sum, and the fftshift/ifftshift pair becomes integer coordinate offsets
 (reduced modulo N), so no padded grid is materialised.
 """
+import math
+
 import numpy as np
 import torch
 
@@ -68,16 +70,22 @@ def field_geometry(field, wavelength, dx, du, z, prop_shape_out, out_ext, oversa
     Returns dict(alpha, shape, shift, offset, out_offset).
     """
     sh = field.shift(z=z, wavelength=wavelength, pixelscale=du, oversample=oversample, indexing='ij')
-    fix = np.fix(sh)
-    sub = np.asarray(sh) - fix
+    if isinstance(sh[0], float) and isinstance(sh[1], float):
+        # truncated toward zero on the scalars themselves
+        fix = math.trunc(sh[0]), math.trunc(sh[1])
+        sub = sh[0] - fix[0], sh[1] - fix[1]
+    else:
+        fix = np.fix(sh)
+        sub = np.asarray(sh) - fix
     pext = _ext.array_extent(prop_shape_out, fix)
     if not _ext.intersect(out_ext, pext):
         return None
     ishape = _ext.intersection_shape(out_ext, pext)
     ishift = _ext.intersection_shift(out_ext, pext)
     iext = _ext.array_extent(ishape, ishift)
-    pshift = np.array(_ext.array_center(pext)) - np.array(_ext.array_center(iext))
-    return dict(alpha=_dft_alpha(dx, du, wavelength, z, oversample), shape=ishape, shift=pshift + sub,
+    (pr, pc), (ir, ic) = _ext.array_center(pext), _ext.array_center(iext)
+    return dict(alpha=_dft_alpha(dx, du, wavelength, z, oversample), shape=ishape,
+                shift=(pr - ir + sub[0], pc - ic + sub[1]),
                 offset=field.offset, out_offset=ishift)
 
 
@@ -92,7 +100,8 @@ def propagate_dft(wavefront, pixelscale, shape=None, prop_shape=None, oversample
     dx = wavefront.pixelscale
     du = np.broadcast_to(pixelscale, (2,))
     z = wavefront.focal_length
-    out = Wavefront.empty(wavelength=wavefront.wavelength, pixelscale=du / oversample,
+    pitch = du / oversample
+    out = Wavefront.empty(wavelength=wavefront.wavelength, pixelscale=pitch,
                           focal_length=wavefront.focal_length, shape=shape_out, ptype=ptype_out)
     for field in wavefront.data:
         g = field_geometry(field, wavefront.wavelength, dx, du, z, prop_shape_out, out_ext, oversample)
@@ -100,7 +109,7 @@ def propagate_dft(wavefront, pixelscale, shape=None, prop_shape=None, oversample
             continue
         data = fourier.dft2(to_dev(_as_2d(field.data)), alpha=g['alpha'], shape=g['shape'], shift=g['shift'],
                             offset=g['offset'], unitary=True, precision=precision)
-        out.data.append(Field(data=data, pixelscale=du / oversample, offset=g['out_offset']))
+        out.data.append(Field(data=data, pixelscale=pitch, offset=g['out_offset']))
     return out
 
 

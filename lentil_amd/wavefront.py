@@ -4,7 +4,7 @@ import torch
 
 from . import _lib, field as _field
 from .ptype import ptype as as_ptype, none as PT_NONE, pupil as PT_PUPIL, image as PT_IMAGE
-from ._arrays import is_dev, write_back
+from ._arrays import is_dev, two, write_back
 from .field import Field
 
 
@@ -16,7 +16,7 @@ class Wavefront:
         self.diameter = diameter
         self.shape = ()
         self._wavelength = wavelength
-        self._pixelscale = None if pixelscale is None else np.broadcast_to(pixelscale, (2,))
+        self._pixelscale = None if pixelscale is None else two(pixelscale)
         self.ptype = as_ptype(ptype)
         if tilt is not None:
             if len(tilt) != 2:
