@@ -161,6 +161,17 @@ int mftx_phase_grad_many(mftx_ctx* ctx, const void* amp, int amp_dtype, int64_t 
                          int32_t nwave, const void* D, int64_t ldD, int64_t strideD, double* grad_opd,
                          int64_t ld_gopd, double* grad_amp, int64_t ld_gamp);
 
+/* mftx_phase_grad_many summed over nopd OPDs too (opd_d at opd + d * strideO
+ * elements, D_dw at D + (d * nwave + w) * strideD), in one launch that writes
+ * the gradients (float32 or float64 by gopd_dtype / gamp_dtype; summed in
+ * float64) instead of adding to them.  inv_wavelengths holds the nwave
+ * reciprocal wavelengths in device memory, so nothing is uploaded. */
+int mftx_phase_grad_stack(mftx_ctx* ctx, const void* amp, int amp_dtype, int64_t ld_amp, const void* opd,
+                          int opd_dtype, int64_t ld_opd, int64_t strideO, int32_t nopd, int64_t m, int64_t n,
+                          const double* inv_wavelengths, int32_t nwave, const void* D, int64_t ldD, int64_t strideD,
+                          void* grad_opd, int gopd_dtype, int64_t ld_gopd, void* grad_amp, int gamp_dtype,
+                          int64_t ld_gamp);
+
 /* ---------------------------------------------------------------------------
  * Many independent MFTs in one grouped call (no reference counterpart: the
  * reference runs one fourier.dft2 per call).  Each entry is one mftx_dft2

@@ -83,6 +83,9 @@ SIGNATURES = {
     'mftx_mft_plan_destroy': (c_int, [c_vp]),
     'mftx_phase_grad_many': (c_int, [c_vp, c_vp, c_int, c_i64, c_vp, c_int, c_i64, c_i64, c_i64, c_vp,
                                      ctypes.c_int32, c_vp, c_i64, c_i64, c_vp, c_i64, c_vp, c_i64]),
+    'mftx_phase_grad_stack': (c_int, [c_vp, c_vp, c_int, c_i64, c_vp, c_int, c_i64, c_i64, ctypes.c_int32, c_i64, c_i64,
+                                      c_vp, ctypes.c_int32, c_vp, c_i64, c_i64, c_vp, c_int, c_i64, c_vp, c_int,
+                                      c_i64]),
     'mftx_zero': (c_int, [c_vp, c_vp, c_i64]),
     'mftx_rebin': (c_int, [c_vp, c_vp, c_int, c_i64, c_i64, c_i64, c_i64, c_i64, c_vp, c_int]),
     'mftx_fft_filter': (c_int, [c_vp, c_vp, c_int, c_i64, c_i64, c_i64, c_vp, c_int, c_i64, c_int, c_vp, c_int,

@@ -19,7 +19,7 @@ The forward runs as one batched PSFPlan over every diversity.  The backward
 takes the weighted forward fields from that plan's own stage-1 operands
 (PSFPlan.fields: one complex-output GEMM), runs the adjoint MFTs as one
 persistent grouped plan (mftx_mft_plan, conjugate twiddles) and one
-mftx_phase_grad_many per diversity.
+mftx_phase_grad_stack over every diversity and wavelength.
 """
 import ctypes
 
@@ -50,7 +50,8 @@ class BroadbandPSFModel:
         self.M = self.npix * self.oversample
         self.precision = precision
         self.amp = torch.from_numpy(amp.copy()).to(self.dev)
-        self.div = [torch.as_tensor(np.asarray(d, dtype=float)).to(self.dev) for d in diversity]
+        div = [np.broadcast_to(np.asarray(d, dtype=float), self.shape) for d in diversity]
+        self.div = torch.from_numpy(np.array(div).reshape((len(div),) + self.shape)).to(self.dev)
         # a full-grid mask keeps the tile the whole array at offset (0, 0)
         pupil = Pupil(amplitude=amp, opd=np.zeros(self.shape), mask=np.ones(self.shape), pixelscale=dx,
                       focal_length=z)
@@ -63,9 +64,7 @@ class BroadbandPSFModel:
         self._gen = 0  # forward calls so far: the plan's operands belong to the last one
         # the backward reads opd + diversity from the plan's own OPD buffers
         # (tile 0 of every copy is the whole pupil: the mask is the full grid)
-        for d in range(len(self.div)):
-            ob = self.plan.opd_buffer(0, copy=d)
-            assert tuple(ob.shape) == self.shape and ob.stride(1) == 1
+        assert tuple(self.plan.opd_stack(0).shape) == (len(self.div),) + self.shape
         # the amplitude last written into the plan and into the backward's
         # buffer: (source tensor, its version) -- the source is kept, so its
         # memory cannot be reused by another tensor while it is cached
@@ -91,8 +90,9 @@ class BroadbandPSFModel:
 
     # ---------------------------------------------------------------- forward
     def forward_images(self, opd, amp):
-        for d, div in enumerate(self.div):
-            torch.add(opd, div, out=self.plan.opd_buffer(0, copy=d))
+        if opd.dim() > 2:
+            raise ValueError(f'opd must have shape {self.shape}, got {tuple(opd.shape)}')
+        torch.add(opd, self.div, out=self.plan.opd_stack(0))
         if not self._same(self._amp_in_plan, amp):
             amp32 = amp.to(torch.float32)  # converted once for every copy
             for d in range(len(self.div)):
@@ -127,7 +127,7 @@ class BroadbandPSFModel:
                 r.alpha_r = r.alpha_c = a
                 r.scale, r.conj = float(abs(a)), 1     # sqrt(|a * a|), the unitary scale
         st['adj'] = adj
-        st['wls'] = (ctypes.c_double * nw)(*[float(w) for w in self.wavelengths])
+        st['inv_wl'] = torch.from_numpy(1.0 / self.wavelengths).to(dev)
         # the weighted forward fields Y = unit w_l g_d F come out of the forward
         # plan (problem order: diversity-major copies of one tile per wavelength)
         Ys, Ws, scales = [], [], []
@@ -165,7 +165,7 @@ class BroadbandPSFModel:
         except Exception:
             pass
 
-    def backward_grads(self, opd, amp, grad_images, need_amp, gen=None):
+    def backward_grads(self, opd, amp, grad_images, need_amp, gen=None, dtypes=(torch.float64, torch.float64)):
         """Gradients of sum_d <g_d, I_d> with respect to opd (and amp).
 
         Two GEMM passes cover every (diversity, wavelength) pair: the forward
@@ -173,7 +173,8 @@ class BroadbandPSFModel:
         (restaged from opd and amp when a later forward call replaced them)
         with the weighted cotangent w_l * g_d folded into the store,
         Y = w_l g_d F, then the adjoint MFT D = dft2_adjoint(Y); one
-        phase-gradient launch per diversity sums the wavelengths."""
+        phase-gradient launch sums diversities and wavelengths in float64.
+        ``dtypes``: types of the two gradients (float32 or float64)."""
         lib = _lib.load()
         ctx = _lib.context()
         m, n = self.shape
@@ -185,8 +186,8 @@ class BroadbandPSFModel:
             st['amp'].copy_(amp)
             self._amp_in_bw = (amp, amp._version)
         st['gI'].copy_(grad_images.detach())
-        g_opd = torch.zeros((m, n), dtype=torch.float64, device=self.dev)
-        g_amp = torch.zeros((m, n), dtype=torch.float64, device=self.dev) if need_amp else None
+        g_opd = torch.empty((m, n), dtype=dtypes[0], device=self.dev)
+        g_amp = torch.empty((m, n), dtype=dtypes[1], device=self.dev) if need_amp else None
         if gen is None or gen != self._gen:
             self.forward_images(opd.detach(), amp)
         # from here on the plan's operands and OPD buffers (opd + diversity d)
@@ -194,12 +195,12 @@ class BroadbandPSFModel:
         self.plan.fields()
         (adj_plan,) = st['plans']
         _lib.check(lib.mftx_mft_plan_execute(adj_plan), ctx, 'mftx_mft_plan_execute (adjoint)')
-        for d in range(nd):
-            tot = self.plan.opd_buffer(0, copy=d)
-            _lib.check(lib.mftx_phase_grad_many(ctx, _ptr(st['amp']), _lib.DT_F64, n, _ptr(tot),
-                                                _lib.DT_F64, tot.stride(0), m, n, st['wls'], nw, _ptr(st['D'][d * nw]), n, m * n,
-                                                _ptr(g_opd), n, _ptr(g_amp) if need_amp else None, n),
-                       ctx, 'mftx_phase_grad_many')
+        tot = self.plan.opd_stack(0)
+        _lib.check(lib.mftx_phase_grad_stack(ctx, _ptr(st['amp']), _lib.DT_F64, n, _ptr(tot), _lib.DT_F64, n, m * n, nd,
+                                             m, n, _ptr(st['inv_wl']), nw, _ptr(st['D']), n, m * n, _ptr(g_opd),
+                                             _lib.dtype_code(g_opd), n, _ptr(g_amp) if need_amp else None,
+                                             _lib.dtype_code(g_amp) if need_amp else _lib.DT_F64, n),
+                   ctx, 'mftx_phase_grad_stack')
         return g_opd, g_amp
 
 
@@ -215,6 +216,9 @@ class _PSFStack(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_images):
         opd, amp = ctx.saved_tensors
-        g_opd, g_amp = ctx.model.backward_grads(opd, amp, grad_images, ctx.needs_input_grad[1], gen=ctx.gen)
+        # the kernel writes the leaf's own type where it can
+        dtypes = [t.dtype if t.dtype == torch.float32 else torch.float64 for t in (opd, amp)]
+        g_opd, g_amp = ctx.model.backward_grads(opd, amp, grad_images, ctx.needs_input_grad[1], gen=ctx.gen,
+                                                dtypes=dtypes)
         return (g_opd.to(opd.dtype) if ctx.needs_input_grad[0] else None,
                 g_amp.to(amp.dtype) if g_amp is not None else None, None)

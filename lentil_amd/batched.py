@@ -334,9 +334,12 @@ class PSFPlan:
         dev = _lib.device()
         self._amp_opd = []
         tiles = []
-        for amp, opd in geo['tiles']:
+        # the copies of a tile's OPD lie one after the other (see opd_stack)
+        self._opd_stack = [torch.from_numpy(np.array(opd, dtype=np.float64, order='C', copy=True)).to(dev)
+                           .repeat(copies, 1, 1) for _, opd in geo['tiles'][:ntile0]]
+        for t, (amp, _) in enumerate(geo['tiles']):
             ta = torch.from_numpy(np.array(amp, dtype=np.float32, order='C', copy=True)).to(dev)
-            to = torch.from_numpy(np.array(opd, dtype=np.float64, order='C', copy=True)).to(dev)
+            to = self._opd_stack[t % ntile0][t // ntile0]
             self._amp_opd.append((ta, to))
             tiles.append(_lib.MftxTile(ta.data_ptr(), to.data_ptr(), _lib.DT_F32, _lib.DT_F64, ta.stride(0),
                                        to.stride(0), amp.shape[0], amp.shape[1]))
@@ -464,6 +467,10 @@ class PSFPlan:
     def opd_buffer(self, tile, copy=0):
         """The float64 device OPD a tile (of one copy) is read from, for in-place updates."""
         return self._amp_opd[copy * self._ntile0 + tile][1]
+
+    def opd_stack(self, tile):
+        """The OPD buffers of a tile's copies as one contiguous (copies, m, n) tensor."""
+        return self._opd_stack[tile]
 
     def set_amplitude(self, tile, amp, copy=0):
         """Overwrite a tile's (masked) amplitude (of one copy) in place."""

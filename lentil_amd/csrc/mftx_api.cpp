@@ -262,13 +262,8 @@ struct mftx_plan {
   int n_phasor_ops = 0;
   OperandSplit split{2, 1};
   long long phasor_threads = 0;
-  struct Reduce {
-    float* partial;
-    long long gstride, ldp;
-    int ngroups, rows, cols;
-    long long r0, c0;
-  };
-  std::vector<Reduce> reduces;
+  std::vector<ReduceOp> reduces;   // regions of the image written from partial images
+  ReduceOp* reduce_ops = nullptr;  // ... on the device
   // coherent groups whose Fields have several output grids: complex outputs,
   // summed and squared into the image by one launch (field.py:331-346)
   CoherentGroup* cgroups = nullptr;
@@ -1136,8 +1131,9 @@ int mftx_phase_grad(mftx_ctx* ctx, const void* amp, int amp_dtype, int64_t ld_am
     return fail(ctx, MFTX_EINVAL, "bad gradient shape");
   if (!(wavelength > 0)) return fail(ctx, MFTX_EINVAL, "wavelength must be positive");
   HIPCHK(ctx, hipSetDevice(ctx->device));
-  HIPCHK(ctx, launch_phase_grad(amp, amp_dtype, ld_amp, opd, opd_dtype, ld_opd, (int)m, (int)n, nullptr,
-                                1.0 / wavelength, 1, D, ldD, 0, grad_opd, ld_gopd, grad_amp, ld_gamp, ctx->stream));
+  HIPCHK(ctx, launch_phase_grad(PhaseGrad{amp, opd, amp_dtype, opd_dtype, ld_amp, ld_opd, 0, 1, (int)m, (int)n, 1, nullptr,
+                                          1.0 / wavelength, D, ldD, 0, grad_opd, grad_amp, 3, 3, ld_gopd, ld_gamp, 1},
+                                ctx->stream));
   return MFTX_OK;
 }
 
@@ -1166,8 +1162,33 @@ int mftx_phase_grad_many(mftx_ctx* ctx, const void* amp, int amp_dtype, int64_t 
   void* dev = nullptr;
   const int rc = upload_desc(ctx, inv.data(), sizeof(double) * inv.size(), &dev);
   if (rc) return rc;
-  HIPCHK(ctx, launch_phase_grad(amp, amp_dtype, ld_amp, opd, opd_dtype, ld_opd, (int)m, (int)n, (const double*)dev,
-                                0.0, nwave, D, ldD, strideD, grad_opd, ld_gopd, grad_amp, ld_gamp, ctx->stream));
+  HIPCHK(ctx, launch_phase_grad(PhaseGrad{amp, opd, amp_dtype, opd_dtype, ld_amp, ld_opd, 0, 1, (int)m, (int)n, nwave,
+                                          (const double*)dev, 0.0, D, ldD, strideD, grad_opd, grad_amp, 3, 3, ld_gopd,
+                                          ld_gamp, 1},
+                                ctx->stream));
+  return MFTX_OK;
+}
+
+int mftx_phase_grad_stack(mftx_ctx* ctx, const void* amp, int amp_dtype, int64_t ld_amp, const void* opd,
+                          int opd_dtype, int64_t ld_opd, int64_t strideO, int32_t nopd, int64_t m, int64_t n,
+                          const double* inv_wavelengths, int32_t nwave, const void* D, int64_t ldD, int64_t strideD,
+                          void* grad_opd, int gopd_dtype, int64_t ld_gopd, void* grad_amp, int gamp_dtype,
+                          int64_t ld_gamp) {
+  if (!ctx) return MFTX_EHANDLE;
+  if (!amp || !opd || !D || !grad_opd || !inv_wavelengths) return fail(ctx, MFTX_EINVAL, "null array pointer");
+  if ((amp_dtype != 1 && amp_dtype != 3) || (opd_dtype != 1 && opd_dtype != 3) ||
+      (gopd_dtype != 1 && gopd_dtype != 3) || (grad_amp && gamp_dtype != 1 && gamp_dtype != 3))
+    return fail(ctx, MFTX_EINVAL, "amp, opd and gradients must be float32 or float64");
+  if (m <= 0 || n <= 0 || ld_amp < n || ld_opd < n || ldD < n || ld_gopd < n || (grad_amp && ld_gamp < n) ||
+      m > (1 << 20) || n > (1 << 20))
+    return fail(ctx, MFTX_EINVAL, "bad gradient shape");
+  if (nwave < 1 || nopd < 1 || ((int64_t)nwave * nopd > 1 && strideD < m * ldD) || (nopd > 1 && strideO < m * ld_opd))
+    return fail(ctx, MFTX_EINVAL, "bad wavelength or OPD count or stride");
+  HIPCHK(ctx, hipSetDevice(ctx->device));
+  HIPCHK(ctx, launch_phase_grad(PhaseGrad{amp, opd, amp_dtype, opd_dtype, ld_amp, ld_opd, strideO, nopd, (int)m, (int)n,
+                                          nwave, inv_wavelengths, 0.0, D, ldD, strideD, grad_opd, grad_amp, gopd_dtype,
+                                          gamp_dtype, ld_gopd, ld_gamp, 0},
+                                ctx->stream));
   return MFTX_OK;
 }
 
@@ -1956,6 +1977,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
                                     problems[cls[kv.second[0]].members[0]].weight});
     cadd_class.insert(cadd_class.end(), kv.second.begin(), kv.second.end());
   }
+  const size_t o_red = lay.take(sizeof(ReduceOp) * std::max<size_t>(geos.size(), 1));
   const size_t o_cg = lay.take(sizeof(CoherentGroup) * std::max<size_t>(cgroups.size(), 1));
   const size_t o_ca = lay.take(sizeof(CoherentAdd) * std::max<size_t>(cadd_class.size(), 1));
 
@@ -2093,9 +2115,15 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   }
   for (auto& gi : geos) {
     const ClassInfo& c0 = cls[gi.lgroups[0][0]];
-    plan->reduces.push_back(mftx_plan::Reduce{(float*)(base + gi.partial), (long long)(gi.prow * gi.pcol),
-                                              (long long)gi.pcol, (int)gi.lgroups.size(), c0.key.M, c0.key.N,
-                                              c0.key.r0, c0.key.c0});
+    plan->reduces.push_back(ReduceOp{(const float*)(base + gi.partial), (long long)(gi.prow * gi.pcol),
+                                     (long long)gi.pcol, (int)gi.lgroups.size(), c0.key.M, c0.key.N, (int)c0.key.r0,
+                                     (int)c0.key.c0, 0});
+  }
+  plan->reduce_ops = (ReduceOp*)(base + o_red);
+  if (!plan->reduces.empty())
+    e = hipMemcpy(plan->reduce_ops, plan->reduces.data(), sizeof(ReduceOp) * plan->reduces.size(), hipMemcpyHostToDevice);
+  if (e != hipSuccess) {
+    return hipfail(ctx, e, "plan descriptor upload");
   }
   // ---- info: algorithmic FLOPs are 8 per complex MAC of the cheaper order -------
   double fl = 0, g1 = 0, g2 = 0;
@@ -2123,8 +2151,9 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     bph += (double)ph.m * ph.n * ((ph.amp_dtype == MFTX_DTYPE_F64 ? 8.0 : 4.0) + (ph.opd_dtype == MFTX_DTYPE_F64 ? 8.0 : 4.0)) +
            (double)ph.wave_stride * ph.nwave;
   for (auto& r : plan->reduces) {
-    const double vr = (double)std::max<int64_t>(0, std::min<int64_t>(r.r0 + r.rows, image_rows) - std::max<int64_t>(r.r0, 0));
-    const double vc = (double)std::max<int64_t>(0, std::min<int64_t>(r.c0 + r.cols, image_cols) - std::max<int64_t>(r.c0, 0));
+    const int64_t r1 = (int64_t)r.r0 + r.rows, c1 = (int64_t)r.c0 + r.cols;
+    const double vr = (double)std::max<int64_t>(0, std::min<int64_t>(r1, image_rows) - std::max(r.r0, 0));
+    const double vc = (double)std::max<int64_t>(0, std::min<int64_t>(c1, image_cols) - std::max(r.c0, 0));
     bre += 4.0 * r.ngroups * vr * vc + 4.0 * vr * vc;
   }
   plan->info.bytes_phasor = bph;
@@ -2134,7 +2163,8 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   plan->info.n_stage2 = (int)cls.size();
   plan->info.n_work1 = plan->nwork1;
   plan->info.n_work2 = plan->nwork2 + plan->nwork2c;
-  int nl = (maxes.empty() ? 0 : 1) + (ops.empty() ? 0 : 1) + 1 + (w2.empty() ? 0 : 1) + (w2c.empty() ? 0 : 1) + (int)plan->reduces.size();
+  int nl = (maxes.empty() ? 0 : 1) + (ops.empty() ? 0 : 1) + 1 + (w2.empty() ? 0 : 1) + (w2c.empty() ? 0 : 1) +
+           (plan->reduces.empty() ? 0 : 1);
   nl += plan->n_cgroups ? 1 : 0;
   plan->info.n_launch = nl;
   *out = owned.release();
@@ -2150,28 +2180,6 @@ static hipError_t launch_phasors(const mftx_plan* plan, hipStream_t s) {
   return launch_operands(plan->prec, false, plan->split, plan->phasor_ops, plan->n_phasor_ops, plan->phasor_threads, s);
 }
 
-static hipError_t launch_reduces(const mftx_plan* plan, void* image, int dtype, int64_t ldi, int accumulate,
-                                 hipStream_t s) {
-  const size_t esz = dtype == 3 ? 8 : 4;
-  bool first = true;
-  for (auto& r : plan->reduces) {
-    int acc = accumulate;
-    if (!accumulate && first && !(r.r0 == 0 && r.c0 == 0 && r.rows == plan->img_rows && r.cols == plan->img_cols)) {
-      hipError_t e = launch_zero_rows(image, (int)esz, plan->img_rows, plan->img_cols, ldi, s);
-      if (e != hipSuccess) return e;
-      acc = 1;
-    } else if (!accumulate && !first) {
-      acc = 1;
-    }
-    first = false;
-    hipError_t e = launch_reduce_partials(r.partial, r.gstride, r.ngroups, r.rows, r.cols, r.ldp, image, dtype, ldi,
-                                          (int)plan->img_rows, (int)plan->img_cols, (int)r.r0, (int)r.c0, acc, s);
-    if (e != hipSuccess) return e;
-  }
-  if (!accumulate && plan->reduces.empty()) return launch_zero_rows(image, (int)esz, plan->img_rows, plan->img_cols, ldi, s);
-  return hipSuccess;
-}
-
 // Stage 2: the intensity launch (classes alone in their coherent group) and
 // the complex-store launch (the classes of several-class groups).
 static hipError_t launch_stage2(const mftx_plan* plan, hipStream_t s) {
@@ -2184,14 +2192,14 @@ static hipError_t launch_stage2(const mftx_plan* plan, hipStream_t s) {
   return e;
 }
 
-// The image: the reductions write (or clear and add) it, then the
-// several-class groups add their |sum of fields|^2.
+// The image: one launch sums the partial images into it (or clears it where a
+// plan has none), then the several-class groups add their |sum of fields|^2.
 static hipError_t launch_finish(const mftx_plan* plan, void* image, int dtype, int64_t ldi, int accumulate,
                                 hipStream_t s) {
-  if (!plan->n_cgroups) return launch_reduces(plan, image, dtype, ldi, accumulate, s);
-  if (!plan->reduces.empty()) {
-    const hipError_t e = launch_reduces(plan, image, dtype, ldi, accumulate, s);
-    if (e != hipSuccess) return e;
+  if (!plan->reduces.empty() || !plan->n_cgroups) {
+    const hipError_t e = launch_reduce(plan->reduce_ops, (int)plan->reduces.size(), image, dtype, ldi,
+                                       (int)plan->img_rows, (int)plan->img_cols, accumulate, s);
+    if (e != hipSuccess || !plan->n_cgroups) return e;
     accumulate = 1;
   }
   return launch_coherent(plan->cgroups, plan->n_cgroups, plan->cadds, image, dtype, ldi, (int)plan->img_rows,

@@ -257,10 +257,15 @@ hipError_t launch_row_phases(const RowPhase* ops_dev, int nops, int most_rows, h
 hipError_t launch_phasor_field(const void* amp, int amp_dtype, long long ld_amp, const void* opd,
                                int opd_dtype, long long ld_opd, int m, int n, double inv_wavelength,
                                void* dst, hipStream_t s);
-hipError_t launch_reduce_partials(const float* partial, long long group_stride, int ngroups,
-                                  int rows, int cols, long long ldp, void* out, int out_dtype,
-                                  long long ldo, int out_rows, int out_cols, int r0, int c0,
-                                  int accumulate, hipStream_t s);
+// One region of the image: ngroups partial images of rows x cols (row stride
+// ldp, gstride floats apart) whose first pixel lies at (r0, c0).
+struct ReduceOp {
+  const float* partial;
+  long long gstride, ldp;
+  int ngroups, rows, cols, r0, c0, pad_;
+};
+hipError_t launch_reduce(const ReduceOp* ops, int nops, void* image, int dtype, long long ldi, int rows, int cols,
+                         int accumulate, hipStream_t s);
 // Coherent groups of a plan whose Fields have several output grids: group g's
 // Fields are adds[first .. first + count) of the launch.
 struct CoherentAdd {
@@ -286,10 +291,21 @@ hipError_t launch_zero_rows(void* p, int esz, long long rows, long long cols, lo
 hipError_t launch_weight_field(const void* F, long long ldF, const void* w, int w_dtype, long long ldw,
                                double scale, void* out, long long ldo, int h, int wd, hipStream_t s);
 // nwave wavelengths (inv_wls on the device, or inv_wl0 alone when null), D_w at D + w * strideD
-hipError_t launch_phase_grad(const void* amp, int amp_dtype, long long ld_amp, const void* opd, int opd_dtype,
-                             long long ld_opd, int m, int n, const double* inv_wls, double inv_wl0, int nwave,
-                             const void* D, long long ldD, long long strideD, double* g_opd, long long ldg,
-                             double* g_amp, long long ldga, hipStream_t s);
+struct PhaseGrad {
+  const void *amp, *opd;
+  int amp_dtype, opd_dtype;        // 1 = f32, 3 = f64, also of the gradients
+  long long ld_amp, ld_opd, strideO;
+  int nopd, m, n, nwave;
+  const double* inv_wls;           // device, or null: inv_wl0 and one wavelength
+  double inv_wl0;
+  const void* D;
+  long long ldD, strideD;
+  void *g_opd, *g_amp;             // g_amp may be null
+  int go_dtype, ga_dtype;
+  long long ld_go, ld_ga;
+  int accumulate;
+};
+hipError_t launch_phase_grad(const PhaseGrad& q, hipStream_t s);
 
 // detector-grid post-processing (mftx_detector.hip)
 hipError_t launch_rebin(const void* src, int dtype, long long nimg, long long rows, long long cols, long long ld,
