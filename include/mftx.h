@@ -124,6 +124,21 @@ int mftx_insert(mftx_ctx* ctx, const void* field, int64_t ldf, int64_t fr0, int6
                 int64_t or0, int64_t oc0, int intensity, double weight);
 
 /*
+ * out[r][c] += weight * |sum_i F_i at (r, c)|^2 for a coherent group of up to 64
+ * complex64 Fields: F_i is h x w with row stride ld, its first sample at output
+ * pixel (r0, c0), which may lie outside (Fields are clipped to rows x cols; out is
+ * float32/float64 with row stride ldo).  Replaces field._merge followed by
+ * field.insert(intensity=True) (field.py:331-346, 301-304) without the merged
+ * array: the Fields are summed in FP32 in list order.
+ */
+typedef struct {
+  const void* F;
+  int64_t ld, h, w, r0, c0;
+} mftx_field;
+int mftx_insert_group(mftx_ctx* ctx, const mftx_field* fields, int32_t count, void* out, int out_dtype, int64_t rows,
+                      int64_t cols, int64_t ldo, double weight);
+
+/*
  * out = a * b elementwise over h x w complex64 arrays (row strides lda, ldb, ldo).
  * Replaces the Field product of Field.__mul__ (field.py:142) on the
  * intersection slices computed by the host (field.py:130-147).
@@ -312,6 +327,11 @@ typedef struct {
   int64_t ld_amp, ld_opd;
   int64_t m, n;
 } mftx_tile;
+
+/* mftx_phasor of every tile at one wavelength, out[i] dense m_i x n_i
+ * complex64: the phasors of a segmented plane (plane.py:495-514) in one launch
+ * per 32 tiles. */
+int mftx_phasor_many(mftx_ctx* ctx, const mftx_tile* tiles, int32_t count, double wavelength, void* const* out);
 
 typedef struct {
   int32_t tile;        /* index into tiles */

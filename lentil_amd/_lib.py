@@ -51,6 +51,10 @@ class MftxPlanInfo(ctypes.Structure):
                 ('n_work1', ctypes.c_int32), ('n_work2', ctypes.c_int32)]
 
 
+class MftxField(ctypes.Structure):
+    _fields_ = [('F', c_vp), ('ld', c_i64), ('h', c_i64), ('w', c_i64), ('r0', c_i64), ('c0', c_i64)]
+
+
 class MftxMft(ctypes.Structure):
     _fields_ = [('f', c_vp), ('amp', c_vp), ('opd', c_vp), ('f_dtype', ctypes.c_int32), ('amp_dtype', ctypes.c_int32),
                 ('opd_dtype', ctypes.c_int32), ('conj', ctypes.c_int32), ('m', c_i64), ('n', c_i64), ('ldf', c_i64),
@@ -75,6 +79,9 @@ SIGNATURES = {
     'mftx_phasor': (c_int, [c_vp, c_vp, c_int, c_i64, c_vp, c_int, c_i64, c_i64, c_i64, c_dbl, c_vp]),
     'mftx_insert': (c_int, [c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_i64, c_vp, c_int, c_i64,
                             c_i64, c_i64, c_int, c_dbl]),
+    'mftx_phasor_many': (c_int, [c_vp, ctypes.POINTER(MftxTile), ctypes.c_int32, c_dbl, ctypes.POINTER(c_vp)]),
+    'mftx_insert_group': (c_int, [c_vp, ctypes.POINTER(MftxField), ctypes.c_int32, c_vp, c_int, c_i64, c_i64, c_i64,
+                                  c_dbl]),
     'mftx_multiply': (c_int, [c_vp, c_vp, c_i64, c_vp, c_i64, c_vp, c_i64, c_i64, c_i64]),
     'mftx_dft2_many': (c_int, [c_vp, ctypes.POINTER(MftxMft), ctypes.c_int32, ctypes.c_int32]),
     'mftx_mft_plan_create': (c_int, [c_vp, ctypes.POINTER(MftxMft), ctypes.c_int32, ctypes.c_int32,

@@ -1074,9 +1074,32 @@ int mftx_phasor(mftx_ctx* ctx, const void* amp, int amp_dtype, int64_t ld_amp, c
     return fail(ctx, MFTX_EINVAL, "bad phasor shape");
   if (!(wavelength > 0)) return fail(ctx, MFTX_EINVAL, "wavelength must be positive");
   HIPCHK(ctx, hipSetDevice(ctx->device));
-  HIPCHK(ctx, launch_phasor_field(amp, amp_dtype, ld_amp, opd, opd_dtype, ld_opd, (int)m, (int)n, 1.0 / wavelength,
-                                  out, ctx->stream));
+  const PhasorField q{amp, opd, (float2*)out, ld_amp, ld_opd, (int)m, (int)n, amp_dtype, opd_dtype};
+  HIPCHK(ctx, launch_phasor_fields(&q, 1, 1.0 / wavelength, ctx->stream));
   return MFTX_OK;
+}
+
+int mftx_phasor_many(mftx_ctx* ctx, const mftx_tile* tiles, int32_t count, double wavelength, void* const* out) {
+  if (!ctx) return MFTX_EHANDLE;
+  return guarded(ctx, [&]() -> int {
+    if (count < 0 || (count > 0 && (!tiles || !out))) return fail(ctx, MFTX_EINVAL, "null array pointer");
+    if (!(wavelength > 0)) return fail(ctx, MFTX_EINVAL, "wavelength must be positive");
+    std::vector<PhasorField> items;
+    items.reserve(count);
+    for (int32_t i = 0; i < count; ++i) {
+      const mftx_tile& T = tiles[i];
+      if (!T.amp || !T.opd || !out[i]) return fail(ctx, MFTX_EINVAL, "null array pointer");
+      if ((T.amp_dtype != 1 && T.amp_dtype != 3) || (T.opd_dtype != 1 && T.opd_dtype != 3))
+        return fail(ctx, MFTX_EINVAL, "amp/opd must be float32 or float64");
+      if (T.m <= 0 || T.n <= 0 || T.ld_amp < T.n || T.ld_opd < T.n || T.m > (1 << 20) || T.n > (1 << 20))
+        return fail(ctx, MFTX_EINVAL, "bad phasor shape");
+      items.push_back(PhasorField{T.amp, T.opd, (float2*)out[i], T.ld_amp, T.ld_opd, (int)T.m, (int)T.n, T.amp_dtype,
+                                  T.opd_dtype});
+    }
+    HIPCHK(ctx, hipSetDevice(ctx->device));
+    HIPCHK(ctx, launch_phasor_fields(items.data(), count, 1.0 / wavelength, ctx->stream));
+    return MFTX_OK;
+  });
 }
 
 int mftx_insert(mftx_ctx* ctx, const void* field, int64_t ldf, int64_t fr0, int64_t fc0, int64_t h, int64_t w,
@@ -1094,6 +1117,38 @@ int mftx_insert(mftx_ctx* ctx, const void* field, int64_t ldf, int64_t fr0, int6
   HIPCHK(ctx, launch_insert(field, ldf, (int)fr0, (int)fc0, (int)h, (int)w, out, out_dtype, ldo, (int)or0,
                             (int)oc0, intensity, weight, ctx->stream));
   return MFTX_OK;
+}
+
+int mftx_insert_group(mftx_ctx* ctx, const mftx_field* fields, int32_t count, void* out, int out_dtype, int64_t rows,
+                      int64_t cols, int64_t ldo, double weight) {
+  if (!ctx) return MFTX_EHANDLE;
+  return guarded(ctx, [&]() -> int {
+    if (!out || count < 0 || (count > 0 && !fields)) return fail(ctx, MFTX_EINVAL, "null array pointer");
+    if (count > kGroupFields) return fail(ctx, MFTX_EINVAL, "too many Fields in one group");
+    if (out_dtype != 1 && out_dtype != 3) return fail(ctx, MFTX_EINVAL, "intensity output must be real");
+    if (rows < 0 || cols < 0 || rows > (1 << 20) || cols > (1 << 20) || ldo < cols)
+      return fail(ctx, MFTX_EINVAL, "bad output shape");
+    std::vector<FieldItem> items;
+    int64_t r0 = rows, r1 = 0, c0 = cols, c1 = 0;
+    for (int32_t i = 0; i < count; ++i) {
+      const mftx_field& f = fields[i];
+      if (!f.F) return fail(ctx, MFTX_EINVAL, "null array pointer");
+      if (f.h <= 0 || f.w <= 0 || f.h > (1 << 20) || f.w > (1 << 20) || f.ld < f.w)
+        return fail(ctx, MFTX_EINVAL, "bad Field shape");
+      // a Field beside the output adds nothing
+      if (f.r0 >= rows || f.c0 >= cols || f.r0 + f.h <= 0 || f.c0 + f.w <= 0) continue;
+      items.push_back(FieldItem{f.F, f.ld, (int)f.h, (int)f.w, (int)f.r0, (int)f.c0});
+      r0 = std::min(r0, std::max<int64_t>(f.r0, 0));
+      c0 = std::min(c0, std::max<int64_t>(f.c0, 0));
+      r1 = std::max(r1, std::min(f.r0 + f.h, rows));
+      c1 = std::max(c1, std::min(f.c0 + f.w, cols));
+    }
+    if (items.empty()) return MFTX_OK;
+    HIPCHK(ctx, hipSetDevice(ctx->device));
+    HIPCHK(ctx, launch_insert_group(items.data(), (int)items.size(), (int)r0, (int)c0, (int)(r1 - r0), (int)(c1 - c0),
+                                    out, out_dtype, ldo, weight, ctx->stream));
+    return MFTX_OK;
+  });
 }
 
 int mftx_multiply(mftx_ctx* ctx, const void* a, int64_t lda, const void* b, int64_t ldb, void* out, int64_t ldo,

@@ -254,9 +254,14 @@ struct RowPhase {
 };
 hipError_t launch_row_phases(const RowPhase* ops_dev, int nops, int most_rows, hipStream_t s);
 // launchers (mftx_gemm.hip, mftx_kernels.hip)
-hipError_t launch_phasor_field(const void* amp, int amp_dtype, long long ld_amp, const void* opd,
-                               int opd_dtype, long long ld_opd, int m, int n, double inv_wavelength,
-                               void* dst, hipStream_t s);
+// A phasor Field of a list: dst = amp exp(2 pi i opd inv_wl), m x n, dense.
+struct PhasorField {
+  const void *amp, *opd;
+  float2* dst;
+  long long ld_amp, ld_opd;
+  int m, n, amp_dtype, opd_dtype;
+};
+hipError_t launch_phasor_fields(const PhasorField* items, int count, double inv_wl, hipStream_t s);
 // One region of the image: ngroups partial images of rows x cols (row stride
 // ldp, gstride floats apart) whose first pixel lies at (r0, c0).
 struct ReduceOp {
@@ -283,6 +288,16 @@ hipError_t launch_coherent(const CoherentGroup* groups_dev, int ngroups, const C
 hipError_t launch_insert(const void* field, long long ldf, int fr0, int fc0, int h, int w,
                          void* out, int out_dtype, long long ldo, int or0, int oc0,
                          int intensity, double weight, hipStream_t s);
+// A Field of a coherent group: h x w samples at F (row stride ld) whose first
+// lies at output pixel (r0, c0).
+struct FieldItem {
+  const void* F;
+  long long ld;
+  int h, w, r0, c0;
+};
+constexpr int kGroupFields = 64;  // per launch (2 KiB of kernel arguments)
+hipError_t launch_insert_group(const FieldItem* items, int count, int r0, int c0, int h, int w, void* out,
+                               int out_dtype, long long ldo, double weight, hipStream_t s);
 hipError_t launch_multiply(const void* a, long long lda, const void* b, long long ldb, void* out,
                            long long ldo, int h, int w, hipStream_t s);
 hipError_t launch_zero(void* p, size_t bytes, hipStream_t s);

@@ -253,6 +253,48 @@ def _device_insert(data, fr0, fc0, h, w, out, or0, oc0, intensity, weight):
         _lib.check(rc, ctx, 'mftx_insert')
 
 
+def insert_reduced(fields, out, weight=1):
+    """``insert`` the intensity of every Field of ``reduce(fields)``.  A group
+    of device Fields that would be merged is summed and squared into a device
+    ``out`` by one launch, without the merged array."""
+    for g in _reduce(fields):
+        fs = g['field']
+        if len(fs) == 1:
+            out = insert(fs[0], out, intensity=True, weight=weight)
+        elif len(fs) <= _GROUP_MAX and is_dev(out) and out.dim() == 2 and out.dtype in (torch.float32, torch.float64) \
+                and all(is_dev(f.data) and f.data.dim() == 2 for f in fs):
+            _insert_group(fs, out, weight)
+        else:
+            out = insert(_merge(fs), out, intensity=True, weight=weight)
+    return out
+
+
+_GROUP_MAX = 64     # Fields per mftx_insert_group call
+
+
+def _insert_group(fields, out, weight):
+    _check_pixelscales(fields)
+    rows, cols = out.shape
+    items, keep = [], []
+    for f in fields:
+        t = (f.data if f.data.dtype == torch.complex64 else f.data.to(torch.complex64)).contiguous()
+        keep.append(t)
+        h, w = t.shape
+        if h and w:
+            items.append((t.data_ptr(), w, h, w, rows // 2 + f.extent[0], cols // 2 + f.extent[2]))
+    ctx = _lib.context()
+    rc = _lib.load().mftx_insert_group(ctx, (_lib.MftxField * len(items))(*items), len(items), out.data_ptr(),
+                                       _lib.DTYPE_CODE[out.dtype], rows, cols, row_stride(out), float(np.real(weight)))
+    if rc != _lib.OK:
+        _lib.check(rc, ctx, 'mftx_insert_group')
+
+
+def _check_pixelscales(fields):
+    p0 = fields[0].pixelscale
+    if not all(f.pixelscale is p0 for f in fields) and not np.all([f.pixelscale == p0 for f in fields]):
+        raise ValueError("Can't merge: pixelscales must be equal")
+
+
 def merge(a, b, enforce_overlap=True):
     """Coherently merge two Fields (field.py:308-327)."""
     if enforce_overlap and not overlap((a, b)):
@@ -262,8 +304,7 @@ def merge(a, b, enforce_overlap=True):
 
 def _merge(fields):
     """Sum Fields into their union box (field.py:331-346, 349-386)."""
-    if not np.all([f.pixelscale == fields[0].pixelscale for f in fields]):
-        raise ValueError("Can't merge: pixelscales must be equal")
+    _check_pixelscales(fields)
     rmin, rmax, cmin, cmax = boundary(fields)
     nrow, ncol = rmax - rmin + 1, cmax - cmin + 1
     offset = (rmin + nrow // 2, cmin + ncol // 2)

@@ -327,11 +327,13 @@ class Plane(_PlaneBase):
         out = Wavefront.empty(wavelength=wavefront.wavelength, pixelscale=pixelscale,
                               focal_length=wavefront.focal_length, shape=shape, ptype=ptype)
         phasors = []
-        for n, s, camp, sopd, ta, to in self._device_tiles(mask):
+        tiles = self._device_tiles(mask)
+        arrays = device_phasors([t[4:] for t in tiles if t[4] is not None], wavefront.wavelength)
+        for n, s, camp, sopd, ta, to in tiles:
             if ta is None:  # scalar amplitude and OPD
                 data = camp * np.exp(2 * np.pi * 1j * sopd / wavefront.wavelength)
             else:
-                data = device_phasor(ta, to, wavefront.wavelength)
+                data = next(arrays)
                 if camp is not None:  # complex amplitude: restore its phase
                     ph = torch.from_numpy(np.ascontiguousarray(np.exp(1j * np.angle(camp))).astype(np.complex64))
                     data = data * ph.to(data.device)
@@ -356,6 +358,20 @@ def device_phasor(amp, opd, wavelength):
     if rc != _lib.OK:
         _lib.check(rc, ctx, 'mftx_phasor')
     return out
+
+
+def device_phasors(pairs, wavelength):
+    """Iterator over ``device_phasor`` of every (amp, opd) pair, from one call."""
+    if len(pairs) < 2:
+        return iter([device_phasor(a, o, wavelength) for a, o in pairs])
+    out = [torch.empty(a.shape, dtype=torch.complex64, device=a.device) for a, _ in pairs]
+    ctx = _lib.context()
+    tiles = (_lib.MftxTile * len(pairs))(*[
+        (a.data_ptr(), o.data_ptr(), _lib.dtype_code(a), _lib.dtype_code(o), a.stride(0), o.stride(0), *a.shape)
+        for a, o in pairs])
+    ptrs = (ctypes.c_void_p * len(pairs))(*[t.data_ptr() for t in out])
+    _lib.check(_lib.load().mftx_phasor_many(ctx, tiles, len(pairs), float(wavelength), ptrs), ctx, 'mftx_phasor_many')
+    return iter(out)
 
 
 def _mul_pixelscale(a, b):

@@ -103,12 +103,13 @@ def propagate_dft(wavefront, pixelscale, shape=None, prop_shape=None, oversample
     pitch = du / oversample
     out = Wavefront.empty(wavelength=wavefront.wavelength, pixelscale=pitch,
                           focal_length=wavefront.focal_length, shape=shape_out, ptype=ptype_out)
+    geometry, jobs = [], []
     for field in wavefront.data:
         g = field_geometry(field, wavefront.wavelength, dx, du, z, prop_shape_out, out_ext, oversample)
-        if g is None:
-            continue
-        data = fourier.dft2(to_dev(_as_2d(field.data)), alpha=g['alpha'], shape=g['shape'], shift=g['shift'],
-                            offset=g['offset'], unitary=True, precision=precision)
+        if g is not None:
+            geometry.append(g)
+            jobs.append((to_dev(_as_2d(field.data)), g['alpha'], g['shape'], g['shift'], g['offset']))
+    for data, g in zip(fourier.dft2_list(jobs, precision=precision), geometry):
         out.data.append(Field(data=data, pixelscale=pitch, offset=g['out_offset']))
     return out
 

@@ -79,9 +79,7 @@ class Wavefront:
     def intensity_tensor(self, dtype=torch.float32):
         """Device-resident intensity (no host copy)."""
         acc = torch.zeros(tuple(self.shape), dtype=dtype, device=_lib.device())
-        for f in _field.reduce(self.data):
-            _field.insert(f, acc, intensity=True)
-        return acc
+        return _field.insert_reduced(self.data, acc)
 
     @classmethod
     def empty(cls, wavelength, pixelscale=None, diameter=None, focal_length=None, tilt=None, shape=None,
@@ -99,13 +97,9 @@ class Wavefront:
         ``out`` may be a NumPy array or a device tensor; with a device tensor
         the accumulation stays on the device.
         """
-        fields = _field.reduce(self.data)
         if is_dev(out) or len(np.shape(out)) < 2:
-            for f in fields:
-                out = _field.insert(f, out, intensity=True, weight=weight)
-            return out
+            return _field.insert_reduced(self.data, out, weight)
         dev = torch.from_numpy(np.ascontiguousarray(out)).to(_lib.device())
-        for f in fields:
-            _field.insert(f, dev, intensity=True, weight=weight)
+        _field.insert_reduced(self.data, dev, weight)
         write_back(out, dev)
         return out
