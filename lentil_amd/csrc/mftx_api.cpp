@@ -155,9 +155,11 @@ struct OutGrid {
   double y0, fold;
 };
 
-OutGrid make_grid(double alpha, double shift, int N) {
+// (`about`: the shift of the core to pair about, where grids of several
+// shifts have to share their slots.)
+OutGrid make_grid(double alpha, double shift, int N, double about) {
   const int h = N / 2;
-  const double core = h + shift;
+  const double core = h + about;
   const double mid = 0.5 * (N - 1);
   double c;
   if (std::fabs(core - mid) <= 1.0) {
@@ -174,6 +176,8 @@ OutGrid make_grid(double alpha, double shift, int N) {
   g.fold = -alpha * (shift + h - c);
   return g;
 }
+
+OutGrid make_grid(double alpha, double shift, int N) { return make_grid(alpha, shift, N, shift); }
 
 // Twiddle tables of a launch, shared by every problem with the same rate, slot
 // origin and sample parity (x' = k' + 1/2 for an even number of samples, k'
@@ -255,6 +259,9 @@ struct mftx_plan {
   // stage 2 of the classes whose coherent group has several output grids:
   // their complex fields, summed by the coherent launch (every other class
   // runs the intensity launch above)
+  Work* works2w = nullptr;  // groups whose Fields are windows of one grid
+  Problem* probs2w = nullptr;
+  int nwork2w = 0;
   Work* works2c = nullptr;
   Problem* probs2c = nullptr;
   int nwork2c = 0;
@@ -497,7 +504,6 @@ void mft_problems(const MftGeo& g, int prec, double scale, Problem& a, Problem& 
   a = Problem{};
   a.rblocks = pair_blocks(g.r1);
   a.sblocks = (int)blocks32(g.g1.slots);
-  a.rows = 32 * a.rblocks;
   a.cols = g.g1.slots;
   a.ncols = (int)g.c1;
   a.cp = g.g1.cp;
@@ -509,7 +515,8 @@ void mft_problems(const MftGeo& g, int prec, double scale, Problem& a, Problem& 
   b = Problem{};
   b.rblocks = (int)blocks32(g.c1);
   b.sblocks = (int)blocks32(g.g2.slots);
-  b.rows = (int)g.c1;
+  b.i1 = (int)g.c1;
+  b.j1 = (int)g.c2;
   b.cols = g.g2.slots;
   b.ncols = (int)g.c2;
   b.cp = g.g2.cp;
@@ -1578,8 +1585,40 @@ struct ClassInfo {
   int64_t pairs1 = 0;       // K pairs of its longest stage-1 problem
   std::vector<int> nkb;     // stage-2 K blocks per member
   std::vector<size_t> abuf; // stage-2 operand per member
-  size_t fbuf = 0;    // complex F (partial-overlap groups)
+  size_t fbuf = 0;    // complex F (groups of the coherent launch)
   int p2 = -1;        // index of its stage-2 problem
+  // its output grid: that of the key, or the box shared by its group's windows
+  int M = 0, N = 0;
+  double sr = 0, sc = 0;            // the key's shift seen from the grid's centre
+  double about_r = 0, about_c = 0;  // shift of the core the grid is paired about
+  int wr0 = 0, wc0 = 0;             // where the key's window starts in the grid
+
+  void grids(OutGrid& g1, OutGrid& g2) const {
+    g1 = make_grid(-(col_first ? key.ar : key.ac), col_first ? sr : sc, col_first ? M : N, col_first ? about_r : about_c);
+    g2 = make_grid(-(col_first ? key.ac : key.ar), col_first ? sc : sr, col_first ? N : M, col_first ? about_c : about_r);
+  }
+};
+
+// Whether `classes` windows of one box, of `nkb` stage-2 K blocks each on
+// average, are better summed in registers on the box's grid (box samples over
+// window samples: `waste`) than stored as Fields and summed by the coherent
+// launch.  Per 32 x 32 block and class, in ns on a full chip: in registers 0.65
+// per K block (its fragments come from L2 for each block) and 1.5 for its end,
+// four waves taking the classes in turn; as a Field 0.34 per K block (128 x 128
+// tiles) and 11.5 for storing, reading and adding it.  Measured (whole image,
+// as Fields -> in registers): 18 segments, K = 4: 160 -> 78 us at waste 1.0,
+// 83 -> 57 at 2.0; K = 7: 2169 -> 805 at 1.0, 690 -> 396 at 1.45, 691 -> 505 at
+// 2.0; 6 segments, K = 22: 621 -> 515 at 1.0, 282 -> 286 at 1.29.
+bool sum_windows(double waste, double nkb, int classes) {
+  const double turns = 4.0 * ((classes + 3) / 4) / classes;
+  return waste * (0.65 * nkb * turns + 1.5) <= 0.34 * nkb + 11.5;
+}
+
+// How a class reaches the image.
+enum ClassPath {
+  PATH_INTENSITY,  // alone in its group: |F|^2 summed in registers
+  PATH_WINDOWS,    // one of several windows of one grid: summed in registers, then squared
+  PATH_FIELDS      // one of several grids: F stored, summed and squared by the coherent launch
 };
 
 }  // namespace
@@ -1640,26 +1679,83 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   }
   std::map<std::pair<int, int>, std::vector<int>> groups;  // (wave, group) -> classes
   for (size_t c = 0; c < cls.size(); ++c) groups[{cls[c].key.wave, cls[c].group}].push_back((int)c);
-  // A group with one class runs the intensity path (|F|^2 summed in
-  // registers); the classes of a group with several are summed as complex
-  // fields first (the fallback), and only they.
+  // A group with one class runs the intensity path.  The classes of a group
+  // with several are windows of one grid, the box around them, where the box
+  // is little larger than they are (their shifts differ by a few pixels, as
+  // segment tilts do): transformed on that grid they are summed in registers.
+  // Far apart, each would compute mostly what it drops; then their Fields are
+  // stored and summed by the coherent launch (sum_windows draws the line).
   bool fast = true;  // every group has one class
-  std::vector<char> cfast(cls.size(), 1);
-  for (auto& g : groups)
-    if (g.second.size() > 1) {
-      fast = false;
-      for (int c : g.second) cfast[c] = 0;
-    }
-
-  // contraction order per class (all members share M, N)
+  std::vector<ClassPath> path(cls.size(), PATH_INTENSITY);
+  struct Box { int64_t r0, r1, c0, c1; };
+  std::map<std::pair<int, int>, Box> boxes;  // of the groups of windows
   for (auto& c : cls) {
-    double row_first = 0, col_first = 0;
+    c.M = c.key.M;
+    c.N = c.key.N;
+    c.sr = c.about_r = c.key.sr;
+    c.sc = c.about_c = c.key.sc;
+  }
+  for (auto& g : groups) {
+    if (g.second.size() < 2) continue;
+    fast = false;
+    const ClassKey& k0 = cls[g.second[0]].key;
+    Box b{k0.r0, k0.r0, k0.c0, k0.c0};
+    double area = 0, nkb = 0;
+    bool same = true;
+    for (int c : g.second) {
+      const ClassKey& k = cls[c].key;
+      for (int i : cls[c].members) {
+        const mftx_tile& T = tiles[problems[i].tile];
+        nkb += 0.5 * (pair_blocks(T.m) + pair_blocks(T.n)) / (double)g.second.size();
+      }
+      b.r0 = std::min(b.r0, k.r0);
+      b.r1 = std::max(b.r1, k.r0 + k.M);
+      b.c0 = std::min(b.c0, k.c0);
+      b.c1 = std::max(b.c1, k.c0 + k.N);
+      area += (double)k.M * k.N;
+      same = same && k.ar == k0.ar && k.ac == k0.ac;
+    }
+    const double all = (double)(b.r1 - b.r0) * (double)(b.c1 - b.c0) * (double)g.second.size();
+    const bool windows = same && sum_windows(all / area, nkb, (int)g.second.size()) && b.r1 - b.r0 <= (1 << 20) && b.c1 - b.c0 <= (1 << 20);
+    for (int c : g.second) path[c] = windows ? PATH_WINDOWS : PATH_FIELDS;
+    if (!windows) continue;
+    boxes[g.first] = b;
+    double mr = 0, mc = 0;
+    for (int ci : g.second) {
+      ClassInfo& c = cls[ci];
+      c.M = (int)(b.r1 - b.r0);
+      c.N = (int)(b.c1 - b.c0);
+      c.wr0 = (int)(c.key.r0 - b.r0);
+      c.wc0 = (int)(c.key.c0 - b.c0);
+      // output coordinate (u - M / 2) - shift of one detector pixel in both grids
+      c.sr = c.key.sr + c.wr0 + c.key.M / 2 - c.M / 2;
+      c.sc = c.key.sc + c.wc0 + c.key.N / 2 - c.N / 2;
+      mr += c.sr / (double)g.second.size();
+      mc += c.sc / (double)g.second.size();
+    }
+    for (int ci : g.second) {
+      cls[ci].about_r = mr;
+      cls[ci].about_c = mc;
+    }
+  }
+
+  // contraction order per class (all members share M, N), one for the classes of a group of windows
+  auto costs = [&](const ClassInfo& c, double& row_first, double& col_first) {
     for (int i : c.members) {
       const mftx_tile& T = tiles[problems[i].tile];
-      row_first += cost_row_first(T.m, T.n, c.key.M, c.key.N);
-      col_first += cost_col_first(T.m, T.n, c.key.M, c.key.N);
+      row_first += cost_row_first(T.m, T.n, c.M, c.N);
+      col_first += cost_col_first(T.m, T.n, c.M, c.N);
     }
-    c.col_first = col_first < row_first;
+  };
+  for (auto& g : groups) {
+    double row_first = 0, col_first = 0;
+    for (int c : g.second) {
+      if (path[c] != PATH_WINDOWS) row_first = col_first = 0;
+      costs(cls[c], row_first, col_first);
+      cls[c].col_first = col_first < row_first;
+    }
+    if (path[g.second[0]] == PATH_WINDOWS)
+      for (int c : g.second) cls[c].col_first = col_first < row_first;
   }
 
   // Each problem's stage-1 operand is its tile's phasor at its wavelength,
@@ -1671,13 +1767,12 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   using Slot = std::tuple<int, double, double, double, double>;  // wave, fold1, x01, fold2, x02
   std::vector<Slot> pslot(nprob);
   for (auto& c : cls) {
-    const ClassKey& K = c.key;
     const bool cf = c.col_first;
     for (int i : c.members) {
       const mftx_problem& P = problems[i];
       const mftx_tile& T = tiles[P.tile];
-      const OutGrid g1 = make_grid(-(cf ? P.alpha_r : P.alpha_c), cf ? K.sr : K.sc, cf ? K.M : K.N);
-      const OutGrid g2 = make_grid(-(cf ? K.ac : K.ar), cf ? K.sc : K.sr, cf ? K.N : K.M);
+      OutGrid g1, g2;
+      c.grids(g1, g2);
       pslot[i] = Slot{P.wave, g1.fold, cf ? -centre(T.m) + P.offset_r : -centre(T.n) + P.offset_c, g2.fold,
                       cf ? -centre(T.n) + P.offset_c : -centre(T.m) + P.offset_r};
     }
@@ -1712,7 +1807,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   }
   // stage-2 operands per class and member
   for (auto& c : cls) {
-    const int64_t rows2 = c.col_first ? c.key.M : c.key.N;
+    const int64_t rows2 = c.col_first ? c.M : c.N;
     c.rblocks2 = (int)blocks32(rows2);
     for (int i : c.members) {
       const mftx_tile& T = tiles[problems[i].tile];
@@ -1721,7 +1816,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
       c.abuf.push_back(lay.take(plain_bytes(rows2, nkb)));
       c.pairs1 = std::max<int64_t>(c.pairs1, pairs(c.col_first ? T.m : T.n));
     }
-    if (!cfast[&c - cls.data()]) c.fbuf = lay.take(sizeof(float2) * (size_t)c.key.M * c.key.N);
+    if (path[&c - cls.data()] == PATH_FIELDS) c.fbuf = lay.take(sizeof(float2) * (size_t)c.key.M * c.key.N);
   }
   // f16 form: one scale for all tiles that meet in a coherent group (connected
   // through classes), from the maxima of their amplitudes, which lie together
@@ -1784,11 +1879,11 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     ClassInfo& c = cls[ci];
     const ClassKey& K = c.key;
     const bool cf = c.col_first;
-    const bool single = cfast[ci] && c.members.size() == 1;
+    const bool single = path[ci] == PATH_INTENSITY && c.members.size() == 1;
     const double a1 = -(cf ? K.ar : K.ac), a2 = -(cf ? K.ac : K.ar);
-    const int n1 = cf ? K.M : K.N, n2 = cf ? K.N : K.M;  // output columns of the stages
-    const OutGrid g1 = make_grid(a1, cf ? K.sr : K.sc, n1);
-    const OutGrid g2 = make_grid(a2, cf ? K.sc : K.sr, n2);
+    const int n1 = cf ? c.M : c.N, n2 = cf ? c.N : c.M;  // output columns of the stages
+    OutGrid g1, g2;
+    c.grids(g1, g2);
     double xc2 = 0;
     // stage 1, one problem per member
     for (size_t j = 0; j < c.members.size(); ++j) {
@@ -1801,7 +1896,6 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
       q.send = q.sbeg + 1;
       q.rblocks = pair_blocks(op.R);
       q.sblocks = (int)blocks32(g1.slots);
-      q.rows = 32 * q.rblocks;
       q.cols = g1.slots;
       q.ncols = n1;
       q.cp = g1.cp;
@@ -1834,7 +1928,10 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     Problem q = {};
     q.rblocks = c.rblocks2;
     q.sblocks = (int)blocks32(g2.slots);
-    q.rows = n1;
+    q.i0 = cf ? c.wr0 : c.wc0;
+    q.i1 = q.i0 + (cf ? K.M : K.N);
+    q.j0 = cf ? c.wc0 : c.wr0;
+    q.j1 = q.j0 + (cf ? K.N : K.M);
     q.cols = g2.slots;
     q.ncols = n2;
     q.cp = g2.cp;
@@ -1845,8 +1942,8 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     q.wrows = K.M;
     q.wcols = K.N;
     const double unit = std::sqrt(std::fabs(K.ar * K.ac));  // unitary scale (fourier.py:100-101)
-    const bool cl_fast = cfast[ci];
-    if (cl_fast) {  // the scale is a power of two, so the weight is rounded once
+    const bool stored = path[ci] == PATH_FIELDS;
+    if (!stored) {  // the scale is a power of two, so the weight is rounded once
       q.scale = (float)stage2_scale(prec, c.pairs1);
       q.weight = (float)(unit * unit * problems[c.members[0]].weight);
     } else {
@@ -1854,7 +1951,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
       q.ldd = K.N;  // F[u][v]
     }
     c.p2 = (int)p2.size();
-    patch2.push_back(Patch{cl_fast ? 0 : c.fbuf, prec == PREC_FP32 ? comps[root(problems[c.members[0]].tile)].inv : 0});
+    patch2.push_back(Patch{stored ? c.fbuf : 0, prec == PREC_FP32 ? comps[root(problems[c.members[0]].tile)].inv : 0});
     p2.push_back(q);
   }
   bool multi = false;  // a class of several segments along K
@@ -1895,7 +1992,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     using Grid = std::tuple<int, int, int>;  // stage-2 (cp, cm, slots)
     std::map<std::tuple<int, int, int64_t, int64_t, int>, std::map<Grid, std::vector<int>>> geo;
     for (size_t c = 0; c < cls.size(); ++c) {
-      if (!cfast[c]) continue;
+      if (path[c] != PATH_INTENSITY) continue;
       const Problem& q = p2[cls[c].p2];
       geo[{cls[c].key.M, cls[c].key.N, cls[c].key.r0, cls[c].key.c0, cls[c].col_first ? 1 : 0}][{q.cp, q.cm, q.cols}]
           .push_back((int)c);
@@ -1933,9 +2030,9 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   }
   // stage-2 problem lists in launch order (λ-groups contiguous), intensity and
   // complex-store, each problem followed by copies of its class's segments
-  std::vector<Problem> p2_launch, p2c_launch;
-  std::vector<Patch> patch2_launch, patch2c_launch;
-  std::vector<Work> w2, w2c, wf;
+  std::vector<Problem> p2_launch, p2c_launch, p2w_launch;
+  std::vector<Patch> patch2_launch, patch2c_launch, patch2w_launch;
+  std::vector<Work> w2, w2c, w2w, wf;
   auto push2 = [&](std::vector<Problem>& list, std::vector<Patch>& patches, int c) {
     Problem q = p2[cls[c].p2];
     q.sbeg = (int)segs.size();
@@ -1961,6 +2058,38 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
       add_tiles(w2, plan->tile2, pb, (int)p2_launch.size(), nch, c0.rblocks2, p2[c0.p2].sblocks,
                 (float*)(uintptr_t)poff, (long long)gi.pcol, c0.key.M, c0.key.N);
     }
+  // groups of windows: a partial image per group, those of one box together
+  struct WindowGeo { Box box; size_t partial; int64_t prow, pcol; int n; };
+  std::vector<WindowGeo> wgeos;
+  {
+    std::map<std::tuple<int64_t, int64_t, int64_t, int64_t>, std::vector<std::pair<int, int>>> by_box;
+    for (auto& kv : boxes) by_box[{kv.second.r0, kv.second.r1, kv.second.c0, kv.second.c1}].push_back(kv.first);
+    for (auto& kv : by_box) {
+      WindowGeo wg;
+      wg.box = boxes[kv.second[0]];
+      wg.n = (int)kv.second.size();
+      wg.prow = round_up(wg.box.r1 - wg.box.r0, 128);
+      wg.pcol = round_up(wg.box.c1 - wg.box.c0, 128);
+      wg.partial = lay.take(sizeof(float) * wg.prow * wg.pcol * wg.n);
+      for (int i = 0; i < wg.n; ++i) {
+        const std::vector<int>& cl = groups[kv.second[i]];
+        const int pb = (int)p2w_launch.size();
+        int nch = 0;
+        for (int c : cl) {
+          push2(p2w_launch, patch2w_launch, c);
+          nch += class_nkb(c);
+        }
+        const ClassInfo& c0 = cls[cl[0]];
+        const Problem& q = p2[c0.p2];
+        // the partial image offset rides in the pointer field until the workspace exists
+        float* partial = (float*)(uintptr_t)(wg.partial + sizeof(float) * wg.prow * wg.pcol * i);
+        for (int r = 0; r < c0.rblocks2; ++r)
+          for (int t = 0; t < q.sblocks; ++t)
+            w2w.push_back(Work{pb, (int)p2w_launch.size(), r, t, partial, (long long)wg.pcol, c0.M, c0.N, nch, 0});
+      }
+      wgeos.push_back(wg);
+    }
+  }
   {
     // complex stores: one problem per work item
     auto cplx_tile = [&](const std::vector<int>& cl) {
@@ -1976,7 +2105,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     std::vector<int> slow, every;
     for (size_t c = 0; c < cls.size(); ++c) {
       every.push_back((int)c);
-      if (!cfast[c]) slow.push_back((int)c);
+      if (path[c] == PATH_FIELDS) slow.push_back((int)c);
     }
     if (!slow.empty()) plan->tile2c = cplx_tile(slow);
     if (!every.empty()) plan->tile_f = cplx_tile(every);
@@ -2000,10 +2129,12 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     for (auto& w : ws) f += (double)w.nch * tile_rows(tile) * tile_slots(tile) * 12.0 * 32768.0;
     return f;
   };
-  const double mf1 = mfma(w1, plan->tile1), mf2 = mfma(w2, plan->tile2) + mfma(w2c, plan->tile2c);
+  const double mf1 = mfma(w1, plan->tile1), mf2 = mfma(w2, plan->tile2) + mfma(w2c, plan->tile2c) +
+                     mfma(w2w, TILE_SMALL);
   w1 = xcd_order(w1);
   w2 = xcd_order(w2);
   w2c = xcd_order(w2c);
+  w2w = xcd_order(w2w);
   wf = xcd_order(wf);
 
   const size_t o_tab = lay.total;
@@ -2016,6 +2147,8 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   const size_t o_p2 = lay.take(sizeof(Problem) * std::max<size_t>(p2_launch.size(), 1));
   const size_t o_w2c = lay.take(sizeof(Work) * std::max<size_t>(w2c.size(), 1));
   const size_t o_p2c = lay.take(sizeof(Problem) * std::max<size_t>(p2c_launch.size(), 1));
+  const size_t o_w2w = lay.take(sizeof(Work) * std::max<size_t>(w2w.size(), 1));
+  const size_t o_p2w = lay.take(sizeof(Problem) * std::max<size_t>(p2w_launch.size(), 1));
   const size_t o_segs = lay.take(sizeof(Seg) * std::max<size_t>(segs.size(), 1));
   const size_t o_iw = lay.take(sizeof(PhasorWave) * std::max<size_t>(wave_slots.size(), 1));
   const size_t o_ops = lay.take(sizeof(PhasorOp) * std::max<size_t>(tops.size(), 1));
@@ -2027,12 +2160,12 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   std::vector<CoherentGroup> cgroups;
   std::vector<int> cadd_class;
   for (auto& kv : groups) {
-    if (kv.second.size() < 2) continue;
+    if (path[kv.second[0]] != PATH_FIELDS) continue;
     cgroups.push_back(CoherentGroup{(int)cadd_class.size(), (int)kv.second.size(),
                                     problems[cls[kv.second[0]].members[0]].weight});
     cadd_class.insert(cadd_class.end(), kv.second.begin(), kv.second.end());
   }
-  const size_t o_red = lay.take(sizeof(ReduceOp) * std::max<size_t>(geos.size(), 1));
+  const size_t o_red = lay.take(sizeof(ReduceOp) * std::max<size_t>(geos.size() + wgeos.size(), 1));
   const size_t o_cg = lay.take(sizeof(CoherentGroup) * std::max<size_t>(cgroups.size(), 1));
   const size_t o_ca = lay.take(sizeof(CoherentAdd) * std::max<size_t>(cadd_class.size(), 1));
 
@@ -2056,8 +2189,10 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   rebase(p1, patch1);
   rebase(p2_launch, patch2_launch);
   rebase(p2c_launch, patch2c_launch);
-  for (auto& w : w2)
-    if (w.partial) w.partial = (float*)(base + (size_t)(uintptr_t)w.partial);
+  rebase(p2w_launch, patch2w_launch);
+  for (auto* ws : {&w2, &w2w})
+    for (auto& w : *ws)
+      if (w.partial) w.partial = (float*)(base + (size_t)(uintptr_t)w.partial);
   {
     float2* rp = (float2*)(base + o_rowph);
     for (size_t c = 0; c < cls.size(); ++c) {
@@ -2095,6 +2230,9 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   plan->works2c = (Work*)(base + o_w2c);
   plan->probs2c = (Problem*)(base + o_p2c);
   plan->nwork2c = (int)w2c.size();
+  plan->works2w = (Work*)(base + o_w2w);
+  plan->probs2w = (Problem*)(base + o_p2w);
+  plan->nwork2w = (int)w2w.size();
   plan->works_f = (Work*)(base + o_wf);
   plan->probs_f = (Problem*)(base + o_pf);
   plan->nwork_f = (int)wf.size();
@@ -2111,6 +2249,8 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   up(plan->probs2, p2_launch.data(), sizeof(Problem) * p2_launch.size());
   up(plan->works2c, w2c.data(), sizeof(Work) * w2c.size());
   up(plan->probs2c, p2c_launch.data(), sizeof(Problem) * p2c_launch.size());
+  up(plan->works2w, w2w.data(), sizeof(Work) * w2w.size());
+  up(plan->probs2w, p2w_launch.data(), sizeof(Problem) * p2w_launch.size());
   up(plan->segs, segs.data(), sizeof(Seg) * segs.size());
   up(plan->waves, iw.data(), sizeof(PhasorWave) * iw.size());
   std::vector<CoherentAdd> cadds;
@@ -2174,6 +2314,10 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
                                      (long long)gi.pcol, (int)gi.lgroups.size(), c0.key.M, c0.key.N, (int)c0.key.r0,
                                      (int)c0.key.c0, 0});
   }
+  for (auto& wg : wgeos)
+    plan->reduces.push_back(ReduceOp{(const float*)(base + wg.partial), (long long)(wg.prow * wg.pcol), (long long)wg.pcol,
+                                     wg.n, (int)(wg.box.r1 - wg.box.r0), (int)(wg.box.c1 - wg.box.c0), (int)wg.box.r0,
+                                     (int)wg.box.c0, 0});
   plan->reduce_ops = (ReduceOp*)(base + o_red);
   if (!plan->reduces.empty())
     e = hipMemcpy(plan->reduce_ops, plan->reduces.data(), sizeof(ReduceOp) * plan->reduces.size(), hipMemcpyHostToDevice);
@@ -2217,9 +2361,9 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   plan->info.n_stage1 = (int)p1.size();
   plan->info.n_stage2 = (int)cls.size();
   plan->info.n_work1 = plan->nwork1;
-  plan->info.n_work2 = plan->nwork2 + plan->nwork2c;
+  plan->info.n_work2 = plan->nwork2 + plan->nwork2c + plan->nwork2w;
   int nl = (maxes.empty() ? 0 : 1) + (ops.empty() ? 0 : 1) + 1 + (w2.empty() ? 0 : 1) + (w2c.empty() ? 0 : 1) +
-           (plan->reduces.empty() ? 0 : 1);
+           (w2w.empty() ? 0 : 1) + (plan->reduces.empty() ? 0 : 1);
   nl += plan->n_cgroups ? 1 : 0;
   plan->info.n_launch = nl;
   *out = owned.release();
@@ -2235,12 +2379,15 @@ static hipError_t launch_phasors(const mftx_plan* plan, hipStream_t s) {
   return launch_operands(plan->prec, false, plan->split, plan->phasor_ops, plan->n_phasor_ops, plan->phasor_threads, s);
 }
 
-// Stage 2: the intensity launch (classes alone in their coherent group) and
-// the complex-store launch (the classes of several-class groups).
+// Stage 2: the intensity launch (classes alone in their coherent group), the
+// launch of the groups of windows and the complex-store launch (the classes of
+// the other groups).
 static hipError_t launch_stage2(const mftx_plan* plan, hipStream_t s) {
   hipError_t e = hipSuccess;
   if (plan->nwork2)
     e = launch_gemm(plan->prec, EPI_INTENSITY, plan->tile2, plan->works2, plan->nwork2, plan->probs2, plan->segs, s);
+  if (e == hipSuccess && plan->nwork2w)
+    e = launch_gemm_coherent(plan->prec, plan->works2w, plan->nwork2w, plan->probs2w, plan->segs, s);
   if (e == hipSuccess && plan->nwork2c)
     e = launch_gemm(plan->prec, EPI_STORE_CPLX, plan->tile2c, plan->works2c, plan->nwork2c, plan->probs2c, plan->segs,
                     s);
@@ -2440,7 +2587,7 @@ int mftx_plan_set_fields(mftx_plan* plan, void* const* dst, int64_t ldd, const v
     for (size_t c = 0; c < plan->pf.size(); ++c) {
       const Problem& q = plan->pf[c];
       const int i = plan->class_first[c];
-      const int64_t N = q.trans ? q.rows : q.ncols;  // the class's F is M x N, row stride ldd
+      const int64_t N = q.trans ? q.i1 - q.i0 : q.j1 - q.j0;  // the class's F is M x N, row stride ldd
       if (!dst[i]) return fail(ctx, MFTX_EINVAL, "null field pointer for problem " + std::to_string(i));
       if (ldd < N || (wmap && wmap[i] && ldw < N)) return fail(ctx, MFTX_EINVAL, "field row stride too small");
       if (!std::isfinite(scale[i])) return fail(ctx, MFTX_EINVAL, "non-finite field scale");

@@ -106,7 +106,8 @@ template <int PREC, int EPI>
 __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int side, int slot, int lane, float sc,
                                            float2 ph, float (&re)[8], float (&im)[8]) {
   const int j = side ? P.cm - slot : P.cp + slot;
-  const bool has = side ? (j >= 0 && j < P.ncols && j != P.cp + slot) : j < P.ncols;
+  const bool has = j >= (EPI == EPI_STORE_CPLX ? P.j0 : 0) && j < (EPI == EPI_STORE_CPLX ? P.j1 : P.ncols) &&
+                   !(side && j == P.cp + slot);
   if (P.xrot != 0.0) {
     const float ps = side ? -ph.y : ph.y;
 #pragma unroll
@@ -125,7 +126,7 @@ __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int 
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int row = row0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-        const v2f32 r = ((gptr<const v2f32>)P.rowph)[row < P.rows ? row : 0];
+        const v2f32 r = ((gptr<const v2f32>)P.rowph)[row < P.i1 ? row : 0];
         const float2 v = cmul(make_float2(re[q], im[q]), make_float2(r.x, r.y));
         re[q] = v.x;
         im[q] = v.y;
@@ -137,15 +138,15 @@ __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int 
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int row = row0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-        wi[q] = has && row < P.rows ? weight_index(P, row, j) : 0;
+        wi[q] = has && row >= P.i0 && row < P.i1 ? weight_index(P, row - P.i0, j - P.j0) : 0;
       }
       float wv[8];
       load_weights(P, wi, wv);
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int row = row0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-        if (has && row < P.rows)
-          ((gptr<v2f32>)dst)[(long long)row * P.ldd + j] = v2f32{re[q] * sc * wv[q], im[q] * sc * wv[q]};
+        if (has && row >= P.i0 && row < P.i1)
+          ((gptr<v2f32>)dst)[(long long)(row - P.i0) * P.ldd + (j - P.j0)] = v2f32{re[q] * sc * wv[q], im[q] * sc * wv[q]};
       }
       return;
     }
@@ -162,14 +163,14 @@ __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int 
       o[9 + 2 * q] = __uint_as_float(b[1]);
     }
     if (!has) return;
-    const int r0 = row0 + 8 * (lane >> 5);  // first of this lane's 8 rows
-    long long wi[8];  // rows past P.rows (not stored) read the column's row 0
+    const int r0 = row0 + 8 * (lane >> 5) - P.i0, nr = P.i1 - P.i0;  // first of this lane's 8 rows, in the window
+    long long wi[8];  // rows outside the window (not stored) read the column's row 0
 #pragma unroll
-    for (int t = 0; t < 8; ++t) wi[t] = weight_index(P, j, r0 + t < P.rows ? r0 + t : 0);
+    for (int t = 0; t < 8; ++t) wi[t] = weight_index(P, j - P.j0, r0 + t >= 0 && r0 + t < nr ? r0 + t : 0);
     float wv[8];
     load_weights(P, wi, wv);
-    float2* d = dst + (long long)j * P.ldd + r0;
-    if (r0 + 8 <= P.rows && (((uintptr_t)d) & 15) == 0) {
+    float2* d = dst + (long long)(j - P.j0) * P.ldd + r0;
+    if (r0 >= 0 && r0 + 8 <= nr && (((uintptr_t)d) & 15) == 0) {
 #pragma unroll
       for (int t = 0; t < 4; ++t)
         ((gptr<v4f32>)d)[t] = v4f32{o[4 * t] * wv[2 * t], o[4 * t + 1] * wv[2 * t], o[4 * t + 2] * wv[2 * t + 1],
@@ -177,7 +178,7 @@ __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int 
     } else {
 #pragma unroll
       for (int t = 0; t < 8; ++t)
-        if (r0 + t < P.rows) ((gptr<v2f32>)d)[t] = v2f32{o[2 * t] * wv[t], o[2 * t + 1] * wv[t]};
+        if (r0 + t >= 0 && r0 + t < nr) ((gptr<v2f32>)d)[t] = v2f32{o[2 * t] * wv[t], o[2 * t + 1] * wv[t]};
     }
     return;
   }
@@ -643,6 +644,197 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const Work* __restri
     }
   }
   if (EPI == EPI_INTENSITY) store_partial<2>(wk, probs[wk.pbeg], wk.tr * 32 + 16 * h, side, slot, lane, isum);
+}
+
+// ---------------------------------------------------------------------------
+// Coherent groups whose Fields have their own windows of one output grid
+// ---------------------------------------------------------------------------
+// Work item: the 32 x 32 block (tr, tc) of the grid and the problems of one
+// group (a Field each, its windows in i0 .. j1).  The four waves take the
+// Fields in turn; a wave adds each Field's (P + iQ, P - iQ), turned by its
+// phase and cut to its window, to its complex sum in LDS (in registers it would
+// spill), and the weighted |sum|^2 of the four goes into the group's partial
+// image.
+// No Field is stored.  Bound by the fragments' way from L2 (12 KiB per K block
+// and wave, double-buffered).  A Field has few K blocks (a segment's box) and
+// its window few blocks, so more of them per work item leave the chip idle:
+// 18 segments, 8 wavelengths of 384^2 take 38 us, with 32 x 64 per item (one
+// wave per SIMD) 69, and 121 when the Fields were stored and summed.
+template <int PREC>
+__global__ __launch_bounds__(256, 2) void gemm_coherent_kernel(const Work* __restrict__ works,
+                                                               const Problem* __restrict__ probs,
+                                                               const Seg* __restrict__ segs) {
+  using N = Num<PREC>;
+  typedef typename N::frag frag;
+  // the waves' sums so far: [wave][side, re / im, row group][lane][element]
+  __shared__ alignas(16) float sum[4][16][64][4];
+  const Work wk = works[blockIdx.x];
+  if (wk.pbeg >= wk.pend) return;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) *(v4f32*)sum[wid][i][lane] = v4f32{};
+
+  // Load cursor: the K block the next fragments come from.  Uniform, in SGPRs.
+  struct Cursor {
+    int pc, sg, send, kb, nkb;
+    const char *a, *b;
+  } ld;
+  auto open = [&](Cursor& c) {
+    const Seg& sg = segs[c.sg];
+    c.kb = 0;
+    c.nkb = sg.nkb;
+    c.a = (const char*)sg.a + (long long)wk.tr * sg.a_nkb * A_BLOCK;
+    c.b = (const char*)sg.b + (long long)wk.tc * sg.b_nkb * B_BLOCK;
+  };
+  auto begin = [&](Cursor& c, int pc) {
+    c.pc = pc;
+    c.sg = probs[pc].sbeg;
+    c.send = probs[pc].send;
+    open(c);
+  };
+  const unsigned voff = 16u * lane;
+  frag af[2][8], bf[2][4];
+  // the fragments of the wave's next K block: of the segment, the problem's
+  // next segment, the wave's next problem
+  auto get = [&](int buf) {
+#pragma unroll
+    for (int f = 0; f < 8; ++f) af[buf][f] = *(gptr<const frag>)((gptr<const char>)ld.a + f * FRAG + voff);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) bf[buf][f] = *(gptr<const frag>)((gptr<const char>)ld.b + f * FRAG + voff);
+    if (++ld.kb < ld.nkb) {
+      ld.a += A_BLOCK;
+      ld.b += B_BLOCK;
+    } else if (++ld.sg < ld.send) {
+      open(ld);
+    } else if (ld.pc + 4 < wk.pend) {
+      begin(ld, ld.pc + 4);
+    }  // past the wave's last block the cursor stays: valid memory, read and unused
+  };
+  f32x16 acc[4];
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = f32x16{};
+  };
+  auto mul = [&](int buf) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      const int ia = t == 2 ? 1 : 0, ib = t == 0 ? 1 : 0;  // hi*lo, hi*hi, lo*hi
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        acc[2 * p] = N::mfma(af[buf][4 * p + ia], bf[buf][2 * p + ib], acc[2 * p]);
+        acc[2 * p + 1] = N::mfma(af[buf][4 * p + 2 + ia], bf[buf][2 * p + ib], acc[2 * p + 1]);
+      }
+    }
+  };
+  auto finish = [&](const Problem& P) {
+    const float scale = P.inv ? P.scale * *(cptr<const float>)P.inv : P.scale;
+    const int slot = wk.tc * 32 + (lane & 31);
+    float2 ph = slot_phase(P, slot);
+    ph.x *= scale;
+    ph.y *= scale;
+    const int jp = P.cp + slot, jm = P.cm - slot;
+    const bool hp = jp >= P.j0 && jp < P.j1, hm = jm >= P.j0 && jm < P.j1 && jm != jp;
+    int row0 = wk.tr * 32 + 4 * (lane >> 5);
+    asm volatile("" : "+v"(row0));
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      v4f32* f = (v4f32*)sum[wid][g][lane];  // plus side re, then im, minus side re, im, 256 vectors apart
+      v4f32 ar = f[0], ai = f[256], br = f[512], bi = f[768];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int e = 4 * g + q, row = row0 + 8 * g + q;
+        const bool in = row >= P.i0 && row < P.i1;
+        const float pr = acc[0][e], pi = acc[1][e], qr = acc[2][e], qi = acc[3][e];
+        const float2 a = cmul(make_float2(pr - qi, pi + qr), ph);                       // P + iQ
+        const float2 b = cmul(make_float2(pr + qi, pi - qr), make_float2(ph.x, -ph.y));  // P - iQ
+        ar[q] += in && hp ? a.x : 0.f;
+        ai[q] += in && hp ? a.y : 0.f;
+        br[q] += in && hm ? b.x : 0.f;
+        bi[q] += in && hm ? b.y : 0.f;
+      }
+      f[0] = ar;
+      f[256] = ai;
+      f[512] = br;
+      f[768] = bi;
+    }
+  };
+  // one segment after the other; the next K block's fragments, whichever
+  // segment they belong to, load while one multiplies
+  int pc = wk.pbeg + wid, sg = 0, left = 0;
+  clear();
+  if (pc < wk.pend) {
+    begin(ld, pc);
+    sg = ld.sg;
+    left = ld.nkb;
+    get(0);
+  }
+  while (pc < wk.pend) {
+    for (;;) {
+      get(1);
+      mul(0);
+      if (--left == 0) {  // the next block is in the second buffer
+#pragma unroll
+        for (int f = 0; f < 8; ++f) af[0][f] = af[1][f];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) bf[0][f] = bf[1][f];
+        break;
+      }
+      get(0);
+      mul(1);
+      if (--left == 0) break;
+    }
+    const Problem& P = probs[pc];
+    if (++sg < P.send) {  // the next segment's midpoint: turn (P, Q) by its rotation
+      left = segs[sg].nkb;
+      const float2 r = cis_turns(segs[sg].rot * (P.y0 + (double)(wk.tc * 32 + (lane & 31))));
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float p = acc[i][e], q = acc[2 + i][e];
+          acc[i][e] = r.x * p - r.y * q;
+          acc[2 + i][e] = r.y * p + r.x * q;
+        }
+    } else {
+      finish(P);
+      clear();
+      pc += 4;
+      if (pc < wk.pend) {
+        sg = probs[pc].sbeg;
+        left = segs[sg].nkb;
+      }
+    }
+  }
+  // ---- the four sums, this wave's quarter of the block: rows 16 h .. 16 h + 15 of one side ----
+  __syncthreads();
+  const int h = wid & 1, side = wid >> 1;
+  const Problem& P = probs[wk.pbeg];
+  float v[8];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int i = 8 * side + 2 * h + g;
+    v4f32 re = *(const v4f32*)sum[0][i][lane], im = *(const v4f32*)sum[0][i + 4][lane];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+      re += *(const v4f32*)sum[w][i][lane];
+      im += *(const v4f32*)sum[w][i + 4][lane];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[4 * g + e] = (float)(((double)re[e] * re[e] + (double)im[e] * im[e]) * (double)P.weight);
+  }
+  store_partial<2>(wk, P, wk.tr * 32 + 16 * h, side, wk.tc * 32 + (lane & 31), lane, v);
+}
+
+hipError_t launch_gemm_coherent(int prec, const Work* work, int nwork, const Problem* probs, const Seg* segs,
+                                hipStream_t s) {
+  if (nwork <= 0) return hipSuccess;
+  if (prec == PREC_BF16X3)
+    hipLaunchKernelGGL((gemm_coherent_kernel<PREC_BF16X3>), dim3(nwork), dim3(256), 0, s, work, probs, segs);
+  else
+    hipLaunchKernelGGL((gemm_coherent_kernel<PREC_FP32>), dim3(nwork), dim3(256), 0, s, work, probs, segs);
+  return hipGetLastError();
 }
 
 template <int PREC, int EPI>

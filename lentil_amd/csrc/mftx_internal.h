@@ -73,9 +73,10 @@ struct Seg {
 struct Problem {
   int sbeg, send;       // K segments
   int rblocks, sblocks; // 32-row blocks of the operand, 32-slot blocks of the twiddle table
-  int rows;             // valid C rows (EPI_STORE_CPLX)
   int cols;             // slots
   int ncols;            // N: output columns
+  int i0, i1, j0, j1;   // EPI_STORE_CPLX and coherent sums: the C rows and columns that count (a window
+                        //   of C; the stored array starts at (i0, j0))
   int cp, cm;           // output columns of slot 0 (P + iQ, P - iQ)
   int trans;            // EPI_STORE_CPLX / EPI_INTENSITY: write C transposed
   double y0;            // Y of slot 0
@@ -221,6 +222,8 @@ hipError_t launch_gemm(int prec, int epi, int tile, const Work* work, int nwork,
                        const Seg* segs, hipStream_t s);
 // one problem (on the device, with its one segment of nch K blocks) over row
 // blocks [0, rblocks) and slot blocks [sb0, sb1), sb0 on a tile boundary
+hipError_t launch_gemm_coherent(int prec, const Work* work, int nwork, const Problem* probs, const Seg* segs,
+                                hipStream_t s);
 hipError_t launch_gemm_one(int prec, int epi, int tile, int rblocks, int sb0, int sb1, int nch, const Problem* prob,
                            const Seg* seg, hipStream_t s);
 // every operand source of a plan in one launch (ops_dev on the device, sorted
