@@ -387,8 +387,10 @@ int mftx_plan_execute(mftx_plan* plan, void* image, int32_t image_dtype, int64_t
 int mftx_plan_set_fields(mftx_plan* plan, void* const* dst, int64_t ldd, const void* const* wmap, int32_t wmap_dtype,
                          int64_t ldw, const double* scale);
 int mftx_plan_execute_fields(mftx_plan* plan);
-/* Capture the plan's launches in a hipGraph for this image pointer and replay it
- * on later executes with the same pointer (use_graph != 0), or run eagerly. */
+/* use_graph != 0: capture the plan's launches in a hipGraph when two executes in
+ * a row have one destination (pointer, stride, type, accumulate), and replay it
+ * on later executes with that destination; 0, and on a stream that is being
+ * captured: launch. */
 int mftx_plan_set_graph(mftx_plan* plan, int32_t use_graph);
 int mftx_plan_get_info(const mftx_plan* plan, mftx_plan_info* info);
 /* Time the plan's launch groups (phasors, stage-1 GEMM, stage-2 GEMM,

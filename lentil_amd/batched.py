@@ -290,7 +290,7 @@ class PSFPlan:
     or 128 slots, 0 = chosen per launch); ``autotune`` times every
     (lambda_group, tile_n) candidate on this device and keeps the fastest
     (remembered per problem shape for the process); ``use_graph`` replays the
-    launches from a hipGraph after the first call.  ``copies`` > 1 makes that
+    launches from a hipGraph once two calls in a row write the same buffer.  ``copies`` > 1 makes that
     many independent copies of the pupil's tiles (each with its own device
     amplitude and OPD, see ``set_opd``) whose images lie side by side in one
     (rows, copies * cols) detector, all computed by the same launches.

@@ -280,9 +280,14 @@ struct mftx_plan {
   int use_graph = 0;
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
-  void* g_image = nullptr;
-  int g_dtype = -1, g_accum = -1;
-  int64_t g_ld = -1;
+  struct Target {  // where a call puts the image, and how
+    void* image = nullptr;
+    int dtype = -1, accumulate = -1;
+    int64_t ld = -1;
+    bool operator==(const Target& o) const {
+      return image == o.image && dtype == o.dtype && accumulate == o.accumulate && ld == o.ld;
+    }
+  } captured, last;  // of the graph, of the last call
   // complex fields of every class from the stage-1 operands already in the
   // workspace (mftx_plan_set_fields / mftx_plan_execute_fields)
   Work* works_f = nullptr;
@@ -2429,8 +2434,21 @@ int mftx_plan_execute(mftx_plan* plan, void* image, int32_t image_dtype, int64_t
   if (ldi < plan->img_cols) return fail(ctx, MFTX_EINVAL, "image row stride too small");
   HIPCHK(ctx, hipSetDevice(ctx->device));
   if (!plan->use_graph) return plan_launch(plan, image, image_dtype, ldi, accumulate);
-  if (!plan->gexec || plan->g_image != image || plan->g_dtype != image_dtype || plan->g_ld != ldi ||
-      plan->g_accum != accumulate) {
+  // A graph is made when a destination comes up a second time in a row: the
+  // launches of a call that is not repeated cost 15 us of host time, capturing
+  // and instantiating them 150.  On a stream that is being captured the
+  // launches become part of the caller's graph.
+  const mftx_plan::Target t{image, image_dtype, accumulate, ldi};
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    cs = hipStreamCaptureStatusNone;
+  }
+  if (cs != hipStreamCaptureStatusNone) return plan_launch(plan, image, image_dtype, ldi, accumulate);
+  if (!plan->gexec || !(plan->captured == t)) {
+    const bool again = plan->last == t;
+    plan->last = t;
+    if (!again) return plan_launch(plan, image, image_dtype, ldi, accumulate);
     if (plan->gexec) (void)hipGraphExecDestroy(plan->gexec);
     if (plan->graph) (void)hipGraphDestroy(plan->graph);
     plan->gexec = nullptr;
@@ -2452,11 +2470,9 @@ int mftx_plan_execute(mftx_plan* plan, void* image, int32_t image_dtype, int64_t
     if (e != hipSuccess) return hipfail(ctx, e, "graph capture");
     plan->graph = g;
     HIPCHK(ctx, hipGraphInstantiate(&plan->gexec, g, nullptr, nullptr, 0));
-    plan->g_image = image;
-    plan->g_dtype = image_dtype;
-    plan->g_ld = ldi;
-    plan->g_accum = accumulate;
+    plan->captured = t;
   }
+  plan->last = t;
   HIPCHK(ctx, hipGraphLaunch(plan->gexec, ctx->stream));
   return MFTX_OK;
   });

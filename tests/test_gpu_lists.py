@@ -88,3 +88,34 @@ def test_insert_group_refuses(L, bad):
     out = torch.zeros((8, 8), device='cuda')
     items = (L._lib.MftxField * 65)(*[(F.data_ptr(), q['ld'], q['h'], 4, 0, 0)] * 65)
     assert lib.mftx_insert_group(ctx, items, q['count'], out.data_ptr(), q['dtype'], 8, 8, q['ldo'], 1.0) == L._lib.EINVAL
+
+
+def test_plan_graph_follows_the_destination(L):
+    """The first call of a destination launches, the second captures, later ones replay; changing the
+    destination, the type or adding in between gives the same image every time, and a call on a stream
+    that is being captured becomes part of that graph."""
+    n = 48
+    y, x = np.mgrid[:n, :n] / n - 0.5
+    pupil = L.Pupil(amplitude=(np.hypot(x, y) < 0.45).astype(float), opd=2e-7 * x * y, pixelscale=1 / n, focal_length=10.0)
+    wl = np.linspace(5e-7, 7e-7, 3)
+    plan = L.PSFPlan(pupil, wl, None, pixelscale=5e-6, shape=40, oversample=2, precision='fp32')
+    want = L.PSFPlan(pupil, wl, None, pixelscale=5e-6, shape=40, oversample=2, precision='fp32', use_graph=False)()
+    a, b = torch.empty_like(want), torch.empty_like(want)
+    d = torch.empty(want.shape, dtype=torch.float64, device='cuda')
+    for dst in (a, a, a, b, a, b, b, b, d, d, d, a, a):
+        dst.fill_(float('nan'))
+        plan(out=dst)
+        assert torch.equal(dst.float(), want)
+    plan(out=a, accumulate=True)
+    plan(out=a, accumulate=True)
+    assert float((a - 3 * want).abs().max()) <= 1e-6 * float(want.max())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        plan(out=b)
+    for _ in range(3):
+        b.fill_(float('nan'))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(b, want)
+        plan(out=a)
+        assert torch.equal(a, want)
