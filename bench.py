@@ -8,8 +8,8 @@ stage-2 GEMM with |E|^2 accumulated over wavelengths, detector reduction.
 Inputs are resident in HBM before the timed region.
 
 Printed: one JSON line with PSFs/s, the roofline of the dominant kernel
-(stage-2 GEMM, timed as it runs in the replayed graph: stream events around
-back-to-back replays of prefix graphs), the relative-L2 error
+(stage-2 GEMM, timed right after its producer: stream events around
+back-to-back replays of graphs of the plan's first launches), the relative-L2 error
 of the image against the complex128 reference loop, the plain per-wavelength
 FP32 GPU path and the CPU baseline (the complex128 oracle of the reference
 loop on this host's cores).
@@ -52,7 +52,7 @@ def parse():
                     help='segmented workloads: segment tiles one by one, summed into their union box, or '
                          'whichever executes fewer MACs')
     ap.add_argument('--eager', action='store_true',
-                    help='launch the plan straight onto the stream each step instead of replaying a hipGraph')
+                    help='time the stages by events between launches instead of replays of prefix graphs')
     ap.add_argument('--copy-mib', type=int, default=0,
                     help='after the timed steps, run one plain device copy of this many MiB (a known-size '
                          'kernel that scales hardware byte counters)')
@@ -314,8 +314,8 @@ def main():
         torch.cuda.synchronize()
         del src, dst, evict
 
-    # per launch group in the mode the steps ran in (graph replay): differences
-    # of replayed prefix graphs, after the clocks have settled again
+    # per launch group: differences of replayed prefix graphs, after the clocks
+    # have settled again
     scratch = torch.empty_like(out)
     warm_up(lambda: plan(scratch), 0, torch.cuda.synchronize)
     stage_ms = plan.profile(scratch, repeats=60)
@@ -418,7 +418,7 @@ def main():
         'config': {'workload': 'broadband_512', 'pupil': 512, 'detector': 1024, 'wavelengths': nwave,
                    'psfs_per_step': nwave, 'precision': args.precision, 'lambda_group': plan.lambda_group,
                    'tile_n': plan.tile_n, 'autotuned': tuned, 'autotune_source': plan.tuned_from,
-                   'launch': 'eager' if args.eager else 'graph replay',
+                   'launch': 'stream', 'stage_timing': stage_ms['mode'],
                    'parallelism': 'single GPU'},
         'warmup_executed': warmed,
         'tflops_algorithmic': total_flops * args.steps / dt / 1e12,

@@ -85,7 +85,7 @@ int mftx_dft2(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, i
  * reference: this is for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  Same arguments, results and errors as mftx_dft2, but the
- * packed operands live in a fixed array of device memory that the library
+ * operands and twiddle tables live in a fixed array of device memory that the library
  * holds on every GPU it runs on until the process ends (its address is looked
  * up once per device, at mftx_create).  A transform whose operands, counted as
  * complex64 with padded rows, need more than MFTX_NOALLOC_SCRATCH_BYTES (about a 1024^2 -> 2048^2
@@ -196,7 +196,8 @@ int mftx_phase_grad_stack(mftx_ctx* ctx, const void* amp, int amp_dtype, int64_t
  *   - when w is not NULL the output is multiplied elementwise by the real
  *     M x N map w (float32/float64, row stride ldw): the weighted cotangent
  *     of an intensity for the adjoint pass of phase retrieval.
- * All entries run in one pack launch and one launch per GEMM stage.
+ * All entries run in one operand launch (one more for complex inputs beside
+ * phasors) and one launch per GEMM stage.
  * ------------------------------------------------------------------------- */
 typedef struct {
   const void* f;       /* input m x n (f_dtype, row stride ldf), or NULL for a phasor */
@@ -387,15 +388,15 @@ int mftx_plan_execute(mftx_plan* plan, void* image, int32_t image_dtype, int64_t
 int mftx_plan_set_fields(mftx_plan* plan, void* const* dst, int64_t ldd, const void* const* wmap, int32_t wmap_dtype,
                          int64_t ldw, const double* scale);
 int mftx_plan_execute_fields(mftx_plan* plan);
-/* use_graph != 0: capture the plan's launches in a hipGraph when two executes in
- * a row have one destination (pointer, stride, type, accumulate), and replay it
- * on later executes with that destination; 0, and on a stream that is being
- * captured: launch. */
+/* How mftx_plan_profile times the plan: use_graph != 0 by replaying graphs of
+ * its first launches, 0 by events between launches.  An execute always queues
+ * its 3 to 8 launches directly (replaying them from a graph took longer), also
+ * on a stream that is being captured, where they join the caller's graph. */
 int mftx_plan_set_graph(mftx_plan* plan, int32_t use_graph);
 int mftx_plan_get_info(const mftx_plan* plan, mftx_plan_info* info);
 /* Time the plan's launch groups (phasors, stage-1 GEMM, stage-2 GEMM,
- * detector reduction) in the mode executes run in, `repeats` times each (at
- * most 4096).  When the plan replays a graph: one graph per prefix of the
+ * detector reduction), `repeats` times each (at most 4096).  After
+ * mftx_plan_set_graph(plan, 1): one graph per prefix of the
  * groups (the first k, k = 1..4) is replayed `repeats` times back to back
  * between two stream events, after two full replays, the prefixes in the
  * order 1 2 3 4 4 3 2 1 so a slow clock drift cancels; a group's time is the

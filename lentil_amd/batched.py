@@ -11,8 +11,7 @@
 
 as a handful of grouped launches (phasors for every (segment, wavelength),
 one stage-1 GEMM launch, one stage-2 GEMM launch with |E|^2 accumulated in
-registers across wavelengths, one reduction onto the detector), optionally
-replayed from a hipGraph.  The per-Field geometry is the same host code as
+registers across wavelengths, one reduction onto the detector).  The per-Field geometry is the same host code as
 ``propagate_dft`` (``propagate.field_geometry``), so both paths agree on
 every shift, clip and offset.
 """
@@ -289,8 +288,8 @@ class PSFPlan:
     tile accumulation in registers; ``tile_n`` is the GEMM workgroup width (64
     or 128 slots, 0 = chosen per launch); ``autotune`` times every
     (lambda_group, tile_n) candidate on this device and keeps the fastest
-    (remembered per problem shape for the process); ``use_graph`` replays the
-    launches from a hipGraph once two calls in a row write the same buffer.  ``copies`` > 1 makes that
+    (remembered per problem shape for the process); ``use_graph`` says how
+    ``profile`` times the launches.  ``copies`` > 1 makes that
     many independent copies of the pupil's tiles (each with its own device
     amplitude and OPD, see ``set_opd``) whose images lie side by side in one
     (rows, copies * cols) detector, all computed by the same launches.
@@ -442,10 +441,10 @@ class PSFPlan:
 
     def profile(self, out=None, repeats=5):
         """Mean milliseconds of (phasors, stage-1 GEMM, stage-2 GEMM, reduction)
-        in the mode calls run in: with ``use_graph``, differences of the mean
+        with ``use_graph`` by differences of the mean
         replay times of prefix graphs (the first k launch groups, ``repeats``
         back-to-back replays each between two stream events), so each group
-        runs right after its producer as in a replayed call; otherwise HIP
+        runs right after its producer as in a call; otherwise by HIP
         events between eagerly queued groups.  ``mode`` says which was used."""
         if out is None:
             out = torch.empty(self.shape_out, dtype=torch.float32, device=_lib.device())

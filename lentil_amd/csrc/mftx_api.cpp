@@ -1,7 +1,7 @@
 // C-ABI of the mftx library (declared in include/mftx.h).
 //
 // An MFT F = c * E1 . f . E2 (lentil fourier.py:97) runs as two launches of
-// the complex GEMM C = A . B (A packed data, B generated twiddles):
+// the complex GEMM C = A . B (A an operand of paired samples, B twiddle tables):
 //   order B (row-first):    G   = f . E2        -> stored as G^T
 //                           F^T = G^T . E1^T    -> F or |F|^2
 //   order A (column-first): T^T = f^T . E1^T    -> stored as T
@@ -9,7 +9,8 @@
 // Order B costs m*n*N + M*m*N complex MACs, order A M*m*n + M*n*N; the
 // cheaper one is used.  Several Fields summed coherently share one output
 // grid, so their stage-2 GEMMs concatenate along K (one GEMM per coherent
-// group, each K segment with its own twiddle coordinate origin).
+// group, each K segment with its own midpoint), or run as windows of one grid
+// that are summed on chip (sum_windows).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -277,17 +278,7 @@ struct mftx_plan {
   CoherentAdd* cadds = nullptr;
   int n_cgroups = 0;
   mftx_plan_info info = {};
-  int use_graph = 0;
-  hipGraphExec_t gexec = nullptr;
-  hipGraph_t graph = nullptr;
-  struct Target {  // where a call puts the image, and how
-    void* image = nullptr;
-    int dtype = -1, accumulate = -1;
-    int64_t ld = -1;
-    bool operator==(const Target& o) const {
-      return image == o.image && dtype == o.dtype && accumulate == o.accumulate && ld == o.ld;
-    }
-  } captured, last;  // of the graph, of the last call
+  int use_graph = 0;  // mftx_plan_profile times prefix graphs
   // complex fields of every class from the stage-1 operands already in the
   // workspace (mftx_plan_set_fields / mftx_plan_execute_fields)
   Work* works_f = nullptr;
@@ -2433,53 +2424,14 @@ int mftx_plan_execute(mftx_plan* plan, void* image, int32_t image_dtype, int64_t
   if (image_dtype != 1 && image_dtype != 3) return fail(ctx, MFTX_EINVAL, "image must be float32 or float64");
   if (ldi < plan->img_cols) return fail(ctx, MFTX_EINVAL, "image row stride too small");
   HIPCHK(ctx, hipSetDevice(ctx->device));
-  if (!plan->use_graph) return plan_launch(plan, image, image_dtype, ldi, accumulate);
-  // A graph is made when a destination comes up a second time in a row: the
-  // launches of a call that is not repeated cost 15 us of host time, capturing
-  // and instantiating them 150.  On a stream that is being captured the
-  // launches become part of the caller's graph.
-  const mftx_plan::Target t{image, image_dtype, accumulate, ldi};
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess) {
-    (void)hipGetLastError();
-    cs = hipStreamCaptureStatusNone;
-  }
-  if (cs != hipStreamCaptureStatusNone) return plan_launch(plan, image, image_dtype, ldi, accumulate);
-  if (!plan->gexec || !(plan->captured == t)) {
-    const bool again = plan->last == t;
-    plan->last = t;
-    if (!again) return plan_launch(plan, image, image_dtype, ldi, accumulate);
-    if (plan->gexec) (void)hipGraphExecDestroy(plan->gexec);
-    if (plan->graph) (void)hipGraphDestroy(plan->graph);
-    plan->gexec = nullptr;
-    plan->graph = nullptr;
-    hipStream_t cap = nullptr;
-    HIPCHK(ctx, hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
-    hipStream_t saved = ctx->stream;
-    ctx->stream = cap;
-    hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
-    int rc = e == hipSuccess ? plan_launch(plan, image, image_dtype, ldi, accumulate) : MFTX_OK;
-    hipGraph_t g = nullptr;
-    if (e == hipSuccess) e = hipStreamEndCapture(cap, &g);
-    ctx->stream = saved;
-    (void)hipStreamDestroy(cap);
-    if (rc) {
-      if (g) (void)hipGraphDestroy(g);
-      return rc;
-    }
-    if (e != hipSuccess) return hipfail(ctx, e, "graph capture");
-    plan->graph = g;
-    HIPCHK(ctx, hipGraphInstantiate(&plan->gexec, g, nullptr, nullptr, 0));
-    plan->captured = t;
-  }
-  plan->last = t;
-  HIPCHK(ctx, hipGraphLaunch(plan->gexec, ctx->stream));
-  return MFTX_OK;
+  // Launched one by one: a plan is 3 to 8 launches, 3 to 4 us of host time each,
+  // and replaying them from a graph took longer on either side (host 13 -> 28 us
+  // and 324 -> 329 us an image for 64 wavelengths of 1024^2, 17 -> 23 and 19 ->
+  // 25 us for three of 64^2), besides 150 us to capture and instantiate one.
+  return plan_launch(plan, image, image_dtype, ldi, accumulate);
   });
 }
 
-// One execute's launch groups with a timing event before, between and after
-// them (ev[0..4]) on stream s.
 // The plan's launch groups in execute order (phasors, stage-1 GEMM, stage-2
 // GEMM, reduction), the first `upto` of them; with `ev`, an event
 // is recorded before the first and after each.
@@ -2501,8 +2453,8 @@ static hipError_t profile_launches(mftx_plan* plan, void* image, int dtype, int6
 // Graph mode of mftx_plan_profile: one graph per prefix of the launch groups
 // (the first k of them, k = 1..4), each replayed `repeats` times back to back
 // between two stream events, twice; group k's time is the difference of the
-// mean replay times of prefixes k + 1 and k, so every launch runs as in a
-// replayed execute, after its producer, with no event between launches.
+// mean replay times of prefixes k + 1 and k, so every launch runs as in an
+// execute, after its producer, with no event between launches.
 // Returns the runtime's error when it cannot capture.
 static hipError_t profile_graphs(mftx_plan* plan, void* image, int dtype, int64_t ldi, int repeats, double* ms) {
   hipStream_t s = plan->ctx->stream;
@@ -2657,8 +2609,6 @@ int mftx_plan_destroy(mftx_plan* plan) {
     (void)hipSetDevice(plan->ctx->device);
     (void)hipStreamSynchronize(plan->ctx->stream);
   }
-  if (plan->gexec) (void)hipGraphExecDestroy(plan->gexec);
-  if (plan->graph) (void)hipGraphDestroy(plan->graph);
   if (plan->ws) (void)hipFree(plan->ws);
   delete plan;
   return MFTX_OK;

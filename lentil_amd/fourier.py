@@ -1,7 +1,7 @@
 """Matrix Fourier transforms on the HIP device (lentil fourier.py).
 
 ``dft2`` and ``idft2`` keep lentil's signatures and semantics; the work runs
-in ``mftx_dft2`` (two complex GEMMs with on-the-fly twiddles on MFMA).
+in ``mftx_dft2`` (two complex GEMMs against twiddle tables on MFMA).
 
 Returned types follow the input: a NumPy input gives a complex128 NumPy
 result (the drop-in contract), a device tensor gives a complex64 device

@@ -91,9 +91,8 @@ def test_insert_group_refuses(L, bad):
 
 
 def test_plan_graph_follows_the_destination(L):
-    """The first call of a destination launches, the second captures, later ones replay; changing the
-    destination, the type or adding in between gives the same image every time, and a call on a stream
-    that is being captured becomes part of that graph."""
+    """Repeating and changing the destination, the type or adding in between gives the same image every
+    time, and a call on a stream that is being captured becomes part of that graph."""
     n = 48
     y, x = np.mgrid[:n, :n] / n - 0.5
     pupil = L.Pupil(amplitude=(np.hypot(x, y) < 0.45).astype(float), opd=2e-7 * x * y, pixelscale=1 / n, focal_length=10.0)
