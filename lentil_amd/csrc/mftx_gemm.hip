@@ -58,6 +58,7 @@ template <> struct Num<PREC_FP32> {
 };
 
 typedef __attribute__((address_space(3))) void lds_void;
+typedef float v4f32a8 __attribute__((ext_vector_type(4), aligned(8)));  // two complex64 at any element offset
 
 // Weight-map values at map offsets idx[0..n-1] (1 without a map).  No load
 // sits behind a branch, so they are in flight together.
@@ -75,13 +76,12 @@ __device__ __forceinline__ void load_weights(const Problem& P, const long long (
   }
 }
 
+// Index i of the map's n rows or columns, i < 2 n.
+__device__ __forceinline__ int wrapped(int i, int n) { return i >= n ? i - n : i; }
+
 // Map offset of F's element (u, v).
 __device__ __forceinline__ long long weight_index(const Problem& P, int u, int v) {
-  u += P.wrow;
-  v += P.wcol;
-  if (u >= P.wrows) u -= P.wrows;
-  if (v >= P.wcols) v -= P.wcols;
-  return (long long)u * P.ldw + v;
+  return (long long)wrapped(u + P.wrow, P.wrows) * P.ldw + wrapped(v + P.wcol, P.wcols);
 }
 
 // A lane's (cos, sin) of the store's output phase for its slot: column cp + s
@@ -94,6 +94,35 @@ __device__ __forceinline__ float store_scale(const Problem& P) {
   return P.inv ? P.scale * *(cptr<const float>)P.inv : P.scale;
 }
 
+// Four 16-byte pieces per lane, transposed within each quad of lanes: piece t
+// of lane q becomes piece q of lane t.
+__device__ __forceinline__ void quad_transpose(float (&v)[16]) {
+  const int lane = threadIdx.x;
+  const bool b0 = lane & 1, b1 = lane & 2;
+  auto flip1 = [](float x) {  // the value of lane ^ 1
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xb1, 0xf, 0xf, true));
+  };
+  auto flip2 = [](float x) {  // of lane ^ 2
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4e, 0xf, 0xf, true));
+  };
+#pragma unroll
+  for (int t = 0; t < 4; t += 2)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = v[4 * t + e], y = v[4 * t + 4 + e], fx = flip1(x), fy = flip1(y);
+      v[4 * t + e] = b0 ? fy : x;
+      v[4 * t + 4 + e] = b0 ? y : fx;
+    }
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = v[4 * t + e], y = v[4 * t + 8 + e], fx = flip2(x), fy = flip2(y);
+      v[4 * t + e] = b1 ? fy : x;
+      v[4 * t + 8 + e] = b1 ? y : fx;
+    }
+}
+
 // Store one side (0: column cp + s from P + iQ, 1: cm - s from P - iQ) of half
 // h of a 32 x 32 block: this lane's slot and the 8 rows 16 h + 8 g + 4 (lane /
 // 32) + e, g = 0, 1, e = 0 .. 3 of row block rb; re, im hold them unscaled.
@@ -101,7 +130,12 @@ __device__ __forceinline__ float store_scale(const Problem& P) {
 // Lane l holds rows 0-3 and 8-11 of the 16, lane l + 32 rows 4-7 and 12-15.
 // One lane swap per word (v_permlane32_swap: the high half of the first
 // operand trades places with the low half of the second) gives lane l rows 0-7
-// and lane l + 32 rows 8-15, so a lane stores 16-byte pieces.
+// and lane l + 32 rows 8-15, so a lane stores 16-byte pieces.  The operand's
+// pieces of 32 lanes are contiguous.  Those of a transposed field lie a row
+// stride apart, so quads of lanes trade theirs first: a store instruction then
+// writes 128 contiguous bytes of 8 rows instead of 32 of 32, and its loads of a
+// weight map touch 8 rows instead of 32 (64 adjoint fields of 512^2 91 -> 83 us,
+// a 1024^2 -> 2048^2 transform 64 -> 60.5).
 template <int PREC, int EPI>
 __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int side, int slot, int lane, float sc,
                                            float2 ph, float (&re)[8], float (&im)[8]) {
@@ -162,23 +196,41 @@ __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int 
       o[8 + 2 * q] = __uint_as_float(a[1]);
       o[9 + 2 * q] = __uint_as_float(b[1]);
     }
-    if (!has) return;
-    const int r0 = row0 + 8 * (lane >> 5) - P.i0, nr = P.i1 - P.i0;  // first of this lane's 8 rows, in the window
-    long long wi[8];  // rows outside the window (not stored) read the column's row 0
+    // lane q of a quad: rows 2 q, 2 q + 1 of the 8, of the quad's four columns in turn
+    quad_transpose(o);
+    const int r = row0 + 8 * (lane >> 5) + 2 * (lane & 3) - P.i0, nr = P.i1 - P.i0;  // first of the two, in the window
+    const bool in0 = r >= 0 && r < nr, in1 = r + 1 >= 0 && r + 1 < nr;
+    int jt[4];  // the columns; -1: not stored
 #pragma unroll
-    for (int t = 0; t < 8; ++t) wi[t] = weight_index(P, j - P.j0, r0 + t >= 0 && r0 + t < nr ? r0 + t : 0);
-    float wv[8];
-    load_weights(P, wi, wv);
-    float2* d = dst + (long long)(j - P.j0) * P.ldd + r0;
-    if (r0 >= 0 && r0 + 8 <= nr && (((uintptr_t)d) & 15) == 0) {
+    for (int t = 0; t < 4; ++t) {
+      const int st = (slot & ~3) + t, j = side ? P.cm - st : P.cp + st;
+      jt[t] = j >= P.j0 && j < P.j1 && !(side && j == P.cp + st) ? j - P.j0 : -1;
+    }
+    if (P.wmap) {
+      // rows and columns that are not stored read the map's first ones
+      const int v0 = in0 ? wrapped(r + P.wcol, P.wcols) : 0, v1 = in1 ? wrapped(r + 1 + P.wcol, P.wcols) : 0;
+      long long wi[8];
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        ((gptr<v4f32>)d)[t] = v4f32{o[4 * t] * wv[2 * t], o[4 * t + 1] * wv[2 * t], o[4 * t + 2] * wv[2 * t + 1],
-                                    o[4 * t + 3] * wv[2 * t + 1]};
-    } else {
+      for (int t = 0; t < 4; ++t) {
+        const long long u = jt[t] >= 0 ? (long long)wrapped(jt[t] + P.wrow, P.wrows) * P.ldw : 0;
+        wi[2 * t] = u + v0;
+        wi[2 * t + 1] = u + v1;
+      }
+      float wv[8];
+      load_weights(P, wi, wv);
 #pragma unroll
-      for (int t = 0; t < 8; ++t)
-        if (r0 + t >= 0 && r0 + t < nr) ((gptr<v2f32>)d)[t] = v2f32{o[2 * t] * wv[t], o[2 * t + 1] * wv[t]};
+      for (int q = 0; q < 16; ++q) o[q] *= wv[q >> 1];
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if (jt[t] < 0) continue;
+      float2* d = dst + (long long)jt[t] * P.ldd + r;
+      if (in0 && in1) {
+        *(gptr<v4f32a8>)d = v4f32a8{o[4 * t], o[4 * t + 1], o[4 * t + 2], o[4 * t + 3]};
+      } else {
+        if (in0) ((gptr<v2f32>)d)[0] = v2f32{o[4 * t], o[4 * t + 1]};
+        if (in1) ((gptr<v2f32>)d)[1] = v2f32{o[4 * t + 2], o[4 * t + 3]};
+      }
     }
     return;
   }
