@@ -432,11 +432,11 @@ static std::vector<std::pair<int, int>> group_runs(const std::vector<Problem>& p
   return runs;
 }
 
-// Schedule and works of a list of independent problems (one segment each,
-// nkb[i] K blocks): the tile is chosen for the whole launch by the summed
-// estimate of its shapes; runs of equal problems share work items.
+// Schedule and works of a list of independent problems (of one segment each
+// unless multi, nkb[i] K blocks): the tile is chosen for the whole launch by
+// the summed estimate of its shapes; runs of equal problems share work items.
 static int list_works(std::vector<Work>& works, const std::vector<Problem>& ps, const std::vector<int>& nkb, int fixed,
-                      int64_t most) {
+                      int64_t most, bool multi = false) {
   struct Shape { int rb, sb, nkb; };
   std::map<std::tuple<int, int, int>, int64_t> shapes;
   for (size_t i = 0; i < ps.size(); ++i) ++shapes[{ps[i].rblocks, (int)blocks32(ps[i].cols), nkb[i]}];
@@ -452,7 +452,7 @@ static int list_works(std::vector<Work>& works, const std::vector<Problem>& ps, 
     }
     total += kv.second;
   }
-  const Schedule sch = pick_schedule(fixed, false, std::get<0>(top), std::get<1>(top), std::get<2>(top), total, most);
+  const Schedule sch = pick_schedule(fixed, multi, std::get<0>(top), std::get<1>(top), std::get<2>(top), total, most);
   for (const auto& r : group_runs(ps, nkb, sch.run)) {
     int nch = 0;
     for (int i = r.first; i < r.second; ++i) nch += nkb[i];
@@ -2087,36 +2087,33 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     }
   }
   {
-    // complex stores: one problem per work item
-    auto cplx_tile = [&](const std::vector<int>& cl) {
-      int rb = 0, sb = 0, nk = 0;
+    // Complex stores: neighbouring classes of one shape share a work item, so
+    // its load pipeline runs on under the stores (64 weighted fields of 512^2,
+    // two rounds of workgroups with one class each: 111 us, now 90).
+    auto cplx_works = [&](const std::vector<int>& cl, std::vector<Work>& works) {
+      if (cl.empty()) return 0;
+      std::vector<Problem> ps;
+      std::vector<int> nkb;
       for (int c : cl) {
-        rb = std::max(rb, p2[cls[c].p2].rblocks);
-        sb = std::max(sb, p2[cls[c].p2].sblocks);
-        nk = std::max(nk, class_nkb(c));
+        ps.push_back(p2[cls[c].p2]);
+        nkb.push_back(class_nkb(c));
       }
-      const int fixed = multi && (fixed_tile == TILE_BIG || fixed_tile == TILE_MID) ? TILE_MULTI : fixed_tile;
-      return pick_schedule(fixed, multi, rb, sb, nk, cl.size(), 1).tile;
+      return list_works(works, ps, nkb, multi && fixed_tile >= 0 ? TILE_MULTI : fixed_tile, 8, multi);
     };
     std::vector<int> slow, every;
     for (size_t c = 0; c < cls.size(); ++c) {
       every.push_back((int)c);
       if (path[c] == PATH_FIELDS) slow.push_back((int)c);
     }
-    if (!slow.empty()) plan->tile2c = cplx_tile(slow);
-    if (!every.empty()) plan->tile_f = cplx_tile(every);
-    for (int c : slow) {
-      const int pb = (int)p2c_launch.size();
-      push2(p2c_launch, patch2c_launch, c);
-      add_tiles(w2c, plan->tile2c, pb, pb + 1, class_nkb(c), cls[c].rblocks2, p2[cls[c].p2].sblocks);
-    }
+    for (int c : slow) push2(p2c_launch, patch2c_launch, c);
     // the complex-field set: each class's stage-2 problem
     std::vector<Patch> patch_f;
     for (int c : every) {
       push2(plan->pf, patch_f, c);
       plan->class_first.push_back(cls[c].members[0]);
-      add_tiles(wf, plan->tile_f, c, c + 1, class_nkb(c), cls[c].rblocks2, p2[cls[c].p2].sblocks);
     }
+    plan->tile2c = cplx_works(slow, w2c);
+    plan->tile_f = cplx_works(every, wf);
   }
   // executed MFMA FLOPs of the two launches: 12 instructions of 32 x 32 x 16
   // per 32 x 32 block and K block
