@@ -94,6 +94,22 @@ __device__ __forceinline__ float store_scale(const Problem& P) {
   return P.inv ? P.scale * *(cptr<const float>)P.inv : P.scale;
 }
 
+// Sum of intensities plus weight * |scale * (re, im)|^2, given w =
+// intensity_weight(weight, scale).  The f16 form's scale undoes the operand's
+// scaling: for an amplitude near 1e-16 it is about 2^-66, and its square would
+// leave FP32's range although the intensity does not.  So one factor of it
+// meets the large sums before the other meets the weight; a power of two, it
+// rounds nothing.  (The bf16 form's scale is 1.)
+template <int PREC>
+__device__ __forceinline__ float intensity_weight(float weight, float scale) {
+  return PREC == PREC_FP32 ? weight * scale : weight * scale * scale;
+}
+template <int PREC>
+__device__ __forceinline__ float add_intensity(float sum, float w, float scale, float re, float im) {
+  const float i2 = __builtin_fmaf(re, re, im * im);
+  return __builtin_fmaf(w, PREC == PREC_FP32 ? i2 * scale : i2, sum);
+}
+
 // Four 16-byte pieces per lane, transposed within each quad of lanes: piece t
 // of lane q becomes piece q of lane t.
 __device__ __forceinline__ void quad_transpose(float (&v)[16]) {
@@ -549,14 +565,14 @@ __global__ __launch_bounds__((Cfg<WR, WC, S>::NT), (Cfg<WR, WC, S>::WG_PER_CU)) 
       for (int s = 0; s < S; ++s) {
         const int slot = (wk.tc * C::SB + wc * S + s) * 32 + (lane & 31);
         if (EPI == EPI_INTENSITY) {
-          const float w = P.weight * scale * scale;
+          const float w = intensity_weight<PREC>(P.weight, scale);
 #pragma unroll
           for (int e = 0; e < 16; ++e) {
             const float pr = acc[s][0][e], pi = acc[s][1][e], qr = acc[s][2][e], qi = acc[s][3][e];
             const float ar = pr - qi, ai = pi + qr;   // P + iQ
             const float br = pr + qi, bi = pi - qr;   // P - iQ
-            ip[s][e] = __builtin_fmaf(w, __builtin_fmaf(ar, ar, ai * ai), ip[s][e]);
-            im[s][e] = __builtin_fmaf(w, __builtin_fmaf(br, br, bi * bi), im[s][e]);
+            ip[s][e] = add_intensity<PREC>(ip[s][e], w, scale, ar, ai);
+            im[s][e] = add_intensity<PREC>(im[s][e], w, scale, br, bi);
           }
         } else {
           const float2 ph = slot_phase(P, slot);
@@ -688,9 +704,9 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const Work* __restri
     }
     const float scale = store_scale(P);
     if (EPI == EPI_INTENSITY) {
-      const float w = P.weight * scale * scale;
+      const float w = intensity_weight<PREC>(P.weight, scale);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) isum[q] = __builtin_fmaf(w, __builtin_fmaf(re[q], re[q], imv[q] * imv[q]), isum[q]);
+      for (int q = 0; q < 8; ++q) isum[q] = add_intensity<PREC>(isum[q], w, scale, re[q], imv[q]);
     } else {
       store_half<PREC, EPI>(P, wk.tr, h, side, slot, lane, scale, slot_phase(P, slot), re, imv);
     }

@@ -1,0 +1,40 @@
+"""Values far from 1, and far from each other: the FP32 form's operands are f16
+pairs scaled by powers of two, and its results keep FP32's range.  Against the
+complex128 oracle at the gates of the forms (fields 2e-6, images 1e-5)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import optics
+from tests.conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def L():
+    import lentil_amd
+    assert torch.cuda.is_available()
+    return lentil_amd
+
+
+# an image of (1e-18)^2 times unit weights is still a normal float32 in the
+# core; 1e9 squared is far from float32's end
+@pytest.mark.parametrize('nseg, tile_n', [(1, 0), (1, 64), (1, 128), (3, 0), (3, 64)])
+@pytest.mark.parametrize('level', [1e-18, 1e-16, 1e-13, 1.0, 1e9])
+def test_plan_images_of_any_amplitude(L, nseg, tile_n, level):
+    """Every tile's intensity epilogue (one segment, several along K)."""
+    n, os, du, z = 72, 2, 5e-6, 10.0
+    masks = np.zeros((nseg, n, n))
+    for k in range(nseg):
+        masks[k, 3 + 24 * k:21 + 24 * k, 5:60] = 1
+    yy, xx = np.mgrid[:n, :n] / n - 0.5
+    amp, opd = masks.sum(axis=0) * (1 + xx * yy), 3e-7 * (yy ** 2 - yy * xx)
+    wl, wt = np.array([5.2e-7, 6e-7, 7e-7]), np.array([0.5, 0.2, 0.3])
+    mask = masks if nseg > 1 else None
+    plan = L.PSFPlan(L.Pupil(amplitude=amp * level, opd=opd, mask=mask, pixelscale=1 / n, focal_length=z), wl, wt,
+                     pixelscale=du, shape=(60, 45), oversample=os, precision='fp32', tile_n=tile_n,
+                     contraction='per_tile')
+    ref = optics.broadband_image(optics.Pupil(amp, opd, 1 / n, z, mask=mask), wl, wt, du, (60, 45), os)
+    img = plan(out=torch.empty(plan.shape_out, dtype=torch.float64, device='cuda'))
+    assert rel_l2(img.cpu().numpy() / level / level, ref) < 1e-5
