@@ -460,18 +460,25 @@ __global__ void resample_kernel(const double* __restrict__ C, long long P0, long
       // the columns' taps and weights once, every load of a row before its sum
       long long cc[6];
       double wx[6];
+      unsigned past = 0;  // taps outside the line (EX_ZERO): they read column 0, which may not be finite
 #pragma unroll
       for (int b = 0; b < 6; ++b) {
         cc[b] = b <= order ? extend_index(sx + b, P1, rule) : -1;
         wx[b] = cc[b] >= 0 ? bspline(order, cx - (double)(sx + b)) : 0.0;
+        if (cc[b] < 0) past |= 1u << b;
         cc[b] = max(cc[b], 0LL);
       }
+      past &= (2u << order) - 1;
       for (int a = 0; a <= order; ++a) {
         const long long rr = extend_index(sy + a, P0, rule);
         if (rr < 0) continue;
         double e[6], row = 0.0;
 #pragma unroll
         for (int b = 0; b < 6; ++b) e[b] = C[rr * P1 + cc[b]];
+        if (past) {
+#pragma unroll
+          for (int b = 0; b < 6; ++b) e[b] = past >> b & 1 ? 0.0 : e[b];
+        }
 #pragma unroll
         for (int b = 0; b < 6; ++b)
           if (b <= order) row += wx[b] * e[b];
