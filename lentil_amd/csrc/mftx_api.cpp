@@ -1814,19 +1814,19 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     }
     if (path[&c - cls.data()] == PATH_FIELDS) c.fbuf = lay.take(sizeof(float2) * (size_t)c.key.M * c.key.N);
   }
-  // f16 form: one scale for all tiles that meet in a coherent group (connected
-  // through classes), from the maxima of their amplitudes, which lie together
+  // f16 form: one scale for all tiles that meet in a class (their products are
+  // summed unscaled along K), from the maxima of their amplitudes, which lie
+  // together.  Classes of one group undo their own scales before they are added:
+  // with one scale for the group a segment 1e-7 as bright as its neighbour kept
+  // 13 of its 22 bits, and its Field was 8e-5 off.
   std::vector<int> comp(ntiles);
   for (int t = 0; t < ntiles; ++t) comp[t] = t;
   auto root = [&](int t) {
     while (comp[t] != t) t = comp[t] = comp[comp[t]];
     return t;
   };
-  for (auto& kv : groups) {
-    const int t0 = problems[cls[kv.second[0]].members[0]].tile;
-    for (int c : kv.second)
-      for (int i : cls[c].members) comp[root(problems[i].tile)] = root(t0);
-  }
+  for (auto& c : cls)
+    for (int i : c.members) comp[root(problems[i].tile)] = root(problems[c.members[0]].tile);
   struct Comp { size_t part = 0, inv = 0; int n = 0; };  // workspace offsets of the maxima and the inverse scale
   std::map<int, Comp> comps;
   std::vector<MaxOp> maxes;
@@ -1834,9 +1834,11 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   long long max_total = 0;
   if (prec == PREC_FP32) {
     for (int t = 0; t < ntiles; ++t) comps[root(t)].n += max_blocks(tiles[t].m, tiles[t].n);
+    size_t inv = lay.take(sizeof(float) * comps.size());  // side by side: the stores of a group read them all
     for (auto& kv : comps) {
-      kv.second.part = lay.take(sizeof(float) * (kv.second.n + 1));
-      kv.second.inv = kv.second.part + sizeof(float) * kv.second.n;
+      kv.second.part = lay.take(sizeof(float) * kv.second.n);
+      kv.second.inv = inv;
+      inv += sizeof(float);
       size_t at = kv.second.part;
       for (int t = 0; t < ntiles; ++t) {
         if (root(t) != kv.first) continue;

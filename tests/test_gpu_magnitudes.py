@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from oracle import optics
+from oracle import mft, optics
 from tests.conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -38,3 +38,40 @@ def test_plan_images_of_any_amplitude(L, nseg, tile_n, level):
     ref = optics.broadband_image(optics.Pupil(amp, opd, 1 / n, z, mask=mask), wl, wt, du, (60, 45), os)
     img = plan(out=torch.empty(plan.shape_out, dtype=torch.float64, device='cuda'))
     assert rel_l2(img.cpu().numpy() / level / level, ref) < 1e-5
+
+
+@pytest.mark.parametrize('tilt', [1.0, 9.0])
+def test_fields_of_unequal_segments(L, tilt):
+    """Segments of one coherent group on grids of their own (windows of one
+    grid, and Fields far apart): a dim one keeps its own 22 bits.  Two segments
+    share a grid and a class."""
+    n, os, du, z = 64, 2, 5e-6, 10.0
+    level = np.array([1.0, 1e-7, 1e-12, 1e3, 0.5])
+    masks = np.zeros((5, n, n))
+    for k in range(5):
+        masks[k, 1 + 20 * (k // 2):20 + 20 * (k // 2), 2 + 31 * (k % 2):30 + 31 * (k % 2)] = 1
+    yy, xx = np.mgrid[:n, :n] / n - 0.5
+    amp, opd = (masks * level[:, None, None]).sum(axis=0), 3e-7 * (yy ** 2 - yy * xx)
+    wl = np.array([5e-7, 6.5e-7])
+    px = np.random.default_rng(1).uniform(-tilt, tilt, (5, 2))
+    px[4] = px[0]
+    pupil = L.Pupil(amplitude=amp, opd=opd, mask=masks, pixelscale=1 / n, focal_length=z)
+    pupil.tilt.extend(L.Tilt(*a) for a in px * du / os / z)
+    plan = L.PSFPlan(pupil, wl, None, pixelscale=du, shape=(30, 47), prop_shape=(20, 20), oversample=os,
+                     precision='fp32', contraction='per_tile')
+    assert plan.info['coherent_fast'] == 0 and plan.info['n_stage2'] == 8
+    F = [torch.zeros((p['M'], p['N']), dtype=torch.complex64, device='cuda') for p in plan.problems]
+    plan()
+    plan.set_fields(F, [1.0] * len(F))
+    plan.fields()
+    tiles = list(pupil.phasor_tiles())
+    field = {}
+    for p in plan.problems:
+        _, _, a, o = tiles[p['tile']]
+        field[p['tile'], p['wave']] = mft.dft2(a * np.exp(2j * np.pi * o / wl[p['wave']]), p['alpha'],
+                                               (p['M'], p['N']), p['shift'], p['offset'], unitary=False)
+    for p, f in zip(plan.problems, F):
+        if p['tile'] == 4:
+            continue    # written with its class's first segment
+        ref = field[p['tile'], p['wave']] + (field[4, p['wave']] if p['tile'] == 0 else 0)
+        assert rel_l2(f.cpu().numpy(), ref) < 2e-6, p['tile']
