@@ -64,9 +64,13 @@ __device__ __forceinline__ float block_max(float v) {
   return v;
 }
 
+constexpr float kMaxFloat = 3.4028234663852886e38f;
+
 // Bound over elements [first, m * n) in steps of `step` of an m x n array:
 // |re| + |im|, 0 for an element that is not finite (it makes its results
-// non-finite whatever the scale).  The dtype is tested outside the loop, so
+// non-finite whatever the scale), FP32's largest number where the sum of two
+// finite parts is past it (at most twice that: scaled operands then reach 2^15
+// instead of 2^14, still half of f16's range).  The dtype is tested outside the loop, so
 // the loads of 8 elements are in flight together.
 template <typename Get>
 __device__ __forceinline__ float bound_of(long long m, long long n, long long ld, long long first, long long step,
@@ -76,8 +80,8 @@ __device__ __forceinline__ float bound_of(long long m, long long n, long long ld
   auto one = [&](long long i) {
     const float2 e = get(ld == n ? i : total < (1LL << 31) ? (long long)((unsigned)i / (unsigned)n) * ld + (unsigned)i % (unsigned)n
                                                            : i / n * ld + i % n);
-    const float b = fabsf(e.x) + fabsf(e.y);
-    return b <= 3.4028234e38f ? b : 0.f;
+    const float ax = fabsf(e.x), ay = fabsf(e.y);
+    return ax <= kMaxFloat && ay <= kMaxFloat ? fminf(ax + ay, kMaxFloat) : 0.f;
   };
   long long i = first;
   for (; i + 7 * step < total; i += 8 * step) {

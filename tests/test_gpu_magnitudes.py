@@ -75,3 +75,14 @@ def test_fields_of_unequal_segments(L, tilt):
             continue    # written with its class's first segment
         ref = field[p['tile'], p['wave']] + (field[4, p['wave']] if p['tile'] == 0 else 0)
         assert rel_l2(f.cpu().numpy(), ref) < 2e-6, p['tile']
+
+
+@pytest.mark.parametrize('n', [16, 120])
+@pytest.mark.parametrize('sample', [2e38 + 2e38j, 3.4028234e38 - 3.4028234e38j, 3.4e38j])
+def test_samples_at_the_ends_of_float32(L, n, sample):
+    """One sample whose parts are finite and whose |re| + |im| may not be."""
+    f = torch.zeros((n, n), dtype=torch.complex64, device='cuda')
+    f[n // 2, n // 2] = sample
+    got = L.fourier.dft2(f, 1 / (2 * n), (20, 30)).cpu().numpy().astype(complex)
+    ref = mft.dft2(f.cpu().numpy().astype(complex), 1 / (2 * n), (20, 30))
+    assert rel_l2(got / abs(sample), ref / abs(sample)) < 2e-6
