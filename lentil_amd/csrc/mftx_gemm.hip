@@ -89,10 +89,9 @@ __device__ __forceinline__ long long weight_index(const Problem& P, int u, int v
 __device__ __forceinline__ float2 slot_phase(const Problem& P, int slot) {
   return P.xrot != 0.0 ? cis_turns(P.xrot * (P.y0 + (double)slot)) : make_float2(1.0f, 0.0f);
 }
+// What undoes the operand's scaling, 1 without one.
 // (a scalar load: a vector load's wait would drain the operand loads in flight)
-__device__ __forceinline__ float store_scale(const Problem& P) {
-  return P.inv ? P.scale * *(cptr<const float>)P.inv : P.scale;
-}
+__device__ __forceinline__ float unscale(const Problem& P) { return P.inv ? *(cptr<const float>)P.inv : 1.0f; }
 
 // Sum of intensities plus weight * |scale * (re, im)|^2, given w =
 // intensity_weight(weight, scale).  The f16 form's scale undoes the operand's
@@ -154,7 +153,7 @@ __device__ __forceinline__ void quad_transpose(float (&v)[16]) {
 // a 1024^2 -> 2048^2 transform 64 -> 60.5).
 template <int PREC, int EPI>
 __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int side, int slot, int lane, float sc,
-                                           float2 ph, float (&re)[8], float (&im)[8]) {
+                                           float inv, float2 ph, float (&re)[8], float (&im)[8]) {
   const int j = side ? P.cm - slot : P.cp + slot;
   const bool has = j >= (EPI == EPI_STORE_CPLX ? P.j0 : 0) && j < (EPI == EPI_STORE_CPLX ? P.j1 : P.ncols) &&
                    !(side && j == P.cp + slot);
@@ -182,6 +181,9 @@ __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int 
         im[q] = v.y;
       }
     }
+    // one after the other: their product may be below the smallest denormal
+    // where the results are not (sources near 1e-38)
+    auto out = [&](float x) { return PREC == PREC_FP32 ? x * sc * inv : x * sc; };
     float2* dst = (float2*)P.dst;
     if (!P.trans) {
       long long wi[8];
@@ -196,16 +198,16 @@ __device__ __forceinline__ void store_half(const Problem& P, int rb, int h, int 
       for (int q = 0; q < 8; ++q) {
         const int row = row0 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
         if (has && row >= P.i0 && row < P.i1)
-          ((gptr<v2f32>)dst)[(long long)(row - P.i0) * P.ldd + (j - P.j0)] = v2f32{re[q] * sc * wv[q], im[q] * sc * wv[q]};
+          ((gptr<v2f32>)dst)[(long long)(row - P.i0) * P.ldd + (j - P.j0)] = v2f32{out(re[q]) * wv[q], out(im[q]) * wv[q]};
       }
       return;
     }
     float o[16];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(re[q] * sc), __float_as_uint(re[4 + q] * sc),
+      const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(out(re[q])), __float_as_uint(out(re[4 + q])),
                                                       false, false);
-      const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(im[q] * sc), __float_as_uint(im[4 + q] * sc),
+      const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(out(im[q])), __float_as_uint(out(im[4 + q])),
                                                       false, false);
       o[2 * q] = __uint_as_float(a[0]);
       o[2 * q + 1] = __uint_as_float(b[0]);
@@ -560,7 +562,7 @@ __global__ __launch_bounds__((Cfg<WR, WC, S>::NT), (Cfg<WR, WC, S>::WG_PER_CU)) 
       continue;
     }
     if (mf) {
-      const float scale = store_scale(P);
+      const float inv = unscale(P), sc0 = P.scale, scale = sc0 * inv;
 #pragma unroll
       for (int s = 0; s < S; ++s) {
         const int slot = (wk.tc * C::SB + wc * S + s) * 32 + (lane & 31);
@@ -588,7 +590,7 @@ __global__ __launch_bounds__((Cfg<WR, WC, S>::NT), (Cfg<WR, WC, S>::WG_PER_CU)) 
                 re[q] = side ? pr + qi : pr - qi;
                 imv[q] = side ? pi - qr : pi + qr;
               }
-              store_half<PREC, EPI>(P, rb, h, side, slot, lane, scale, ph, re, imv);
+              store_half<PREC, EPI>(P, rb, h, side, slot, lane, sc0, inv, ph, re, imv);
             }
         }
 #pragma unroll
@@ -702,13 +704,13 @@ __global__ __launch_bounds__(256, 2) void gemm_small_kernel(const Work* __restri
       re[q] = side ? t[0][q] + t[3][q] : t[0][q] - t[3][q];
       imv[q] = side ? t[1][q] - t[2][q] : t[1][q] + t[2][q];
     }
-    const float scale = store_scale(P);
+    const float inv = unscale(P), sc0 = P.scale, scale = sc0 * inv;
     if (EPI == EPI_INTENSITY) {
       const float w = intensity_weight<PREC>(P.weight, scale);
 #pragma unroll
       for (int q = 0; q < 8; ++q) isum[q] = add_intensity<PREC>(isum[q], w, scale, re[q], imv[q]);
     } else {
-      store_half<PREC, EPI>(P, wk.tr, h, side, slot, lane, scale, slot_phase(P, slot), re, imv);
+      store_half<PREC, EPI>(P, wk.tr, h, side, slot, lane, sc0, inv, slot_phase(P, slot), re, imv);
     }
   }
   if (EPI == EPI_INTENSITY) store_partial<2>(wk, probs[wk.pbeg], wk.tr * 32 + 16 * h, side, slot, lane, isum);
@@ -796,7 +798,7 @@ __global__ __launch_bounds__(256, 2) void gemm_coherent_kernel(const Work* __res
     }
   };
   auto finish = [&](const Problem& P) {
-    const float scale = P.inv ? P.scale * *(cptr<const float>)P.inv : P.scale;
+    const float scale = P.scale * unscale(P);
     const int slot = wk.tc * 32 + (lane & 31);
     float2 ph = slot_phase(P, slot);
     ph.x *= scale;

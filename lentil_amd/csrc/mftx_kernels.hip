@@ -122,21 +122,23 @@ hipError_t launch_absmax(const MaxOp* ops, int nops, long long total_blocks, hip
   return hipGetLastError();
 }
 
-// Power of two that takes 4 * bound to at most 2^14 (1 for bound 0).
-__device__ __forceinline__ float operand_scale(float bound) {
-  if (!(bound > 0.f)) return 1.0f;
-  const int e = 12 - __builtin_amdgcn_frexp_expf(bound);  // bound < 2^frexp_exp
-  return __uint_as_float((uint32_t)(127 + min(max(e, -126), 126)) << 23);
+// Exponent of the power of two that takes 4 * bound to at most 2^14 (0 for
+// bound 0): -116 to 149, whose inverse is the smallest denormal.  Up to 2^-137
+// it is the one wanted; the denormals below have few bits to lose.
+__device__ __forceinline__ int operand_exponent(float bound) {
+  return bound > 0.f ? min(12 - __builtin_amdgcn_frexp_expf(bound), 149) : 0;  // bound < 2^frexp_exp
 }
+// x * 2^e, exact (past 2^127 no float holds the factor)
+__device__ __forceinline__ float scaled(float x, int e) { return __builtin_amdgcn_ldexpf(x, e); }
 
-// The scale of an operand source (every thread of the block calls it).
-__device__ __forceinline__ float block_scale(const ScaleSrc& sc, bool first) {
-  if (sc.n == 0) return 1.0f;
+// The scale (its exponent) of an operand source (every thread of the block calls it).
+__device__ __forceinline__ int block_scale(const ScaleSrc& sc, bool first) {
+  if (sc.n == 0) return 0;
   float v = 0.f;
   for (int i = threadIdx.x; i < sc.n; i += kGroupBlock) v = fmaxf(v, sc.part[i]);
-  const float s = operand_scale(block_max(v));
-  if (first && threadIdx.x == 0) *sc.inv = 1.0f / s;
-  return s;
+  const int e = operand_exponent(block_max(v));
+  if (first && threadIdx.x == 0) *sc.inv = scaled(1.0f, -e);
+  return e;
 }
 
 // --------------------------------------------------------------------------
@@ -180,7 +182,8 @@ __device__ __forceinline__ PhasorWave load_wave(cptr<const PhasorWave> p) {
 // phases are skipped.
 // DT: the dtype of a complex source.
 template <int PREC, bool CPLX, int NP, int DT, typename Waves>
-__device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave, int waves, long long u, float scale) {
+__device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave, int waves, long long u, int scale) {
+  auto fit = [&](float x) { return PREC == PREC_FP32 ? scaled(x, scale) : x; };
   static_assert(NP == 2 || NP == 4 || NP == 8, "a thread's pairs lie in one half of a K block");
   constexpr int SUB = 8 / NP;  // threads per (row pair, half K block)
   const int R = op.trans ? op.n : op.m, K = op.trans ? op.m : op.n;
@@ -226,8 +229,8 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
           const float2 e = load_elem(op.amp, DT, ia[i]);
-          a[rs][ks][i] = in[i] ? e.x * scale : 0.f;
-          ci[rs][ks][i] = in[i] ? e.y * (op.conj ? -scale : scale) : 0.f;
+          a[rs][ks][i] = in[i] ? fit(e.x) : 0.f;
+          ci[rs][ks][i] = in[i] ? fit(op.conj ? -e.y : e.y) : 0.f;
         }
       } else {
         if (op.amp_dtype == 3) {
@@ -252,7 +255,7 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
         }
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
-          a[rs][ks][i] = in[i] ? a[rs][ks][i] * scale : 0.f;
+          a[rs][ks][i] = in[i] ? fit(a[rs][ks][i]) : 0.f;
           o[rs][ks][i] = in[i] ? o[rs][ks][i] : 0.0;
         }
       }
@@ -344,7 +347,7 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
 // operand_thread for the op's source dtype (tested once per thread: a test per
 // load would wait for each)
 template <int PREC, bool CPLX, int NP, typename Waves>
-__device__ __forceinline__ void operand_source(const PhasorOp& op, Waves&& wave, int waves, long long u, float scale) {
+__device__ __forceinline__ void operand_source(const PhasorOp& op, Waves&& wave, int waves, long long u, int scale) {
   if constexpr (!CPLX) {
     operand_thread<PREC, false, NP, 0>(op, wave, waves, u, scale);
   } else {
@@ -364,7 +367,7 @@ __global__ __launch_bounds__(kGroupBlock, 4) void operand_group_kernel(const Pha
                                                                        int waves) {
   const long long b0 = (long long)blockIdx.x * kGroupBlock;
   const PhasorOp& op = ops[block_op(ops, nops, b0)];
-  const float scale = block_scale(op.sc, b0 == op.begin);
+  const int scale = block_scale(op.sc, b0 == op.begin);
   const long long u = b0 + threadIdx.x - op.begin;
   if (u >= operand_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, op.nwave, OperandSplit{NP, waves})) return;
   operand_source<PREC, CPLX, NP>(op, [&](int w) { return load_wave((cptr<const PhasorWave>)op.waves + w); }, waves, u,
@@ -498,12 +501,12 @@ __global__ __launch_bounds__(kGroupBlock, 4) void prepare_one_kernel(PhasorOp op
                                                                      int op_blocks, int tab_blocks) {
   const int b = (int)blockIdx.x;
   if (b < op_blocks) {
-    float scale = 1.0f;
+    int scale = 0;
     if (PREC == PREC_FP32) {
       if (op.sc.n == 0) {  // a small source: every block takes its maximum
-        scale = operand_scale(block_max(array_bound(op.amp, op.amp_dtype, op.m, op.n, op.ld_amp, threadIdx.x,
-                                                    kGroupBlock)));
-        if (b == 0 && threadIdx.x == 0) *op.sc.inv = 1.0f / scale;
+        scale = operand_exponent(block_max(array_bound(op.amp, op.amp_dtype, op.m, op.n, op.ld_amp, threadIdx.x,
+                                                       kGroupBlock)));
+        if (b == 0 && threadIdx.x == 0) *op.sc.inv = scaled(1.0f, -scale);
       } else {
         scale = block_scale(op.sc, b == 0);
       }

@@ -86,3 +86,19 @@ def test_samples_at_the_ends_of_float32(L, n, sample):
     got = L.fourier.dft2(f, 1 / (2 * n), (20, 30)).cpu().numpy().astype(complex)
     ref = mft.dft2(f.cpu().numpy().astype(complex), 1 / (2 * n), (20, 30))
     assert rel_l2(got / abs(sample), ref / abs(sample)) < 2e-6
+
+
+@pytest.mark.parametrize('n', [40, 130])
+@pytest.mark.parametrize('level', [1e-36, 1e-38, 1e-40, 3e-43])
+def test_sources_at_the_lower_end_of_float32(L, n, level):
+    """Sources near FP32's smallest normal number and among the denormals, as
+    one transform and in a list; results are rounded to steps of 1.4e-45."""
+    rng = np.random.default_rng(n)
+    f = ((1 + rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))) * level).astype(np.complex64)
+    t = torch.from_numpy(f).cuda()
+    jobs = [(t, (1 / (2 * n),) * 2, (31, 44), (0.3, 1.7), (0, 0))] * 2
+    for got, unitary in [(L.fourier.dft2(t, 1 / (2 * n), (31, 44), (0.3, 1.7), unitary=False), False)] + [
+            (g, True) for g in L.fourier.dft2_list(jobs, precision='fp32')]:
+        ref = mft.dft2(f.astype(complex), 1 / (2 * n), (31, 44), (0.3, 1.7), unitary=unitary)
+        err = np.linalg.norm((got.cpu().numpy().astype(complex) - ref) / level)
+        assert err < 2e-6 * np.linalg.norm(ref / level) + 1.5e-45 / level * ref.size ** 0.5
