@@ -157,6 +157,8 @@ def check(rc, ctx=None, what=''):
 
 
 _devices = {}     # torch.device by index, filled once a HIP device has been seen
+# a forked child asks again: torch refuses a HIP runtime that its parent has initialised
+os.register_at_fork(after_in_child=_devices.clear)
 
 
 def device_index():
@@ -186,7 +188,9 @@ def device():
 def context(dev=None):
     """Per-device mftx context bound to torch's current stream."""
     lib = _lib or load()
-    idx = device_index() if dev is None or dev.index is None else dev.index
+    idx = device_index()
+    if dev is not None and dev.index is not None:
+        idx = dev.index
     ctx = _ctx.get(idx)
     if ctx is None:
         with _lock:  # one context per device, also when threads race here
