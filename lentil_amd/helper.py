@@ -32,4 +32,9 @@ def slice_offset(slc, shape):
             return (0, 0)
         raise ValueError(f"Can't compute offset from slice {slc}")
     r, c = slc[0], slc[1]
-    return (r.start + (r.stop - r.start) // 2 - shape[0] // 2, c.start + (c.stop - c.start) // 2 - shape[1] // 2)
+    if isinstance(shape, tuple) and len(shape) == 2 \
+            and all(isinstance(v, (int, np.int64)) for v in (r.start, r.stop, c.start, c.stop)):
+        return (r.start + (r.stop - r.start) // 2 - shape[0] // 2, c.start + (c.stop - c.start) // 2 - shape[1] // 2)
+    # other shapes and indices as numpy broadcasts and promotes them
+    size = np.array((r.stop - r.start, c.stop - c.start))
+    return tuple(np.array((r.start + size[0] // 2, c.start + size[1] // 2)) - np.asarray(shape) // 2)
