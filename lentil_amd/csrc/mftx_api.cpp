@@ -187,7 +187,7 @@ class Tables {
  public:
   // index of the table for `samples` input samples and `slots` output slots
   int get(double alpha, double y0, int64_t samples, int64_t slots) {
-    const std::tuple<double, double, int> key{alpha, y0, (int)(samples & 1)};
+    const Key key{bits(alpha), bits(y0), (int)(samples & 1)};
     auto it = index_.find(key);
     if (it == index_.end()) {
       it = index_.emplace(key, (int)ops.size()).first;
@@ -220,7 +220,15 @@ class Tables {
   long long threads = 0;
 
  private:
-  std::map<std::tuple<double, double, int>, int> index_;
+  // the rates' bits: a NaN rate compares equal to every other one, and a
+  // transform of a list would then use its neighbour's table
+  using Key = std::tuple<uint64_t, uint64_t, int>;
+  static uint64_t bits(double v) {
+    uint64_t u;
+    std::memcpy(&u, &v, sizeof u);
+    return u;
+  }
+  std::map<Key, int> index_;
 };
 
 }  // namespace
