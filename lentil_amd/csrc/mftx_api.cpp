@@ -910,7 +910,7 @@ int mftx_dft2(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, i
               int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r, double shift_c,
               double offset_r, double offset_c, double scale, int conj, int precision) {
   return mftx::dft2_on_workspace(ctx, f, f_dtype, m, n, ldf, F, M, N, ldF, alpha_r, alpha_c, shift_r, shift_c,
-                                 offset_r, offset_c, scale, conj, precision, nullptr, 0, 0);
+                                 offset_r, offset_c, scale, conj, precision, nullptr, 0, 0, 0);
 }
 
 }  // extern "C"
@@ -936,8 +936,8 @@ struct OneSpec {
 };
 }  // namespace
 
-// One transform on the caller's workspace `ws`, or on the context's growable
-// workspace when ws is null.  Three launches and nothing uploaded: the source's
+// One transform on the caller's workspace `ws` of ws_bytes, or on the context's
+// growable workspace when ws is null.  Three launches and nothing uploaded: the source's
 // maximum (f16 form, larger sources only), then operand, twiddle tables and
 // descriptors (launch_prepare_one), then the two GEMMs.  A table larger than
 // `table_cap` bytes is made and used in pieces of whole tile columns.
@@ -950,7 +950,7 @@ struct OneSpec {
 // then stage 1's output for every K the second stage reads), so the workspace
 // needs no clearing; padding rows beyond the output only feed output rows that
 // are never stored.
-static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t cap, size_t table_cap) {
+static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t ws_bytes, size_t cap, size_t table_cap) {
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const int prec = q.precision;
   const int64_t m = q.m, n = q.n;
@@ -989,6 +989,10 @@ static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t cap, size_t
     rc = ensure_ws(ctx, need);
     if (rc) return rc;
     ws = ctx->ws;
+  } else if (need > ws_bytes) {
+    // a transform within the cap takes two thirds of the array at most; this keeps the kernels inside it whatever changes
+    return fail(ctx, MFTX_EINVAL, "transform needs " + std::to_string(need) + " bytes of workspace, more than the " +
+                                      std::to_string(ws_bytes) + " available");
   }
   if (too_large(g, false)) return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
   char* base = (char*)ws;
@@ -1059,7 +1063,7 @@ static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t cap, size_t
 int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, int64_t ldf, void* F,
                             int64_t M, int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r,
                             double shift_c, double offset_r, double offset_c, double scale, int conj, int precision,
-                            void* ws, size_t cap, size_t table_cap) {
+                            void* ws, size_t ws_bytes, size_t cap, size_t table_cap) {
   if (!ctx) return MFTX_EHANDLE;
   if (!f || !F) return fail(ctx, MFTX_EINVAL, "null array pointer");
   if (m <= 0 || n <= 0 || M <= 0 || N <= 0) return fail(ctx, MFTX_EINVAL, "shapes must be positive");
@@ -1070,7 +1074,7 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
     return fail(ctx, MFTX_EINVAL, "dimension too large");
   OneSpec q{f, f_dtype, m, n, ldf, F, M, N, ldF, alpha_r, alpha_c, shift_r, shift_c, offset_r, offset_c, scale, conj,
             precision};
-  return run_one(ctx, q, ws, cap, table_cap);
+  return run_one(ctx, q, ws, ws_bytes, cap, table_cap);
 }
 
 extern "C" {
@@ -1377,7 +1381,7 @@ int mftx_fft_filter(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int
   q.ldw = ldk;
   q.wrow = (int)((rows - hr) % rows);
   q.wcol = (int)((cols - hc) % cols);
-  rc = run_one(ctx, q, nullptr, 0, 0);
+  rc = run_one(ctx, q, nullptr, 0, 0, 0);
   if (rc) return rc;
   OneSpec b = q;
   b.f = F;
@@ -1389,7 +1393,7 @@ int mftx_fft_filter(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int
   b.w = nullptr;
   b.conj_input = true;
   b.reuse_tables = true;
-  rc = run_one(ctx, b, nullptr, 0, 0);
+  rc = run_one(ctx, b, nullptr, 0, 0, 0);
   if (rc) return rc;
   HIPCHK(ctx, launch_magnitude(Y, cols, rows, cols, hr, hc, out, out_dtype, ldo, part, ctx->stream));
   if (normalize) {

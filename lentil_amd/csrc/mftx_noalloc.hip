@@ -62,5 +62,6 @@ extern "C" int mftx_dft2_noalloc(mftx_ctx* ctx, const void* f, int f_dtype, int6
     return mftx::set_error(ctx, MFTX_EDEVICE,
                            (std::string("scratch address lookup: ") + hipGetErrorString(e)).c_str());
   return mftx::dft2_on_workspace(ctx, f, f_dtype, m, n, ldf, F, M, N, ldF, alpha_r, alpha_c, shift_r, shift_c,
-                                 offset_r, offset_c, scale, conj, precision, ws, mftx::kScratchBytes, mftx::kTableBytes);
+                                 offset_r, offset_c, scale, conj, precision, ws, sizeof(mftx::scratch),
+                                 mftx::kScratchBytes, mftx::kTableBytes);
 }
