@@ -35,6 +35,7 @@ namespace {
 constexpr int kRingSlots = 16;
 constexpr size_t kTableCap = 64u << 20;  // twiddle table bytes per stage of one mftx_dft2
 constexpr size_t kSlotBytes = 512 * 1024;
+constexpr size_t kListTables = 1u << 30;  // twiddle table bytes of one launch of a list
 
 int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 double centre(int64_t k) { return (double)(k / 2); }  // floor(k/2), k >= 0 (fourier.py:117-120)
@@ -560,6 +561,7 @@ bool too_large(const MftGeo& g, bool list_entry) {
 struct ManyBatch {
   int tile1 = 0, tile2 = 0;
   size_t ws = 0, bytes = 0;  // workspace and descriptor block sizes
+  size_t table_bytes = 0;    // the workspace's part for twiddle tables
   size_t o_wv = 0, o_ph = 0, o_pk = 0, o_mx = 0, o_tb = 0, o_p1 = 0, o_p2 = 0, o_s1 = 0, o_s2 = 0, o_w1 = 0, o_w2 = 0;
   std::vector<MftGeo> geo;
   std::vector<PhasorWave> waves;
@@ -595,7 +597,8 @@ static void many_build(const mftx_mft* mfts, int32_t count, int prec, int fixed,
     mb.tab1.push_back(mb.tables.get(g.alpha1, g.g1.y0, g.k1, g.g1.slots));
     mb.tab2.push_back(mb.tables.get(g.alpha2, g.g2.y0, g.r1, g.g2.slots));
   }
-  ws += mb.tables.place(ws);
+  mb.table_bytes = mb.tables.place(ws);
+  ws += mb.table_bytes;
 
   // ---- sources -----------------------------------------------------------------
   long long ph_quads = 0, pk_quads = 0;
@@ -764,24 +767,31 @@ static hipError_t many_launch(const ManyBatch& mb, int prec, const char* d, hipS
   return e;
 }
 
+// One entry of a list by itself (below, beside mftx_dft2's code).
+static int run_entry(mftx_ctx* ctx, const mftx_mft& q, int prec);
+
 // All entries [0, count) on the context stream with the context workspace and
-// one descriptor ring slot; a batch whose descriptors exceed a slot is split.
+// one descriptor ring slot; a batch whose descriptors exceed a slot is split,
+// and so is one whose tables exceed kListTables: they hold 2 bytes per input
+// sample and output pixel of an axis (1 x 100000 -> 1 x 100000: 20 GB, for
+// arrays of 1.6 MB), where an entry alone makes its own in pieces.
 static int dft2_many_run(mftx_ctx* ctx, const mftx_mft* mfts, int32_t count, int prec) {
   std::unique_ptr<ManyBatch> mb(new ManyBatch());
   many_build(mfts, count, prec, -1, *mb);
+  auto halves = [&]() {
+    const int32_t h = count / 2;
+    const int rc = dft2_many_run(ctx, mfts, h, prec);
+    return rc ? rc : dft2_many_run(ctx, mfts + h, count - h, prec);
+  };
   if (mb->bytes > kSlotBytes || (count == 1 && too_large(mb->geo[0], true))) {
-    if (count == 1) {
-      // the widest tiles need the fewest descriptors
-      mb.reset(new ManyBatch());
-      many_build(mfts, count, prec, TILE_BIG, *mb);
-      if (mb->bytes > kSlotBytes || too_large(mb->geo[0], true))
-        return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
-    } else {
-      const int32_t h = count / 2;
-      const int rc = dft2_many_run(ctx, mfts, h, prec);
-      return rc ? rc : dft2_many_run(ctx, mfts + h, count - h, prec);
-    }
+    if (count > 1) return halves();
+    // the widest tiles need the fewest descriptors
+    mb.reset(new ManyBatch());
+    many_build(mfts, count, prec, TILE_BIG, *mb);
+    if (mb->bytes > kSlotBytes || too_large(mb->geo[0], true))
+      return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
   }
+  if (mb->table_bytes > kListTables) return count > 1 ? halves() : run_entry(ctx, mfts[0], prec);
   int rc = ensure_ws(ctx, mb->ws);
   if (rc) return rc;
   // the slot is reserved first: the descriptors hold device addresses inside it
@@ -1058,6 +1068,25 @@ static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t ws_bytes, s
     }
   }
   return MFTX_OK;
+}
+
+// A phasor source is made as a complex64 array first.
+static int run_entry(mftx_ctx* ctx, const mftx_mft& q, int prec) {
+  OneSpec one{q.f, q.f_dtype, q.m, q.n, q.ldf, q.F, q.M, q.N, q.ldF, q.alpha_r, q.alpha_c, q.shift_r, q.shift_c,
+              q.offset_r, q.offset_c, q.scale, q.conj, prec};
+  one.w = q.w;
+  one.w_dtype = q.w_dtype;
+  one.ldw = q.ldw;
+  if (!q.f) {
+    const int rc = ensure_aux(ctx, sizeof(float2) * (size_t)q.m * q.n);
+    if (rc) return rc;
+    const PhasorField ph{q.amp, q.opd, (float2*)ctx->aux, q.ld_amp, q.ld_opd, (int)q.m, (int)q.n, q.amp_dtype, q.opd_dtype};
+    HIPCHK(ctx, launch_phasor_fields(&ph, 1, q.inv_wl, ctx->stream));
+    one.f = ctx->aux;
+    one.f_dtype = MFTX_DTYPE_C64;
+    one.ldf = q.n;
+  }
+  return run_one(ctx, one, nullptr, 0, 0, 0);
 }
 
 int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, int64_t ldf, void* F,

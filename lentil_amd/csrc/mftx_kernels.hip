@@ -461,19 +461,25 @@ __device__ __forceinline__ void table_thread(const TableOp& op, long long u) {
 }
 
 template <int PREC>
-__global__ void table_group_kernel(const TableOp* __restrict__ ops, int nops) {
-  const long long b0 = (long long)blockIdx.x * kGroupBlock;
+__global__ void table_group_kernel(const TableOp* __restrict__ ops, int nops, long long first) {
+  const long long b0 = first + (long long)blockIdx.x * kGroupBlock;
   const TableOp& op = ops[block_op(ops, nops, b0)];
   const long long u = b0 + threadIdx.x - op.begin;
   if (u < table_threads(op.nsb, op.nkb)) table_thread<PREC>(op, u);
 }
 
 hipError_t launch_tables(int prec, const TableOp* ops, int nops, long long total, hipStream_t s) {
-  if (total <= 0 || nops <= 0) return hipSuccess;
-  const dim3 grid((unsigned)((total + kGroupBlock - 1) / kGroupBlock)), block(kGroupBlock);
-  if (prec == PREC_BF16X3) hipLaunchKernelGGL((table_group_kernel<PREC_BF16X3>), grid, block, 0, s, ops, nops);
-  else hipLaunchKernelGGL((table_group_kernel<PREC_FP32>), grid, block, 0, s, ops, nops);
-  return hipGetLastError();
+  if (nops <= 0) return hipSuccess;
+  // a launch holds fewer than 2^32 threads: 64 GiB of tables (more were cut off without an error)
+  constexpr long long kMost = 1LL << 31;
+  for (long long first = 0; first < total; first += kMost) {
+    const dim3 grid((unsigned)((std::min(total - first, kMost) + kGroupBlock - 1) / kGroupBlock)), block(kGroupBlock);
+    if (prec == PREC_BF16X3) hipLaunchKernelGGL((table_group_kernel<PREC_BF16X3>), grid, block, 0, s, ops, nops, first);
+    else hipLaunchKernelGGL((table_group_kernel<PREC_FP32>), grid, block, 0, s, ops, nops, first);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 __global__ void row_phase_kernel(const RowPhase* __restrict__ ops) {
