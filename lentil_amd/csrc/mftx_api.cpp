@@ -143,6 +143,15 @@ double stage2_scale(int prec, int64_t k_pairs) {
   return prec != PREC_FP32 ? 1.0 : 1.0 / (tw_scale(prec) * tw_scale(prec)) / stage1_scale(prec, k_pairs);
 }
 
+// Beyond kLongPairs that worst case, every pair as bright as the brightest,
+// leaves too little of f16's range: stage 1's output for a few bright samples
+// would be below 2^-2, where the pair's lo part runs out (one sample among
+// 500000: results 3.1e-6 off).  Such a transform takes the sum of its samples'
+// magnitudes too, and scales the operand so that stage 1 stays below 2^14 with
+// the factor of kLongPairs (OneMft::sums): 7e-8, as for short ones.
+constexpr int64_t kLongPairs = 1 << 14;
+bool is_long(int prec, int64_t k_pairs) { return prec == PREC_FP32 && k_pairs > kLongPairs; }
+
 // Output grid of one MFT stage with N columns, signed twiddle scale alpha and
 // output shift: the slots and pairing centre the GEMM runs on (see Problem)
 // and the fold of its A operand.  Outputs are paired about the PSF core
@@ -504,8 +513,9 @@ MftGeo mft_geometry(int64_t m, int64_t n, int64_t M, int64_t N, double alpha_r, 
   return g;
 }
 
-// The two GEMM problems of one transform (addresses filled by the caller).
-void mft_problems(const MftGeo& g, int prec, double scale, Problem& a, Problem& b) {
+// The two GEMM problems of one transform (addresses filled by the caller);
+// k_pairs: how many pairs of the operand's largest value stage 1's sums reach.
+void mft_problems(const MftGeo& g, int prec, double scale, int64_t k_pairs, Problem& a, Problem& b) {
   a = Problem{};
   a.rblocks = pair_blocks(g.r1);
   a.sblocks = (int)blocks32(g.g1.slots);
@@ -515,7 +525,7 @@ void mft_problems(const MftGeo& g, int prec, double scale, Problem& a, Problem& 
   a.cm = g.g1.cm;
   a.y0 = g.g1.y0;
   a.xrot = g.alpha1 * g.xc1();
-  a.scale = (float)stage1_scale(prec, pairs(g.k1));
+  a.scale = (float)stage1_scale(prec, k_pairs);
   a.ldd = pair_blocks(g.r1);
   b = Problem{};
   b.rblocks = (int)blocks32(g.c1);
@@ -528,7 +538,7 @@ void mft_problems(const MftGeo& g, int prec, double scale, Problem& a, Problem& 
   b.cm = g.g2.cm;
   b.y0 = g.g2.y0;
   b.xrot = g.alpha2 * g.xc2();
-  b.scale = (float)(scale * stage2_scale(prec, pairs(g.k1)));
+  b.scale = (float)(scale * stage2_scale(prec, k_pairs));
   b.trans = g.col_first ? 0 : 1;  // C is F (column-first) or F^T (row-first)
   b.wrows = (int)(g.col_first ? g.c1 : g.c2);
   b.wcols = (int)(g.col_first ? g.c2 : g.c1);
@@ -670,7 +680,7 @@ static void many_build(const mftx_mft* mfts, int32_t count, int prec, int fixed,
     const MftGeo& g = geo[i];
     Problem& a = mb.p1[i];
     Problem& b = mb.p2[i];
-    mft_problems(g, prec, q.scale, a, b);
+    mft_problems(g, prec, q.scale, pairs(g.k1), a, b);
     a.sbeg = b.sbeg = i;
     a.send = b.send = i + 1;
     b.dst = q.F;
@@ -774,7 +784,8 @@ static int run_entry(mftx_ctx* ctx, const mftx_mft& q, int prec);
 // one descriptor ring slot; a batch whose descriptors exceed a slot is split,
 // and so is one whose tables exceed kListTables: they hold 2 bytes per input
 // sample and output pixel of an axis (1 x 100000 -> 1 x 100000: 20 GB, for
-// arrays of 1.6 MB), where an entry alone makes its own in pieces.
+// arrays of 1.6 MB), where an entry alone makes its own in pieces.  So is one
+// with an entry that needs a sum of its samples (is_long).
 static int dft2_many_run(mftx_ctx* ctx, const mftx_mft* mfts, int32_t count, int prec) {
   std::unique_ptr<ManyBatch> mb(new ManyBatch());
   many_build(mfts, count, prec, -1, *mb);
@@ -791,7 +802,9 @@ static int dft2_many_run(mftx_ctx* ctx, const mftx_mft* mfts, int32_t count, int
     if (mb->bytes > kSlotBytes || too_large(mb->geo[0], true))
       return fail(ctx, MFTX_EINVAL, "descriptor block too large (output too big for one call)");
   }
-  if (mb->table_bytes > kListTables) return count > 1 ? halves() : run_entry(ctx, mfts[0], prec);
+  bool alone = mb->table_bytes > kListTables;
+  for (const MftGeo& g : mb->geo) alone = alone || is_long(prec, pairs(g.k1));
+  if (alone) return count > 1 ? halves() : run_entry(ctx, mfts[0], prec);
   int rc = ensure_ws(ctx, mb->ws);
   if (rc) return rc;
   // the slot is reserved first: the descriptors hold device addresses inside it
@@ -947,8 +960,8 @@ struct OneSpec {
 }  // namespace
 
 // One transform on the caller's workspace `ws` of ws_bytes, or on the context's
-// growable workspace when ws is null.  Three launches and nothing uploaded: the source's
-// maximum (f16 form, larger sources only), then operand, twiddle tables and
+// growable workspace when ws is null.  Nothing is uploaded: the source's maximum
+// (f16 form, larger sources only; one launch more for a long one), then operand, twiddle tables and
 // descriptors (launch_prepare_one), then the two GEMMs.  A table larger than
 // `table_cap` bytes is made and used in pieces of whole tile columns.
 //
@@ -979,7 +992,8 @@ static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t ws_bytes, s
   OneMft one = {};
   Problem& p1 = one.desc.prob[0];
   Problem& p2 = one.desc.prob[1];
-  mft_problems(g, prec, q.scale, p1, p2);
+  const bool long_k = is_long(prec, pairs(g.k1));
+  mft_problems(g, prec, q.scale, long_k ? kLongPairs : pairs(g.k1), p1, p2);
   const int tile[2] = {pick_schedule(-1, false, p1.rblocks, p1.sblocks, nkb1, 1, 1).tile,
                        pick_schedule(-1, false, p2.rblocks, p2.sblocks, nkb2, 1, 1).tile};
   // slot blocks of a stage whose table fits the cap (whole tiles)
@@ -989,8 +1003,9 @@ static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t ws_bytes, s
     return (int)std::min<int64_t>(sblocks, std::max<int64_t>(fit, tile_slots(t)));
   };
   const int piece1 = piece(p1.sblocks, nkb1, tile[0]), piece2 = piece(p2.sblocks, nkb2, tile[1]);
-  // workspace: descriptors, maxima and inverse scale, operands, tables
-  const size_t o_max = round_up(sizeof(OneDesc), 256), o_a1 = o_max + 2048;
+  // workspace: descriptors, maxima and inverse scale (and sums), operands, tables
+  const size_t o_max = round_up(sizeof(OneDesc), 256), o_sum = o_max + 2048;
+  const size_t o_a1 = o_sum + (long_k ? sizeof(double) * kMaxBlocks : 0);
   const size_t o_a2 = o_a1 + folded_bytes(g.r1, g.k1), o_t1 = o_a2 + plain_bytes(g.c1, nkb2);
   const size_t o_t2 = o_t1 + table_bytes(piece1, nkb1), need = o_t2 + table_bytes(piece2, nkb2);
   static_assert((kMaxBlocks + 1) * sizeof(float) <= 2048, "maxima and inverse scale fit their space");
@@ -1030,6 +1045,7 @@ static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t ws_bytes, s
     // a source of up to 8192 elements is read whole by every operand block
     // instead: cheaper than a launch of its own
     one.op.sc = ScaleSrc{part, inv, m * n <= 8192 ? 0 : mx.nblk, 0};
+    if (long_k) one.sums = (double*)(base + o_sum);
     p2.inv = inv;
   }
   one.wave = PhasorWave{0.0, 4.0 * g.g1.fold, g.x01, 4.0 * g.g2.fold, g.x02};

@@ -246,6 +246,7 @@ struct OneMft {
   TableOp tab[2];
   OneDesc desc;
   OneDesc* desc_dev;    // device copy for the GEMM launches
+  double* sums;         // f16 form of a long transform: space for the source's block sums, else null
 };
 hipError_t launch_prepare_one(int prec, const OneMft& one, const MaxOp& mx, hipStream_t s);
 hipError_t launch_table_one(int prec, const TableOp& op, hipStream_t s);

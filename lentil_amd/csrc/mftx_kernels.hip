@@ -71,11 +71,13 @@ constexpr float kMaxFloat = 3.4028234663852886e38f;
 // non-finite whatever the scale), FP32's largest number where the sum of two
 // finite parts is past it (at most twice that: scaled operands then reach 2^15
 // instead of 2^14, still half of f16's range).  The dtype is tested outside the loop, so
-// the loads of 8 elements are in flight together.
-template <typename Get>
+// the loads of 8 elements are in flight together.  SUM: the elements' bounds are
+// added up in *sum too.
+template <bool SUM, typename Get>
 __device__ __forceinline__ float bound_of(long long m, long long n, long long ld, long long first, long long step,
-                                          Get&& get) {
+                                          double* sum, Get&& get) {
   float v = 0.f;
+  double total_bound = 0.0;
   const long long total = m * n;
   auto one = [&](long long i) {
     const float2 e = get(ld == n ? i : total < (1LL << 31) ? (long long)((unsigned)i / (unsigned)n) * ld + (unsigned)i % (unsigned)n
@@ -89,23 +91,38 @@ __device__ __forceinline__ float bound_of(long long m, long long n, long long ld
 #pragma unroll
     for (int q = 0; q < 8; ++q) b[q] = one(i + q * step);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v = fmaxf(v, b[q]);
+    for (int q = 0; q < 8; ++q) {
+      v = fmaxf(v, b[q]);
+      if (SUM) total_bound += (double)b[q];
+    }
   }
-  for (; i < total; i += step) v = fmaxf(v, one(i));
+  for (; i < total; i += step) {
+    const float b = one(i);
+    v = fmaxf(v, b);
+    if (SUM) total_bound += (double)b;
+  }
+  if (SUM) *sum = total_bound;
   return v;
 }
-__device__ __forceinline__ float array_bound(const void* src, int dtype, long long m, long long n, long long ld,
-                                             long long first, long long step) {
+template <bool SUM>
+__device__ __forceinline__ float array_bound_sum(const void* src, int dtype, long long m, long long n, long long ld,
+                                                 long long first, long long step, double* sum) {
   switch (dtype) {
     case 0:
-      return bound_of(m, n, ld, first, step, [&](long long i) {
+      return bound_of<SUM>(m, n, ld, first, step, sum, [&](long long i) {
         const v2f32 e = ((gptr<const v2f32>)src)[i];
         return make_float2(e.x, e.y);
       });
-    case 1: return bound_of(m, n, ld, first, step, [&](long long i) { return make_float2(((gptr<const float>)src)[i], 0.f); });
-    case 2: return bound_of(m, n, ld, first, step, [&](long long i) { return load_elem(src, 2, i); });
-    default: return bound_of(m, n, ld, first, step, [&](long long i) { return load_elem(src, 3, i); });
+    case 1:
+      return bound_of<SUM>(m, n, ld, first, step, sum,
+                           [&](long long i) { return make_float2(((gptr<const float>)src)[i], 0.f); });
+    case 2: return bound_of<SUM>(m, n, ld, first, step, sum, [&](long long i) { return load_elem(src, 2, i); });
+    default: return bound_of<SUM>(m, n, ld, first, step, sum, [&](long long i) { return load_elem(src, 3, i); });
   }
+}
+__device__ __forceinline__ float array_bound(const void* src, int dtype, long long m, long long n, long long ld,
+                                             long long first, long long step) {
+  return array_bound_sum<false>(src, dtype, m, n, ld, first, step, nullptr);
 }
 
 __global__ void absmax_kernel(const MaxOp* __restrict__ ops, int nops) {
@@ -538,15 +555,49 @@ __global__ void table_one_kernel(TableOp op) {
   if (u < table_threads(op.nsb, op.nkb)) table_thread<PREC>(op, u);
 }
 
-__global__ void absmax_one_kernel(MaxOp op) {
-  const float v = block_max(array_bound(op.src, op.dtype, op.m, op.n, op.ld,
-                                        (long long)blockIdx.x * kGroupBlock + threadIdx.x,
-                                        (long long)op.nblk * kGroupBlock));
-  if (threadIdx.x == 0) op.part[blockIdx.x] = v;
+// Sum of v over the block (every thread calls it once).
+__device__ double block_sum(double v) {
+  __shared__ double w[kGroupBlock / 64];
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = v;
+  __syncthreads();
+  v = 0.0;
+  for (int i = 0; i < kGroupBlock / 64; ++i) v += w[i];
+  return v;
 }
 
+// SUM: also sums[b], the sum of block b's element bounds.
+template <bool SUM>
+__global__ void absmax_one_kernel(MaxOp op, double* __restrict__ sums) {
+  double sum = 0.0;
+  const float v = block_max(array_bound_sum<SUM>(op.src, op.dtype, op.m, op.n, op.ld,
+                                                 (long long)blockIdx.x * kGroupBlock + threadIdx.x,
+                                                 (long long)op.nblk * kGroupBlock, &sum));
+  if (threadIdx.x == 0) op.part[blockIdx.x] = v;
+  if (SUM) {
+    sum = block_sum(sum);
+    if (threadIdx.x == 0) sums[blockIdx.x] = sum;
+  }
+}
+
+// Raises the source's bound to 2^-16 of the sum S of its samples: the operand's
+// scale 2^e then keeps S 2^e, and so stage 1's sums over any number of pairs,
+// below 2^28, 2^14 after the store's 2^-14 (one block, n <= kGroupBlock).
+__global__ void long_bound_kernel(float* __restrict__ part, const double* __restrict__ sums, int n) {
+  const double s = block_sum((int)threadIdx.x < n ? sums[threadIdx.x] : 0.0);
+  if (threadIdx.x == 0) part[0] = fmaxf(part[0], (float)fmin(s * 0x1p-16, (double)kMaxFloat));
+}
+static_assert(kMaxBlocks <= kGroupBlock, "one block adds every sum");
+
 hipError_t launch_prepare_one(int prec, const OneMft& one, const MaxOp& mx, hipStream_t s) {
-  if (prec == PREC_FP32 && one.op.sc.n > 0) hipLaunchKernelGGL(absmax_one_kernel, dim3(mx.nblk), dim3(kGroupBlock), 0, s, mx);
+  if (prec == PREC_FP32 && one.op.sc.n > 0) {
+    if (one.sums) {
+      hipLaunchKernelGGL((absmax_one_kernel<true>), dim3(mx.nblk), dim3(kGroupBlock), 0, s, mx, one.sums);
+      hipLaunchKernelGGL(long_bound_kernel, dim3(1), dim3(kGroupBlock), 0, s, mx.part, one.sums, mx.nblk);
+    } else {
+      hipLaunchKernelGGL((absmax_one_kernel<false>), dim3(mx.nblk), dim3(kGroupBlock), 0, s, mx, nullptr);
+    }
+  }
   const PhasorOp& op = one.op;
   const int op_blocks =
       (int)((operand_threads(op.trans ? op.n : op.m, op.trans ? op.m : op.n, 1, OperandSplit{2, 1}) + kGroupBlock - 1) /
