@@ -33,7 +33,12 @@ using namespace mftx;
 namespace {
 
 constexpr int kRingSlots = 16;
-constexpr size_t kTableCap = 64u << 20;  // twiddle table bytes per stage of one mftx_dft2
+// Twiddle table bytes per stage of one mftx_dft2: a larger table is used in
+// pieces.  Pieces of kTableCap where those give every CU two tiles; of up to
+// kTableMost where they do not (long, thin transforms: with pieces of 64 MiB
+// 1 x 40000 -> 1 x 40000 took 25 launches of 25 workgroups, 9.3 ms, now 3.1,
+// and 1 x 500000 -> 1 x 3001 47 launches of one, 82 ms, now 10.7).
+constexpr size_t kTableCap = 64u << 20, kTableMost = 1u << 30;
 constexpr size_t kSlotBytes = 512 * 1024;
 constexpr size_t kListTables = 1u << 30;  // twiddle table bytes of one launch of a list
 
@@ -933,7 +938,7 @@ int mftx_dft2(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, i
               int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r, double shift_c,
               double offset_r, double offset_c, double scale, int conj, int precision) {
   return mftx::dft2_on_workspace(ctx, f, f_dtype, m, n, ldf, F, M, N, ldF, alpha_r, alpha_c, shift_r, shift_c,
-                                 offset_r, offset_c, scale, conj, precision, nullptr, 0, 0, 0);
+                                 offset_r, offset_c, scale, conj, precision, nullptr, 0, 0);
 }
 
 }  // extern "C"
@@ -961,19 +966,19 @@ struct OneSpec {
 
 // One transform on the caller's workspace `ws` of ws_bytes, or on the context's
 // growable workspace when ws is null.  Nothing is uploaded: the source's maximum
-// (f16 form, larger sources only; one launch more for a long one), then operand, twiddle tables and
-// descriptors (launch_prepare_one), then the two GEMMs.  A table larger than
-// `table_cap` bytes is made and used in pieces of whole tile columns.
+// (f16 form, larger sources only; one launch more for a long one), then operand,
+// twiddle tables and descriptors (launch_prepare_one), then the two GEMMs.  A
+// table larger than its space is made and used in pieces of whole tile columns.
 //
 // `cap` bounds the transform as the no-allocation entry point documents it:
 // complex64-sized operands with rows padded to 128 and K to 16 or 32.  The
 // workspace then holds operands of up to twice that (K is padded to 32 and
-// paired), two tables of table_cap and the descriptors.  The operands are fully
+// paired), the descriptors, and tables in the rest.  The operands are fully
 // written before they are read (the source's operand with its zero padding,
 // then stage 1's output for every K the second stage reads), so the workspace
 // needs no clearing; padding rows beyond the output only feed output rows that
 // are never stored.
-static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t ws_bytes, size_t cap, size_t table_cap) {
+static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t ws_bytes, size_t cap) {
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const int prec = q.precision;
   const int64_t m = q.m, n = q.n;
@@ -996,17 +1001,21 @@ static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t ws_bytes, s
   mft_problems(g, prec, q.scale, long_k ? kLongPairs : pairs(g.k1), p1, p2);
   const int tile[2] = {pick_schedule(-1, false, p1.rblocks, p1.sblocks, nkb1, 1, 1).tile,
                        pick_schedule(-1, false, p2.rblocks, p2.sblocks, nkb2, 1, 1).tile};
-  // slot blocks of a stage whose table fits the cap (whole tiles)
-  if (!ws) table_cap = kTableCap;
-  auto piece = [&](int sblocks, int nkb, int t) {
-    const int64_t fit = (int64_t)(table_cap / table_bytes(1, nkb)) / tile_slots(t) * tile_slots(t);
-    return (int)std::min<int64_t>(sblocks, std::max<int64_t>(fit, tile_slots(t)));
-  };
-  const int piece1 = piece(p1.sblocks, nkb1, tile[0]), piece2 = piece(p2.sblocks, nkb2, tile[1]);
   // workspace: descriptors, maxima and inverse scale (and sums), operands, tables
   const size_t o_max = round_up(sizeof(OneDesc), 256), o_sum = o_max + 2048;
   const size_t o_a1 = o_sum + (long_k ? sizeof(double) * kMaxBlocks : 0);
   const size_t o_a2 = o_a1 + folded_bytes(g.r1, g.k1), o_t1 = o_a2 + plain_bytes(g.c1, nkb2);
+  // slot blocks of a stage whose table fits its space (whole tiles): kTableCap,
+  // more where that gives a CU less than two tiles, half of what the operands
+  // leave of a caller's workspace at most
+  const size_t room = !ws ? kTableMost : o_t1 < ws_bytes ? (ws_bytes - o_t1) / 2 : 0;
+  auto piece = [&](const Problem& p, int nkb, int t) {
+    const int64_t tr = (p.rblocks + tile_rows(t) - 1) / tile_rows(t);
+    const size_t fill = table_bytes((int)((2 * kCUs + tr - 1) / tr) * tile_slots(t), nkb);
+    const int64_t fit = (int64_t)(std::min(room, std::max(kTableCap, fill)) / table_bytes(1, nkb)) / tile_slots(t) * tile_slots(t);
+    return (int)std::min<int64_t>(p.sblocks, std::max<int64_t>(fit, tile_slots(t)));
+  };
+  const int piece1 = piece(p1, nkb1, tile[0]), piece2 = piece(p2, nkb2, tile[1]);
   const size_t o_t2 = o_t1 + table_bytes(piece1, nkb1), need = o_t2 + table_bytes(piece2, nkb2);
   static_assert((kMaxBlocks + 1) * sizeof(float) <= 2048, "maxima and inverse scale fit their space");
   int rc = MFTX_OK;
@@ -1015,7 +1024,7 @@ static int run_one(mftx_ctx* ctx, const OneSpec& q, void* ws, size_t ws_bytes, s
     if (rc) return rc;
     ws = ctx->ws;
   } else if (need > ws_bytes) {
-    // a transform within the cap takes two thirds of the array at most; this keeps the kernels inside it whatever changes
+    // the array is made so that a transform within the cap fits; this keeps the kernels inside it whatever changes
     return fail(ctx, MFTX_EINVAL, "transform needs " + std::to_string(need) + " bytes of workspace, more than the " +
                                       std::to_string(ws_bytes) + " available");
   }
@@ -1102,13 +1111,13 @@ static int run_entry(mftx_ctx* ctx, const mftx_mft& q, int prec) {
     one.f_dtype = MFTX_DTYPE_C64;
     one.ldf = q.n;
   }
-  return run_one(ctx, one, nullptr, 0, 0, 0);
+  return run_one(ctx, one, nullptr, 0, 0);
 }
 
 int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, int64_t ldf, void* F,
                             int64_t M, int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r,
                             double shift_c, double offset_r, double offset_c, double scale, int conj, int precision,
-                            void* ws, size_t ws_bytes, size_t cap, size_t table_cap) {
+                            void* ws, size_t ws_bytes, size_t cap) {
   if (!ctx) return MFTX_EHANDLE;
   if (!f || !F) return fail(ctx, MFTX_EINVAL, "null array pointer");
   if (m <= 0 || n <= 0 || M <= 0 || N <= 0) return fail(ctx, MFTX_EINVAL, "shapes must be positive");
@@ -1119,7 +1128,7 @@ int mftx::dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m
     return fail(ctx, MFTX_EINVAL, "dimension too large");
   OneSpec q{f, f_dtype, m, n, ldf, F, M, N, ldF, alpha_r, alpha_c, shift_r, shift_c, offset_r, offset_c, scale, conj,
             precision};
-  return run_one(ctx, q, ws, ws_bytes, cap, table_cap);
+  return run_one(ctx, q, ws, ws_bytes, cap);
 }
 
 extern "C" {
@@ -1426,7 +1435,7 @@ int mftx_fft_filter(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int
   q.ldw = ldk;
   q.wrow = (int)((rows - hr) % rows);
   q.wcol = (int)((cols - hc) % cols);
-  rc = run_one(ctx, q, nullptr, 0, 0, 0);
+  rc = run_one(ctx, q, nullptr, 0, 0);
   if (rc) return rc;
   OneSpec b = q;
   b.f = F;
@@ -1438,7 +1447,7 @@ int mftx_fft_filter(mftx_ctx* ctx, const void* img, int dtype, int64_t rows, int
   b.w = nullptr;
   b.conj_input = true;
   b.reuse_tables = true;
-  rc = run_one(ctx, b, nullptr, 0, 0, 0);
+  rc = run_one(ctx, b, nullptr, 0, 0);
   if (rc) return rc;
   HIPCHK(ctx, launch_magnitude(Y, cols, rows, cols, hr, hc, out, out_dtype, ldo, part, ctx->stream));
   if (normalize) {

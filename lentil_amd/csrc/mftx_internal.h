@@ -374,12 +374,12 @@ hipError_t launch_zernike(const double* rho, const double* theta, const void* ma
 
 // host side of the C ABI (mftx_api.cpp)
 // mftx_dft2 on the caller's workspace ws of ws_bytes (for transforms of up to
-// cap bytes, see the definition, with table_cap bytes per twiddle table), or on the
-// context's own growable workspace when ws is null
+// cap bytes, see the definition), or on the context's own growable workspace when
+// ws is null
 int dft2_on_workspace(mftx_ctx* ctx, const void* f, int f_dtype, int64_t m, int64_t n, int64_t ldf, void* F,
                       int64_t M, int64_t N, int64_t ldF, double alpha_r, double alpha_c, double shift_r,
                       double shift_c, double offset_r, double offset_c, double scale, int conj, int precision,
-                      void* ws, size_t ws_bytes, size_t cap, size_t table_cap);
+                      void* ws, size_t ws_bytes, size_t cap);
 // record msg as the context's last error and return code
 int set_error(mftx_ctx* ctx, int code, const char* msg);
 // the device a context was created on

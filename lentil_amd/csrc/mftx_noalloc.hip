@@ -23,7 +23,8 @@ namespace mftx {
 
 // The documented limit counts complex64-sized operands; what the kernels lay
 // out for a transform within it takes at most twice that (K padded to pairs of
-// 32), two twiddle tables and the descriptors (dft2_on_workspace).
+// 32), two pieces of twiddle tables (K is 32768 at most: a piece of four slot
+// blocks takes 16 MiB) and the descriptors (dft2_on_workspace).
 constexpr size_t kScratchBytes = MFTX_NOALLOC_SCRATCH_BYTES;
 constexpr size_t kTableBytes = 16u << 20;
 constexpr int kMaxDevices = 64;
@@ -63,5 +64,5 @@ extern "C" int mftx_dft2_noalloc(mftx_ctx* ctx, const void* f, int f_dtype, int6
                            (std::string("scratch address lookup: ") + hipGetErrorString(e)).c_str());
   return mftx::dft2_on_workspace(ctx, f, f_dtype, m, n, ldf, F, M, N, ldF, alpha_r, alpha_c, shift_r, shift_c,
                                  offset_r, offset_c, scale, conj, precision, ws, sizeof(mftx::scratch),
-                                 mftx::kScratchBytes, mftx::kTableBytes);
+                                 mftx::kScratchBytes);
 }

@@ -1,7 +1,8 @@
-"""Transforms whose twiddle table is larger than its space (16 MiB of the
-no-allocation array, 64 MiB of the context workspace): the table is made and
-used in pieces of whole tile columns, the last of them a remainder.  Against
-the complex128 oracle at the fields' gates, and against each other."""
+"""Transforms whose twiddle table is larger than its space (what the operands
+leave of the no-allocation array, 64 MiB to 1 GiB of the context workspace): the
+table is made and used in pieces of whole tile columns, the last of them a
+remainder.  Against the complex128 oracle at the fields' gates, and against each
+other."""
 import ctypes
 
 import numpy as np
@@ -26,9 +27,11 @@ def _call(name, f, F, alpha, shift, prec):
 @pytest.mark.parametrize('prec', [0, 1])
 @pytest.mark.parametrize('flip', [False, True])
 @pytest.mark.parametrize('names, shape_in, shape_out', [
-    (('mftx_dft2_noalloc', 'mftx_dft2'), (64, 1024), (16, 20001)),   # stage 2, 128 KiB per 32 slots: 3 pieces, 1 on
-    (('mftx_dft2_noalloc', 'mftx_dft2'), (16, 1024), (64, 20001)),   # the context; the same in stage 1
-    (('mftx_dft2',), (5, 1200), (3, 30001))])                        # 152 KiB: 2 pieces on the context
+    (('mftx_dft2_noalloc', 'mftx_dft2'), (64, 1024), (16, 20001)),   # stage 2, a table of 41 MB
+    (('mftx_dft2_noalloc', 'mftx_dft2'), (16, 1024), (64, 20001)),   # the same in stage 1
+    (('mftx_dft2_noalloc', 'mftx_dft2'), (2, 9000), (3, 7001)),      # 126 MB: 3 pieces on the array, 1 on the context
+    (('mftx_dft2_noalloc', 'mftx_dft2'), (3, 9000), (2, 7001)),      # the same in stage 2
+    (('mftx_dft2',), (5, 1200), (3, 30001))])                        # 73 MB
 def test_tables_in_pieces(names, shape_in, shape_out, flip, prec):
     rng = np.random.default_rng(shape_in[0])
     x = (rng.standard_normal(shape_in) + 1j * rng.standard_normal(shape_in)).astype(np.complex64)
