@@ -282,6 +282,8 @@ def _insert_group(fields, out, weight):
         h, w = t.shape
         if h and w:
             items.append((t.data_ptr(), w, h, w, rows // 2 + f.extent[0], cols // 2 + f.extent[2]))
+    if not (rows and cols and items):   # nothing to add to
+        return
     ctx = _lib.context()
     rc = _lib.load().mftx_insert_group(ctx, (_lib.MftxField * len(items))(*items), len(items), out.data_ptr(),
                                        _lib.DTYPE_CODE[out.dtype], rows, cols, row_stride(out), float(np.real(weight)))
