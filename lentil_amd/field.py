@@ -293,7 +293,9 @@ def _insert_group(fields, out, weight):
 
 def _check_pixelscales(fields):
     p0 = fields[0].pixelscale
-    if not all(f.pixelscale is p0 for f in fields) and not np.all([f.pixelscale == p0 for f in fields]):
+    if all(f.pixelscale is p0 for f in fields) and (p0 is None or np.all(p0 == p0)):
+        return      # one object, compared once
+    if not np.all([f.pixelscale == p0 for f in fields]):
         raise ValueError("Can't merge: pixelscales must be equal")
 
 
