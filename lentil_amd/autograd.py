@@ -35,6 +35,15 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr())
 
 
+def _plane(x):
+    """x without leading axes of length 1: an array of at most two dimensions."""
+    if x.ndim > 2:
+        if any(n != 1 for n in x.shape[:-2]):
+            raise ValueError(f'expected one array of two dimensions, got shape {tuple(x.shape)}')
+        x = x.reshape(x.shape[-2:])
+    return x
+
+
 class BroadbandPSFModel:
     """Multi-diversity broadband PSF model on the device with gradients."""
 
@@ -50,7 +59,7 @@ class BroadbandPSFModel:
         self.M = self.npix * self.oversample
         self.precision = precision
         self.amp = torch.from_numpy(amp.copy()).to(self.dev)
-        div = [np.broadcast_to(np.asarray(d, dtype=float), self.shape) for d in diversity]
+        div = [np.broadcast_to(_plane(np.asarray(d, dtype=float)), self.shape) for d in diversity]
         self.div = torch.from_numpy(np.array(div).reshape((len(div),) + self.shape)).to(self.dev)
         # a full-grid mask keeps the tile the whole array at offset (0, 0)
         pupil = Pupil(amplitude=amp, opd=np.zeros(self.shape), mask=np.ones(self.shape), pixelscale=dx,
@@ -90,9 +99,7 @@ class BroadbandPSFModel:
 
     # ---------------------------------------------------------------- forward
     def forward_images(self, opd, amp):
-        if opd.dim() > 2:
-            raise ValueError(f'opd must have shape {self.shape}, got {tuple(opd.shape)}')
-        torch.add(opd, self.div, out=self.plan.opd_stack(0))
+        torch.add(_plane(opd), self.div, out=self.plan.opd_stack(0))
         if not self._same(self._amp_in_plan, amp):
             amp32 = amp.to(torch.float32)  # converted once for every copy
             for d in range(len(self.div)):
@@ -220,5 +227,7 @@ class _PSFStack(torch.autograd.Function):
         dtypes = [t.dtype if t.dtype == torch.float32 else torch.float64 for t in (opd, amp)]
         g_opd, g_amp = ctx.model.backward_grads(opd, amp, grad_images, ctx.needs_input_grad[1], gen=ctx.gen,
                                                 dtypes=dtypes)
+        if opd.dim() > 2:   # leading axes of length 1
+            g_opd = g_opd.reshape(opd.shape[:-2] + g_opd.shape)
         return (g_opd.to(opd.dtype) if ctx.needs_input_grad[0] else None,
                 g_amp.to(amp.dtype) if g_amp is not None else None, None)
