@@ -295,6 +295,7 @@ struct mftx_plan {
   long long phasor_threads = 0;
   std::vector<ReduceOp> reduces;   // regions of the image written from partial images
   ReduceOp* reduce_ops = nullptr;  // ... on the device
+  double unit = 1.0;               // what one unit of the partial images is worth
   // coherent groups whose Fields have several output grids: complex outputs,
   // summed and squared into the image by one launch (field.py:331-346)
   CoherentGroup* cgroups = nullptr;
@@ -1925,6 +1926,13 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     }
   }
 
+  // Weights all below 2^-60 meet the FP32 sums without their common power of
+  // two, which the reduction multiplies in: the unitary scale and the f16 form's
+  // would take them out of FP32's range.
+  double most_weight = 0;
+  for (int i = 0; i < nprob; ++i) most_weight = std::max(most_weight, std::fabs(problems[i].weight));
+  const int wexp = most_weight > 0 && most_weight < 0x1p-60 ? std::ilogb(most_weight) : 0;
+
   // ---- descriptors ---------------------------------------------------------------
   // Segment addresses are workspace offsets (operand) and table indices until
   // the workspace exists.
@@ -2009,7 +2017,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
     const bool stored = path[ci] == PATH_FIELDS;
     if (!stored) {  // the scale is a power of two, so the weight is rounded once
       q.scale = (float)stage2_scale(prec, c.pairs1);
-      q.weight = (float)(unit * unit * problems[c.members[0]].weight);
+      q.weight = (float)(unit * unit * std::ldexp(problems[c.members[0]].weight, -wexp));
     } else {
       q.scale = (float)(unit * stage2_scale(prec, c.pairs1));
       q.ldd = K.N;  // F[u][v]
@@ -2380,6 +2388,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
                                      wg.n, (int)(wg.box.r1 - wg.box.r0), (int)(wg.box.c1 - wg.box.c0), (int)wg.box.r0,
                                      (int)wg.box.c0, 0});
   plan->reduce_ops = (ReduceOp*)(base + o_red);
+  plan->unit = std::ldexp(1.0, wexp);
   if (!plan->reduces.empty())
     e = hipMemcpy(plan->reduce_ops, plan->reduces.data(), sizeof(ReduceOp) * plan->reduces.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) {
@@ -2461,7 +2470,7 @@ static hipError_t launch_finish(const mftx_plan* plan, void* image, int dtype, i
                                 hipStream_t s) {
   if (!plan->reduces.empty() || !plan->n_cgroups) {
     const hipError_t e = launch_reduce(plan->reduce_ops, (int)plan->reduces.size(), image, dtype, ldi,
-                                       (int)plan->img_rows, (int)plan->img_cols, accumulate, s);
+                                       (int)plan->img_rows, (int)plan->img_cols, accumulate, plan->unit, s);
     if (e != hipSuccess || !plan->n_cgroups) return e;
     accumulate = 1;
   }

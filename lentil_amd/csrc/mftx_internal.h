@@ -273,8 +273,9 @@ struct ReduceOp {
   long long gstride, ldp;
   int ngroups, rows, cols, r0, c0, pad_;
 };
+// image (+)= unit times the sum of the regions
 hipError_t launch_reduce(const ReduceOp* ops, int nops, void* image, int dtype, long long ldi, int rows, int cols,
-                         int accumulate, hipStream_t s);
+                         int accumulate, double unit, hipStream_t s);
 // Coherent groups of a plan whose Fields have several output grids: group g's
 // Fields are adds[first .. first + count) of the launch.
 struct CoherentAdd {

@@ -673,7 +673,7 @@ hipError_t launch_phasor_fields(const PhasorField* items, int count, double inv_
 // one launch for all regions: 4 side by side (512^2, 8 partials each) took a
 // clear and 4 launches of 4.7 us, 24 us in all.
 __global__ void reduce_kernel(const ReduceOp* __restrict__ ops, int nops, void* __restrict__ image, int dtype,
-                              long long ldi, int rows, int cols, int accumulate) {
+                              long long ldi, int rows, int cols, int accumulate, double unit) {
   const unsigned per_row = (unsigned)(cols + 255) / 256;
   const int r = (int)(blockIdx.x / per_row), c = (int)(blockIdx.x % per_row) * 256 + (int)threadIdx.x;
   if (c >= cols) return;
@@ -687,6 +687,7 @@ __global__ void reduce_kernel(const ReduceOp* __restrict__ ops, int nops, void* 
 #pragma unroll 8
     for (int g = 0; g < n; ++g) acc += (double)p[(long long)g * step];
   }
+  acc *= unit;
   const long long o = (long long)r * ldi + c;
   if (dtype == 3) {
     double* d = (double*)image;
@@ -698,10 +699,10 @@ __global__ void reduce_kernel(const ReduceOp* __restrict__ ops, int nops, void* 
 }
 
 hipError_t launch_reduce(const ReduceOp* ops, int nops, void* image, int dtype, long long ldi, int rows, int cols,
-                         int accumulate, hipStream_t s) {
+                         int accumulate, double unit, hipStream_t s) {
   if (rows <= 0 || cols <= 0 || (nops == 0 && accumulate)) return hipSuccess;
   hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)rows * (unsigned)((cols + 255) / 256)), dim3(256), 0, s, ops, nops,
-                     image, dtype, ldi, rows, cols, accumulate);
+                     image, dtype, ldi, rows, cols, accumulate, unit);
   return hipGetLastError();
 }
 
