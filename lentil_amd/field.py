@@ -293,8 +293,10 @@ def _insert_group(fields, out, weight):
 
 def _check_pixelscales(fields):
     p0 = fields[0].pixelscale
-    if all(f.pixelscale is p0 for f in fields) and (p0 is None or np.all(p0 == p0)):
-        return      # one object, compared once
+    if all(f.pixelscale is p0 for f in fields):     # one object, compared once
+        same = p0 == p0
+        if same is True or (same.all() if isinstance(same, np.ndarray) else np.all(same)):
+            return
     if not np.all([f.pixelscale == p0 for f in fields]):
         raise ValueError("Can't merge: pixelscales must be equal")
 

@@ -23,6 +23,9 @@ def boundary_slice(x, threshold=0, pad=(0, 0)):
                  max(cmin - pad[1], 0):min(cmax + pad[1] + 1, x.shape[1])]
 
 
+_INTS = frozenset((int, np.int64))
+
+
 def slice_offset(slc, shape):
     """Offset of a slice's centre from the centre of its parent (helper.py:65-123)."""
     if slc is Ellipsis:
@@ -32,9 +35,10 @@ def slice_offset(slc, shape):
             return (0, 0)
         raise ValueError(f"Can't compute offset from slice {slc}")
     r, c = slc[0], slc[1]
-    if isinstance(shape, tuple) and len(shape) == 2 \
-            and all(isinstance(v, (int, np.int64)) for v in (r.start, r.stop, c.start, c.stop)):
-        return (r.start + (r.stop - r.start) // 2 - shape[0] // 2, c.start + (c.stop - c.start) // 2 - shape[1] // 2)
+    ends = r.start, r.stop, c.start, c.stop
+    if type(shape) is tuple and len(shape) == 2 and _INTS.issuperset(map(type, ends)):
+        r0, r1, c0, c1 = map(int, ends)
+        return r0 + (r1 - r0) // 2 - shape[0] // 2, c0 + (c1 - c0) // 2 - shape[1] // 2
     # other shapes and indices as numpy broadcasts and promotes them
     size = np.array((r.stop - r.start, c.stop - c.start))
     return tuple(np.array((r.start + size[0] // 2, c.start + size[1] // 2)) - np.asarray(shape) // 2)
