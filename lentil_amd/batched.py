@@ -11,9 +11,9 @@
 
 as a handful of grouped launches (phasors for every (segment, wavelength),
 one stage-1 GEMM launch, one stage-2 GEMM launch with |E|^2 accumulated in
-registers across wavelengths, one reduction onto the detector).  The per-Field geometry is the same host code as
-``propagate_dft`` (``propagate.field_geometry``), so both paths agree on
-every shift, clip and offset.
+registers across wavelengths, one reduction onto the detector).  The per-Field
+geometry is the same host code as ``propagate_dft`` (``propagate.field_geometry``),
+so both paths agree on every shift, clip and offset.
 """
 import ctypes
 import hashlib

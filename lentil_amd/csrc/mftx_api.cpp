@@ -1663,13 +1663,13 @@ struct ClassInfo {
 };
 
 // Whether `classes` windows of one box, of `nkb` stage-2 K blocks each on
-// average, are better summed in registers on the box's grid (box samples over
+// average, are better summed on chip on the box's grid (box samples over
 // window samples: `waste`) than stored as Fields and summed by the coherent
-// launch.  Per 32 x 32 block and class, in ns on a full chip: in registers 0.65
+// launch.  Per 32 x 32 block and class, in ns on a full chip: on chip 0.65
 // per K block (its fragments come from L2 for each block) and 1.5 for its end,
 // four waves taking the classes in turn; as a Field 0.34 per K block (128 x 128
 // tiles) and 11.5 for storing, reading and adding it.  Measured (whole image,
-// as Fields -> in registers): 18 segments, K = 4: 160 -> 78 us at waste 1.0,
+// as Fields -> on chip): 18 segments, K = 4: 160 -> 78 us at waste 1.0,
 // 83 -> 57 at 2.0; K = 7: 2169 -> 805 at 1.0, 690 -> 396 at 1.45, 691 -> 505 at
 // 2.0; 6 segments, K = 22: 621 -> 515 at 1.0, 282 -> 286 at 1.29.
 bool sum_windows(double waste, double nkb, int classes) {
@@ -1680,7 +1680,7 @@ bool sum_windows(double waste, double nkb, int classes) {
 // How a class reaches the image.
 enum ClassPath {
   PATH_INTENSITY,  // alone in its group: |F|^2 summed in registers
-  PATH_WINDOWS,    // one of several windows of one grid: summed in registers, then squared
+  PATH_WINDOWS,    // one of several windows of one grid: summed in LDS, then squared
   PATH_FIELDS      // one of several grids: F stored, summed and squared by the coherent launch
 };
 
@@ -1745,7 +1745,7 @@ int mftx_plan_psf(mftx_ctx* ctx, const mftx_tile* tiles, int32_t ntiles, const d
   // A group with one class runs the intensity path.  The classes of a group
   // with several are windows of one grid, the box around them, where the box
   // is little larger than they are (their shifts differ by a few pixels, as
-  // segment tilts do): transformed on that grid they are summed in registers.
+  // segment tilts do): transformed on that grid they are summed on chip.
   // Far apart, each would compute mostly what it drops; then their Fields are
   // stored and summed by the coherent launch (sum_windows draws the line).
   bool fast = true;  // every group has one class

@@ -20,9 +20,11 @@ constexpr int B_BLOCK = 4 * FRAG;      // twiddle bytes per (32 slots, K block):
 // Number formats of the split operands: every value is hi + lo of one 16-bit
 // type, a real product is hi*hi + hi*lo + lo*hi with FP32 accumulation.
 //   PREC_FP32   : f16 pairs (22 bits).  The operand is scaled by a power of two
-//                 per launch so its largest value fits f16 (see ScaleSrc); the
-//                 result's error is below that of FP32 MFMAs, whose rounding
-//                 grows with the K / 2 accumulations of a K = 2 instruction.
+//                 per launch so its largest value fits f16 (see ScaleSrc).  From
+//                 about 24 samples an axis on, the result's error is below that
+//                 of FP32 MFMAs, whose rounding grows with the K / 2 accumulations
+//                 of a K = 2 instruction; a handful of samples or of bright ones
+//                 adds few roundings, and there the 22 bits show (1.4e-7, not 8e-8).
 //   PREC_BF16X3 : bf16 pairs (16 bits), no scaling.
 enum Precision { PREC_FP32 = 0, PREC_BF16X3 = 1 };
 
@@ -187,7 +189,7 @@ struct PhasorOp {
   ScaleSrc sc;
   long long begin;
 };
-// How an operand launch splits its work: K pairs (2, 4 or 8) and wavelengths
+// How an operand launch splits its work: K pairs (2 or 4) and wavelengths
 // per thread.
 struct OperandSplit {
   int np, waves;
@@ -220,10 +222,11 @@ inline long long group_begin(long long total) { return (total + kGroupBlock - 1)
 // launchers (mftx_gemm.hip, mftx_kernels.hip)
 hipError_t launch_gemm(int prec, int epi, int tile, const Work* work, int nwork, const Problem* probs,
                        const Seg* segs, hipStream_t s);
-// one problem (on the device, with its one segment of nch K blocks) over row
-// blocks [0, rblocks) and slot blocks [sb0, sb1), sb0 on a tile boundary
+// groups of windows of one grid (gemm_coherent_kernel)
 hipError_t launch_gemm_coherent(int prec, const Work* work, int nwork, const Problem* probs, const Seg* segs,
                                 hipStream_t s);
+// one problem (on the device, with its one segment of nch K blocks) over row
+// blocks [0, rblocks) and slot blocks [sb0, sb1), sb0 on a tile boundary
 hipError_t launch_gemm_one(int prec, int epi, int tile, int rblocks, int sb0, int sb1, int nch, const Problem* prob,
                            const Seg* seg, hipStream_t s);
 // every operand source of a plan in one launch (ops_dev on the device, sorted
@@ -257,7 +260,6 @@ struct RowPhase {
   int rows, pad_;
 };
 hipError_t launch_row_phases(const RowPhase* ops_dev, int nops, int most_rows, hipStream_t s);
-// launchers (mftx_gemm.hip, mftx_kernels.hip)
 // A phasor Field of a list: dst = amp exp(2 pi i opd inv_wl), m x n, dense.
 struct PhasorField {
   const void *amp, *opd;

@@ -194,14 +194,14 @@ __device__ __forceinline__ PhasorWave load_wave(cptr<const PhasorWave> p) {
 //
 // Bound by the arithmetic of the phases (about 40 instructions per sample and
 // wavelength, several FP64) beside the stores.  NP = 4 holds 48 registers of
-// source and 32 of result, four waves per SIMD; NP = 8 left room for two.
+// source and 32 of result, four waves per SIMD; 8 pairs left room for two.
 // Where every sample of a wave is outside the aperture (amplitude 0) the
 // phases are skipped.
 // DT: the dtype of a complex source.
 template <int PREC, bool CPLX, int NP, int DT, typename Waves>
 __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave, int waves, long long u, int scale) {
   auto fit = [&](float x) { return PREC == PREC_FP32 ? scaled(x, scale) : x; };
-  static_assert(NP == 2 || NP == 4 || NP == 8, "a thread's pairs lie in one half of a K block");
+  static_assert(NP == 2 || NP == 4, "a thread's pairs lie in one half of a K block, its pieces are one or two words");
   constexpr int SUB = 8 / NP;  // threads per (row pair, half K block)
   const int R = op.trans ? op.n : op.m, K = op.trans ? op.m : op.n;
   const int nrb = pair_blocks(R), nkb = pair_blocks(K);
@@ -354,8 +354,7 @@ __device__ __forceinline__ void operand_thread(const PhasorOp& op, Waves&& wave,
         for (int pl = 0; pl < 4; ++pl) {
           const uint32_t (&x)[NP / 2] = w[par][part][pl];
           char* dp = d + (part * 4 + pl) * FRAG + par * 256;
-          if constexpr (NP == 8) *(gptr<v4u32>)dp = v4u32{x[0], x[1], x[2], x[3]};
-          else if constexpr (NP == 4) *(gptr<v2u32>)dp = v2u32{x[0], x[1]};
+          if constexpr (NP == 4) *(gptr<v2u32>)dp = v2u32{x[0], x[1]};
           else *(gptr<uint32_t>)dp = x[0];
         }
   }
