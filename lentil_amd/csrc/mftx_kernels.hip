@@ -666,15 +666,22 @@ hipError_t launch_phasor_fields(const PhasorField* items, int count, double inv_
 // detector accumulation
 // --------------------------------------------------------------------------
 
+// Rows of an image that one launch of a thread per pixel covers: a launch of
+// 2^32 threads or more is cut off without an error.
+static int image_rows(int rows, int cols) {
+  const int per_row = (cols + 255) / 256;
+  return std::min(rows, std::max(1, (1 << 23) / per_row));
+}
+
 // One thread per image pixel: the partial images of every region that covers
 // it are summed in FP64 and the pixel is written (or added to) once, regions
 // or not, so nothing is cleared first.  Bound by reading the partial images;
 // one launch for all regions: 4 side by side (512^2, 8 partials each) took a
 // clear and 4 launches of 4.7 us, 24 us in all.
 __global__ void reduce_kernel(const ReduceOp* __restrict__ ops, int nops, void* __restrict__ image, int dtype,
-                              long long ldi, int rows, int cols, int accumulate, double unit) {
+                              long long ldi, int row0, int cols, int accumulate, double unit) {
   const unsigned per_row = (unsigned)(cols + 255) / 256;
-  const int r = (int)(blockIdx.x / per_row), c = (int)(blockIdx.x % per_row) * 256 + (int)threadIdx.x;
+  const int r = row0 + (int)(blockIdx.x / per_row), c = (int)(blockIdx.x % per_row) * 256 + (int)threadIdx.x;
   if (c >= cols) return;
   double acc = 0.0;
   for (int i = 0; i < nops; ++i) {
@@ -700,8 +707,10 @@ __global__ void reduce_kernel(const ReduceOp* __restrict__ ops, int nops, void* 
 hipError_t launch_reduce(const ReduceOp* ops, int nops, void* image, int dtype, long long ldi, int rows, int cols,
                          int accumulate, double unit, hipStream_t s) {
   if (rows <= 0 || cols <= 0 || (nops == 0 && accumulate)) return hipSuccess;
-  hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)rows * (unsigned)((cols + 255) / 256)), dim3(256), 0, s, ops, nops,
-                     image, dtype, ldi, rows, cols, accumulate, unit);
+  const int step = image_rows(rows, cols);
+  for (int r = 0; r < rows; r += step)
+    hipLaunchKernelGGL(reduce_kernel, dim3((unsigned)std::min(step, rows - r) * (unsigned)((cols + 255) / 256)), dim3(256),
+                       0, s, ops, nops, image, dtype, ldi, r, cols, accumulate, unit);
   return hipGetLastError();
 }
 
@@ -713,9 +722,9 @@ hipError_t launch_reduce(const ReduceOp* ops, int nops, void* image, int dtype, 
 // Field was added to an accumulator and every accumulator to the image.
 __global__ void coherent_kernel(const CoherentGroup* __restrict__ groups, int ngroups,
                                 const CoherentAdd* __restrict__ adds, void* __restrict__ image, int dtype,
-                                long long ldi, int rows, int cols, int accumulate) {
+                                long long ldi, int row0, int cols, int accumulate) {
   const unsigned per_row = (unsigned)(cols + 255) / 256;
-  const int r = (int)(blockIdx.x / per_row), c = (int)(blockIdx.x % per_row) * 256 + (int)threadIdx.x;
+  const int r = row0 + (int)(blockIdx.x / per_row), c = (int)(blockIdx.x % per_row) * 256 + (int)threadIdx.x;
   if (c >= cols) return;
   double acc = 0.0;
   for (int g = 0; g < ngroups; ++g) {
@@ -744,8 +753,10 @@ __global__ void coherent_kernel(const CoherentGroup* __restrict__ groups, int ng
 hipError_t launch_coherent(const CoherentGroup* groups, int ngroups, const CoherentAdd* adds, void* image, int dtype,
                            long long ldi, int rows, int cols, int accumulate, hipStream_t s) {
   if (rows <= 0 || cols <= 0) return hipSuccess;
-  hipLaunchKernelGGL(coherent_kernel, dim3((unsigned)rows * (unsigned)((cols + 255) / 256)), dim3(256), 0, s, groups,
-                     ngroups, adds, image, dtype, ldi, rows, cols, accumulate);
+  const int step = image_rows(rows, cols);
+  for (int r = 0; r < rows; r += step)
+    hipLaunchKernelGGL(coherent_kernel, dim3((unsigned)std::min(step, rows - r) * (unsigned)((cols + 255) / 256)), dim3(256),
+                       0, s, groups, ngroups, adds, image, dtype, ldi, r, cols, accumulate);
   return hipGetLastError();
 }
 
