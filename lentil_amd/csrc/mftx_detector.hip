@@ -438,7 +438,11 @@ __global__ __launch_bounds__(256) void fir_rows_kernel(const double* __restrict_
 // (mask_mode 1: img != 0; 2: a real mask array) is sampled with order 1,
 // mode 'nearest', on the unpadded grid and zeroed below eps
 // (util.py:338-339).  raw = interpolated value, part = block sums of raw.
-__global__ void resample_kernel(const double* __restrict__ C, long long P0, long long P1, int npad, int order,
+// The order is a template parameter, so a low one loads no taps that it has not: a
+// rescale from 2000^2 to 3200^2 at order 0 takes 171.8 us, 267 with six taps for every
+// order (and every block of the last launch adding the partial sums for 256 pixels).
+template <int order>
+__global__ void resample_kernel(const double* __restrict__ C, long long P0, long long P1, int npad,
                                 int mode, long long rows, long long cols, double scale, long long orows,
                                 long long ocols, const void* __restrict__ msrc, int mask_mode, int mdt, long long ldm,
                                 double eps, double* __restrict__ raw, double* __restrict__ mval,
@@ -458,30 +462,28 @@ __global__ void resample_kernel(const double* __restrict__ C, long long P0, long
       const int rule = tap_rule(mode);
       const long long sy = first_tap(cy, order), sx = first_tap(cx, order);
       // the columns' taps and weights once, every load of a row before its sum
-      long long cc[6];
-      double wx[6];
+      long long cc[order + 1];
+      double wx[order + 1];
       unsigned past = 0;  // taps outside the line (EX_ZERO): they read column 0, which may not be finite
 #pragma unroll
-      for (int b = 0; b < 6; ++b) {
-        cc[b] = b <= order ? extend_index(sx + b, P1, rule) : -1;
+      for (int b = 0; b <= order; ++b) {
+        cc[b] = extend_index(sx + b, P1, rule);
         wx[b] = cc[b] >= 0 ? bspline(order, cx - (double)(sx + b)) : 0.0;
         if (cc[b] < 0) past |= 1u << b;
         cc[b] = max(cc[b], 0LL);
       }
-      past &= (2u << order) - 1;
       for (int a = 0; a <= order; ++a) {
         const long long rr = extend_index(sy + a, P0, rule);
         if (rr < 0) continue;
-        double e[6], row = 0.0;
+        double e[order + 1], row = 0.0;
 #pragma unroll
-        for (int b = 0; b < 6; ++b) e[b] = C[rr * P1 + cc[b]];
+        for (int b = 0; b <= order; ++b) e[b] = C[rr * P1 + cc[b]];
         if (past) {
 #pragma unroll
-          for (int b = 0; b < 6; ++b) e[b] = past >> b & 1 ? 0.0 : e[b];
+          for (int b = 0; b <= order; ++b) e[b] = past >> b & 1 ? 0.0 : e[b];
         }
 #pragma unroll
-        for (int b = 0; b < 6; ++b)
-          if (b <= order) row += wx[b] * e[b];
+        for (int b = 0; b <= order; ++b) row += wx[b] * e[b];
         v += bspline(order, cy - (double)(sy + a)) * row;
       }
     }
@@ -517,29 +519,31 @@ __global__ void rescale_finish_kernel(const double* __restrict__ raw, const doub
   if (unitary)
     for (int q = 0; q < 4; ++q)
       if (raw_im || !(q & 1)) sums[q] = total(part + q * kMaxPart, q < 2 ? ni : nr);
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= orows * ocols) return;
-  const long long o = (t / ocols) * ldo + t % ocols;
-  if (!raw_im) {
-    double v = raw[t];
-    if (unitary) v *= sums[0] / sums[2];
-    store_real(out, odt, o, v * mval[t]);
-    return;
+  const double ratio = sums[0] / sums[2];
+  const long long n = orows * ocols, step = (long long)gridDim.x * kBlock;
+  for (long long t = (long long)blockIdx.x * kBlock + threadIdx.x; t < n; t += step) {
+    const long long o = (t / ocols) * ldo + t % ocols;
+    if (!raw_im) {
+      double v = raw[t];
+      if (unitary) v *= ratio;
+      store_real(out, odt, o, v * mval[t]);
+      continue;
+    }
+    double re = raw[t], im = raw_im[t];
+    if (unitary) {
+      // (a + ib) / (c + id) with a, b = sum(img), c, d = sum(raw)
+      const double a = sums[0], b = sums[1], c = sums[2], d = sums[3];
+      const double den = c * c + d * d;
+      const double qr = (a * c + b * d) / den, qi = (b * c - a * d) / den;
+      const double nr = re * qr - im * qi;
+      im = re * qi + im * qr;
+      re = nr;
+    }
+    re *= mval[t];
+    im *= mval[t];
+    if (odt == 2) ((double2*)out)[o] = make_double2(re, im);
+    else ((float2*)out)[o] = make_float2((float)re, (float)im);
   }
-  double re = raw[t], im = raw_im[t];
-  if (unitary) {
-    // (a + ib) / (c + id) with a, b = sum(img), c, d = sum(raw)
-    const double a = sums[0], b = sums[1], c = sums[2], d = sums[3];
-    const double den = c * c + d * d;
-    const double qr = (a * c + b * d) / den, qi = (b * c - a * d) / den;
-    const double nr = re * qr - im * qi;
-    im = re * qi + im * qr;
-    re = nr;
-  }
-  re *= mval[t];
-  im *= mval[t];
-  if (odt == 2) ((double2*)out)[o] = make_double2(re, im);
-  else ((float2*)out)[o] = make_float2((float)re, (float)im);
 }
 
 // The order's prefilter response h[|k|], k <= kPrefilterTaps, computed once
@@ -621,11 +625,14 @@ hipError_t launch_rescale(const void* img, int dtype, long long rows, long long 
       hipLaunchKernelGGL(rescale_load_kernel, dim3(blocks_for(P0 * P1)), dim3(kBlock), 0, s, img, dtype, comp, rows,
                          cols, ld, npad, zero, P);
     }
-    hipLaunchKernelGGL(resample_kernel, dim3(nr), dim3(kBlock), 0, s, (const double*)P, P0, P1, npad, order, mode,
+    const auto resample = order == 0 ? resample_kernel<0> : order == 1 ? resample_kernel<1> : order == 2 ? resample_kernel<2>
+                          : order == 3 ? resample_kernel<3> : order == 4 ? resample_kernel<4> : resample_kernel<5>;
+    hipLaunchKernelGGL(resample, dim3(nr), dim3(kBlock), 0, s, (const double*)P, P0, P1, npad, mode,
                        rows, cols, scale, orows, ocols, msrc, mask_mode, mdt, ldm, eps, comp ? raw_im : raw,
                        comp ? (double*)nullptr : mval, part + (2 + comp) * kMaxPart);
   }
-  hipLaunchKernelGGL(rescale_finish_kernel, dim3(blocks_for(orows * ocols)), dim3(kBlock), 0, s, (const double*)raw,
+  // every block adds the partial sums, so there are no more blocks than fill the chip
+  hipLaunchKernelGGL(rescale_finish_kernel, dim3(std::min(blocks_for(orows * ocols), 2048u)), dim3(kBlock), 0, s, (const double*)raw,
                      cplx ? (const double*)raw_im : nullptr, (const double*)mval, orows, ocols, unitary,
                      (const double*)part, ni, nr, out, odt, ldo);
   return hipGetLastError();
