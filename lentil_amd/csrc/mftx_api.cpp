@@ -202,20 +202,20 @@ class Tables {
  public:
   // index of the table for `samples` input samples and `slots` output slots
   int get(double alpha, double y0, int64_t samples, int64_t slots) {
-    const Key key{bits(alpha), bits(y0), (int)(samples & 1)};
-    auto it = index_.find(key);
-    if (it == index_.end()) {
-      it = index_.emplace(key, (int)ops.size()).first;
+    if (2 * ops.size() >= index_.size()) grow();
+    int& at = index_[find(alpha, y0, samples & 1 ? 0.0 : 0.5)];
+    if (at < 0) {
+      at = (int)ops.size();
       TableOp op = {};
       op.alpha = alpha;
       op.x0 = samples & 1 ? 0.0 : 0.5;
       op.y0 = y0;
       ops.push_back(op);
     }
-    TableOp& op = ops[it->second];
+    TableOp& op = ops[at];
     op.nsb = std::max(op.nsb, (int)blocks32(slots));
     op.nkb = std::max(op.nkb, pair_blocks(samples));
-    return it->second;
+    return at;
   }
   // thread ranges of the launch and offsets of the tables from `base`; the total bytes
   size_t place(size_t base) {
@@ -235,15 +235,28 @@ class Tables {
   long long threads = 0;
 
  private:
-  // the rates' bits: a NaN rate compares equal to every other one, and a
-  // transform of a list would then use its neighbour's table
-  using Key = std::tuple<uint64_t, uint64_t, int>;
+  // Open hashing over indices of ops (-1: free).  Rates are compared by their
+  // bits: a NaN rate is unequal to itself, and in an ordered container equal to
+  // every other one.
   static uint64_t bits(double v) {
     uint64_t u;
     std::memcpy(&u, &v, sizeof u);
     return u;
   }
-  std::map<Key, int> index_;
+  size_t find(double alpha, double y0, double x0) const {
+    uint64_t h = (bits(alpha) ^ bits(y0) * 3 ^ bits(x0) * 5) * 0x9E3779B97F4A7C15ull;
+    for (h ^= h >> 32;; ++h) {
+      const size_t i = h & (index_.size() - 1);
+      if (index_[i] < 0) return i;
+      const TableOp& op = ops[index_[i]];
+      if (bits(op.alpha) == bits(alpha) && bits(op.y0) == bits(y0) && bits(op.x0) == bits(x0)) return i;
+    }
+  }
+  void grow() {
+    index_.assign(std::max<size_t>(16, 4 * index_.size()), -1);
+    for (size_t k = 0; k < ops.size(); ++k) index_[find(ops[k].alpha, ops[k].y0, ops[k].x0)] = (int)k;
+  }
+  std::vector<int> index_;  // a power of two, at most half of it used
 };
 
 }  // namespace
@@ -597,6 +610,15 @@ struct ManyBatch {
 static void many_build(const mftx_mft* mfts, int32_t count, int prec, int fixed, ManyBatch& mb) {
   std::vector<MftGeo>& geo = mb.geo;
   geo.clear();
+  for (auto* v : {&mb.op_of, &mb.tab1, &mb.tab2}) v->reserve(count);
+  geo.reserve(count);
+  mb.waves.reserve(count);
+  mb.s1.reserve(count);
+  mb.s2.reserve(count);
+  const int nsource = (int)std::count_if(mfts, mfts + count, [](const mftx_mft& q) { return q.f != nullptr; });
+  mb.packs.reserve(nsource);
+  mb.phops.reserve(count - nsource);
+  if (prec == PREC_FP32) mb.maxes.reserve(count);
   size_t ws = 0;
   for (int32_t i = 0; i < count; ++i) {
     const mftx_mft& q = mfts[i];
@@ -679,6 +701,8 @@ static void many_build(const mftx_mft* mfts, int32_t count, int prec, int fixed,
 
   // ---- problems and works ------------------------------------------------------
   std::vector<int> nkb1, nkb2;
+  nkb1.reserve(count);
+  nkb2.reserve(count);
   mb.p1.resize(count);
   mb.p2.resize(count);
   for (int32_t i = 0; i < count; ++i) {
@@ -845,25 +869,25 @@ static int check_mfts(mftx_ctx* ctx, const mftx_mft* mfts, int32_t count, int32_
   if (precision != MFTX_PREC_FP32 && precision != MFTX_PREC_BF16X3) return fail(ctx, MFTX_EINVAL, "unknown precision");
   for (int32_t i = 0; i < count; ++i) {
     const mftx_mft& q = mfts[i];
-    const std::string at = "MFT " + std::to_string(i) + ": ";
-    if (!q.F) return fail(ctx, MFTX_EINVAL, at + "null output pointer");
-    if (q.m <= 0 || q.n <= 0 || q.M <= 0 || q.N <= 0) return fail(ctx, MFTX_EINVAL, at + "shapes must be positive");
+    auto bad = [&](const char* what) { return fail(ctx, MFTX_EINVAL, "MFT " + std::to_string(i) + ": " + what); };
+    if (!q.F) return bad("null output pointer");
+    if (q.m <= 0 || q.n <= 0 || q.M <= 0 || q.N <= 0) return bad("shapes must be positive");
     if (q.m > (1 << 20) || q.n > (1 << 20) || q.M > (1 << 20) || q.N > (1 << 20))
-      return fail(ctx, MFTX_EINVAL, at + "dimension too large");
-    if (q.ldF < q.N) return fail(ctx, MFTX_EINVAL, at + "output row stride smaller than row length");
+      return bad("dimension too large");
+    if (q.ldF < q.N) return bad("output row stride smaller than row length");
     if (q.f) {
-      if (q.f_dtype < 0 || q.f_dtype > 3) return fail(ctx, MFTX_EINVAL, at + "unknown input dtype");
-      if (q.ldf < q.n) return fail(ctx, MFTX_EINVAL, at + "input row stride smaller than row length");
+      if (q.f_dtype < 0 || q.f_dtype > 3) return bad("unknown input dtype");
+      if (q.ldf < q.n) return bad("input row stride smaller than row length");
     } else {
-      if (!q.amp || !q.opd) return fail(ctx, MFTX_EINVAL, at + "phasor input needs amp and opd");
+      if (!q.amp || !q.opd) return bad("phasor input needs amp and opd");
       if ((q.amp_dtype != 1 && q.amp_dtype != 3) || (q.opd_dtype != 1 && q.opd_dtype != 3))
-        return fail(ctx, MFTX_EINVAL, at + "amp/opd must be float32 or float64");
-      if (q.ld_amp < q.n || q.ld_opd < q.n) return fail(ctx, MFTX_EINVAL, at + "phasor row stride too small");
-      if (!(q.inv_wl > 0) || !std::isfinite(q.inv_wl)) return fail(ctx, MFTX_EINVAL, at + "inv_wl must be positive");
+        return bad("amp/opd must be float32 or float64");
+      if (q.ld_amp < q.n || q.ld_opd < q.n) return bad("phasor row stride too small");
+      if (!(q.inv_wl > 0) || !std::isfinite(q.inv_wl)) return bad("inv_wl must be positive");
     }
     if (q.w) {
-      if (q.w_dtype != 1 && q.w_dtype != 3) return fail(ctx, MFTX_EINVAL, at + "weight must be float32 or float64");
-      if (q.ldw < q.N) return fail(ctx, MFTX_EINVAL, at + "weight row stride smaller than row length");
+      if (q.w_dtype != 1 && q.w_dtype != 3) return bad("weight must be float32 or float64");
+      if (q.ldw < q.N) return bad("weight row stride smaller than row length");
     }
   }
   return MFTX_OK;
