@@ -4,6 +4,7 @@
 #include "mftx_device.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mftx {
 
@@ -875,14 +876,12 @@ hipError_t launch_weight_field(const void* F, long long ldF, const void* w, int 
   return hipGetLastError();
 }
 
-__device__ inline void put_grad(void* g, int dtype, long long i, double v, int accumulate) {
-  if (dtype == 3) {
-    double* d = (double*)g;
-    d[i] = accumulate ? d[i] + v : v;
-  } else {
-    float* d = (float*)g;
-    d[i] = (float)(accumulate ? (double)d[i] + v : v);
-  }
+__device__ __forceinline__ double get_real(const void* p, int dtype, long long i) {
+  return dtype == 3 ? ((gptr<const double>)p)[i] : (double)((gptr<const float>)p)[i];
+}
+__device__ __forceinline__ void put_grad(void* g, int dtype, long long i, double v) {
+  if (dtype == 3) ((gptr<double>)g)[i] = v;
+  else ((gptr<float>)g)[i] = (float)v;
 }
 
 // Given D_dw = dL/d conj(f_dw) for f_dw = amp * exp(2 pi i opd_d / lambda_w),
@@ -895,25 +894,39 @@ __device__ inline void put_grad(void* g, int dtype, long long i, double v, int a
 // flight and sums in FP64 over every OPD, so the gradient is written once.
 // 4 OPDs x 16 wavelengths of 512^2 (134 MB): one launch per OPD, each with its
 // wavelengths uploaded first and the gradient read back and added to, took 88 us.
+// BATCH: wavelengths whose loads are in flight together.  8 of them take registers
+// and loads that a gradient of fewer lacks, and a loop waits for what was loaded
+// before it, so one OPD (ONE) and one wavelength (BATCH 0) have none: one of 8000^2
+// took 566 us in the general form, 326 in its own.
+template <int BATCH, bool ONE>
 __global__ void phase_grad_kernel(PhaseGrad q) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long long)q.m * q.n) return;
   const long long r = t / q.n, c = t % q.n;
   const long long ia = r * q.ld_amp + c, io = r * q.ld_opd + c;
-  const double a = q.amp_dtype == 3 ? ((const double*)q.amp)[ia] : (double)((const float*)q.amp)[ia];
+  const double a = get_real(q.amp, q.amp_dtype, ia);
+  // what the sums are added to, loaded with the rest
+  const long long jo = r * q.ld_go + c, ja = r * q.ld_ga + c;
+  double go0 = 0.0, ga0 = 0.0;
+  if (q.accumulate) {
+    go0 = get_real(q.g_opd, q.go_dtype, jo);
+    if (q.g_amp) ga0 = get_real(q.g_amp, q.ga_dtype, ja);
+  }
   double go = 0.0, ga = 0.0;
   gptr<const v2f32> D = (gptr<const v2f32>)q.D + (r * q.ldD + c);
-  for (int d = 0; d < q.nopd; ++d, D += q.nwave * q.strideD) {
+  for (int d = 0; d < (ONE ? 1 : q.nopd); ++d, D += q.nwave * q.strideD) {
     const long long id = io + d * q.strideO;
-    const double o = q.opd_dtype == 3 ? ((const double*)q.opd)[id] : (double)((const float*)q.opd)[id];
-    for (int w0 = 0; w0 < q.nwave; w0 += 8) {
-      v2f32 v[8];
+    const double o = get_real(q.opd, q.opd_dtype, id);
+    int w = 0;
+    // the next N wavelengths, their loads in flight together
+    auto batch = [&](auto count) {
+      constexpr int N = decltype(count)::value;
+      v2f32 v[N];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = D[(w0 + i < q.nwave ? w0 + i : q.nwave - 1) * q.strideD];
+      for (int i = 0; i < N; ++i) v[i] = D[(w + i) * q.strideD];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (w0 + i >= q.nwave) break;
-        const double inv_wl = q.inv_wls ? q.inv_wls[w0 + i] : q.inv_wl0;
+      for (int i = 0; i < N; ++i) {
+        const double inv_wl = q.inv_wls ? q.inv_wls[w + i] : q.inv_wl0;
         const float2 e = cis_turns(o * inv_wl);
         // conj(D) * e = (x - i y)(e.x + i e.y)
         const double re = (double)v[i].x * e.x + (double)v[i].y * e.y;
@@ -921,17 +934,30 @@ __global__ void phase_grad_kernel(PhaseGrad q) {
         go += -4.0 * 3.14159265358979323846 * inv_wl * a * im;
         ga += 2.0 * re;
       }
-    }
+      w += N;
+    };
+    if constexpr (BATCH == 8)
+      while (w + 8 <= q.nwave) batch(std::integral_constant<int, 8>());
+    if constexpr (BATCH >= 4)
+      while (w + 4 <= q.nwave) batch(std::integral_constant<int, 4>());
+    if constexpr (BATCH == 0) batch(std::integral_constant<int, 1>());
+    else
+      while (w < q.nwave) batch(std::integral_constant<int, 1>());
   }
-  put_grad(q.g_opd, q.go_dtype, r * q.ld_go + c, go, q.accumulate);
-  if (q.g_amp) put_grad(q.g_amp, q.ga_dtype, r * q.ld_ga + c, ga, q.accumulate);
+  put_grad(q.g_opd, q.go_dtype, jo, q.accumulate ? go0 + go : go);
+  if (q.g_amp) put_grad(q.g_amp, q.ga_dtype, ja, q.accumulate ? ga0 + ga : ga);
 }
 
 hipError_t launch_phase_grad(const PhaseGrad& q, hipStream_t s) {
   const long long total = (long long)q.m * q.n;
   if (total <= 0 || q.nwave <= 0 || q.nopd <= 0) return hipSuccess;
   const int bs = 256;
-  hipLaunchKernelGGL(phase_grad_kernel, dim3((unsigned)((total + bs - 1) / bs)), dim3(bs), 0, s, q);
+  const auto one = q.nwave >= 8 ? phase_grad_kernel<8, true> : q.nwave >= 4 ? phase_grad_kernel<4, true>
+                   : q.nwave > 1 ? phase_grad_kernel<1, true> : phase_grad_kernel<0, true>;
+  const auto several = q.nwave >= 8 ? phase_grad_kernel<8, false> : q.nwave >= 4 ? phase_grad_kernel<4, false>
+                                                                                 : phase_grad_kernel<1, false>;
+  const auto kernel = q.nopd == 1 ? one : several;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((total + bs - 1) / bs)), dim3(bs), 0, s, q);
   return hipGetLastError();
 }
 
