@@ -293,9 +293,11 @@ def _insert_group(fields, out, weight):
 
 def _check_pixelscales(fields):
     p0 = fields[0].pixelscale
-    if all(f.pixelscale is p0 for f in fields):     # one object, compared once
-        same = p0 == p0
-        if same is True or (same.all() if isinstance(same, np.ndarray) else np.all(same)):
+    for f in fields:
+        if f.pixelscale is not p0:
+            break
+    else:   # one object, equal to itself unless it is not a number
+        if p0 is None or (not any(v != v for v in p0.flat) if isinstance(p0, np.ndarray) else np.all(p0 == p0)):
             return
     if not np.all([f.pixelscale == p0 for f in fields]):
         raise ValueError("Can't merge: pixelscales must be equal")

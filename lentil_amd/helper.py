@@ -35,10 +35,11 @@ def slice_offset(slc, shape):
             return (0, 0)
         raise ValueError(f"Can't compute offset from slice {slc}")
     r, c = slc[0], slc[1]
-    ends = r.start, r.stop, c.start, c.stop
-    if type(shape) is tuple and len(shape) == 2 and _INTS.issuperset(map(type, ends)):
-        r0, r1, c0, c1 = map(int, ends)
-        return r0 + (r1 - r0) // 2 - shape[0] // 2, c0 + (c1 - c0) // 2 - shape[1] // 2
+    r0, r1, c0, c1 = r.start, r.stop, c.start, c.stop
+    if type(shape) is tuple and len(shape) == 2 and type(r0) in _INTS and type(r1) in _INTS and type(c0) in _INTS \
+            and type(c1) in _INTS:
+        r0, c0 = int(r0), int(c0)
+        return r0 + (int(r1) - r0) // 2 - shape[0] // 2, c0 + (int(c1) - c0) // 2 - shape[1] // 2
     # other shapes and indices as numpy broadcasts and promotes them
     size = np.array((r.stop - r.start, c.stop - c.start))
     return tuple(np.array((r.start + size[0] // 2, c.start + size[1] // 2)) - np.asarray(shape) // 2)
