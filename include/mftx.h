@@ -199,7 +199,9 @@ int mftx_phase_grad_stack(mftx_ctx* ctx, const void* amp, int amp_dtype, int64_t
  *     M x N map w (float32/float64, row stride ldw): the weighted cotangent
  *     of an intensity for the adjoint pass of phase retrieval.
  * All entries run in one operand launch (one more for complex inputs beside
- * phasors) and one launch per GEMM stage.
+ * phasors) and one launch per GEMM stage.  Lists whose twiddle tables (2 bytes per
+ * input sample and output pixel of an axis) exceed 1 GiB, or with FP32 entries of
+ * more than 32768 samples along an axis, are split, down to single entries.
  * ------------------------------------------------------------------------- */
 typedef struct {
   const void* f;       /* input m x n (f_dtype, row stride ldf), or NULL for a phasor */
